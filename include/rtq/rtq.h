@@ -276,7 +276,8 @@ rtq_status rtq_trace_stats(rtq_ctx* ctx, uint32_t scene_id, const rtq_ray* rays_
  * process ends (rtq_create looks up its address once per device).  The
  * persistent grid takes as many workgroups as that array holds stacks for, so
  * very deep trees trace with fewer workgroups; RTQ_ECAPACITY when not even one
- * workgroup's stacks fit.  Every call clears the counters first.  All calls on
+ * workgroup's stacks fit.  A call that uses the counters clears them first
+ * (one more small launch; a few hundred thousand rays need none).  All calls on
  * one GPU share the array: calls that overlap on one GPU (any context, any
  * stream) race, and the caller must serialise them.  Asynchronous on `stream`;
  * device buffers. */
@@ -328,7 +329,8 @@ void rtq_batch_destroy(rtq_batch* batch);
 
 typedef struct rtq_launch_params {
     uint32_t refill;       /* refill a wave's idle lanes once this many (1..64) are idle */
-    uint32_t chunk;        /* consecutive rays a wave takes per atomic (1..4096) */
+    uint32_t chunk;        /* most consecutive rays a wave takes at a time (1..4096); launches of
+                              fewer than about 1,000 rays per wave take 64 or fewer */
     uint32_t prefer_wide;  /* trace 8-wide nodes when a scene has them */
     uint32_t spec_slack;   /* speculative traversal: a wave switches from node visits to
                               leaf tests once at most this many (0..63) of its lanes

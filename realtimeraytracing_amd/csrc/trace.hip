@@ -44,18 +44,29 @@ namespace {
 constexpr int kTraceThreads = 256;
 // Work distribution: every ray set (item) of a launch is split into kXcds
 // contiguous parts and part j of each item belongs to XCD j.  Workgroups are
-// dispatched to the XCDs round-robin, so a wave of block b drains XCD b %
-// kXcds's part of every item first (its rays then share nodes in that XCD's
-// L2), then steals parts of the other XCDs.  Part (item i, j) has counter
-// p = i * kXcds + j, 64 B apart; counter[kDry..] is a bit mask of exhausted
-// parts; counter[kArrive] counts finished blocks.
+// dispatched to the XCDs round-robin, so the waves of block b drain XCD b %
+// kXcds's queue (its part of every item, item by item, in chunks of
+// consecutive rays) first, so that its rays share nodes in that XCD's L2, then
+// take chunks of the other XCDs' queues.  Chunk number i of queue j, below the
+// number of waves of XCD j, belongs to that XCD's wave i from the start; the
+// chunks after those are handed out by the queue's counter, one atomic each.
+// A wave whose queue ran out tries the others in turn, but not those that a
+// wave of its workgroup has found empty.  Atomics of many waves on one word
+// serialise (about 12 ns each), and with one counter per item and XCD, each
+// tried by every wave at the end of the launch, a launch took 60 us or more
+// however few its rays (2.1M camera rays 0.461 ms, 0.418 now; a batch of 10
+// scenes and 1.3M rays 1.51 ms, 0.54 now).  Counters lie 256 B apart: two in
+// one 128-B line move it between their XCDs' L2s on every atomic (0.524 against
+// 0.499 ms, with the probing above), and so does looking at another XCD's
+// counter with a load before trying it (0.499 against 0.424 ms).
+// counter[kArrive] counts finished blocks.
 constexpr uint32_t kXcds = 8;
-constexpr uint32_t kMaxBatchItems = 64;
-constexpr uint32_t kMaxParts = kMaxBatchItems * kXcds;
-constexpr uint32_t kPartStride = 16;
-constexpr uint32_t kDry = kMaxParts * kPartStride;
-constexpr uint32_t kArrive = kDry + kMaxParts / 32;
-constexpr uint32_t kCounterWords = kArrive + kPartStride;
+constexpr uint32_t kWavesPerBlock = kTraceThreads / 64;
+constexpr uint32_t kSimdsPerCu = 4;
+constexpr uint32_t kMaxBatchItems = 64;   // one lane of a wave per item (chunk_rays)
+constexpr uint32_t kQueueStride = 64;
+constexpr uint32_t kArrive = kXcds * kQueueStride;
+constexpr uint32_t kCounterWords = kArrive + kQueueStride;
 
 // Relative widening of a box's far distance (tn <= tf + |tf| * kSlabRel):
 // 32 units of 2^-24, twice the sum of the distance-proportional errors of the
@@ -89,9 +100,11 @@ struct BatchItem {
     rtq_hit* hits;
     uint32_t begin;
     uint32_t n;
-    uint32_t any;
-    uint32_t learned;  // take the learned child order where the nodes hold it
+    uint32_t mode;       // kItemAny | kItemLearned
+    uint32_t chunk_end;  // chunks of an XCD's queue through this item
 };
+constexpr uint32_t kItemAny = 1;      // any-hit rays
+constexpr uint32_t kItemLearned = 2;  // take the learned child order where the nodes hold it
 static_assert(sizeof(BatchItem) == 48, "batch descriptor is 48 B");
 
 // Item descriptors of a batched launch, passed by value (3 KB of kernel
@@ -116,7 +129,9 @@ struct TraceArgs {
     uint32_t* spill;
     uint32_t spill_stride;
     uint32_t refill;     // refill once this many lanes of a wave are idle
-    uint32_t chunk;      // rays taken from a work counter per atomic
+    uint32_t chunk;      // consecutive rays of a chunk
+    uint32_t queue;      // chunks in each XCD's queue
+    uint32_t dynamic;    // a queue has more chunks than its XCD has waves
     uint32_t slack;      // leaf tests start once at most this many lanes still descend
     uint32_t leaf_slack; // node visits resume once at most this many lanes test triangles
     uint32_t* stat_nodes;
@@ -260,6 +275,39 @@ enum Layout : int {
 __host__ __device__ constexpr bool wide_layout(int layout) { return layout == kWide || layout == kWideOrdered; }
 __host__ __device__ constexpr bool learned_layout(int layout) { return layout == kOrdered || layout == kWideOrdered; }
 
+// Waves of XCD j in this launch.
+__device__ __forceinline__ uint32_t xcd_waves(uint32_t j) {
+    return kWavesPerBlock * ((gridDim.x + kXcds - 1u - j) / kXcds);
+}
+
+// Rays of each XCD's part of a ray set of n rays, and the chunks of a part: the
+// same for every XCD, so that the last parts of a small set may be short or
+// empty.
+__host__ __device__ __forceinline__ uint32_t part_rays(uint32_t n) { return (n + kXcds - 1) / kXcds; }
+__host__ __device__ __forceinline__ uint32_t part_chunks(uint32_t n, uint32_t chunk) {
+    return (part_rays(n) + chunk - 1) / chunk;
+}
+
+// Rays [lo, hi) and item of chunk c of XCD j's queue (c and j wave-uniform, c
+// below the queue's chunks; every lane of the wave takes part).  With several
+// items lane i holds the chunks through item i; the item is the first one
+// whose count exceeds c.
+template <bool MULTI>
+__device__ __forceinline__ void chunk_rays(const TraceArgs& a, const BatchItem* items, uint32_t lane, uint32_t j,
+                                           uint32_t c, uint32_t& lo, uint32_t& hi, uint32_t& item) {
+    uint32_t begin = 0, n = a.n;
+    if constexpr (MULTI) {
+        item = (uint32_t)__builtin_ctzll(__ballot(lane < a.n_items && items[lane].chunk_end > c));
+        if (item > 0) c -= __builtin_amdgcn_readfirstlane(items[item - 1].chunk_end);
+        begin = __builtin_amdgcn_readfirstlane(items[item].begin);
+        n = __builtin_amdgcn_readfirstlane(items[item].n);
+    }
+    const uint32_t part = part_rays(n);
+    lo = min(j * part + c * a.chunk, n);
+    hi = begin + min(min(lo + a.chunk, (j + 1) * part), n);
+    lo += begin;
+}
+
 // MODE: 0 closest hit, 1 any hit, 2 per batch item.  MULTI: 0 one ray set;
 // 1 several items (ray sets over any scenes), each lane takes its scene from
 // its item; 2 several items over one scene, whose nodes and triangles are
@@ -276,6 +324,8 @@ __device__ __forceinline__ void trace_waves(const TraceArgs& a, const ItemTable<
     // the top of the binary tree, read from LDS instead of L2 by every ray
     constexpr uint32_t kTopSlots = (wide_layout(LAYOUT) || kTopNodes == 0) ? 1u : kTopNodes;
     __shared__ float4 s_top[4 * kTopSlots];
+    __shared__ uint32_t s_gone;   // bit j: XCD j's queue was found empty
+    constexpr uint32_t kAllGone = (1u << kXcds) - 1u;
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u;
     uint32_t* const lds = s_stack + tid;  // entry k at lds[k * kTraceThreads]: lanes on distinct banks
@@ -286,7 +336,8 @@ __device__ __forceinline__ void trace_waves(const TraceArgs& a, const ItemTable<
     if constexpr (MULTI)
         for (uint32_t i = tid; i < a.n_items; i += kTraceThreads) s_items[i] = table.item[i];
     for (uint32_t i = tid; i < 4 * n_top; i += kTraceThreads) s_top[i] = a.top[i];
-    if (MULTI || n_top) __syncthreads();
+    if (tid == 0) s_gone = 0;
+    __syncthreads();
     // the lane's scene and ray set (kernel arguments unless batched)
     const float4* nodes_p = a.nodes;
     const float4* tris_p = a.tris;
@@ -300,14 +351,12 @@ __device__ __forceinline__ void trace_waves(const TraceArgs& a, const ItemTable<
     uint32_t order_bit = 0, order_mask = 0xFFFFFFFFu;
 
     int rid = -1;
-    // wave-uniform ray pool [pool_next, pool_end) of item pool_item, taken
-    // from the seq-th part of the wave's order; dry once every part is
-    // exhausted
+    // wave-uniform ray pool [pool_next, pool_end) of item pool_item, a chunk of
+    // XCD `queue`'s queue; own: the chunk the wave starts with (kNone once
+    // taken); dry once every queue is exhausted
     uint32_t pool_next = 0, pool_end = 0, pool_item = 0;
-    const uint32_t xcd = blockIdx.x % kXcds;
-    const uint32_t n_items = MULTI ? a.n_items : 1u;
-    const uint32_t n_parts = n_items * kXcds;
-    uint32_t seq = 0;
+    uint32_t queue = blockIdx.x % kXcds;
+    uint32_t own = (blockIdx.x / kXcds) * kWavesPerBlock + __builtin_amdgcn_readfirstlane(tid >> 6);
     bool dry = false;
     float ox = 0, oy = 0, oz = 0, dx = 0, dy = 0, dz = 0;
     float ix = 0, iy = 0, iz = 0, oix = 0, oiy = 0, oiz = 0;
@@ -552,60 +601,32 @@ __device__ __forceinline__ void trace_waves(const TraceArgs& a, const ItemTable<
         const bool need = (rid < 0) && !dry;
         const uint64_t need_mask = __ballot(need);
         if (need_mask) {
-            if (pool_next == pool_end) {
-                const uint32_t leader = (uint32_t)__ffsll((unsigned long long)need_mask) - 1u;
-                uint32_t lo = 0, hi = 0, item = 0;
-                if (lane == leader) {
-                    // the current part, then the next ones of the wave's order
-                    // (own XCD's part of each item, then the next XCD's);
-                    // parts marked exhausted are skipped without an atomic
-                    const unsigned long long* dry_mask =
-                        reinterpret_cast<const unsigned long long*>(a.counter + kDry);
-                    unsigned long long gone = 0;
-                    uint32_t gone_word = kNone;
-                    for (const uint32_t first = seq; seq < n_parts; ++seq) {
-                        item = seq % n_items;
-                        const uint32_t j = (xcd + seq / n_items) % kXcds;
-                        const uint32_t p = item * kXcds + j;
-                        // up to 16 parts are probed with their own atomics; more
-                        // (large batches) consult the exhausted-part mask so a
-                        // wave's end-of-launch probing stays short
-                        if (n_parts > 16 && seq != first) {
-                            if (p / 64 != gone_word) {
-                                gone_word = p / 64;
-                                gone = __hip_atomic_load(dry_mask + gone_word, __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_AGENT);
-                            }
-                            if ((gone >> (p % 64)) & 1ull) continue;
-                        }
-                        uint32_t ib = 0, in = a.n;
-                        if constexpr (MULTI) {
-                            ib = s_items[item].begin;
-                            in = s_items[item].n;
-                        }
-                        const uint32_t pb = ib + (uint32_t)(((uint64_t)in * j) / kXcds);
-                        const uint32_t pe = ib + (uint32_t)(((uint64_t)in * (j + 1)) / kXcds);
-                        const uint32_t base = atomicAdd(a.counter + p * kPartStride, a.chunk);
-                        if (base < pe - pb) {
-                            lo = pb + base;
-                            hi = min(lo + a.chunk, pe);
-                            break;
-                        }
-                        if (n_parts > 16)
-                            atomicOr(const_cast<unsigned long long*>(dry_mask) + p / 64, 1ull << (p % 64));
-                    }
-                }
-                lo = __shfl(lo, (int)leader);
-                hi = __shfl(hi, (int)leader);
-                item = __shfl(item, (int)leader);
-                seq = __shfl(seq, (int)leader);
-                if (lo == hi) {
+            // (a short or empty part's chunk may hold no rays: another one then)
+            while (pool_next == pool_end && !dry) {
+                uint32_t c = own;
+                own = kNone;
+                if (c >= a.queue) {
                     dry = true;
-                } else {
-                    pool_next = lo;
-                    pool_end = hi;
-                    pool_item = item;
+                    if (!a.dynamic) break;
+                    // from this wave's queue on, the first one that no wave of
+                    // the workgroup has found empty
+                    uint32_t gone = __hip_atomic_load(&s_gone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    gone = __builtin_amdgcn_readfirstlane(gone);
+                    while (gone != kAllGone) {
+                        queue = (queue + __builtin_ctz(~((gone | (gone << kXcds)) >> queue))) % kXcds;
+                        uint32_t got = 0;
+                        if (lane == 0) got = atomicAdd(a.counter + queue * kQueueStride, 1u);
+                        c = xcd_waves(queue) + __builtin_amdgcn_readfirstlane(got);
+                        if (c < a.queue) break;
+                        if (lane == 0)
+                            __hip_atomic_fetch_or(&s_gone, 1u << queue, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        gone = __builtin_amdgcn_readfirstlane(
+                            __hip_atomic_load(&s_gone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) | (1u << queue));
+                    }
+                    if (c >= a.queue) break;
+                    dry = false;
                 }
+                chunk_rays<MULTI != 0>(a, s_items, lane, queue, c, pool_next, pool_end, pool_item);
             }
             if (!dry) {
                 const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(need_mask >> 32),
@@ -626,8 +647,8 @@ __device__ __forceinline__ void trace_waves(const TraceArgs& a, const ItemTable<
                         rays_p = it.rays;
                         lane_item = pool_item;
                         local = r - it.begin;
-                        lane_any = it.any != 0;
-                        order_mask = it.learned ? 0xFFFFFFFFu : 0u;
+                        lane_any = (it.mode & kItemAny) != 0;
+                        order_mask = (it.mode & kItemLearned) ? 0xFFFFFFFFu : 0u;
                     }
                     const float4* rp = reinterpret_cast<const float4*>(rays_p + local);
                     const float4 r0 = load_stream(rp), r1 = load_stream(rp + 1);
@@ -748,10 +769,11 @@ __device__ __forceinline__ void trace_waves(const TraceArgs& a, const ItemTable<
             if (active == 0 || (!dry && (uint32_t)__popcll(idle) >= a.refill)) break;
         }
     }
-    // A wave leaves the loop only after every part ran dry for it, so when
+    // A wave leaves the loop only after every queue ran dry for it, so when
     // every block has arrived here no fetch is outstanding: the last block
-    // resets the part counters, the exhausted-part mask and the arrival counter
-    // for the next launch on the stream.
+    // resets the counters for the next launch on the stream.  A launch whose
+    // chunks all had their wave from the start touched none.
+    if (!a.dynamic) return;
     __shared__ uint32_t s_last;
     __syncthreads();
     if (tid == 0) {
@@ -760,8 +782,7 @@ __device__ __forceinline__ void trace_waves(const TraceArgs& a, const ItemTable<
     }
     __syncthreads();
     if (s_last) {
-        for (uint32_t p = tid; p < n_parts; p += kTraceThreads) atomicExch(a.counter + p * kPartStride, 0u);
-        if (tid < (n_parts + 31) / 32) atomicExch(a.counter + kDry + tid, 0u);
+        if (tid < kXcds) atomicExch(a.counter + tid * kQueueStride, 0u);
         if (tid == 0) atomicExch(a.counter + kArrive, 0u);
     }
 }
@@ -782,11 +803,10 @@ __global__ __launch_bounds__(kTraceThreads) __attribute__((amdgpu_waves_per_eu(W
 
 // Occupancy hints by layout (0 = the compiler's own choice), from timings on
 // the 2M-triangle terrain: the batched binary kernels at least 7 waves per
-// SIMD (no spill), the single-scene 8-wide kernels at 7 instead of 6 (74 -> 72
-// VGPRs, no spill), the one-scene batched 8-wide kernel at 6 instead of 5
-// (80 VGPRs, no spill: +10% on the batched form); the single-scene binary
-// kernels were slower when pushed from 7 to 8 waves, and the multi-scene
-// batched 8-wide kernel (89 VGPRs, per-lane scene pointers) spills at 6.
+// SIMD (no spill), the single-scene 8-wide kernels at 7 (69 VGPRs), the
+// one-scene batched 8-wide kernel at 6 instead of 5 (78 VGPRs, no spill: +10%
+// on the batched form), the multi-scene batched 8-wide kernel at 5 (95 VGPRs,
+// per-lane scene pointers; without the hint it takes 97 and 4 waves).
 #ifndef RTQ_OCC_BATCH
 #define RTQ_OCC_BATCH 7
 #endif
@@ -794,7 +814,7 @@ __global__ __launch_bounds__(kTraceThreads) __attribute__((amdgpu_waves_per_eu(W
 #define RTQ_OCC_WIDE 7
 #endif
 #ifndef RTQ_OCC_BATCH_WIDE
-#define RTQ_OCC_BATCH_WIDE 0
+#define RTQ_OCC_BATCH_WIDE 5
 #endif
 #ifndef RTQ_OCC_BATCH_WIDE_ONE
 #define RTQ_OCC_BATCH_WIDE_ONE 6
@@ -831,17 +851,73 @@ constexpr int stack_choice(int k) {
     return (int)(wide_layout(LAYOUT) ? kStackChoicesWide[k] : kStackChoicesBinary[k]);
 }
 
+__global__ void k_zero_u32(uint32_t* __restrict__ p, uint32_t n) {
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0u;
+}
+
+// Waves of a launch of n rays (at most the resident ones) and the rays of a
+// chunk (at most the context's setting).
+//  - Fewer rays than one full wave per SIMD holds: one wave per SIMD with as
+//    few rays each as that gives, at least 2.  Such a launch lasts as long as
+//    its slowest wave, and a wave of few rays waits for fewer of them (1,021
+//    rays on a 960-triangle mesh: 31 us with 2 rays a wave, 35 with 4, 45 with
+//    16; 76 us with 128-ray chunks on waves of 64).
+//  - More: full waves, up to 4 per SIMD, then waves of about 200 rays up to
+//    the resident ones, which trace incoherent rays faster than a lane for
+//    every ray: they keep their lanes filled and share the caches among fewer
+//    waves (700,000 random rays on a 200,000-triangle soup: 0.88 ms on 4,096
+//    waves, 1.10 ms on 7,168; 300,000 rays: 0.36 ms against 0.46).
+//  - Chunks of 64 rays keep the waves evenly loaded at the end of a launch;
+//    where a wave takes 1,024 rays or more, the atomics weigh more than the
+//    end (10.4M terrain rays: 1.20 ms with 64-ray chunks, 1.12 with 128; 2.1M
+//    camera rays: 0.418 against 0.426 ms).
+struct WaveSplit {
+    uint64_t waves;
+    uint32_t chunk;
+};
+WaveSplit split_rays(uint32_t n, uint64_t simds, uint64_t resident, uint32_t max_chunk) {
+    WaveSplit w{};
+    uint64_t chunk = 64;
+    if (n < 64 * simds) {
+        chunk = std::max<uint64_t>((n + simds - 1) / simds, 2);
+        w.waves = (n + chunk - 1) / chunk;
+    } else {
+        w.waves = std::min<uint64_t>(n / 64, std::max<uint64_t>(4 * simds, n / 200));
+    }
+    w.waves = std::min(w.waves, resident);
+    if (n / w.waves >= 1024) chunk = max_chunk;
+    w.chunk = (uint32_t)std::min<uint64_t>(chunk, max_chunk);
+    return w;
+}
+
+// Chunks of an XCD's queue: of the launch's ray set, or through each item of a
+// batch (which its table then holds).
+uint32_t queue_chunks(ItemTable<false>&, uint32_t, uint32_t n, uint32_t chunk) { return part_chunks(n, chunk); }
+uint32_t queue_chunks(ItemTable<true>& table, uint32_t n_items, uint32_t, uint32_t chunk) {
+    uint32_t q = 0;
+    for (uint32_t i = 0; i < n_items; ++i) {
+        q += part_chunks(table.item[i].n, chunk);
+        table.item[i].chunk_end = q;
+    }
+    return q;
+}
+
 // Persistent grid sized from occupancy, spill column sized from the stack
 // bound `depth_entries`, one launch (or only the scratch sizing).
 template <int LEAF, int MODE, bool STATS, int LAYOUT, int MULTI, int STACK = stack_choice<LAYOUT>(1)>
 rtq_status launch(rtq_ctx* ctx, TraceScratch& sc, uint64_t depth_entries, const TraceArgs& base,
-                  const ItemTable<(MULTI != 0)>& table, uint32_t n, bool size_only, hipStream_t st) {
+                  ItemTable<(MULTI != 0)>& table, uint32_t n, bool size_only, hipStream_t st) {
     const auto kern = trace_kernel<LEAF, MODE, STATS, LAYOUT, MULTI, STACK>();
     int per_cu = 0;
     hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kTraceThreads, 0);
     if (e != hipSuccess || per_cu <= 0) per_cu = 4;
-    uint64_t blocks = std::min<uint64_t>((n + kTraceThreads - 1) / kTraceThreads,
-                                         (uint64_t)per_cu * (uint64_t)std::max(ctx->n_cu, 1));
+    const uint64_t resident = (uint64_t)per_cu * (uint64_t)std::max(ctx->n_cu, 1);
+    const WaveSplit split =
+        split_rays(n, (uint64_t)kSimdsPerCu * std::max(ctx->n_cu, 1), resident * kWavesPerBlock, ctx->chunk);
+    const uint32_t queue = queue_chunks(table, base.n_items, n, split.chunk);
+    // whole rounds of the XCDs: every XCD's queue has the same chunks
+    auto rounds = [](uint64_t waves) { return (waves + kXcds * kWavesPerBlock - 1) / (kXcds * kWavesPerBlock); };
+    uint64_t blocks = std::min<uint64_t>(kXcds * std::min(rounds(split.waves), rounds((uint64_t)kXcds * queue)), resident);
     if (blocks == 0) blocks = 1;
     constexpr uint32_t kStackLds = STACK;
     const uint64_t column = depth_entries > kStackLds ? depth_entries - kStackLds : 0;  // spill words per thread
@@ -856,7 +932,10 @@ rtq_status launch(rtq_ctx* ctx, TraceScratch& sc, uint64_t depth_entries, const 
         blocks = std::min(blocks, fit);
     }
     const uint64_t threads = blocks * kTraceThreads;
-    const uint64_t spill_words = column ? column * threads : 1;
+    // sized for one wave per SIMD at least: a launch of fewer rays may take
+    // more workgroups than one of more rays does (split_rays), up to that many
+    const uint64_t least = std::min<uint64_t>((uint64_t)std::max(ctx->n_cu, 1) * kSimdsPerCu / kWavesPerBlock, resident);
+    const uint64_t spill_words = column ? column * (sc.fixed ? threads : std::max(threads, least * kTraceThreads)) : 1;
     if (spill_words > sc.spill_words) {
         if (sc.fixed) return fail(ctx, RTQ_EINTERNAL, "trace: fixed scratch sizing");
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -879,7 +958,15 @@ rtq_status launch(rtq_ctx* ctx, TraceScratch& sc, uint64_t depth_entries, const 
     args.spill = sc.spill;
     args.spill_stride = (uint32_t)threads;
     args.refill = ctx->refill;
-    args.chunk = ctx->chunk;
+    args.chunk = split.chunk;
+    args.queue = queue;
+    // the last XCD has the fewest workgroups
+    args.dynamic = queue > kWavesPerBlock * (blocks / kXcds) ? 1u : 0u;
+    if (sc.fixed && args.dynamic) {
+        // the fixed scratch is shared by every context: its counters start at zero
+        hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(256), 0, st, sc.counter, (uint32_t)kCounterWords);
+        RTQ_HIP(ctx, hipGetLastError());
+    }
     args.slack = ctx->spec_slack;
     args.leaf_slack = ctx->leaf_slack;
     hipLaunchKernelGGL(kern, dim3((uint32_t)blocks), dim3(kTraceThreads), 0, st, args, table);
@@ -899,7 +986,7 @@ uint64_t stack_bound(const Scene* s, bool wide) {
 template <int LEAF, int MODE, bool STATS>
 rtq_status launch_single(rtq_ctx* ctx, const Scene* s, TraceArgs a, uint32_t n, int layout, hipStream_t st,
                          TraceScratch* fixed = nullptr) {
-    const ItemTable<false> none{};
+    ItemTable<false> none{};
     const bool wide = wide_layout(layout);
     a.nodes = wide ? s->wide : s->nodes;
     a.top = wide ? nullptr : s->top;
@@ -971,10 +1058,6 @@ constexpr int kMaxDevices = 64;
 std::mutex g_noalloc_mutex;
 uint32_t* g_noalloc_ptr[kMaxDevices] = {};
 
-__global__ void k_zero_u32(uint32_t* __restrict__ p, uint32_t n) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0u;
-}
-
 }  // namespace
 
 rtq_status noalloc_setup(rtq_ctx* ctx) {
@@ -1006,10 +1089,6 @@ rtq_status trace_noalloc(rtq_ctx* ctx, const Scene* s, const rtq_ray* rays, uint
     sc.spill = base + kNoAllocSpillOffset;
     sc.spill_words = kNoAllocWords - kNoAllocSpillOffset;
     sc.fixed = true;
-    // the counters start at zero (a launch's last block also resets them)
-    hipLaunchKernelGGL(k_zero_u32, dim3((kCounterWords + 255) / 256), dim3(256), 0, st, sc.counter,
-                       (uint32_t)kCounterWords);
-    RTQ_HIP(ctx, hipGetLastError());
     TraceArgs args{};
     args.tris = s->tris;
     args.rays = rays;
@@ -1059,7 +1138,7 @@ rtq_status trace(rtq_ctx* ctx, const Scene* s, const rtq_ray* rays, uint64_t n, 
 // of the other layout family: the default).
 template <int LEAF, int LAYOUT, int MULTI>
 rtq_status launch_batch_stack(rtq_ctx* ctx, TraceScratch& sc, uint64_t depth, const TraceArgs& args,
-                              const ItemTable<true>& table, uint32_t nt, bool size_only, hipStream_t st) {
+                              ItemTable<true>& table, uint32_t nt, bool size_only, hipStream_t st) {
     const int want = (int)ctx->stack_lds;
     if (want == stack_choice<LAYOUT>(0))
         return launch<LEAF, 2, false, LAYOUT, MULTI, stack_choice<LAYOUT>(0)>(ctx, sc, depth, args, table, nt,
@@ -1072,7 +1151,7 @@ rtq_status launch_batch_stack(rtq_ctx* ctx, TraceScratch& sc, uint64_t depth, co
 
 template <int MULTI>
 rtq_status launch_batch(rtq_ctx* ctx, TraceScratch& sc, uint64_t depth, const TraceArgs& args,
-                        const ItemTable<true>& table, uint32_t nt, bool size_only, hipStream_t st, bool refmt,
+                        ItemTable<true>& table, uint32_t nt, bool size_only, hipStream_t st, bool refmt,
                         int layout) {
     if (refmt) {
         if (layout == kWide) return launch_batch_stack<1, kWide, MULTI>(ctx, sc, depth, args, table, nt, size_only, st);
@@ -1156,8 +1235,7 @@ rtq_status trace_batch(rtq_ctx* ctx, const rtq_batch_item* items, uint32_t n_ite
         b.hits = it.hits_dev;
         b.begin = (uint32_t)total;
         b.n = (uint32_t)it.n_rays;
-        b.any = (it.flags & RTQ_TRACE_ANY) ? 1u : 0u;
-        b.learned = learned_decisions(s, it.flags) ? 1u : 0u;
+        b.mode = ((it.flags & RTQ_TRACE_ANY) ? kItemAny : 0u) | (learned_decisions(s, it.flags) ? kItemLearned : 0u);
         total += it.n_rays;
         if (total > 0x80000000ull) return fail(ctx, RTQ_ECAPACITY, "trace_batch: more than 2^31 rays in one launch");
         depth = std::max(depth, stack_bound(s, wide));
