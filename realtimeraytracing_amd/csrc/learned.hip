@@ -7,9 +7,9 @@
 //  - Logs: k_order_log walks sampled rays with the plain traversal and emits,
 //    at nodes where both children are hit, the node's features, the label and
 //    a weight.
-//  - Training: k_mlp_grad (forward + backward of 64 samples per block, FP32,
-//    per-block partial gradients), k_mlp_reduce (deterministic reduction in
-//    block order) and k_mlp_adam, all on the GPU.
+//  - Training: k_mlp_grad (forward + backward of 64 samples per block on FP32
+//    matrix instructions, per-block partial gradients) and k_mlp_step
+//    (deterministic reduction in block order, Adam), all on the GPU.
 //  - Inference: k_order_apply evaluates every (node, octant, mode) with BF16
 //    MFMA tiles (v_mfma_f32_32x32x16_bf16, FP32 accumulation) and stores 16
 //    decision bits and 16 confidence bits in the node's spare word; with
@@ -298,123 +298,202 @@ __global__ __launch_bounds__(256) void k_order_log(const float4* __restrict__ no
 // ---- training ----------------------------------------------------------------
 
 constexpr int kTB = 64;  // samples per block
+constexpr int kGradThreads = 1024;
+// Row lengths of the LDS arrays: 20 or 44 mod 64 words, so that the matrix
+// operands read along a row (16 rows x 4 columns of a wave) lie in 64 distinct
+// banks and the ones read down a column (4 rows x 16 columns) in at most two
+// each.
+constexpr int kLdX = 44, kLdH = 84;
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// 16 x 16 tile of A B + C, FP32: lane l holds A[l % 16][4 t + l / 16] and
+// B[4 t + l / 16][l % 16] of step t, and D[4 (l / 16) + r][l % 16] in register
+// r.  The instruction adds the 4 products of a step in order, each with one
+// rounding, so a chain of steps gives the bits of a loop of fmaf over k
+// (checked for ordinary, subnormal and zero products).
+__device__ __forceinline__ f32x4 mfma_step(float a, float b, f32x4 acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0);
+}
+
+struct GradLds {
+    float x[kTB * kLdX];    // features [sample][feature]
+    float h1[kTB * kLdH];   // activations [sample][unit]
+    float h2[kTB * kLdH];
+    float d1[kTB * kLdH];   // gradients of the layers' inputs to ReLU [sample][unit]
+    float d2[kTB * kLdH];
+    float w2[kH * kLdH];    // [in][out]
+    float y[kTB], w[kTB], dz[kTB], loss[kTB];
+};
+static_assert(sizeof(GradLds) <= 160 * 1024, "one workgroup per CU");
 
 // Forward + backward of up to 64 samples: sample i of the step is
 // samples[(start + i) * mul % n]; writes the block's gradient sums and its sum
 // of weighted losses.  Loss of a sample: weight * BCE(sigmoid(z), label).
-__global__ __launch_bounds__(kTB) void k_mlp_grad(const float* __restrict__ P, const float* __restrict__ samples,
-                                                  uint32_t n, uint64_t start, uint32_t count, uint64_t mul,
-                                                  float* __restrict__ partial, float* __restrict__ loss_part) {
-    __shared__ float sW2[kH * kH];
-    // rows padded to kTB + 1 so a thread walking its own row hits its own bank
-    __shared__ float sX[kIn][kTB + 1];
-    __shared__ float sH1[kH][kTB + 1];
-    __shared__ float sH2[kH][kTB + 1];
-    __shared__ float sDz[kTB];
-    const int t = threadIdx.x;
-    for (int i = t; i < kH * kH; i += kTB) sW2[i] = P[kW2 + i];
-    const uint32_t local = blockIdx.x * kTB + t;
-    const bool valid = local < count;
-    const uint64_t idx = ((start + local) * mul) % n;
-    for (int k = 0; k < kIn; ++k) sX[k][t] = valid ? samples[idx * kSample + k] : 0.0f;
-    const float y = valid ? samples[idx * kSample + kIn] : 0.0f;
-    const float w = valid ? samples[idx * kSample + kIn + 1] : 0.0f;
-    __syncthreads();
-    // forward (one sample per thread)
-    for (int j = 0; j < kH; ++j) {
-        float acc = P[kB1 + j];
-        for (int k = 0; k < kIn; ++k) acc = fmaf(sX[k][t], P[kW1 + k * kH + j], acc);
-        sH1[j][t] = fmaxf(acc, 0.0f);
+// Every layer's product is 16 tiles of 16 x 16, one per wave, on the FP32
+// matrix instruction.  A training step has few blocks (16 at the default batch
+// of 1,024), so its time is one block's chain of phases: 98.6 us a step with a
+// block in one wave (a sample or a column per lane, each product a loop over
+// LDS), 11.5 us now.
+__global__ __launch_bounds__(kGradThreads) void k_mlp_grad(const float* __restrict__ P,
+                                                           const float* __restrict__ samples, uint32_t n,
+                                                           uint64_t start, uint32_t count, uint64_t mul,
+                                                           float* __restrict__ partial,
+                                                           float* __restrict__ loss_part) {
+    __shared__ GradLds L;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c = lane & 15, g = lane >> 4;          // operand column and k group
+    const int mt = 16 * (wave >> 2), nt = 16 * (wave & 3);   // the wave's tile
+    // layer 1's weights straight into operand registers, layer 2's to LDS
+    float w1[kIn / 4];
+#pragma unroll
+    for (int t = 0; t < kIn / 4; ++t) w1[t] = P[kW1 + (4 * t + g) * kH + nt + c];
+    const float b1 = P[kB1 + nt + c], b2 = P[kB2 + nt + c], w3 = P[kW3 + nt + c];
+#pragma unroll
+    for (int r = 0; r < kH * kH / kGradThreads; ++r) {
+        const int i = tid + r * kGradThreads;
+        L.w2[(i / kH) * kLdH + i % kH] = P[kW2 + i];
     }
-    float z = P[kB3];
-    for (int j = 0; j < kH; ++j) {
-        float acc = P[kB2 + j];
-        for (int k = 0; k < kH; ++k) acc = fmaf(sH1[k][t], sW2[k * kH + j], acc);
-        const float h = fmaxf(acc, 0.0f);
-        sH2[j][t] = h;
-        z = fmaf(h, P[kW3 + j], z);
-    }
-    // BCE with logits: max(z, 0) - z y + log(1 + e^-|z|); dL/dz = w (sigmoid(z) - y)
-    const float p = 1.0f / (1.0f + expf(-z));
-    const float loss = w * ((fmaxf(z, 0.0f) - z * y) + log1pf(expf(-fabsf(z))));
-    sDz[t] = valid ? w * (p - y) : 0.0f;
-    __syncthreads();
-    float* g = partial + (size_t)blockIdx.x * kNP;
-    // output layer: dw3[j] = sum_s h2[s][j] dz[s]; db3 = sum dz (thread t owns j = t)
+    // 16 threads per sample
     {
+        const int s = tid >> 4;
+        const uint32_t local = blockIdx.x * kTB + s;
+        const bool valid = local < count;
+        const float* row = samples + (valid ? ((start + local) * mul) % n : 0) * kSample;
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            const int k = (tid & 15) + 16 * r;
+            const float v = valid && k < kSample ? row[k] : 0.0f;
+            if (k < kIn) L.x[s * kLdX + k] = v;
+            if (k == kIn) L.y[s] = v;
+            if (k == kIn + 1) L.w[s] = v;
+        }
+    }
+    __syncthreads();
+    float h1[4], h2[4];   // the wave's tile of both layers
+    {
+        f32x4 acc = {b1, b1, b1, b1};
+#pragma unroll
+        for (int t = 0; t < kIn / 4; ++t) acc = mfma_step(L.x[(mt + c) * kLdX + 4 * t + g], w1[t], acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            h1[r] = fmaxf(acc[r], 0.0f);
+            L.h1[(mt + 4 * g + r) * kLdH + nt + c] = h1[r];
+        }
+    }
+    __syncthreads();
+    {
+        f32x4 acc = {b2, b2, b2, b2};
+#pragma unroll
+        for (int t = 0; t < kH / 4; ++t)
+            acc = mfma_step(L.h1[(mt + c) * kLdH + 4 * t + g], L.w2[(4 * t + g) * kLdH + nt + c], acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            h2[r] = fmaxf(acc[r], 0.0f);
+            L.h2[(mt + 4 * g + r) * kLdH + nt + c] = h2[r];
+        }
+    }
+    __syncthreads();
+    if (tid < kTB) {   // output layer and loss, one sample per lane
+        float z = P[kB3];
+#pragma unroll 8
+        for (int j = 0; j < kH; ++j) z = fmaf(L.h2[tid * kLdH + j], P[kW3 + j], z);
+        // BCE with logits: max(z, 0) - z y + log(1 + e^-|z|); dL/dz = w (sigmoid(z) - y)
+        const float y = L.y[tid], w = L.w[tid];
+        const float p = 1.0f / (1.0f + expf(-z));
+        const float loss = w * ((fmaxf(z, 0.0f) - z * y) + log1pf(expf(-fabsf(z))));
+        const bool valid = blockIdx.x * kTB + tid < count;
+        L.dz[tid] = valid ? w * (p - y) : 0.0f;
+        L.loss[tid] = valid ? loss : 0.0f;
+    }
+    __syncthreads();
+    // dH2 = dz * w3 * (h2 > 0)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int m = mt + 4 * g + r;
+        L.d2[m * kLdH + nt + c] = h2[r] > 0.0f ? L.dz[m] * w3 : 0.0f;
+    }
+    __syncthreads();
+    float* out = partial + (size_t)blockIdx.x * kNP;
+    {   // dH1 = (dH2 W2^T) * (h1 > 0)
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < kH / 4; ++t)
+            acc = mfma_step(L.d2[(mt + c) * kLdH + 4 * t + g], L.w2[(nt + c) * kLdH + 4 * t + g], acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) L.d1[(mt + 4 * g + r) * kLdH + nt + c] = h1[r] > 0.0f ? acc[r] : 0.0f;
+    }
+    {   // dW2[k][j] = sum_s h1[s][k] dh2[s][j]
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < kTB / 4; ++t)
+            acc = mfma_step(L.h1[(4 * t + g) * kLdH + mt + c], L.d2[(4 * t + g) * kLdH + nt + c], acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[kW2 + (mt + 4 * g + r) * kH + nt + c] = acc[r];
+    }
+    __syncthreads();
+    if (wave < 8) {   // dW1[k][j] = sum_s x[s][k] dh1[s][j]
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < kTB / 4; ++t)
+            acc = mfma_step(L.x[(4 * t + g) * kLdX + mt + c], L.d1[(4 * t + g) * kLdH + nt + c], acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[kW1 + (mt + 4 * g + r) * kH + nt + c] = acc[r];
+    } else if (wave == 8) {   // dw3[j] = sum_s h2[s][j] dz[s]
         float acc = 0.0f;
-        for (int s = 0; s < kTB; ++s) acc = fmaf(sH2[t][s], sDz[s], acc);
-        g[kW3 + t] = acc;
-        if (t == 0) {
-            float a = 0.0f;
-            for (int s = 0; s < kTB; ++s) a += sDz[s];
-            g[kB3] = a;
-        }
-    }
-    __syncthreads();
-    // dH2 = dz * w3 * (h2 > 0), in place of H2 (thread t owns sample t)
-    for (int j = 0; j < kH; ++j) sH2[j][t] = sH2[j][t] > 0.0f ? sDz[t] * P[kW3 + j] : 0.0f;
-    __syncthreads();
-    // dW2[k][j] = sum_s h1[s][k] dh2[s][j]; db2[j] = sum_s dh2[s][j]   (thread t owns column j = t)
-    {
-        float db = 0.0f;
-        for (int s = 0; s < kTB; ++s) db += sH2[t][s];
-        g[kB2 + t] = db;
-        for (int k = 0; k < kH; ++k) {
-            float acc = 0.0f;
-            for (int s = 0; s < kTB; ++s) acc = fmaf(sH1[k][s], sH2[t][s], acc);
-            g[kW2 + k * kH + t] = acc;
-        }
-    }
-    __syncthreads();
-    // dH1 = (dH2 W2^T) * (h1 > 0), in place of H1 (thread t owns sample t)
-    for (int k = 0; k < kH; ++k) {
+#pragma unroll 8
+        for (int s = 0; s < kTB; ++s) acc = fmaf(L.h2[s * kLdH + lane], L.dz[s], acc);
+        out[kW3 + lane] = acc;
+    } else if (wave < 11) {   // db2[j] = sum_s dh2[s][j] and db1[j] = sum_s dh1[s][j]
+        const float* d = wave == 9 ? L.d2 : L.d1;
         float acc = 0.0f;
-        for (int j = 0; j < kH; ++j) acc = fmaf(sH2[j][t], sW2[k * kH + j], acc);
-        sH1[k][t] = sH1[k][t] > 0.0f ? acc : 0.0f;
-    }
-    __syncthreads();
-    // dW1[k][j] = sum_s x[s][k] dh1[s][j]; db1[j] = sum_s dh1[s][j]   (thread t owns column j = t)
-    {
-        float db = 0.0f;
-        for (int s = 0; s < kTB; ++s) db += sH1[t][s];
-        g[kB1 + t] = db;
-        for (int k = 0; k < kIn; ++k) {
-            float acc = 0.0f;
-            for (int s = 0; s < kTB; ++s) acc = fmaf(sX[k][s], sH1[t][s], acc);
-            g[kW1 + k * kH + t] = acc;
-        }
-    }
-    // loss sum of the block
-    __shared__ float sL[kTB];
-    sL[t] = valid ? loss : 0.0f;
-    __syncthreads();
-    if (t == 0) {
-        float a = 0.0f;
-        for (int s = 0; s < kTB; ++s) a += sL[s];
-        loss_part[blockIdx.x] = a;
+#pragma unroll 8
+        for (int s = 0; s < kTB; ++s) acc += d[s * kLdH + lane];
+        out[(wave == 9 ? kB2 : kB1) + lane] = acc;
+    } else if (wave == 11) {   // db3 = sum of dz (lane 0) and the block's loss (lane 1)
+        const float* v = lane == 0 ? L.dz : L.loss;
+        float acc = 0.0f;
+        if (lane < 2)
+#pragma unroll 8
+            for (int s = 0; s < kTB; ++s) acc += v[s];
+        if (lane == 0) out[kB3] = acc;
+        if (lane == 1) loss_part[blockIdx.x] = acc;
     }
 }
 
-// Sums the blocks' gradients in block order (deterministic), scales by 1/batch.
-__global__ void k_mlp_reduce(const float* __restrict__ partial, uint32_t blocks, float scale, float* __restrict__ grad) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= kNP) return;
+// The blocks' gradients of parameter j, summed in block order (deterministic)
+// and scaled by 1 / samples.
+__device__ __forceinline__ float grad_of(const float* __restrict__ partial, uint32_t blocks, float scale, int j) {
     float acc = 0.0f;
+#pragma unroll 16
     for (uint32_t b = 0; b < blocks; ++b) acc += partial[(size_t)b * kNP + j];
-    grad[j] = acc * scale;
+    return acc * scale;
 }
 
-__global__ void k_mlp_adam(float* __restrict__ P, float* __restrict__ M, float* __restrict__ V,
-                           const float* __restrict__ grad, float lr, float b1, float b2, float eps, float c1, float c2) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+constexpr int kParamThreads = 64;   // 100 workgroups for the 6,337 parameters
+constexpr uint32_t kParamBlocks = (kNP + kParamThreads - 1) / kParamThreads;
+
+__global__ __launch_bounds__(kParamThreads) void k_mlp_reduce(const float* __restrict__ partial, uint32_t blocks,
+                                                              float scale, float* __restrict__ grad) {
+    const int j = blockIdx.x * kParamThreads + threadIdx.x;
+    if (j < kNP) grad[j] = grad_of(partial, blocks, scale, j);
+}
+
+// The reduction and the Adam update in one launch (two launches took 9.6 us a
+// step at 16 blocks, this one 3.8).
+__global__ __launch_bounds__(kParamThreads) void k_mlp_step(const float* __restrict__ partial, uint32_t blocks,
+                                                            float scale, float* __restrict__ P, float* __restrict__ M,
+                                                            float* __restrict__ V, float lr, float b1, float b2,
+                                                            float eps, float c1, float c2) {
+    const int j = blockIdx.x * kParamThreads + threadIdx.x;
     if (j >= kNP) return;
-    const float g = grad[j];
-    const float m = b1 * M[j] + (1.0f - b1) * g;
-    const float v = b2 * V[j] + (1.0f - b2) * g * g;
+    const float m0 = M[j], v0 = V[j], p0 = P[j];
+    const float g = grad_of(partial, blocks, scale, j);
+    const float m = b1 * m0 + (1.0f - b1) * g;
+    const float v = b2 * v0 + (1.0f - b2) * g * g;
     M[j] = m;
     V[j] = v;
-    P[j] -= lr * (m / c1) / (sqrtf(v / c2) + eps);
+    P[j] = p0 - lr * (m / c1) / (sqrtf(v / c2) + eps);
 }
 
 // ---- BF16 MFMA inference ---------------------------------------------------------
@@ -710,13 +789,13 @@ rtq_status rtq_order_grad(rtq_ctx* ctx, const float* params_dev, const float* sa
     RTQ_HIP(ctx, dev_alloc(&partial, (size_t)blocks * kNP));
     hipError_t e = dev_alloc(&lp, blocks);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_mlp_grad, dim3(blocks), dim3(kTB), 0, st, params_dev, samples_dev, n, 0ull, n, 1ull,
+        hipLaunchKernelGGL(k_mlp_grad, dim3(blocks), dim3(kGradThreads), 0, st, params_dev, samples_dev, n, 0ull, n, 1ull,
                            partial, lp);
         e = hipGetLastError();
     }
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_mlp_reduce, dim3((kNP + 255) / 256), dim3(256), 0, st, partial, blocks, 1.0f / (float)n,
-                           grad_dev);
+        hipLaunchKernelGGL(k_mlp_reduce, dim3(kParamBlocks), dim3(kParamThreads), 0, st, partial, blocks,
+                           1.0f / (float)n, grad_dev);
         e = hipGetLastError();
     }
     std::vector<float> hl(blocks);
@@ -746,10 +825,9 @@ rtq_status rtq_order_train(rtq_ctx* ctx, const float* samples_dev, uint64_t n_sa
     hipStream_t st = ctx->stream;
     const uint32_t n = (uint32_t)n_samples;
     const uint32_t blocks = tp->batch / kTB;
-    float *partial = nullptr, *lp = nullptr, *grad = nullptr;
+    float *partial = nullptr, *lp = nullptr;
     RTQ_HIP(ctx, dev_alloc(&partial, (size_t)blocks * kNP));
     hipError_t e = dev_alloc(&lp, (size_t)blocks * ((n + tp->batch - 1) / tp->batch));
-    if (e == hipSuccess) e = dev_alloc(&grad, kNP);
     const uint32_t steps_per_epoch = (n + tp->batch - 1) / tp->batch;
     for (uint32_t ep = 0; ep < tp->epochs && e == hipSuccess; ++ep) {
         // a permutation of the samples per epoch: i -> i * mul mod n with mul coprime to n
@@ -764,18 +842,15 @@ rtq_status rtq_order_train(rtq_ctx* ctx, const float* samples_dev, uint64_t n_sa
             const uint64_t start = (uint64_t)sidx * tp->batch;
             const uint32_t cnt = (uint32_t)std::min<uint64_t>(tp->batch, n - start);
             const uint32_t bl = (cnt + kTB - 1) / kTB;
-            hipLaunchKernelGGL(k_mlp_grad, dim3(bl), dim3(kTB), 0, st, params_dev, samples_dev, n, start, cnt, mul,
-                               partial, lp + (size_t)sidx * blocks);
-            e = hipGetLastError();
-            if (e != hipSuccess) break;
-            hipLaunchKernelGGL(k_mlp_reduce, dim3((kNP + 255) / 256), dim3(256), 0, st, partial, bl,
-                               1.0f / (float)cnt, grad);
+            hipLaunchKernelGGL(k_mlp_grad, dim3(bl), dim3(kGradThreads), 0, st, params_dev, samples_dev, n, start, cnt,
+                               mul, partial, lp + (size_t)sidx * blocks);
             e = hipGetLastError();
             if (e != hipSuccess) break;
             const uint32_t tstep = ++*step;
             const float c1 = 1.0f - powf(tp->beta1, (float)tstep), c2 = 1.0f - powf(tp->beta2, (float)tstep);
-            hipLaunchKernelGGL(k_mlp_adam, dim3((kNP + 255) / 256), dim3(256), 0, st, params_dev, adam_m_dev,
-                               adam_v_dev, grad, tp->lr, tp->beta1, tp->beta2, 1e-8f, c1, c2);
+            hipLaunchKernelGGL(k_mlp_step, dim3(kParamBlocks), dim3(kParamThreads), 0, st, partial, bl,
+                               1.0f / (float)cnt, params_dev, adam_m_dev, adam_v_dev, tp->lr, tp->beta1, tp->beta2,
+                               1e-8f, c1, c2);
             e = hipGetLastError();
         }
         if (e != hipSuccess) break;
@@ -796,7 +871,6 @@ rtq_status rtq_order_train(rtq_ctx* ctx, const float* samples_dev, uint64_t n_sa
     }
     (void)hipFree(partial);
     (void)hipFree(lp);
-    (void)hipFree(grad);
     if (e != hipSuccess) return hip_fail(ctx, e, "order_train");
     return RTQ_OK;
 }

@@ -1,0 +1,49 @@
+"""The training kernels at the edges of their blocks: gradients with a last
+block of 1, 63 or 64 samples and with more blocks than CUs, and one training
+step (reduction and Adam in one kernel) against the same gradient put through
+Adam's formulas in FP32."""
+import numpy as np
+import pytest
+
+import oracle
+from realtimeraytracing_amd.rtq import ORDER_PARAMS, TrainParams
+from test_gpu_learned import dev, rand_params, rand_samples
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [63, 65, 127, 1025, 20001])
+def test_gradient_at_block_edges(rtq_ctx, torch_mod, n):
+    torch = torch_mod
+    P, S = rand_params(n), rand_samples(n, n + 1)
+    g = torch.zeros(ORDER_PARAMS, dtype=torch.float32, device="cuda")
+    dP, dS = dev(P, torch), dev(S, torch)
+    loss = rtq_ctx.order_grad(dP.data_ptr(), dS.data_ptr(), n, g.data_ptr())
+    want_loss, want = oracle.mlp_grad(P, S)
+    # sums of n terms in FP32: 64 in a chain per block, then the blocks in a chain
+    rel = 2.0 ** -24 * (64 + n / 64) * 4
+    assert loss == pytest.approx(want_loss, rel=rel)
+    assert np.abs(g.cpu().numpy() - want).max() <= max(1e-5, rel) * np.abs(want).max() + 1e-7
+
+
+@pytest.mark.parametrize("n", [1, 64, 1000, 1024])
+def test_step_is_gradient_and_adam(rtq_ctx, torch_mod, n):
+    torch = torch_mod
+    P, S = rand_params(n + 5), rand_samples(n, n + 6)
+    dP, dS = dev(P, torch), dev(S, torch)
+    m, v, g = (torch.zeros(ORDER_PARAMS, dtype=torch.float32, device="cuda") for _ in range(3))
+    torch.cuda.synchronize()
+    rtq_ctx.order_grad(dP.data_ptr(), dS.data_ptr(), n, g.data_ptr())
+    tp = TrainParams(1, 1024, 1e-2, 0.9, 0.999, 0, 3)
+    step, _ = rtq_ctx.order_train(dS.data_ptr(), n, tp, dP.data_ptr(), m.data_ptr(), v.data_ptr())
+    assert step == 1
+    # the epoch visits the samples in another order than the gradient call
+    f = np.float32
+    gh = g.cpu().numpy()
+    b1, b2 = f(0.9), f(0.999)
+    tol = 2.0 ** -24 * (64 + 16) * 4 * np.abs(gh).max()
+    assert np.abs(m.cpu().numpy() - (f(1) - b1) * gh).max() <= tol * 0.2
+    mh, vh = m.cpu().numpy(), v.cpu().numpy()
+    assert np.allclose(vh, (f(1) - b2) * (mh / (f(1) - b1)) ** 2, rtol=1e-5, atol=1e-30)
+    want = P - f(1e-2) * (mh / (f(1) - b1)) / (np.sqrt(vh / (f(1) - b2)) + f(1e-8))
+    assert np.allclose(dP.cpu().numpy(), want, rtol=1e-5, atol=1e-6)
