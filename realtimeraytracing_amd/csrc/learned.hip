@@ -122,7 +122,8 @@ __device__ __forceinline__ void child_hits(float4 n0, float4 n1, float4 n2, cons
     h1 = tn1 <= tf1;
 }
 
-constexpr int kLogStack = 96;
+constexpr uint32_t kLogStack = 96;
+constexpr uint32_t kLogRecords = 32;       // samples of a ray kept until its wave ends
 constexpr uint32_t kLogBudget = 1u << 14;  // node visits + triangle tests per sub-traversal
 
 struct LogRay {
@@ -135,10 +136,10 @@ struct LogRay {
 // Closest (any = false): returns the leaf-order index of the closest hit and
 // shrinks tmax to its t.  Any hit: returns the first hit found.  kNone = no
 // hit.  cost = node visits + triangle tests; ok = false when the walk ran past
-// kLogBudget or its stack.
+// kLogBudget or kLogStack entries.  Stack entry k is stack[k * stride] in LDS.
 __device__ uint32_t log_walk(const float4* __restrict__ nodes, const float4* __restrict__ tris, const LogRay& R,
-                             uint32_t ref, bool any, float& tmax, uint32_t& cost, bool& ok) {
-    uint32_t stack[kLogStack];
+                             uint32_t ref, bool any, uint32_t* stack, uint32_t stride, float& tmax, uint32_t& cost,
+                             bool& ok) {
     uint32_t sp = 0, cur = ref, target = kNone;
     cost = 0;
     ok = true;
@@ -160,7 +161,7 @@ __device__ uint32_t log_walk(const float4* __restrict__ nodes, const float4* __r
                     return kNone;
                 }
                 const bool f0 = tn0 <= tn1;
-                stack[sp++] = f0 ? r1 : r0;
+                stack[sp++ * stride] = f0 ? r1 : r0;
                 cur = f0 ? r0 : r1;
                 continue;
             }
@@ -184,16 +185,19 @@ __device__ uint32_t log_walk(const float4* __restrict__ nodes, const float4* __r
             }
         }
         if (sp == 0) return target;
-        cur = stack[--sp];
+        cur = stack[--sp * stride];
     }
 }
 
-__device__ void emit(float* __restrict__ out, uint32_t cap, uint32_t* __restrict__ count, float4 n0, float4 n1,
-                     float4 n2, float4 n3, uint4 ax4, uint32_t octant, uint32_t any, bool child0_first, float weight) {
-    const uint32_t slot = atomicAdd(count, 1u);
+// Sample `slot`: the features of binary node `node` for the octant and mode,
+// the label and the weight.
+__device__ void emit(float* __restrict__ out, uint32_t cap, uint32_t slot, const float4* __restrict__ nodes,
+                     const uint4* __restrict__ aux, uint32_t node, uint32_t octant, uint32_t any, bool child0_first,
+                     float weight) {
     if (slot >= cap) return;
+    const float4* nd = nodes + 4ull * node;
     float f[kIn];
-    node_features(n0, n1, n2, n3, ax4, octant, any, f);
+    node_features(nd[0], nd[1], nd[2], nd[3], aux[node], octant, any, f);
     float* o = out + (size_t)slot * kSample;
     for (int k = 0; k < kIn; ++k) o[k] = f[k];
     o[kIn] = child0_first ? 1.0f : 0.0f;
@@ -206,92 +210,127 @@ __device__ void emit(float* __restrict__ out, uint32_t cap, uint32_t* __restrict
 // occluder is found for any-hit rays); label = the cheaper child first, weight
 // log2(1 + cost difference), no sample on a tie.  The walk continues into the
 // cheaper child and stops where no hit lies below it.
-__global__ __launch_bounds__(256) void k_order_log(const float4* __restrict__ nodes, const uint4* __restrict__ aux,
-                                                   const float4* __restrict__ tris, const rtq_ray* __restrict__ rays,
-                                                   uint32_t n, uint32_t stride, uint32_t any, float* __restrict__ out,
-                                                   uint32_t cap, uint32_t* __restrict__ count) {
-    const uint64_t r = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * stride;
-    if (r >= n) return;
-    const rtq_ray ray = rays[r];
-    if (!(ray.tmin <= ray.tmax)) return;
-    LogRay R;
-    for (int k = 0; k < 3; ++k) {
-        const float d = fabsf(ray.d[k]) < 1e-30f ? copysignf(1e-30f, ray.d[k]) : ray.d[k];
-        R.o[k] = ray.o[k];
-        R.inv[k] = 1.0f / d;
-    }
-    R.tmin = ray.tmin;
-    R.tmax = ray.tmax;
-    const float ax = fabsf(ray.d[0]), ay = fabsf(ray.d[1]), az = fabsf(ray.d[2]);
-    int kz = 0;
-    float m = ax;
-    if (ay > m) { kz = 1; m = ay; }
-    if (az > m) kz = 2;
-    int kx = kz + 1 == 3 ? 0 : kz + 1;
-    int ky = kx + 1 == 3 ? 0 : kx + 1;
-    const float dkz = ray.d[kz];
-    if (dkz == 0.0f) return;
-    if (dkz < 0.0f) { const int tmp = kx; kx = ky; ky = tmp; }
-    R.kx = kx;
-    R.ky = ky;
-    R.kz = kz;
-    R.sx = ray.d[kx] / dkz;
-    R.sy = ray.d[ky] / dkz;
-    R.sz = 1.0f / dkz;
-    R.opx = ray.o[kx];
-    R.opy = ray.o[ky];
-    R.opz = ray.o[kz];
-    const uint32_t octant = (ray.d[0] < 0.0f ? 1u : 0u) | (ray.d[1] < 0.0f ? 2u : 0u) | (ray.d[2] < 0.0f ? 4u : 0u);
-    // Walk from the root along the child each decision visits first: nothing
-    // has been visited before such a node, so its interval is the ray's own.
-    uint32_t cur = 0;
-    while (!(cur & kLeafBit)) {
-        const float4* nd = nodes + 4ull * cur;
-        const float4 n0 = nd[0], n1 = nd[1], n2 = nd[2], n3 = nd[3];
-        bool h0, h1;
-        float tn0, tn1;
-        child_hits(n0, n1, n2, R.o, R.inv, R.tmin, R.tmax, h0, h1, tn0, tn1);
-        const uint32_t r0 = __float_as_uint(n3.x), r1 = __float_as_uint(n3.y);
-        if (h0 && h1) {
-            uint32_t cost01, cost10;
-            bool f0, f1;
-            if (any) {
-                // an occluder below the first child ends the ray there
-                uint32_t c0, c1;
-                bool ok0, ok1;
-                float t0 = R.tmax, t1 = R.tmax;
-                f0 = log_walk(nodes, tris, R, r0, true, t0, c0, ok0) != kNone;
-                f1 = log_walk(nodes, tris, R, r1, true, t1, c1, ok1) != kNone;
-                if (!ok0 || !ok1) return;
-                cost01 = f0 ? c0 : c0 + c1;
-                cost10 = f1 ? c1 : c1 + c0;
-            } else {
-                // closest hit: the second child is walked with the interval the first left
-                uint32_t a0, a1, b0, b1;
-                bool ok[4];
-                float ta = R.tmax, tb = R.tmax;
-                f0 = log_walk(nodes, tris, R, r0, false, ta, a0, ok[0]) != kNone;
-                log_walk(nodes, tris, R, r1, false, ta, a1, ok[1]);
-                f1 = log_walk(nodes, tris, R, r1, false, tb, b1, ok[2]) != kNone;
-                log_walk(nodes, tris, R, r0, false, tb, b0, ok[3]);
-                if (!ok[0] || !ok[1] || !ok[2] || !ok[3]) return;
-                cost01 = a0 + a1;
-                cost10 = b1 + b0;
+// A pair of lanes per ray: the even one prices child 0 first, the odd one
+// child 1 first.  A launch lasts as long as its longest walks, so a wave takes
+// only `per_wave` rays, and its stacks lie in LDS, `levels` entries per lane.  A
+// ray's samples wait in registers' scratch, so that a wave takes their slots
+// with one atomic at its end: atomics of every sample on one word serialise.
+// 25,000 any-hit rays on 300,000 occluded triangles: 1.04 ms (closest hit
+// 1.60), 2.64 (5.15) with a lane per ray and full waves; 200,000 rays 2.53
+// against 3.26 ms.
+__global__ __launch_bounds__(64) void k_order_log(const float4* __restrict__ nodes, const uint4* __restrict__ aux,
+                                                  const float4* __restrict__ tris, const rtq_ray* __restrict__ rays,
+                                                  uint32_t n, uint32_t stride, uint32_t per_wave, uint32_t levels,
+                                                  uint32_t any, float* __restrict__ out, uint32_t cap,
+                                                  uint32_t* __restrict__ count) {
+    extern __shared__ uint32_t s_log[];
+    const uint32_t lane = threadIdx.x, lanes = 2 * per_wave;
+    const bool second = lane & 1u;          // prices child 1 first
+    uint32_t* const stack = s_log + lane;   // [levels][lanes]
+    uint2 rec[kLogRecords];                 // node | child 0 first << 31, weight (even lanes)
+    const uint64_t r = ((uint64_t)blockIdx.x * per_wave + lane / 2) * stride;
+    uint32_t n_rec = 0, octant = 0;
+    if (lane < lanes && r < n) {
+        const rtq_ray ray = rays[r];
+        LogRay R;
+        for (int k = 0; k < 3; ++k) {
+            const float d = fabsf(ray.d[k]) < 1e-30f ? copysignf(1e-30f, ray.d[k]) : ray.d[k];
+            R.o[k] = ray.o[k];
+            R.inv[k] = 1.0f / d;
+        }
+        R.tmin = ray.tmin;
+        R.tmax = ray.tmax;
+        const float ax = fabsf(ray.d[0]), ay = fabsf(ray.d[1]), az = fabsf(ray.d[2]);
+        int kz = 0;
+        float m = ax;
+        if (ay > m) { kz = 1; m = ay; }
+        if (az > m) kz = 2;
+        int kx = kz + 1 == 3 ? 0 : kz + 1;
+        int ky = kx + 1 == 3 ? 0 : kx + 1;
+        const float dkz = ray.d[kz];
+        if (dkz < 0.0f) { const int tmp = kx; kx = ky; ky = tmp; }
+        R.kx = kx;
+        R.ky = ky;
+        R.kz = kz;
+        R.sx = ray.d[kx] / dkz;
+        R.sy = ray.d[ky] / dkz;
+        R.sz = 1.0f / dkz;
+        R.opx = ray.o[kx];
+        R.opy = ray.o[ky];
+        R.opz = ray.o[kz];
+        octant = (ray.d[0] < 0.0f ? 1u : 0u) | (ray.d[1] < 0.0f ? 2u : 0u) | (ray.d[2] < 0.0f ? 4u : 0u);
+        // Walk from the root along the child each decision visits first: nothing
+        // has been visited before such a node, so its interval is the ray's own.
+        // (An empty interval or a zero direction hits nothing: no walk.)
+        uint32_t cur = ray.tmin <= ray.tmax && dkz != 0.0f ? 0u : kLeafBit;
+        while (!(cur & kLeafBit)) {
+            const float4* nd = nodes + 4ull * cur;
+            const float4 n3 = nd[3];
+            bool h0, h1;
+            float tn0, tn1;
+            child_hits(nd[0], nd[1], nd[2], R.o, R.inv, R.tmin, R.tmax, h0, h1, tn0, tn1);
+            const uint32_t r0 = __float_as_uint(n3.x), r1 = __float_as_uint(n3.y);
+            if (!(h0 || h1)) break;
+            if (!(h0 && h1)) {
+                cur = h0 ? r0 : r1;
+                continue;
             }
+            // the lane's first child, and for closest-hit rays the other one
+            // with the interval the first left (an occluder below the first
+            // child ends an any-hit ray there, and the other lane's walk gives
+            // the other child's cost)
+            uint32_t cost, more = 0;
+            bool ok, ok2 = true;
+            float t = R.tmax;
+            const bool found = log_walk(nodes, tris, R, second ? r1 : r0, any, stack, lanes, t, cost, ok) != kNone;
+            if (!any) log_walk(nodes, tris, R, second ? r0 : r1, false, stack, lanes, t, more, ok2);
+            const int good = ok && ok2, other_good = __shfl_xor(good, 1);
+            const bool other_found = __shfl_xor((int)found, 1) != 0;
+            const uint32_t mine = cost + more, other = __shfl_xor(mine, 1);
+            if (!good || !other_good) break;
+            const uint32_t total = any && !found ? mine + other : mine;
+            const uint32_t other_total = any && !other_found ? other + mine : other;
+            const bool f0 = second ? other_found : found, f1 = second ? found : other_found;
+            const uint32_t cost01 = second ? other_total : total, cost10 = second ? total : other_total;
             // with no hit below either child every order visits the same nodes
-            if (!f0 && !f1) return;
-            if (cost01 != cost10) {
+            if (!f0 && !f1) break;
+            if (cost01 != cost10 && !second) {
                 const float diff = (float)(cost01 > cost10 ? cost01 - cost10 : cost10 - cost01);
-                emit(out, cap, count, n0, n1, n2, n3, aux[cur], octant, any, cost01 < cost10, log2f(1.0f + diff));
+                const float weight = log2f(1.0f + diff);
+                if (n_rec < kLogRecords) {
+                    rec[n_rec++] = make_uint2(cur | (cost01 < cost10 ? kLeafBit : 0u), __float_as_uint(weight));
+                } else {   // a path of more levels than the records hold
+                    emit(out, cap, atomicAdd(count, 1u), nodes, aux, cur, octant, any, cost01 < cost10, weight);
+                }
             }
             const bool go0 = cost01 <= cost10;
-            if (!(go0 ? f0 : f1)) return;
+            if (!(go0 ? f0 : f1)) break;
             cur = go0 ? r0 : r1;
-        } else if (h0 || h1) {
-            cur = h0 ? r0 : r1;
-        } else {
-            return;
         }
+    }
+    // the wave's slots, then each ray's samples by its two lanes in turn
+    uint32_t incl = n_rec;   // in the even lanes; 0 in the odd ones
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = __shfl_up(incl, d, 64);
+        if (lane >= (uint32_t)d) incl += o;
+    }
+    const uint32_t all = __shfl(incl, 63, 64);
+    if (all == 0) return;
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(count, all);
+    base = __shfl(base, 0, 64) + __shfl(incl - n_rec, (int)(lane & ~1u), 64);
+    for (uint32_t k = 0; k < kLogRecords; k += 2) {
+        if (__ballot(k < n_rec) == 0) break;
+        // the even lane's records k and k + 1, one for each lane of the pair
+        const uint2 a0 = rec[k], a1 = rec[k + 1];
+        const uint32_t sx = __shfl(second ? a0.x : a1.x, (int)(lane & ~1u), 64);
+        const uint32_t sy = __shfl(second ? a0.y : a1.y, (int)(lane & ~1u), 64);
+        const uint32_t have = __shfl(n_rec, (int)(lane & ~1u), 64);
+        const uint2 s = second ? make_uint2(sx, sy) : a0;
+        if (k + second < have)
+            emit(out, cap, base + k + second, nodes, aux, s.x & ~kLeafBit, octant, any, (s.x & kLeafBit) != 0,
+                 __uint_as_float(s.y));
     }
 }
 
@@ -763,9 +802,16 @@ rtq_status rtq_order_log(rtq_ctx* ctx, uint32_t scene_id, const rtq_ray* rays_de
     hipError_t e = hipMemsetAsync(cnt, 0, sizeof(uint32_t), st);
     const uint64_t threads = (n_rays + stride - 1) / stride;
     if (e == hipSuccess && threads > 0) {
-        hipLaunchKernelGGL(k_order_log, dim3((uint32_t)((threads + 255) / 256)), dim3(256), 0, st, s->nodes,
-                           s->node_aux, s->tris, rays_dev, (uint32_t)n_rays, stride,
-                           (flags & RTQ_TRACE_ANY) ? 1u : 0u, samples_dev, (uint32_t)capacity, cnt);
+        // four waves per SIMD, of at least 4 rays (25,000 rays on 300,000
+        // occluded triangles: 1.22 ms with one wave per SIMD, 1.04 with four,
+        // 1.18 with eight), then full ones
+        const uint64_t simds = 4 * (uint64_t)std::max(ctx->n_cu, 1);
+        const uint32_t per_wave = (uint32_t)std::min<uint64_t>(32, std::max<uint64_t>(4, threads / (4 * simds)));
+        const uint32_t levels = std::min<uint32_t>(kLogStack, s->depth + 1);
+        hipLaunchKernelGGL(k_order_log, dim3((uint32_t)((threads + per_wave - 1) / per_wave)), dim3(64),
+                           sizeof(uint32_t) * levels * 2 * per_wave, st, s->nodes, s->node_aux, s->tris, rays_dev,
+                           (uint32_t)n_rays, stride, per_wave, levels, (flags & RTQ_TRACE_ANY) ? 1u : 0u, samples_dev,
+                           (uint32_t)capacity, cnt);
         e = hipGetLastError();
     }
     uint32_t h = 0;

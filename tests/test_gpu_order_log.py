@@ -1,0 +1,57 @@
+"""Traversal logs: waves of few rays, pairs of lanes per ray and slots taken per
+wave give the samples that single rays give, at ray counts around the split's
+edges, and a store that is too small keeps what fits."""
+import numpy as np
+import pytest
+
+from realtimeraytracing_amd import ORDER_SAMPLE, devmem, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def scene(rtq_ctx):
+    sc = rtq_ctx.upload(*scenes.soup_scene(3000, seed=4))
+    sc.build()
+    yield sc
+    sc.release()
+
+
+def log(scene, torch, rays, n, any_hit, stride, capacity):
+    out = torch.full((capacity + 1, ORDER_SAMPLE), 7.5, dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    k = scene.order_log(rays.data_ptr(), n, out.data_ptr(), capacity, 1 if any_hit else 0, stride)
+    out = out.cpu().numpy()
+    assert (out[k:] == 7.5).all()
+    return out[:k]
+
+
+def as_sorted(s):
+    return s[np.lexsort(s.T)]
+
+
+@pytest.mark.parametrize("any_hit", [True, False])
+@pytest.mark.parametrize("n,stride", [(1, 1), (3, 1), (9, 2), (257, 1), (1025, 7)])
+def test_samples_are_those_of_single_rays(scene, torch_mod, any_hit, n, stride):
+    rays = scenes.random_rays(n, 12, (0, 0, 0), (1, 1, 1))
+    rays["tmax"][::5] = 0.2
+    rays["tmin"][::11] = 0.5
+    rays["d"][3::97] = 0.0
+    d = devmem.to_device(rays)
+    got = log(scene, torch_mod, d, n, any_hit, stride, 64 * n)
+    one = [log(scene, torch_mod, devmem.to_device(rays[i:i + 1]), 1, any_hit, 1, 64) for i in range(0, n, stride)]
+    want = np.concatenate(one)
+    assert len(got) == len(want)
+    assert np.array_equal(as_sorted(got).view(np.uint32), as_sorted(want).view(np.uint32))
+
+
+def test_full_store(scene, torch_mod):
+    rays = scenes.random_rays(500, 13, (0, 0, 0), (1, 1, 1))
+    d = devmem.to_device(rays)
+    every = log(scene, torch_mod, d, 500, True, 1, 32000)
+    room = len(every) // 2
+    assert room > 10
+    kept = log(scene, torch_mod, d, 500, True, 1, room)
+    assert len(kept) == room
+    rows = {r.tobytes() for r in every}
+    assert all(r.tobytes() in rows for r in kept)
