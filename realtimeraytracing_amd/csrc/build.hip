@@ -337,7 +337,7 @@ __global__ __launch_bounds__(kThreads) void k_morton(const rtq_triangle* __restr
 
 // --------------------------------------------------------------------- PLOC
 
-struct Box6 {
+struct alignas(8) Box6 {   // three 8-B words, so LDS reads take 8 B at a time
     float lo[3], hi[3];
 };
 
@@ -347,6 +347,75 @@ __device__ __forceinline__ float merged_sa(const Box6& a, const Box6& b) {
     float dy = smax(a.hi[1], b.hi[1]) - smin(a.lo[1], b.lo[1]);
     float dz = smax(a.hi[2], b.hi[2]) - smin(a.lo[2], b.lo[2]);
     return 2.0f * ((dx * dy + dy * dz) + dz * dx);
+}
+
+// Half of merged_sa for the comparisons of the neighbour search: the doubling
+// is exact, and the minimum and maximum instructions differ from the compares
+// of smin / smax in the sign of a zero only, so the order of two clusters is
+// the same (vertices are finite).  17 instead of 34 instructions per neighbour
+// with the search's loop unrolled (the first pass of 2M clusters spends 35 us
+// in it, close to the rate of its instructions; 27 us wait in the look-back).
+__device__ __forceinline__ float vmin(float a, float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmax(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float merge_cost(const Box6& a, const Box6& b) {
+    const float dx = vmax(a.hi[0], b.hi[0]) - vmin(a.lo[0], b.lo[0]);
+    const float dy = vmax(a.hi[1], b.hi[1]) - vmin(a.lo[1], b.lo[1]);
+    const float dz = vmax(a.hi[2], b.hi[2]) - vmin(a.lo[2], b.lo[2]);
+    return (dx * dy + dy * dz) + dz * dx;
+}
+
+// A box past the ends of a list: its merge cost with any box is infinite, so
+// the search never takes it.
+__device__ __forceinline__ Box6 far_box() {
+    constexpr float f = 3.0e38f;
+    return Box6{{-f, -f, -f}, {f, f, f}};
+}
+
+// The nearer of (best, arg) and the N boxes from w on, whose list positions are
+// j, j + 1, ...; the first one on ties.
+template <int N>
+__device__ __forceinline__ void nearest_of(const Box6& b, const Box6* w, int j, float& best, uint32_t& arg) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const float d = merge_cost(b, w[k]);
+        const bool take = d < best;
+        best = take ? d : best;
+        arg = take ? (uint32_t)(j + k) : arg;
+    }
+}
+
+// Search radius of the reference (bvh.hpp:66): its window is unrolled.
+constexpr int kRefRadius = 16;
+
+// Nearest neighbour in the window [i - r, i + r] of list position i, the
+// lowest one on ties (bvh.cpp:193-210); w is the box at i - r, with far boxes
+// beside the list's ends when r is kRefRadius, else the list is [lo, hi).
+__device__ __forceinline__ uint32_t nearest_in_window(const Box6* w, int i, int r, int lo, int hi) {
+    float best = INFINITY;
+    uint32_t arg = kNone;
+    if (r == kRefRadius) {
+        const Box6 b = w[kRefRadius];
+        nearest_of<kRefRadius>(b, w, i - kRefRadius, best, arg);
+        nearest_of<kRefRadius>(b, w + kRefRadius + 1, i + 1, best, arg);
+    } else {
+        const Box6 b = w[r];
+        const int start = max(i - r, lo), end = min(i + r + 1, hi);
+        for (int j = start; j < end; ++j) {
+            const float d = merge_cost(b, w[j - i + r]);
+            const bool take = j != i && d < best;
+            best = take ? d : best;
+            arg = take ? (uint32_t)j : arg;
+        }
+    }
+    return arg;
 }
 
 __global__ __launch_bounds__(kThreads) void k_cluster_init(uint32_t n, uint32_t* __restrict__ cparent,
@@ -598,12 +667,26 @@ __device__ __forceinline__ void ploc_merge_write(const PlocClusters& cl, uint32_
     ploc_merge_store(cl, id, cid, cj, count, b, bj);
 }
 
+// Tile of this workgroup.  Workgroups are dispatched to the 8 XCDs in turn, and
+// the ones of each XCD number their tiles by a counter of their own: the k-th
+// one to start of those with blockIdx % 8 == x takes tile 8 k + x.  Every tile
+// before it is then taken by a workgroup that was dispatched before or with it
+// (or waits for a slot that only earlier tiles hold), so the look-back's waits
+// end; atomics on one word serialise (about 12 ns each, 50 us for the 4,361
+// tiles of a 2M-triangle terrain's first pass with one counter).
+constexpr uint32_t kTicketStride = 32;             // words between the counters (128 B)
+constexpr uint32_t kTicketWords = 8 * kTicketStride;
+__device__ __forceinline__ uint32_t take_tile(uint32_t* ctr) {
+    const uint32_t x = blockIdx.x & 7u;
+    return 8u * atomicAdd(ctr + x * kTicketStride, 1u) + x;
+}
+
 struct PlocPassArgs {
     const uint32_t* st_in;
     uint32_t* st_out;
     uint32_t bound;       // clusters at the start of the batch: the grid covers them
     uint32_t radius;
-    uint32_t* tile_ctr;   // zeroed before the pass
+    uint32_t* tile_ctr;   // kTicketWords words, zeroed before the pass
     uint64_t* tile_status;// one word per tile, zeroed before the pass
     uint32_t* err;
     uint4* log;           // (first merge id, merges, clusters, 1 if left to the tail)
@@ -640,7 +723,7 @@ __global__ __launch_bounds__(kPassThreads) void k_ploc_pass(PlocPassArgs a) {
         // counter, whose atomics serialise), so the tiles are 0 .. need - 1
         const uint32_t need = (iter + T - 1) / T;
         if (!skip && blockIdx.x >= need) skip = 1;
-        const uint32_t tile = skip ? 0u : atomicAdd(a.tile_ctr, 1u);
+        const uint32_t tile = skip ? 0u : take_tile(a.tile_ctr);
         s_hdr[0] = tile;
         s_hdr[1] = iter;
         s_hdr[2] = n_total;
@@ -656,7 +739,7 @@ __global__ __launch_bounds__(kPassThreads) void k_ploc_pass(PlocPassArgs a) {
     const int lo = base - 2 * r;
     for (int q = tid; q < kPassThreads + 2 * r; q += kPassThreads) {
         const int p = lo + q;
-        if (p >= 0 && p < (int)iter) s_box[q] = b_in[p];
+        s_box[q] = p >= 0 && p < (int)iter ? b_in[p] : far_box();
     }
     __syncthreads();
 
@@ -666,17 +749,7 @@ __global__ __launch_bounds__(kPassThreads) void k_ploc_pass(PlocPassArgs a) {
     {
         uint32_t arg = kNone;
         if (i >= 0 && i < (int)iter) {
-            const Box6 bi = s_box[tid + r];
-            const int start = max(i - r, 0), end = min(i + r + 1, (int)iter);
-            float best = INFINITY;
-            // branch-free body, unrolled: the LDS reads of several j overlap
-#pragma unroll 4
-            for (int j = start; j < end; ++j) {
-                const float d = merged_sa(bi, s_box[j - lo]);
-                const bool take = j != i && d < best;
-                best = take ? d : best;
-                arg = take ? (uint32_t)j : arg;
-            }
+            arg = nearest_in_window(s_box + tid, i, r, 0, (int)iter);
             if (arg == kNone) atomicOr(a.err, kPlocErrNoNeighbour);
         }
         s_nn[tid] = arg;
@@ -780,21 +853,154 @@ __global__ __launch_bounds__(kPassThreads) void k_ploc_pass(PlocPassArgs a) {
     a.lists.b[cur ^ 1u][oy] = b;
 }
 
+// Lane l's value from lane l ^ X of its group of four.
+template <int X>
+__device__ __forceinline__ uint32_t quad_xor(uint32_t v) {
+    constexpr int ctrl = X == 1 ? 0xB1 : 0x4E;   // quad_perm [1 0 3 2] or [2 3 0 1]
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
+}
+
+// Inclusive sum over the wave's 64 lanes (data-parallel primitives: a step per
+// instruction instead of an LDS round trip).
+__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t x) {
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, false);   // row_shr:1
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, false);   // row_shr:2
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, false);   // row_shr:4
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, false);   // row_shr:8
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xA, 0xF, false);   // row_bcast:15
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xC, 0xF, false);   // row_bcast:31
+    return x;
+}
+
+// kRefRadius search of position i by P = 2 or 4 neighbouring lanes, each with a
+// part of the window (lane part q before lane part q + 1 in list order).
+template <int P>
+__device__ __forceinline__ uint32_t nearest_by_lanes(const Box6* w, int i, int q) {
+    constexpr int kPart = 2 * kRefRadius / P;
+    // the parts before the box, then (one further) those after it
+    const int k = -kRefRadius + q * kPart + (q >= P / 2 ? 1 : 0);
+    float best = INFINITY;
+    uint32_t arg = kNone;
+    nearest_of<kPart>(*w, w + k, i + k, best, arg);
+#pragma unroll
+    for (int x = 1; x < P; x *= 2) {
+        const float d = __uint_as_float(x == 1 ? quad_xor<1>(__float_as_uint(best)) : quad_xor<2>(__float_as_uint(best)));
+        const uint32_t j = x == 1 ? quad_xor<1>(arg) : quad_xor<2>(arg);
+        const bool take = d < best || (d == best && j < arg);
+        best = take ? d : best;
+        arg = take ? j : arg;
+    }
+    return arg;
+}
+
+// The tail's list in LDS, with its triangle counts (no global loads between the
+// passes' barriers) and nearest neighbours.
+struct TailLists {
+    Box6 list[kTailMax + 2 * kRefRadius];   // kRefRadius far boxes, the list's boxes, kRefRadius far boxes
+    uint32_t c[kTailMax];
+    uint32_t n[kTailMax];
+    uint16_t nn[kTailMax];
+    uint32_t w[kTailThreads / 64];
+};
+
+// Flags, scan, merge and compaction of a list of m clusters whose neighbours
+// are found: thread t owns positions K t .. K t + K - 1.  Returns merges << 16 |
+// clusters left.  ONE_WAVE: the first wave alone (m <= 64 K), else every thread
+// (two barriers).  Both partners' state is read before anything depends on
+// it, so that a pass waits for LDS three times, not once per position and step.
+template <int K, bool ONE_WAVE>
+__device__ __forceinline__ uint32_t tail_merge(TailLists& L, int tid, uint32_t m, uint32_t n_total,
+                                               const PlocClusters& cl) {
+    Box6* const s_box = L.list + kRefRadius;
+    uint32_t j[K], back[K], f[K], sum = 0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const uint32_t i = (uint32_t)(K * tid + k);
+        j[k] = L.nn[min(i, m - 1)];
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        j[k] = min(j[k], m - 1);   // in range also where the search found none (which fails the build)
+        back[k] = L.nn[j[k]];
+    }
+    Box6 ob[K], pb[K];
+    uint32_t oc[K], on[K], pc[K], pn[K], opos[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const uint32_t i = min((uint32_t)(K * tid + k), m - 1);
+        ob[k] = s_box[i];
+        oc[k] = L.c[i];
+        on[k] = L.n[i];
+        pb[k] = s_box[j[k]];
+        pc[k] = L.c[j[k]];
+        pn[k] = L.n[j[k]];
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const uint32_t i = (uint32_t)(K * tid + k);
+        const bool mutual = back[k] == i && j[k] != i;
+        f[k] = i < m ? ((mutual && i < j[k]) ? 1u << 16 : 0u) | ((mutual && j[k] < i) ? 0u : 1u) : 0u;
+        sum += f[k];
+    }
+    uint32_t run = wave_inclusive_sum(sum), total = 0;
+    if constexpr (ONE_WAVE) {
+        total = (uint32_t)__builtin_amdgcn_readlane((int)run, 63);
+        run -= sum;
+    } else {
+        if ((tid & 63) == 63) L.w[tid >> 6] = run;
+        __syncthreads();
+        run -= sum;
+#pragma unroll
+        for (int w = 0; w < kTailThreads / 64; ++w) {
+            const uint32_t x = L.w[w];
+            run += w < (tid >> 6) ? x : 0u;
+            total += x;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        opos[k] = (f[k] & 0xFFFFu) ? run & 0xFFFFu : kNone;
+        if (f[k] >> 16) {
+            const uint32_t id = n_total + (run >> 16);
+            on[k] += pn[k];
+            ploc_merge_store(cl, id, oc[k], pc[k], on[k], ob[k], pb[k]);
+            oc[k] = id;
+        }
+        run += f[k];
+    }
+    // every read of this pass's list is done: by the barrier above, or because
+    // one wave's instructions keep their order
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        if (opos[k] != kNone) {
+            s_box[opos[k]] = ob[k];
+            L.c[opos[k]] = oc[k];
+            L.n[opos[k]] = on[k];
+        }
+    if (tid < kRefRadius) s_box[(total & 0xFFFFu) + tid] = far_box();
+    return total;
+}
+
 // All remaining passes once at most kTailMax clusters are left, in one
 // workgroup with the list in LDS (same arithmetic as k_ploc_pass).  Thread t
 // owns positions 4t .. 4t+3 for flags, scan and merge.  Does nothing unless
 // 1 < clusters <= kTailMax.
+// One CU runs it, so its long passes are bound by the search's instructions
+// (merge_cost), its short ones (half of them have under 130 clusters) by a
+// pass's chain of dependent steps: up to 512 or 256 clusters a position's window
+// is shared by 2 or 4 lanes, and up to 256 the first wave alone flags, scans
+// and merges, so that a pass has two barriers.  960 clusters (19 passes): 112
+// us before these and the shorter search, 66 now; the last 33 passes of a
+// 2M-triangle terrain, whose first ones are long, 228 and 206.
 __global__ __launch_bounds__(kTailThreads) void k_ploc_tail(uint32_t* __restrict__ state, uint32_t radius,
                                                             uint32_t* __restrict__ err, uint4* __restrict__ log,
                                                             uint32_t* __restrict__ log_count, PlocLists lists,
                                                             PlocClusters cl) {
-    __shared__ Box6 s_box[kTailMax];
-    __shared__ uint32_t s_c[kTailMax];
-    __shared__ uint32_t s_n[kTailMax];   // triangle counts: no global loads between the passes' barriers
-    __shared__ uint16_t s_nn[kTailMax];
-    __shared__ uint32_t s_w[kTailThreads / 64];
+    __shared__ TailLists L;
     __shared__ uint32_t s_hdr[4];
-    constexpr uint16_t kNone16 = 0xFFFFu;
+    Box6* const s_box = L.list + kRefRadius;
     const int tid = threadIdx.x;
     const int r = (int)radius;
     if (tid == 0) {
@@ -812,74 +1018,43 @@ __global__ __launch_bounds__(kTailThreads) void k_ploc_tail(uint32_t* __restrict
     for (uint32_t q = tid; q < m; q += kTailThreads) {
         s_box[q] = lists.b[cur][q];
         const uint32_t c = lists.c[cur][q];
-        s_c[q] = c;
-        s_n[q] = cl.count[c];
+        L.c[q] = c;
+        L.n[q] = cl.count[c];
+    }
+    if (tid < kRefRadius) {
+        L.list[tid] = far_box();
+        s_box[m + tid] = far_box();
     }
     __syncthreads();
     uint32_t passes = 0;
     while (m > 1) {
-        for (int i = tid; i < (int)m; i += kTailThreads) {
-            const Box6 bi = s_box[i];
-            const int start = max(i - r, 0), end = min(i + r + 1, (int)m);
-            float best = INFINITY;
-            uint16_t arg = kNone16;
-#pragma unroll 4
-            for (int j = start; j < end; ++j) {
-                const float d = merged_sa(bi, s_box[j]);
-                const bool take = j != i && d < best;
-                best = take ? d : best;
-                arg = take ? (uint16_t)j : arg;
-            }
-            if (arg == kNone16) atomicOr(err, kPlocErrNoNeighbour);
-            s_nn[i] = arg;
+        const bool shared = r == kRefRadius;   // window parts need the unrolled search
+        const int split = shared && m <= 256 ? 2 : shared && m <= 512 ? 1 : 0;   // log2 of the lanes per window
+        for (int t = tid; t < (int)m << split; t += kTailThreads) {
+            const int i = t >> split, q = t & ((1 << split) - 1);
+            const uint32_t arg = split == 2   ? nearest_by_lanes<4>(s_box + i, i, q)
+                                 : split == 1 ? nearest_by_lanes<2>(s_box + i, i, q)
+                                              : nearest_in_window(s_box + i - r, i, r, 0, (int)m);
+            if (arg == kNone) atomicOr(err, kPlocErrNoNeighbour);
+            if (q == 0) L.nn[i] = (uint16_t)arg;
         }
         __syncthreads();
-        uint32_t f[4], sum = 0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint32_t i = 4u * tid + k;
-            f[k] = 0;
-            if (i < m) {
-                const uint32_t j = s_nn[i];
-                const bool mutual = j != kNone16 && s_nn[j] == i;
-                f[k] = ((mutual && i < j) ? 1u << 16 : 0u) | ((mutual && j < i) ? 0u : 1u);
-            }
-            sum += f[k];
-        }
+        const bool one_wave = m <= 256;
         uint32_t total = 0;
-        uint32_t run = block_exclusive_sum<kTailThreads>(sum, s_w, total);
-        Box6 ob[4];
-        uint32_t oc[4], on[4], opos[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint32_t i = 4u * tid + k;
-            opos[k] = kNone;
-            if (i < m && (f[k] & 0xFFFFu)) {
-                uint32_t cid = s_c[i], cnt = s_n[i];
-                Box6 b = s_box[i];
-                if (f[k] >> 16) {
-                    const uint32_t j = s_nn[i], id = n_total + (run >> 16);
-                    cnt += s_n[j];
-                    ploc_merge_store(cl, id, cid, s_c[j], cnt, b, s_box[j]);
-                    cid = id;
-                }
-                ob[k] = b;
-                oc[k] = cid;
-                on[k] = cnt;
-                opos[k] = run & 0xFFFFu;
-            }
-            run += f[k];
+        if (m <= 64) {
+            if (tid < 64) total = tail_merge<1, true>(L, tid, m, n_total, cl);
+        } else if (one_wave) {
+            if (tid < 64) total = tail_merge<4, true>(L, tid, m, n_total, cl);
+        } else {
+            total = tail_merge<4, false>(L, tid, m, n_total, cl);
         }
-        __syncthreads();  // every read of this pass's list is done
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (opos[k] != kNone) {
-                s_box[opos[k]] = ob[k];
-                s_c[opos[k]] = oc[k];
-                s_n[opos[k]] = on[k];
-            }
+        if (tid == 0) {
+            s_hdr[0] = total;
+            log[passes] = make_uint4(n_total, total >> 16, m, 0u);
+        }
+        __syncthreads();
+        total = s_hdr[0];
         const uint32_t merges = total >> 16, stays = total & 0xFFFFu;
-        if (tid == 0) log[passes] = make_uint4(n_total, merges, m, 0u);
         if (merges == 0) {  // uniform: no progress, the build reports it
             if (tid == 0) atomicOr(err, kPlocErrNoMerge);
             break;
@@ -887,7 +1062,6 @@ __global__ __launch_bounds__(kTailThreads) void k_ploc_tail(uint32_t* __restrict
         n_total += merges;
         m = stays;
         ++passes;
-        __syncthreads();
     }
     if (tid == 0) {
         state[0] = m;
@@ -1166,7 +1340,8 @@ rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
     const uint32_t T = kPassThreads - 2 * radius;
     const uint32_t max_tiles = (n + T - 1) / T;
     // ctl: kPlocBatch tile counters, then kPlocBatch x max_tiles status words
-    const size_t ctl_words = 2 * kPlocBatch + (size_t)kPlocBatch * max_tiles * 2;
+    constexpr size_t kCtrWords = (size_t)kPlocBatch * kTicketWords;
+    const size_t ctl_words = kCtrWords + (size_t)kPlocBatch * max_tiles * 2;
     uint32_t *ctl = nullptr, *state = nullptr, *err = nullptr, *tail_count = nullptr;
     uint4 *log = nullptr, *tail_log = nullptr;
     RTQ_HIP(ctx, tmp.get(&ctl, ctl_words));
@@ -1189,10 +1364,10 @@ rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
         const uint32_t bound = iter;
         if (iter > kTailMax) {
             const uint32_t tiles = (bound + T - 1) / T;
-            RTQ_HIP(ctx, hipMemsetAsync(ctl, 0, sizeof(uint32_t) * (2ull * kPlocBatch + 2ull * kPlocBatch * tiles), st));
-            uint64_t* status = reinterpret_cast<uint64_t*>(ctl + 2 * kPlocBatch);
+            RTQ_HIP(ctx, hipMemsetAsync(ctl, 0, sizeof(uint32_t) * (kCtrWords + 2ull * kPlocBatch * tiles), st));
+            uint64_t* status = reinterpret_cast<uint64_t*>(ctl + kCtrWords);
             for (uint32_t k = 0; k < kPlocBatch; ++k) {
-                PlocPassArgs a{state + 4 * (k & 1), state + 4 * ((k + 1) & 1), bound, radius, ctl + k,
+                PlocPassArgs a{state + 4 * (k & 1), state + 4 * ((k + 1) & 1), bound, radius, ctl + k * kTicketWords,
                                status + (size_t)k * tiles, err, log + k, lists, cl};
                 hipLaunchKernelGGL(k_ploc_pass, dim3(tiles), dim3(kPassThreads), 0, st, a);
                 RTQ_HIP(ctx, hipGetLastError());
