@@ -8,9 +8,9 @@ namespace rtq {
 namespace {
 
 constexpr int kShadeThreads = 256;
-// BVH overlay stack: a node at depth k < display depth pushes two children, so
-// at most display depth + 1 entries are live.
-constexpr uint32_t kOverlayStack = 64;
+// BVH overlay: a right child waits per level above the display depth, at most
+// 62 of them.
+constexpr uint32_t kOverlayLevels = 63;
 
 // Constants of raytracer.glsl:69-72.
 constexpr float kWireframeWidth = 0.02f;
@@ -51,22 +51,20 @@ __global__ __launch_bounds__(kShadeThreads) void k_shade(const rtq_hit* __restri
 }
 
 // intersectBVH (raytracer.glsl:182-237): 0 miss, 1 hit, 2 hit with the entry
-// point within `threshold` of two slab planes.
+// point within `threshold` of two slab planes.  inv = 1 / d per component.
 __device__ __forceinline__ uint32_t ref_box_hit(float ox, float oy, float oz, float dx, float dy, float dz,
-                                                const rtq_aabb& b, float threshold) {
-    const float inv_x = 1.0f / dx;
+                                                float inv_x, float inv_y, float inv_z, const rtq_aabb& b,
+                                                float threshold) {
     const float tx1 = (b.min[0] - ox) * inv_x;
     const float tx2 = (b.max[0] - ox) * inv_x;
     float tmin = gmin(tx1, tx2);
     float tmax = gmax(tx1, tx2);
     if (tmax < 0.0f || tmin > tmax) return 0;
-    const float inv_y = 1.0f / dy;
     const float ty1 = (b.min[1] - oy) * inv_y;
     const float ty2 = (b.max[1] - oy) * inv_y;
     tmin = gmax(tmin, gmin(ty1, ty2));
     tmax = gmin(tmax, gmax(ty1, ty2));
     if (tmax < 0.0f || tmin > tmax) return 0;
-    const float inv_z = 1.0f / dz;
     const float tz1 = (b.min[2] - oz) * inv_z;
     const float tz2 = (b.max[2] - oz) * inv_z;
     tmin = gmax(tmin, gmin(tz1, tz2));
@@ -79,42 +77,49 @@ __device__ __forceinline__ uint32_t ref_box_hit(float ox, float oy, float oz, fl
     return ((near_x && near_y) || (near_x && near_z) || (near_y && near_z)) ? 2u : 1u;
 }
 
-// One ray per thread; the reference DFS (pop, test, push left then right) cut
-// below the display depth, where nodes no longer change the colour.
+// One ray per thread.  The reference's DFS enters the right child first and
+// the last node it reaches at the display depth sets the colour; that node is
+// the first one a DFS with the left child first reaches, so this walk takes the
+// left child first and ends there (nodes below the display depth cannot change
+// the colour).  A right child waits at its level in LDS, the levels that hold
+// one in a bit mask.  1080p rays on 65,536 triangles at depth 8: 439 us with the
+// reference's order and a stack in scratch, 48 us now.
 __global__ __launch_bounds__(kShadeThreads) void k_bvh_overlay(const rtq_bvh_node* __restrict__ nodes,
                                                                const rtq_ray* __restrict__ rays, uint64_t n,
                                                                uint32_t depth, float threshold,
                                                                float4* __restrict__ out) {
+    extern __shared__ uint32_t s_right[];   // [level of the parent][thread]
     const uint64_t i = (uint64_t)blockIdx.x * kShadeThreads + threadIdx.x;
     if (i >= n) return;
+    uint32_t* const right = s_right + threadIdx.x;
     const float4* rp = reinterpret_cast<const float4*>(rays + i);
     const float4 r0 = rp[0], r1 = rp[1];
-    uint32_t stack[kOverlayStack];
-    uint8_t sdepth[kOverlayStack];
-    uint32_t sp = 0;
-    stack[sp] = 0;
-    sdepth[sp] = 0;
-    ++sp;
+    const float inv_x = 1.0f / r1.x, inv_y = 1.0f / r1.y, inv_z = 1.0f / r1.z;
+    uint32_t cur = 0, d = 0;   // the node to test and its depth
+    uint64_t waiting = 0;      // bit l: a right child waits at level l (its depth is l + 1)
     float4 color = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    while (sp > 0) {
-        --sp;
-        const uint32_t cur = stack[sp];
-        const uint32_t d = sdepth[sp];
+    for (;;) {
         const rtq_bvh_node nd = nodes[cur];
-        const uint32_t h = ref_box_hit(r0.x, r0.y, r0.z, r1.x, r1.y, r1.z, nd.box, threshold);
-        if (h == 0) continue;
-        if (d == depth) {
-            color = h == 2 ? make_float4(0.7f, 0.0f, 0.7f, 0.1f) : make_float4(0.5f, 0.0f, 0.5f, 0.1f);
-            continue;
+        const uint32_t h = ref_box_hit(r0.x, r0.y, r0.z, r1.x, r1.y, r1.z, inv_x, inv_y, inv_z, nd.box, threshold);
+        if (h != 0) {
+            if (d == depth) {
+                color = h == 2 ? make_float4(0.7f, 0.0f, 0.7f, 0.1f) : make_float4(0.5f, 0.0f, 0.5f, 0.1f);
+                break;
+            }
+            if (!(nd.left_child == 0 && nd.right_child == 0)) {
+                // d < depth <= kOverlayLevels - 1 (checked on the host)
+                right[d * kShadeThreads] = nd.right_child;
+                waiting |= 1ull << d;
+                cur = nd.left_child;
+                ++d;
+                continue;
+            }
         }
-        if (nd.left_child == 0 && nd.right_child == 0) continue;
-        // d < depth <= kOverlayStack - 2 (checked on the host), so sp + 2 <= d + 2 fits
-        stack[sp] = nd.left_child;
-        sdepth[sp] = (uint8_t)(d + 1);
-        ++sp;
-        stack[sp] = nd.right_child;
-        sdepth[sp] = (uint8_t)(d + 1);
-        ++sp;
+        if (waiting == 0) break;
+        const uint32_t l = 63u - (uint32_t)__builtin_clzll(waiting);   // the deepest one
+        waiting &= ~(1ull << l);
+        cur = right[l * kShadeThreads];
+        d = l + 1;
     }
     out[i] = color;
 }
@@ -171,14 +176,15 @@ rtq_status rtq_bvh_overlay(rtq_ctx* ctx, uint32_t scene_id, const rtq_ray* rays_
         RTQ_HIP(ctx, hipGetLastError());
         return RTQ_OK;
     }
-    if (depth + 2 > kOverlayStack)
-        return fail(ctx, RTQ_ECAPACITY, "bvh_overlay: depth %u exceeds %u", depth, kOverlayStack - 2);
+    if (depth > kOverlayLevels - 1)
+        return fail(ctx, RTQ_ECAPACITY, "bvh_overlay: depth %u exceeds %u", depth, kOverlayLevels - 1);
     // BVH_LINE_WIDTH / (uDepthDisplayBVH + 1.f), raytracer.glsl:222
     const float threshold = kBvhLineWidth / ((float)depth + 1.0f);
     const rtq_status rs = ensure_ref_nodes(ctx, s, st);
     if (rs != RTQ_OK) return rs;
-    hipLaunchKernelGGL(k_bvh_overlay, dim3(shade_blocks(n)), dim3(kShadeThreads), 0, st, s->ref_nodes, rays_dev, n,
-                       depth, threshold, out);
+    hipLaunchKernelGGL(k_bvh_overlay, dim3(shade_blocks(n)), dim3(kShadeThreads),
+                       sizeof(uint32_t) * kShadeThreads * std::max(depth, 1u), st, s->ref_nodes, rays_dev, n, depth,
+                       threshold, out);
     RTQ_HIP(ctx, hipGetLastError());
     return RTQ_OK;
 }
