@@ -370,6 +370,34 @@ rtq_status ensure_ref_nodes(rtq_ctx* ctx, Scene* s, hipStream_t st);
 rtq_status radix_sort_pairs(rtq_ctx* ctx, uint32_t* keys, uint32_t* vals, uint32_t* tmp_k,
                             uint32_t* tmp_v, uint64_t n, uint32_t key_bits, uint32_t* err, hipStream_t st);
 
+// ---- device helpers shared by the kernels
+
+// Inclusive sum over the wave's 64 lanes (data-parallel primitives: a step per
+// instruction instead of an LDS round trip).
+__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t x) {
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, false);   // row_shr:1
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, false);   // row_shr:2
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, false);   // row_shr:4
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, false);   // row_shr:8
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xA, 0xF, false);   // row_bcast:15
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xC, 0xF, false);   // row_bcast:31
+    return x;
+}
+
+// Tile of this workgroup.  Workgroups are dispatched to the 8 XCDs in turn, and
+// the ones of each XCD number their tiles by a counter of their own: the k-th
+// one to start of those with blockIdx % 8 == x takes tile 8 k + x.  Every tile
+// before it is then taken by a workgroup that was dispatched before or with it
+// (or waits for a slot that only earlier tiles hold), so the look-back's waits
+// end; atomics on one word serialise (about 12 ns each, 50 us for the 4,361
+// tiles of a 2M-triangle terrain's first pass with one counter).
+constexpr uint32_t kTicketStride = 32;             // words between the counters (128 B)
+constexpr uint32_t kTicketWords = 8 * kTicketStride;
+__device__ __forceinline__ uint32_t take_tile(uint32_t* ctr) {
+    const uint32_t x = blockIdx.x & 7u;
+    return 8u * atomicAdd(ctr + x * kTicketStride, 1u) + x;
+}
+
 }  // namespace rtq
 
 #define RTQ_HIP(ctx, call)                                   \
