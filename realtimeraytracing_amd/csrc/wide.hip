@@ -20,6 +20,7 @@
 // (Ylitie, Karras & Laine, "Efficient Incoherent Ray Traversal on GPUs Through
 // Compressed Wide BVHs", HPG 2017, for the quantised-box idea).
 #include <cmath>
+#include <type_traits>
 
 #include "rtq_internal.hpp"
 
@@ -28,12 +29,9 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWidth = 8;
-
-// a child that becomes an 8-wide node of the next level: a merged cluster
-// (ids from nt on) of more than max_leaf triangles
-__device__ __forceinline__ bool expandable(uint32_t c, uint32_t max_leaf, uint32_t nt, const uint32_t* ccount) {
-    return c >= nt && ccount[c] > max_leaf;
-}
+// a level's tile: kLevelNodes nodes of 8 lanes each
+constexpr int kLevelThreads = 512;
+constexpr uint32_t kLevelNodes = kLevelThreads / kWidth;
 
 __device__ __forceinline__ float box_area(const rtq_aabb& b) {
     const float dx = b.max[0] - b.min[0], dy = b.max[1] - b.min[1], dz = b.max[2] - b.min[2];
@@ -169,103 +167,116 @@ __global__ __launch_bounds__(kLdsThreads) void k_dp_lds(const uint2* __restrict_
     }
 }
 
-// The slots of node cluster c as the cost table splits them, children left
-// to right; returns their count.  Clusters below nt are the single triangles
-// (no children), so a step's three loads do not wait for one another.
-__device__ __forceinline__ uint32_t collapse_node(uint32_t c, const uint32_t* __restrict__ cleft,
-                                                  const uint32_t* __restrict__ cright, uint32_t nt,
-                                                  const uint32_t* __restrict__ choice, uint32_t* ch) {
-    uint32_t n = 0;
-    if (c < nt) {
-        ch[n++] = c;  // single-triangle scene: the root itself is the only (leaf) child
-        return n;
-    }
-    const uint32_t kn = ((choice[c - nt] >> 21) & 7u) + 1u;
-    uint32_t sx[kWidth], sj[kWidth];
-    int sp = 0;
-    sx[sp] = cright[c]; sj[sp++] = kWidth - kn;
-    sx[sp] = cleft[c]; sj[sp++] = kn;
-    while (sp > 0) {
-        --sp;
-        const uint32_t x = sx[sp], j = sj[sp];
-        if (j == 1 || x < nt) {
-            ch[n++] = x;
-            continue;
-        }
+// Eight lanes per 8-wide node, one per slot.  A lane's walk from the node's
+// cluster c to the child in slot `slot`, as the cost table splits the slots
+// (children left to right); false if the split leaves the slot empty.  The
+// lanes of one node load the same words, and no lane waits for another: the
+// walk takes as many steps as the slot's child lies below c, where one thread
+// per node takes a step for each cluster opened.
+__device__ __forceinline__ bool slot_child(uint32_t c, uint32_t slot, const uint32_t* __restrict__ cleft,
+                                           const uint32_t* __restrict__ cright, uint32_t nt,
+                                           const uint32_t* __restrict__ choice, uint32_t* child) {
+    uint32_t x = c, j = kWidth, o = slot;   // cluster x fills j slots, this lane's is number o of them
+    bool root = true;
+    while (j > 1 && x >= nt) {
         const uint32_t cw = choice[x - nt], l = cleft[x], r = cright[x];
-        const uint32_t pick = (cw >> (3 * (j - 2))) & 7u;
-        if (pick == 0) {
-            sx[sp] = x; sj[sp++] = j - 1;
+        uint32_t pick;
+        if (root) {
+            pick = ((cw >> 21) & 7u) + 1u;
+            root = false;
         } else {
-            sx[sp] = r; sj[sp++] = j - pick;
-            sx[sp] = l; sj[sp++] = pick;
+            while (j > 1 && (pick = (cw >> (3 * (j - 2))) & 7u) == 0) --j;   // fewer slots: the last ones stay empty
+            if (j == 1) break;
+            if (o >= j) return false;
+        }
+        if (o < pick) {
+            x = l;
+            j = pick;
+        } else {
+            x = r;
+            j -= pick;
+            o -= pick;
         }
     }
-    return n;
+    *child = x;
+    return o == 0;
 }
 
-__device__ int exponent_for(double extent) {
-    // smallest e with 255 * 2^e >= extent, within the normal float range
-    int e = extent > 0.0 ? ilogb(extent) - 7 : -126;
-    if (e < -126) e = -126;
-    while (e < 127 && ldexp(255.0, e) < extent) ++e;
-    while (e > -126 && ldexp(255.0, e - 1) >= extent) --e;
-    return e;
+// Minimum of a value over each 8 lanes, in all of them.
+__device__ __forceinline__ float min_of_8(float x) {
+    const auto dpp = [](float v, auto ctrl) {
+        return __int_as_float(
+            __builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xF, 0xF, false));
+    };
+    x = fminf(x, dpp(x, std::integral_constant<int, 0xB1>{}));    // lanes 1 0 3 2 of each quad
+    x = fminf(x, dpp(x, std::integral_constant<int, 0x4E>{}));    // lanes 2 3 0 1
+    return fminf(x, dpp(x, std::integral_constant<int, 0x141>{}));   // the other quad
 }
 
-// The first four float4 of an 8-wide node with children ch[0..n) in slots
-// 0..n-1: origin and meta (exponents, valid mask), then the x, y and z planes.
-// Child boxes are widened by pad and quantised outward in exact (double)
-// arithmetic, so the decoded box contains the padded child box.
-__device__ void write_wide_boxes(const uint32_t* ch, uint32_t n, const rtq_aabb* __restrict__ cbox, float pad,
-                                 float4* __restrict__ o) {
-    float lo[kWidth][3], hi[kWidth][3];
-    float org[3] = {INFINITY, INFINITY, INFINITY};
-    double top[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (uint32_t i = 0; i < n; ++i) {
-        const rtq_aabb b = cbox[ch[i]];
-        for (int q = 0; q < 3; ++q) {
-            lo[i][q] = b.min[q] - pad;
-            hi[i][q] = b.max[q] + pad;
-            org[q] = fminf(org[q], lo[i][q]);
-            top[q] = fmax(top[q], (double)hi[i][q]);
-        }
-    }
-    int ex[3];
-    double scale[3];
+// Smallest e with 255 * 2^e >= extent, in [-126, 127]: for an extent of
+// m 2^k, 1 <= m < 2, k - 7 if m <= 255 / 128, else k - 6.
+__device__ __forceinline__ int exponent_for(double extent) {
+    if (!(extent > 0.0)) return -126;
+    const uint64_t b = (uint64_t)__double_as_longlong(extent);
+    const int k = (int)(b >> 52) - 1023;
+    const int e = (b & ((1ull << 52) - 1)) <= (127ull << 45) ? k - 7 : k - 6;
+    return e < -126 ? -126 : e > 127 ? 127 : e;
+}
+
+// Words of a node in LDS: 32, and 4 more to spread the nodes over the banks.
+constexpr uint32_t kImageWords = 36;
+
+// The first 16 words of an 8-wide node (origin and meta: exponents and valid
+// mask; then the x, y and z planes) into img, by the node's 8 lanes.  A lane
+// with a child (`has`) gives its slot and box; the others have the slots past
+// the last child, in any order.  Every lane of the wave calls it; live: the
+// lane's node exists.  Child boxes are widened by pad and quantised outward in
+// exact (double) arithmetic, so the decoded box contains the padded child box.
+__device__ __forceinline__ void wide_boxes(bool live, bool has, uint32_t slot, uint32_t n, const rtq_aabb& box,
+                                           float pad, uint32_t* img) {
+    uint8_t* const bytes = reinterpret_cast<uint8_t*>(img);
+    uint32_t meta = n ? ((1u << n) - 1u) << 24 : 0u;
+    float org[3];
+#pragma unroll
     for (int q = 0; q < 3; ++q) {
-        ex[q] = exponent_for(top[q] - (double)org[q]);
-        scale[q] = ldexp(1.0, ex[q]);
-    }
-    uint32_t qlo[3][2] = {{0, 0}, {0, 0}, {0, 0}}, qhi[3][2] = {{0, 0}, {0, 0}, {0, 0}};
-    uint32_t valid = 0;
-    for (uint32_t i = 0; i < n; ++i) {
-        valid |= 1u << i;
-        for (int q = 0; q < 3; ++q) {
-            // exact: float differences and division by a power of two are exact in double
-            double l = floor(((double)lo[i][q] - (double)org[q]) / scale[q]);
-            double h = ceil(((double)hi[i][q] - (double)org[q]) / scale[q]);
-            l = fmin(fmax(l, 0.0), 255.0);
-            h = fmin(fmax(h, 0.0), 255.0);
-            qlo[q][i >> 2] |= (uint32_t)l << (8 * (i & 3));
-            qhi[q][i >> 2] |= (uint32_t)h << (8 * (i & 3));
+        const float lo = has ? box.min[q] - pad : INFINITY;
+        const float hi = has ? box.max[q] + pad : -INFINITY;
+        org[q] = min_of_8(lo);
+        const float top = -min_of_8(-hi);
+        const int e = exponent_for((double)top - (double)org[q]);
+        meta |= (uint32_t)(e + 127) << (8 * q);
+        // exact: float differences and products with a power of two (2^-e is a
+        // normal double) are exact in double
+        const double inv = __longlong_as_double((int64_t)(1023 - e) << 52);
+        const double l = fmin(fmax(floor(((double)lo - (double)org[q]) * inv), 0.0), 255.0);
+        const double h = fmin(fmax(ceil(((double)hi - (double)org[q]) * inv), 0.0), 255.0);
+        // empty slots: an inverted box (lower planes 255, upper 0) that a ray
+        // misses on every axis unless its origin lies more than 2^19 node
+        // extents away; their child ref is then harmless (one triangle test,
+        // see the level kernel), so traversal needs no test of the valid bits
+        if (live) {
+            bytes[16 * (q + 1) + slot] = has ? (uint8_t)(uint32_t)l : (uint8_t)0xFF;
+            bytes[16 * (q + 1) + 8 + slot] = has ? (uint8_t)(uint32_t)h : (uint8_t)0;
         }
     }
-    // empty slots: an inverted box (lower planes 255, upper 0) that a ray
-    // misses on every axis unless its origin lies more than 2^19 node extents
-    // away; their child ref is then harmless (one triangle test, see the
-    // level kernel), so traversal needs no test of the valid bits
-    for (uint32_t i = n; i < kWidth; ++i)
-        for (int q = 0; q < 3; ++q) qlo[q][i >> 2] |= 0xFFu << (8 * (i & 3));
-    const uint32_t meta = (uint32_t)(ex[0] + 127) | ((uint32_t)(ex[1] + 127) << 8) |
-                          ((uint32_t)(ex[2] + 127) << 16) | (valid << 24);
-    o[0] = make_float4(org[0], org[1], org[2], __uint_as_float(meta));
-    o[1] = make_float4(__uint_as_float(qlo[0][0]), __uint_as_float(qlo[0][1]), __uint_as_float(qhi[0][0]),
-                       __uint_as_float(qhi[0][1]));
-    o[2] = make_float4(__uint_as_float(qlo[1][0]), __uint_as_float(qlo[1][1]), __uint_as_float(qhi[1][0]),
-                       __uint_as_float(qhi[1][1]));
-    o[3] = make_float4(__uint_as_float(qlo[2][0]), __uint_as_float(qlo[2][1]), __uint_as_float(qhi[2][0]),
-                       __uint_as_float(qhi[2][1]));
+    if (live && slot == 0) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) img[q] = __float_as_uint(org[q]);
+        img[3] = meta;
+    }
+}
+
+// Float4 i of a node's image, after the wave's writes to it.
+__device__ __forceinline__ float4 image_part(const uint32_t* img, uint32_t i) {
+    const uint4 w = reinterpret_cast<const uint4*>(img)[i];
+    return make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w));
+}
+
+// Orders a wave's LDS writes before its later LDS reads.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Tile status of the level scan: value in the low 32 bits, state on top.
@@ -277,7 +288,9 @@ constexpr uint32_t kLvSpinLimit = 1u << 24;
 enum : uint32_t { kWideErrOverflow = 1, kWideErrScan = 2 };
 
 struct LevelArgs {
-    uint32_t* lv;              // this level's words: count, first node, first status word, tile ticket
+    uint32_t* lv;              // this level's words: count, first node, first status word, unused
+    uint32_t* tickets;         // tile counters of this level, zero before it
+    uint32_t* next_tickets;    // of the next one
     uint64_t* status;          // tile status words, n_status of them, zero before the first level
     uint32_t n_status;
     uint32_t cap;              // node capacity
@@ -300,53 +313,59 @@ struct LevelArgs {
     uint32_t* kids;            // 8 child clusters per node (kNone past the last)
 };
 
-// One level of the collapse in one launch.  Each thread takes one node of the
-// level and picks its slots; the next level's nodes are numbered by an
+// One level of the collapse in one launch, eight lanes per node of the level:
+// each lane finds its slot's child; the next level's nodes are numbered by an
 // exclusive scan of the nodes' expandable children in node order, across
-// workgroups by decoupled look-back (tiles numbered in the order workgroups
-// start, so every tile waited on is running; the wait is bounded and a tile
-// that gives up poisons its status and sets an error bit); then the thread
-// writes its node.  The last tile writes the next level's words (lv[4..7]).
-// The grid covers an upper bound of the level's count; workgroups past the
-// count, and every workgroup of an empty level, return at once.
-__global__ __launch_bounds__(kThreads) void k_wide_level(LevelArgs a) {
-    __shared__ uint32_t s_tile, s_excl, s_bad, s_w[kThreads / 64];
+// workgroups by decoupled look-back (see take_tile; the wait is bounded and a
+// tile that gives up poisons its status and sets an error bit); then each lane
+// quantises its child's box and the lanes of a node write its 128 B together.
+// The last tile writes the next level's words (lv[4..6]).  The grid covers an
+// upper bound of the level's count; workgroups past the count, and every
+// workgroup of an empty level, return at once.
+// The chain of dependent loads down to a slot's child bounds small levels, the
+// children's scattered boxes large ones.  2,095,104 triangles, 12 levels: 354 us
+// with one thread per node (its walk, boxes and quantisation one child after
+// another), 171 us now; a level of a few nodes 20 us and 6 us.
+__global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
+    constexpr uint32_t kWaves = kLevelThreads / 64;
+    __shared__ uint32_t s_tile, s_excl, s_bad, s_w[kWaves];
+    __shared__ __align__(16) uint32_t s_img[kLevelNodes * kImageWords];
     const uint32_t count = a.lv[0];
-    const uint32_t tiles = (count + kThreads - 1) / kThreads;
+    const uint32_t tiles = (count + kLevelNodes - 1) / kLevelNodes;
     if (blockIdx.x >= tiles) return;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    if (tid == 0) s_tile = atomicAdd(a.lv + 3, 1u);
+    if (tid == 0) s_tile = take_tile(a.tickets);
+    if (blockIdx.x == 0 && tid >= 64 && tid < 72) a.next_tickets[(tid - 64) * kTicketStride] = 0;
     __syncthreads();
     const uint32_t tile = s_tile;
-    const uint32_t k = tile * kThreads + tid;
+    const uint32_t k = tile * kLevelNodes + tid / kWidth;
     const uint32_t level_base = a.lv[1], sbase = a.lv[2];
+    const bool live = k < count;
 
-    uint32_t ch[kWidth];
-    uint32_t n = 0, ne = 0, expand = 0;
-    if (k < count) {
-        n = collapse_node(a.items[k], a.cleft, a.cright, a.nt, a.choice, ch);
-        for (uint32_t i = 0; i < n; ++i)
-            if (expandable(ch[i], a.max_leaf, a.nt, a.ccount)) {
-                expand |= 1u << i;
-                ++ne;
-            }
-    }
-    // exclusive sum of ne over the workgroup
-    uint32_t x = ne;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = __shfl_up(x, d, 64);
-        if ((int)lane >= d) x += y;
-    }
-    if (lane == 63) s_w[wave] = x;
+    // the children take the slots 0..n-1 in order, the lanes without one the rest
+    const uint32_t c0 = live ? a.items[k] : 0u;
+    uint32_t c = 0;
+    const bool has = live && slot_child(c0, tid % kWidth, a.cleft, a.cright, a.nt, a.choice, &c);
+    const uint32_t group = lane & ~(kWidth - 1u);
+    const uint32_t mask = (uint32_t)(__ballot(has) >> group) & 0xFFu;
+    const uint32_t below = (1u << (lane - group)) - 1u;
+    const uint32_t n = __popc(mask);
+    const uint32_t slot = has ? __popc(mask & below) : n + __popc(~mask & below);
+    const uint32_t cnt = has ? a.ccount[c] : 0u;
+    const rtq_aabb box = a.cbox[c];
+    const uint32_t first = has ? a.fl[c] : 0u;
+    const bool expand = has && c >= a.nt && cnt > a.max_leaf;   // an 8-wide node of the next level
+    // exclusive sum of the expandable children over the workgroup
+    const uint64_t em = __ballot(expand);
+    const uint32_t in_wave = __builtin_amdgcn_mbcnt_hi((uint32_t)(em >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)em, 0u));
+    if (lane == 0) s_w[wave] = (uint32_t)__popcll(em);
     __syncthreads();
     uint32_t wave_off = 0, total = 0;
 #pragma unroll
-    for (uint32_t w = 0; w < kThreads / 64; ++w) {
+    for (uint32_t w = 0; w < kWaves; ++w) {
         if (w < wave) wave_off += s_w[w];
         total += s_w[w];
     }
-    const uint32_t local = wave_off + x - ne;
 
     // counts before this tile: decoupled look-back by wave 0
     if (wave == 0) {
@@ -413,46 +432,36 @@ __global__ __launch_bounds__(kThreads) void k_wide_level(LevelArgs a) {
         a.lv[4] = next_count;
         a.lv[5] = next_base;
         a.lv[6] = sbase + tiles;
-        a.lv[7] = 0u;
     }
-    if (k >= count) return;
 
-    // the node: children boxes quantised outward against the node's origin
-    // the binary traversal node of this node's root cluster (learned order)
-    a.wide_trav[level_base + k] = a.bidx ? a.bidx[a.pos[a.items[k]]] : kNone;
-    float4* o = a.nodes + 8ull * (level_base + k);
-    write_wide_boxes(ch, n, a.cbox, a.pad, o);
-    uint32_t ref[kWidth];
-    uint32_t rank = 0;
-    for (uint32_t i = 0; i < kWidth; ++i) {
-        // an empty slot's box is inverted (write_wide_boxes); should a far ray
-        // still enter it, its ref is the leaf of traversal triangle 0 alone:
-        // a real triangle, so whatever that test reports is a genuine hit
-        ref[i] = leaf_ref(0u, 1u);
-        if (i >= n) continue;
-        const uint32_t c = ch[i];
-        if ((expand >> i) & 1u) {
-            const uint32_t slot = excl + local + rank++;
-            ref[i] = next_base + slot;
-            if ((uint64_t)next_base + slot < a.cap) {
-                a.next_items[slot] = c;
-            } else {
-                atomicOr(a.err, kWideErrOverflow);
-            }
+    uint32_t* const img = s_img + (tid / kWidth) * kImageWords;
+    wide_boxes(live, has, slot, n, box, a.pad, img);
+    // an empty slot's box is inverted (wide_boxes); should a far ray still enter
+    // it, its ref is the leaf of traversal triangle 0 alone: a real triangle, so
+    // whatever that test reports is a genuine hit
+    uint32_t ref = leaf_ref(0u, 1u);
+    if (expand) {
+        const uint32_t to = excl + wave_off + in_wave;
+        ref = next_base + to;
+        if ((uint64_t)next_base + to < a.cap) {
+            a.next_items[to] = c;
         } else {
-            ref[i] = leaf_ref(a.fl[c], a.ccount[c]);
+            atomicOr(a.err, kWideErrOverflow);
         }
+    } else if (has) {
+        ref = leaf_ref(first, cnt);
     }
-    o[4] = make_float4(__uint_as_float(ref[0]), __uint_as_float(ref[1]), __uint_as_float(ref[2]),
-                       __uint_as_float(ref[3]));
-    o[5] = make_float4(__uint_as_float(ref[4]), __uint_as_float(ref[5]), __uint_as_float(ref[6]),
-                       __uint_as_float(ref[7]));
-    o[6] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    o[7] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    // the node's child clusters, for a refit
-    uint4* kid = reinterpret_cast<uint4*>(a.kids + 8ull * (level_base + k));
-    kid[0] = make_uint4(ch[0], n > 1 ? ch[1] : kNone, n > 2 ? ch[2] : kNone, n > 3 ? ch[3] : kNone);
-    kid[1] = make_uint4(n > 4 ? ch[4] : kNone, n > 5 ? ch[5] : kNone, n > 6 ? ch[6] : kNone, n > 7 ? ch[7] : kNone);
+    if (live) {
+        img[16 + slot] = ref;
+        img[24 + slot] = 0;
+        // the node's child clusters, for a refit
+        a.kids[8ull * (level_base + k) + slot] = has ? c : kNone;
+        // the binary traversal node of this node's root cluster (learned order)
+        if (slot == 0) a.wide_trav[level_base + k] = a.bidx ? a.bidx[a.pos[c0]] : kNone;
+    }
+    wave_lds_fence();
+    if (live)
+        a.nodes[8ull * (level_base + k) + tid % kWidth] = image_part(img, tid % kWidth);
 }
 
 // New boxes for the kept 8-wide nodes after a refit: each node's child
@@ -461,16 +470,21 @@ __global__ __launch_bounds__(kThreads) void k_wide_level(LevelArgs a) {
 __global__ __launch_bounds__(kThreads) void k_wide_refit(uint32_t n_wide, const uint32_t* __restrict__ kids,
                                                          const rtq_aabb* __restrict__ cbox, float pad,
                                                          float4* __restrict__ nodes) {
-    const uint32_t k = blockIdx.x * kThreads + threadIdx.x;
-    if (k >= n_wide) return;
-    const uint4* kp = reinterpret_cast<const uint4*>(kids + 8ull * k);
-    const uint4 k0 = kp[0], k1 = kp[1];
-    const uint32_t ch[kWidth] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
-    uint32_t n = 0;
-    while (n < kWidth && ch[n] != kNone) ++n;
-    float4* o = nodes + 8ull * k;
-    write_wide_boxes(ch, n, cbox, pad, o);
-    o[6] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    __shared__ __align__(16) uint32_t s_img[kThreads / kWidth * kImageWords];
+    const uint32_t tid = threadIdx.x, slot = tid % kWidth;
+    const uint32_t k = blockIdx.x * (kThreads / kWidth) + tid / kWidth;
+    const bool live = k < n_wide;
+    const uint32_t c = live ? kids[8ull * k + slot] : kNone;
+    const bool has = c != kNone;
+    const uint32_t group = tid & 63u & ~(kWidth - 1u);
+    const uint32_t n = __popc((uint32_t)(__ballot(has) >> group) & 0xFFu);
+    const rtq_aabb box = cbox[has ? c : 0u];
+    uint32_t* const img = s_img + (tid / kWidth) * kImageWords;
+    wide_boxes(live, has, slot, n, box, pad, img);
+    if (live) img[24 + slot] = 0;
+    wave_lds_fence();
+    if (live && (slot < 4 || slot == 6))
+        nodes[8ull * k + slot] = image_part(img, slot);
 }
 
 __global__ void k_set_u32(uint32_t* p, uint32_t v) { *p = v; }
@@ -517,11 +531,15 @@ rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const uint
     RTQ_HIP(ctx, tmp.get(&items, cap));
     RTQ_HIP(ctx, tmp.get(&next, cap));
     // tile status words of every level's scan: a level of c nodes takes
-    // ceil(c / kThreads) of them, and there are at most depth + 1 levels
-    const uint32_t n_status = cap / kThreads + s->depth + 2;
+    // ceil(c / kLevelNodes) of them, and there are at most depth + 1 levels
+    const uint32_t n_status = cap / kLevelNodes + s->depth + 2;
     uint64_t* status = nullptr;
-    RTQ_HIP(ctx, tmp.get(&status, n_status));
-    RTQ_HIP(ctx, hipMemsetAsync(status, 0, sizeof(uint64_t) * n_status, st));
+    // and before them two sets of tile counters: a level clears the next one's
+    constexpr uint32_t kTickets = 2 * kTicketWords / 2;
+    RTQ_HIP(ctx, tmp.get(&status, (size_t)kTickets + n_status));
+    RTQ_HIP(ctx, hipMemsetAsync(status, 0, sizeof(uint64_t) * (kTickets + n_status), st));
+    uint32_t* const tickets = reinterpret_cast<uint32_t*>(status);
+    status += kTickets;
     // a refit writes the same buffer again (its size depends on the topology only)
     if (!s->wide) RTQ_HIP(ctx, take(s->kept_wide, &s->wide, 8ull * cap));
     if (!s->wide_trav) RTQ_HIP(ctx, take(s->kept_wide_trav, &s->wide_trav, cap));
@@ -530,10 +548,11 @@ rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const uint
     hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, st, items, root);
     RTQ_HIP(ctx, hipGetLastError());
     // levels top-down, one launch each, kLevelsPerRead of them between host
-    // reads: a level's words (count, first node, first status word, ticket)
+    // reads: a level's words (count, first node, first status word)
     // stay on the device, its launch covers an upper bound of its count (8
     // children per node, at most cap nodes)
     constexpr uint32_t kLevelsPerRead = 6;
+    static_assert(kLevelsPerRead % 2 == 0, "the levels of a group start with the first set of tile counters");
     constexpr uint32_t kLvWords = 4 * (kLevelsPerRead + 1);
     uint32_t* lvl = nullptr;
     RTQ_HIP(ctx, tmp.get(&lvl, kLvWords + 1));
@@ -570,7 +589,10 @@ rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const uint
             la.lv = lvl + 4 * g;
             la.items = items;
             la.next_items = next;
-            hipLaunchKernelGGL(k_wide_level, dim3(blocks_for(ub)), dim3(kThreads), 0, st, la);
+            la.tickets = tickets + (g & 1u) * kTicketWords;
+            la.next_tickets = tickets + (~g & 1u) * kTicketWords;
+            hipLaunchKernelGGL(k_wide_level, dim3((uint32_t)((ub + kLevelNodes - 1) / kLevelNodes)),
+                               dim3(kLevelThreads), 0, st, la);
             RTQ_HIP(ctx, hipGetLastError());
             std::swap(items, next);
             ub = std::min<uint64_t>(8 * ub, cap);
@@ -598,7 +620,7 @@ rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const uint
 rtq_status refit_wide(rtq_ctx* ctx, Scene* s, hipStream_t st) {
     if (!s->wide || !s->wide_kids) return fail(ctx, RTQ_EINTERNAL, "refit: the scene has no 8-wide nodes");
     if (s->n_wide == 0) return RTQ_OK;
-    hipLaunchKernelGGL(k_wide_refit, dim3(blocks_for(s->n_wide)), dim3(kThreads), 0, st, s->n_wide, s->wide_kids,
+    hipLaunchKernelGGL(k_wide_refit, dim3(blocks_for(8ull * s->n_wide)), dim3(kThreads), 0, st, s->n_wide, s->wide_kids,
                        s->cbox, s->box_pad, s->wide);
     RTQ_HIP(ctx, hipGetLastError());
     s->wide_ordered = false;   // the tables were cleared
