@@ -61,6 +61,7 @@ void reset_build(Scene* s) {
     s->wide_ordered = false;
     s->d_passes = nullptr;
     s->lds_from = 0;
+    s->sub_from = 0;
     s->n_top = 0;
     s->built = false;
     s->stale = false;
@@ -101,6 +102,8 @@ void free_build(Scene* s) {
     release(s->preorder);
     release(s->first_leaf);
     release(s->node_depth);
+    release(s->sub_roots);
+    release(s->sub_list);
     release(s->trav_index);
     release(s->top);
     release(s->tris);

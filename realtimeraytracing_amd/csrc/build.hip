@@ -69,25 +69,39 @@ __global__ __launch_bounds__(kThreads) void k_refit_leaves(const rtq_triangle* _
     cbox[i] = a;
 }
 
-// Merged clusters [first, first + count) of one PLOC pass: the box is the
-// merge of the children's (left operand first, as k_ploc_merge).
-__device__ __forceinline__ void refit_merge_one(uint32_t id, const uint32_t* __restrict__ cleft,
-                                                const uint32_t* __restrict__ cright, rtq_aabb* __restrict__ cbox) {
-    const rtq_aabb l = cbox[cleft[id]], r = cbox[cright[id]];
+// A merged cluster's box: the merge of the children's (left operand first, as
+// k_ploc_merge).
+__device__ __forceinline__ rtq_aabb merged_box(const rtq_aabb& l, const rtq_aabb& r) {
     rtq_aabb a{};
     for (int k = 0; k < 3; ++k) {
         a.min[k] = smin(l.min[k], r.min[k]);
         a.max[k] = smax(l.max[k], r.max[k]);
     }
-    cbox[id] = a;
+    return a;
 }
 
+// Merged clusters [first, first + count) of one PLOC pass.
 __global__ __launch_bounds__(kThreads) void k_refit_merge(uint32_t first, uint32_t count,
                                                           const uint32_t* __restrict__ cleft,
                                                           const uint32_t* __restrict__ cright,
                                                           rtq_aabb* __restrict__ cbox) {
     const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-    if (i < count) refit_merge_one(first + i, cleft, cright, cbox);
+    if (i < count) cbox[first + i] = merged_box(cbox[cleft[first + i]], cbox[cright[first + i]]);
+}
+
+// The boxes of one middle subtree per workgroup (one wave), the deepest level
+// first, from the list its placement left.  260,642 triangles with 17 passes
+// below the top ones: a refit and its rays 292 us with a launch per pass, 263 us
+// now.
+__global__ __launch_bounds__(kSubThreads) void k_refit_subtrees(const uint2* __restrict__ roots,
+                                                                const uint32_t* __restrict__ list,
+                                                                const uint32_t* __restrict__ fl,
+                                                                const uint32_t* __restrict__ cleft,
+                                                                const uint32_t* __restrict__ cright, rtq_aabb* cbox) {
+    if (blockIdx.x >= roots[0].x) return;
+    const uint2 root = roots[1 + blockIdx.x];
+    levels_up(list + fl[root.x], root.y,
+              [&](uint32_t c) { cbox[c] = merged_box(cbox[cleft[c]], cbox[cright[c]]); });
 }
 
 // The passes [k0, k1) at the top of the tree in one workgroup, in build order,
@@ -118,12 +132,7 @@ __global__ __launch_bounds__(kLdsThreads) void k_refit_merge_lds(const uint2* __
             if (idx >= R || c < p.x || c >= p.x + p.y) continue;
             const rtq_aabb l = L[q] >= c_lo ? s_box[L[q] - c_lo] : cbox[L[q]];
             const rtq_aabb r = Rc[q] >= c_lo ? s_box[Rc[q] - c_lo] : cbox[Rc[q]];
-            rtq_aabb m{};
-            for (int d = 0; d < 3; ++d) {   // the merge of refit_merge_one
-                m.min[d] = smin(l.min[d], r.min[d]);
-                m.max[d] = smax(l.max[d], r.max[d]);
-            }
-            s_box[idx] = m;
+            s_box[idx] = merged_box(l, r);
         }
         __syncthreads();
     }
@@ -1044,12 +1053,6 @@ __global__ __launch_bounds__(kTailThreads) void k_ploc_tail(uint32_t* __restrict
     }
 }
 
-__global__ void k_root_init(uint32_t root, uint32_t* pos, uint32_t* fl, uint32_t* dep) {
-    pos[root] = 0;
-    fl[root] = 0;
-    dep[root] = 0;
-}
-
 __device__ __forceinline__ void place_one(uint32_t p, const uint32_t* __restrict__ cleft,
                                           const uint32_t* __restrict__ cright, const uint32_t* __restrict__ ccount,
                                           uint32_t* __restrict__ pos, uint32_t* __restrict__ fl,
@@ -1080,22 +1083,94 @@ __global__ __launch_bounds__(kThreads) void k_place_pass(uint32_t first, uint32_
     if (k < count) place_one(first + k, cleft, cright, ccount, pos, fl, dep);
 }
 
+// The middle subtrees' clusters (from c_mid on), level by level from the root,
+// one subtree per workgroup (one wave).  A level's clusters come with their state
+// from the lanes that placed them, through LDS while they fit, else from the
+// list and the arrays.  A subtree's list of clusters takes its first-leaf range
+// of `list`; the order within a level is free, no result depends on it.
+constexpr uint32_t kFront = 256;
+
+__global__ __launch_bounds__(kSubThreads) void k_place_subtrees(uint2* roots, uint32_t c_mid,
+                                                                const uint32_t* __restrict__ cleft,
+                                                                const uint32_t* __restrict__ cright,
+                                                                const uint32_t* __restrict__ ccount, uint32_t* pos,
+                                                                uint32_t* fl, uint32_t* dep, uint32_t* list_base) {
+    __shared__ uint4 s_front[2][kFront];
+    if (blockIdx.x >= roots[0].x) return;
+    const uint32_t lane = threadIdx.x;
+    const uint32_t root = roots[1 + blockIdx.x].x;
+    const uint32_t root_fl = fl[root];
+    uint32_t* const list = list_base + root_fl;
+    if (lane == 0) {
+        s_front[0][0] = make_uint4(root, pos[root], root_fl, dep[root]);
+        list[0] = root | kLevelStart;
+    }
+    __syncthreads();
+    uint32_t begin = 0, end = 1;
+    for (uint32_t k = 0; begin < end; ++k) {
+        const uint4* const front = s_front[k & 1u];
+        uint4* const next = s_front[~k & 1u];
+        uint32_t n_next = 0;
+        for (uint32_t e0 = begin; e0 < end; e0 += kSubThreads) {
+            const uint32_t e = e0 + lane;
+            uint4 f = make_uint4(0, 0, 0, 0);
+            uint32_t l = 0, r = 0, lc = 0;
+            if (e < end) {
+                if (e - begin < kFront) {
+                    f = front[e - begin];
+                } else {
+                    f.x = list[e] & ~kLevelStart;
+                    f.y = pos[f.x];
+                    f.z = fl[f.x];
+                    f.w = dep[f.x];
+                }
+                l = cleft[f.x];
+                r = cright[f.x];
+                lc = ccount[l];
+                pos[l] = f.y + 1;
+                pos[r] = f.y + 2 * lc;
+                fl[l] = f.z;
+                fl[r] = f.z + lc;
+                dep[l] = f.w + 1;
+                dep[r] = f.w + 1;
+            }
+            // children of the middle passes to the next level
+            const bool bl = l >= c_mid, br = r >= c_mid;
+            const uint64_t ml = __ballot(bl), mr = __ballot(br);
+            const uint64_t below = (1ull << lane) - 1u;
+            const auto put = [&](uint32_t i, uint32_t c, uint32_t p, uint32_t first) {
+                list[end + i] = i == 0 ? c | kLevelStart : c;
+                if (i < kFront) next[i] = make_uint4(c, p, first, f.w + 1);
+            };
+            if (bl) put(n_next + (uint32_t)__popcll(ml & below), l, f.y + 1, f.z);
+            n_next += (uint32_t)__popcll(ml);
+            if (br) put(n_next + (uint32_t)__popcll(mr & below), r, f.y + 2 * lc, f.z + lc);
+            n_next += (uint32_t)__popcll(mr);
+        }
+        __syncthreads();
+        begin = end;
+        end += n_next;
+    }
+    if (lane == 0) roots[1 + blockIdx.x].y = end;
+}
+
 // The passes [k0, k1) at the top of the tree in one workgroup, last pass
 // first, with the placement state (position, first leaf, depth) of their
 // clusters [c_lo, nc) in LDS: a pass reads and writes LDS only, a barrier
 // between passes.  Children from earlier passes get their state in global
-// memory; the clusters of the range write theirs back at the end.  Each
+// memory, and those from c_mid on are the roots of the middle subtrees, listed
+// in roots; the clusters of the range write their state back at the end.  Each
 // thread keeps the child ids and left-child triangle counts of its clusters
-// c_lo + t + kLdsThreads * s in registers.  nc - c_lo <= kLdsClusters.
+// c_lo + t + kLdsThreads * s in registers.  1 <= nc - c_lo <= kLdsClusters.
 __global__ __launch_bounds__(kLdsThreads) void k_place_lds(const uint2* __restrict__ passes, uint32_t k0, uint32_t k1,
-                                                           uint32_t c_lo, uint32_t nc,
+                                                           uint32_t c_lo, uint32_t nc, uint32_t c_mid,
                                                            const uint32_t* __restrict__ cleft,
                                                            const uint32_t* __restrict__ cright,
                                                            const uint32_t* __restrict__ ccount,
                                                            uint32_t* __restrict__ pos, uint32_t* __restrict__ fl,
-                                                           uint32_t* __restrict__ dep) {
+                                                           uint32_t* __restrict__ dep, uint2* __restrict__ roots) {
     constexpr int kSlots = kLdsClusters / kLdsThreads;
-    __shared__ uint32_t s_pos[kLdsClusters], s_fl[kLdsClusters], s_dep[kLdsClusters];
+    __shared__ uint32_t s_pos[kLdsClusters], s_fl[kLdsClusters], s_dep[kLdsClusters], s_roots;
     const uint32_t t = threadIdx.x;
     const uint32_t R = nc - c_lo;
     uint32_t L[kSlots], Rc[kSlots], LC[kSlots];
@@ -1106,11 +1181,12 @@ __global__ __launch_bounds__(kLdsThreads) void k_place_lds(const uint2* __restri
         Rc[q] = idx < R ? cright[c_lo + idx] : 0u;
     }
 #pragma unroll
-    for (int q = 0; q < kSlots; ++q) LC[q] = t + kLdsThreads * q < R ? ccount[L[q]] : 0u;
+    for (int q = 0; q < kSlots; ++q) LC[q] = L[q] < nc && t + kLdsThreads * q < R ? ccount[L[q]] : 0u;
     if (t == 0) {  // the root, the last cluster
-        s_pos[R - 1] = pos[nc - 1];
-        s_fl[R - 1] = fl[nc - 1];
-        s_dep[R - 1] = dep[nc - 1];
+        s_pos[R - 1] = 0;
+        s_fl[R - 1] = 0;
+        s_dep[R - 1] = 0;
+        s_roots = 0;
     }
     __syncthreads();
     for (uint32_t k = k1; k > k0; --k) {
@@ -1138,12 +1214,23 @@ __global__ __launch_bounds__(kLdsThreads) void k_place_lds(const uint2* __restri
 #pragma unroll
     for (int q = 0; q < kSlots; ++q) {
         const uint32_t idx = t + kLdsThreads * q;
-        if (idx < R) {
+        const bool in = idx < R;
+        if (in) {
             pos[c_lo + idx] = s_pos[idx];
             fl[c_lo + idx] = s_fl[idx];
             dep[c_lo + idx] = s_dep[idx];
         }
+        const bool bl = in && L[q] >= c_mid && L[q] < c_lo, br = in && Rc[q] >= c_mid && Rc[q] < c_lo;
+        const uint64_t ml = __ballot(bl), mr = __ballot(br);
+        uint32_t at = 0;
+        if ((t & 63u) == 0 && (ml | mr)) at = atomicAdd(&s_roots, (uint32_t)(__popcll(ml) + __popcll(mr)));
+        at = 1u + (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+        const uint64_t below = (1ull << (t & 63u)) - 1u;
+        if (bl) roots[at + __popcll(ml & below)] = make_uint2(L[q], 0u);
+        if (br) roots[at + __popcll(ml) + __popcll(mr & below)] = make_uint2(Rc[q], 0u);
     }
+    __syncthreads();
+    if (t == 0) roots[0] = make_uint2(s_roots, 0u);
 }
 
 // Leaf-ordered traversal triangles, and the depth of each workgroup's deepest
@@ -1510,6 +1597,8 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipSt
     if (!s->preorder) RTQ_HIP(ctx, dev_alloc(&s->preorder, nc));
     if (!s->first_leaf) RTQ_HIP(ctx, dev_alloc(&s->first_leaf, nc));
     if (!s->node_depth) RTQ_HIP(ctx, dev_alloc(&s->node_depth, nc));
+    if (!s->sub_roots) RTQ_HIP(ctx, dev_alloc(&s->sub_roots, kLdsClusters + 2));
+    if (!s->sub_list) RTQ_HIP(ctx, dev_alloc(&s->sub_list, n));
     // so is every cluster's traversal node index: a refit needs no new marks
     if (!s->trav_index) RTQ_HIP(ctx, dev_alloc(&s->trav_index, nc));
     uint32_t* const pos = s->preorder;
@@ -1523,47 +1612,46 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipSt
     RTQ_HIP(ctx, tmp.get(&flag, nc));
     RTQ_HIP(ctx, tmp.get(&ntrav, 1));
     const uint32_t root = nc - 1;
-    // The 8-wide collapse's cost table reads the clusters only: it runs on the
-    // second stream beside the placement and the binary nodes, its launches
-    // queued between the placement's so that both streams start at once.
     float* wcost = nullptr;
     uint32_t* wchoice = nullptr;
     SideWork side(ctx);
-    const uint32_t dp_steps = s->params.node_width == 8 && !refit ? wide_cost_steps(s) : 0u;
-    uint32_t dp_next = 0;
-    auto queue_cost = [&](uint32_t upto) -> rtq_status {
-        upto = std::min(upto, dp_steps);
-        if (dp_next >= upto) return RTQ_OK;
-        const rtq_status r = wide_cost_table(ctx, s, wcost, wchoice, dp_next, upto, ctx->side);
-        dp_next = upto;
-        return r;
-    };
-    if (dp_steps) {
-        RTQ_HIP(ctx, tmp.get(&wcost, (size_t)(nc - n) * 8));
-        RTQ_HIP(ctx, tmp.get(&wchoice, nc - n));
-        RTQ_HIP(ctx, side.fork(st));
-    }
     rtq_status rs = RTQ_OK;
     if (!refit) {
-        hipLaunchKernelGGL(k_root_init, dim3(1), dim3(1), 0, st, root, pos, fl, dep);
-        RTQ_HIP(ctx, hipGetLastError());
-        // the passes at the top of the tree in one launch (their clusters'
-        // state in LDS), then one launch per larger pass, last pass first
         const uint32_t n_passes = (uint32_t)s->passes.size();
-        if (s->lds_from < n_passes) {
-            hipLaunchKernelGGL(k_place_lds, dim3(1), dim3(kLdsThreads), 0, st, s->d_passes, s->lds_from, n_passes,
-                               s->passes[s->lds_from].first, nc, s->cleft, s->cright, s->ccount, pos, fl, dep);
+        const bool cost = s->params.node_width == 8 && n > 1;
+        if (cost) {
+            RTQ_HIP(ctx, tmp.get(&wcost, (size_t)(nc - n) * 8));
+            RTQ_HIP(ctx, tmp.get(&wchoice, nc - n));
+        }
+        // the passes at the top of the tree in one launch (their clusters'
+        // state in LDS), then the middle subtrees, then the larger passes, last
+        // pass first; the collapse's cost table the other way round on the
+        // second stream, where it waits for the subtrees' lists
+        const uint32_t c_lo = n_passes ? s->passes[s->lds_from].first : nc - 1;
+        const uint32_t c_mid = s->sub_from < s->lds_from ? s->passes[s->sub_from].first : c_lo;
+        if (cost) RTQ_HIP(ctx, side.fork(st));
+        hipLaunchKernelGGL(k_place_lds, dim3(1), dim3(kLdsThreads), 0, st, s->d_passes, s->lds_from, n_passes, c_lo,
+                           nc, c_mid, s->cleft, s->cright, s->ccount, pos, fl, dep, s->sub_roots);
+        RTQ_HIP(ctx, hipGetLastError());
+        if (cost) {
+            rs = wide_cost_bottom(ctx, s, wcost, wchoice, ctx->side);
+            if (rs != RTQ_OK) return rs;
+        }
+        if (c_mid < c_lo) {
+            hipLaunchKernelGGL(k_place_subtrees, dim3(nc - c_lo + 1), dim3(kSubThreads), 0, st, s->sub_roots, c_mid,
+                               s->cleft, s->cright, s->ccount, pos, fl, dep, s->sub_list);
             RTQ_HIP(ctx, hipGetLastError());
         }
-        rs = queue_cost(2);
-        if (rs != RTQ_OK) return rs;
-        for (uint32_t k = s->lds_from; k > 0; --k) {
-            const auto& pr = s->passes[k - 1];
-            hipLaunchKernelGGL(k_place_pass, dim3(blocks_for(pr.second)), dim3(kThreads), 0, st, pr.first,
-                               pr.second, s->cleft, s->cright, s->ccount, pos, fl, dep);
-            RTQ_HIP(ctx, hipGetLastError());
-            rs = queue_cost(dp_next + 1);
+        if (cost) {
+            RTQ_HIP(ctx, side.fork(st));
+            rs = wide_cost_top(ctx, s, wcost, wchoice, ctx->side);
             if (rs != RTQ_OK) return rs;
+        }
+        for (uint32_t k = s->sub_from; k > 0; --k) {
+            const auto& pr = s->passes[k - 1];
+            hipLaunchKernelGGL(k_place_pass, dim3(blocks_for(pr.second)), dim3(kThreads), 0, st, pr.first, pr.second,
+                               s->cleft, s->cright, s->ccount, pos, fl, dep);
+            RTQ_HIP(ctx, hipGetLastError());
         }
     }
     hipLaunchKernelGGL(k_write_leaves, dim3(blocks_for(nc)), dim3(kThreads), 0, st, nc, s->ctri, s->cleft, fl,
@@ -1592,8 +1680,6 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipSt
     if (!refit) RTQ_HIP(ctx, rd.add(&h_depth, maxd, sizeof h_depth));
     if (!refit && n > 1) RTQ_HIP(ctx, rd.add(&h_ntrav, ntrav, sizeof h_ntrav));
     if (flag_dev) RTQ_HIP(ctx, rd.add(flag_host, flag_dev, sizeof(uint32_t)));
-    rs = queue_cost(dp_steps);
-    if (rs != RTQ_OK) return rs;
     RTQ_HIP(ctx, rd.wait());
     float extent = 0.0f;
     for (int k = 0; k < 3; ++k)
@@ -1733,6 +1819,8 @@ rtq_status build_scene(rtq_ctx* ctx, Scene* s, const rtq_build_params& prm) {
     // lds_from on create at most kLdsClusters clusters in all
     s->lds_from = s->ploc_passes;
     while (s->lds_from > 0 && nc - s->passes[s->lds_from - 1].first <= kLdsClusters) --s->lds_from;
+    s->sub_from = s->lds_from;
+    while (s->sub_from > 0 && s->passes[s->sub_from - 1].second <= kSubPass) --s->sub_from;
     if (s->ploc_passes > 0) {
         s->h_passes.resize(s->ploc_passes);
         for (uint32_t k = 0; k < s->ploc_passes; ++k)
@@ -1791,10 +1879,16 @@ rtq_status refit_scene(rtq_ctx* ctx, Scene* s) {
                        n, s->cbox);
     RTQ_HIP(ctx, hipGetLastError());
     const uint32_t n_passes = (uint32_t)s->passes.size();
-    for (uint32_t k = 0; k < s->lds_from; ++k) {
+    for (uint32_t k = 0; k < s->sub_from; ++k) {
         const auto& pr = s->passes[k];
         hipLaunchKernelGGL(k_refit_merge, dim3(blocks_for(pr.second)), dim3(kThreads), 0, st, pr.first, pr.second,
                            s->cleft, s->cright, s->cbox);
+        RTQ_HIP(ctx, hipGetLastError());
+    }
+    if (s->sub_from < s->lds_from) {
+        const uint32_t blocks = s->n_clusters - s->passes[s->lds_from].first + 1;
+        hipLaunchKernelGGL(k_refit_subtrees, dim3(blocks), dim3(kSubThreads), 0, st, s->sub_roots, s->sub_list,
+                           s->first_leaf, s->cleft, s->cright, s->cbox);
         RTQ_HIP(ctx, hipGetLastError());
     }
     if (s->lds_from < n_passes) {

@@ -58,6 +58,8 @@ struct Scene {
     uint32_t* preorder = nullptr;       // pre-order position of every cluster (2N - 1)
     uint32_t* first_leaf = nullptr;     // rank of the first leaf below every cluster (2N - 1)
     uint32_t* node_depth = nullptr;     // depth of every cluster (2N - 1)
+    uint2* sub_roots = nullptr;         // .x = number of middle subtrees, then each one's (root, listed clusters)
+    uint32_t* sub_list = nullptr;       // N: each one's clusters level by level, from its first leaf's rank on
     uint32_t* trav_index = nullptr;     // binary traversal node of every cluster (2N - 1), kNone if none
     float4* nodes = nullptr;            // traversal nodes, 4 float4 (64 B) each
     uint4* node_aux = nullptr;          // per traversal node: child leaf ranges [A,B) [B,C), depth
@@ -81,10 +83,12 @@ struct Scene {
     // the same on the device (and its host staging copy); the clusters of the
     // passes from lds_from on fit in one workgroup's LDS together
     // (kLdsClusters): placement, collapse costs and refit merges run those
-    // passes in one launch
+    // passes in one launch, the passes [sub_from, lds_from) as subtrees below
+    // them in another, and each pass before sub_from in its own
     uint2* d_passes = nullptr;
     std::vector<uint2> h_passes;
     uint32_t lds_from = 0;
+    uint32_t sub_from = 0;
     // the memory behind nodes, node_aux, wide, wide_trav, wide_kids and
     // d_passes, kept from build to build
     Kept kept_nodes, kept_aux, kept_wide, kept_wide_trav, kept_wide_kids, kept_passes;
@@ -332,7 +336,7 @@ void scratch_free(TraceScratch* sc);
 // Compressed 8-wide nodes from the cluster arrays (fl: first leaf rank per cluster).
 // pos, bidx: pre-order position of every cluster and binary traversal index
 // of every position (null for a one-triangle scene, which has no binary node).
-// choice: the collapse's cost-table decisions (wide_cost_table), null for a
+// choice: the collapse's cost-table decisions (wide_cost_top), null for a
 // one-triangle scene.
 rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const uint32_t* fl, const uint32_t* pos,
                       const uint32_t* bidx, hipStream_t st);
@@ -341,13 +345,24 @@ rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const uint
 constexpr uint32_t kLdsClusters = 4096;
 constexpr int kLdsThreads = 1024;   // 4 clusters per thread
 
+// Middle subtrees: the clusters of the passes [sub_from, lds_from), hanging from
+// the top ones.  A pass of up to kSubPass merges is shorter than its launch, and
+// a tree has twenty of them: a workgroup takes a subtree through all its levels.
+// Larger passes fill the chip by themselves and keep a launch each.  Rebuild of
+// 2,095,104 triangles (28 passes below the top ones, placed and costed by 56
+// launches): 2,161 us; with the middle ones as subtrees 2,097 us (18 launches),
+// with passes up to 8,192 / 32,768 / 131,072 merges in them 2,127 / 2,104 /
+// 2,128 us, with all 2,267 us: few workgroups then have the long subtrees.
+constexpr uint32_t kSubPass = 65536;
+constexpr int kSubThreads = 64;
+
 // The SAH cost table of the 8-wide collapse (cost: 8 floats, choice: one word
-// per internal cluster), bottom-up over the PLOC passes in wide_cost_steps(s)
-// launches; wide_cost_table queues launches [first, last) of them.  It reads
-// the cluster arrays only, so it can run beside the binary layout's placement.
-uint32_t wide_cost_steps(const Scene* s);
-rtq_status wide_cost_table(rtq_ctx* ctx, const Scene* s, float* cost, uint32_t* choice, uint32_t first,
-                           uint32_t last, hipStream_t st);
+// per merged cluster), bottom-up.  wide_cost_bottom queues the passes before
+// sub_from, wide_cost_top the middle subtrees (from the lists the placement
+// leaves) and the rest; they read the cluster arrays, so they can run beside the
+// binary layout's placement.
+rtq_status wide_cost_bottom(rtq_ctx* ctx, const Scene* s, float* cost, uint32_t* choice, hipStream_t st);
+rtq_status wide_cost_top(rtq_ctx* ctx, const Scene* s, float* cost, uint32_t* choice, hipStream_t st);
 // New boxes for the kept 8-wide nodes after a refit (the cluster boxes and
 // box pad already refitted): one launch over the nodes, child refs kept.
 rtq_status refit_wide(rtq_ctx* ctx, Scene* s, hipStream_t st);
@@ -382,6 +397,26 @@ __device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t x) {
     x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xA, 0xF, false);   // row_bcast:15
     x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xC, 0xF, false);   // row_bcast:31
     return x;
+}
+
+// A middle subtree's list of clusters: each level's first one has this bit.
+constexpr uint32_t kLevelStart = 1u << 31;
+
+// f(cluster) for a subtree's `count` listed clusters, the deepest level first,
+// by one wave: as many of the last level left as there are lanes at a time.
+template <class F>
+__device__ __forceinline__ void levels_up(const uint32_t* list, uint32_t count, F&& f) {
+    const int lane = (int)threadIdx.x & 63;
+    int end = (int)count;
+    while (end > 0) {
+        const int i = end - 64 + lane;
+        const uint32_t w = i >= 0 ? list[i] : 0u;
+        const uint64_t m = __ballot((w & kLevelStart) != 0);
+        const int start = m ? end - 1 - __builtin_clzll(m) : end - 64;   // the first one has the bit
+        if (i >= start) f(w & ~kLevelStart);
+        end = start;
+        __syncthreads();
+    }
 }
 
 // Tile of this workgroup.  Workgroups are dispatched to the 8 XCDs in turn, and

@@ -47,12 +47,13 @@ __device__ __forceinline__ float box_area(const rtq_aabb& b) {
 // slots go either to the cluster with fewer slots or split between its
 // children.  choice[x] keeps, per j = 2..8, 0 (fewer slots) or the left
 // child's share (bits 3(j-2)), and the node's own split (bits 21..23).
-// Rows are computed bottom-up, one PLOC pass at a time (a merge's children
-// come from earlier passes); single triangles have a constant row.
+// Rows are computed bottom-up: the large PLOC passes one at a time (a merge's
+// children come from earlier passes), the middle subtrees in one launch, the
+// top's in another; single triangles have a constant row.
 constexpr float kNodeCost = 1.0f;
 constexpr float kTriCost = 0.6f;  // best of 0.15-4 on the 2M-triangle terrain
 
-__device__ __forceinline__ void dp_row(uint32_t x, uint32_t nt, const float* __restrict__ cost,
+__device__ __forceinline__ void dp_row(uint32_t x, uint32_t nt, const float* cost,
                                        const rtq_aabb* __restrict__ cbox, float* row) {
     if (x < nt) {
         const float a = kTriCost * box_area(cbox[x]);
@@ -92,7 +93,7 @@ __device__ __forceinline__ uint32_t dp_combine(const float* dl, const float* dr,
 __device__ __forceinline__ void dp_cluster(uint32_t c, uint32_t nt, uint32_t max_leaf,
                                            const uint32_t* __restrict__ cleft, const uint32_t* __restrict__ cright,
                                            const uint32_t* __restrict__ ccount, const rtq_aabb* __restrict__ cbox,
-                                           float* __restrict__ cost, uint32_t* __restrict__ choice) {
+                                           float* cost, uint32_t* __restrict__ choice) {
     float dl[kWidth], dr[kWidth], row[kWidth];
     dp_row(cleft[c], nt, cost, cbox, dl);
     dp_row(cright[c], nt, cost, cbox, dr);
@@ -111,6 +112,22 @@ __global__ __launch_bounds__(kThreads) void k_dp_pass(uint32_t first, uint32_t c
                                                       uint32_t* __restrict__ choice) {
     const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
     if (i < count) dp_cluster(first + i, nt, max_leaf, cleft, cright, ccount, cbox, cost, choice);
+}
+
+// The cost rows of one middle subtree per workgroup (one wave), the deepest
+// level first.
+__global__ __launch_bounds__(kSubThreads) void k_dp_subtrees(const uint2* __restrict__ roots,
+                                                             const uint32_t* __restrict__ list,
+                                                             const uint32_t* __restrict__ fl, uint32_t nt,
+                                                             uint32_t max_leaf, const uint32_t* __restrict__ cleft,
+                                                             const uint32_t* __restrict__ cright,
+                                                             const uint32_t* __restrict__ ccount,
+                                                             const rtq_aabb* __restrict__ cbox, float* cost,
+                                                             uint32_t* __restrict__ choice) {
+    if (blockIdx.x >= roots[0].x) return;
+    const uint2 root = roots[1 + blockIdx.x];
+    levels_up(list + fl[root.x], root.y,
+              [&](uint32_t c) { dp_cluster(c, nt, max_leaf, cleft, cright, ccount, cbox, cost, choice); });
 }
 
 // Passes [k0, k1) at the top of the tree in one workgroup, bottom-up, with
@@ -493,27 +510,28 @@ inline uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + kThreads - 1) / 
 
 }  // namespace
 
-uint32_t wide_cost_steps(const Scene* s) {
-    if (s->n_clusters <= s->n_tris) return 0;
-    return s->lds_from + (s->lds_from < (uint32_t)s->passes.size() ? 1u : 0u);
-}
-
-rtq_status wide_cost_table(rtq_ctx* ctx, const Scene* s, float* cost, uint32_t* choice, uint32_t first,
-                           uint32_t last, hipStream_t st) {
-    const uint32_t nt = s->n_tris, max_leaf = s->params.max_leaf_size;
-    const uint32_t n_passes = (uint32_t)s->passes.size();
-    for (uint32_t k = first; k < last; ++k) {
-        if (k < s->lds_from) {
-            const auto& pr = s->passes[k];
-            hipLaunchKernelGGL(k_dp_pass, dim3(blocks_for(pr.second)), dim3(kThreads), 0, st, pr.first, pr.second,
-                               nt, max_leaf, s->cleft, s->cright, s->ccount, s->cbox, cost, choice);
-        } else {
-            hipLaunchKernelGGL(k_dp_lds, dim3(1), dim3(kLdsThreads), 0, st, s->d_passes, s->lds_from, n_passes,
-                               s->passes[s->lds_from].first, s->n_clusters, nt, max_leaf, s->cleft, s->cright,
-                               s->ccount, s->cbox, cost, choice);
-        }
+rtq_status wide_cost_bottom(rtq_ctx* ctx, const Scene* s, float* cost, uint32_t* choice, hipStream_t st) {
+    for (uint32_t k = 0; k < s->sub_from; ++k) {
+        const auto& pr = s->passes[k];
+        hipLaunchKernelGGL(k_dp_pass, dim3(blocks_for(pr.second)), dim3(kThreads), 0, st, pr.first, pr.second,
+                           s->n_tris, s->params.max_leaf_size, s->cleft, s->cright, s->ccount, s->cbox, cost, choice);
         RTQ_HIP(ctx, hipGetLastError());
     }
+    return RTQ_OK;
+}
+
+rtq_status wide_cost_top(rtq_ctx* ctx, const Scene* s, float* cost, uint32_t* choice, hipStream_t st) {
+    const uint32_t nt = s->n_tris, max_leaf = s->params.max_leaf_size, c_lo = s->passes[s->lds_from].first;
+    if (s->sub_from < s->lds_from) {
+        hipLaunchKernelGGL(k_dp_subtrees, dim3(s->n_clusters - c_lo + 1), dim3(kSubThreads), 0, st, s->sub_roots,
+                           s->sub_list, s->first_leaf, nt, max_leaf, s->cleft, s->cright, s->ccount, s->cbox, cost,
+                           choice);
+        RTQ_HIP(ctx, hipGetLastError());
+    }
+    hipLaunchKernelGGL(k_dp_lds, dim3(1), dim3(kLdsThreads), 0, st, s->d_passes, s->lds_from,
+                       (uint32_t)s->passes.size(), c_lo, s->n_clusters, nt, max_leaf, s->cleft, s->cright, s->ccount,
+                       s->cbox, cost, choice);
+    RTQ_HIP(ctx, hipGetLastError());
     return RTQ_OK;
 }
 
