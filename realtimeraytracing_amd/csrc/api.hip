@@ -99,12 +99,10 @@ void free_build(Scene* s) {
     release(s->sorted_idx);
     release(s->sorted_codes);
     release(s->ref_nodes);
-    release(s->preorder);
-    release(s->first_leaf);
-    release(s->node_depth);
+    release(s->ctrav);
+    release(s->placed);
     release(s->sub_roots);
     release(s->sub_list);
-    release(s->trav_index);
     release(s->top);
     release(s->tris);
 }

@@ -95,12 +95,12 @@ __global__ __launch_bounds__(kThreads) void k_refit_merge(uint32_t first, uint32
 // now.
 __global__ __launch_bounds__(kSubThreads) void k_refit_subtrees(const uint2* __restrict__ roots,
                                                                 const uint32_t* __restrict__ list,
-                                                                const uint32_t* __restrict__ fl,
+                                                                const uint4* __restrict__ placed,
                                                                 const uint32_t* __restrict__ cleft,
                                                                 const uint32_t* __restrict__ cright, rtq_aabb* cbox) {
     if (blockIdx.x >= roots[0].x) return;
     const uint2 root = roots[1 + blockIdx.x];
-    levels_up(list + fl[root.x], root.y,
+    levels_up(list + placed[root.x].y, root.y,
               [&](uint32_t c) { cbox[c] = merged_box(cbox[cleft[c]], cbox[cright[c]]); });
 }
 
@@ -155,8 +155,7 @@ __global__ __launch_bounds__(kLdsThreads) void k_refit_merge_lds(const uint2* __
 // before right) order with a wave prefix sum, which is the order a FIFO
 // breadth-first walk appends them; children past kTopNodes keep their refs.
 static_assert(kTopNodes <= 64, "one lane per top-of-tree slot");
-__global__ __launch_bounds__(64) void k_top_nodes(const float4* __restrict__ nodes, float4* __restrict__ top,
-                                                  uint32_t* __restrict__ n_top) {
+__global__ __launch_bounds__(64) void k_top_nodes(const float4* __restrict__ nodes, float4* __restrict__ top) {
     __shared__ uint32_t s_q[64];
     const uint32_t lane = threadIdx.x;
     uint32_t node = 0;                 // node index of slot `lane` once its level is reached
@@ -207,7 +206,6 @@ __global__ __launch_bounds__(64) void k_top_nodes(const float4* __restrict__ nod
         begin = end;
         end = next;
     }
-    if (lane == 0) *n_top = end;
 }
 
 // ------------------------------------------------------------- scene bounds
@@ -518,7 +516,8 @@ __global__ __launch_bounds__(kThreads) void k_ploc_merge(
     const uint2* __restrict__ offs, const uint32_t* __restrict__ c_in, const Box6* __restrict__ b_in,
     uint32_t* __restrict__ c_out, Box6* __restrict__ b_out, rtq_aabb* __restrict__ cbox,
     uint32_t* __restrict__ cleft, uint32_t* __restrict__ cright, uint32_t* __restrict__ cparent,
-    uint32_t* __restrict__ ccount, uint32_t* __restrict__ ctri) {
+    uint32_t* __restrict__ ccount, uint32_t* __restrict__ ctri, uint32_t* __restrict__ ctrav, uint32_t nt,
+    uint32_t max_leaf) {
     const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
     const uint32_t iter = state[0], n_total = state[1];
     if (i >= iter) return;
@@ -546,7 +545,9 @@ __global__ __launch_bounds__(kThreads) void k_ploc_merge(
         cright[id] = cj;
         cparent[cid] = id;
         cparent[cj] = id;
-        ccount[id] = ccount[cid] + ccount[cj];
+        const uint32_t count = ccount[cid] + ccount[cj];
+        ccount[id] = count;
+        ctrav[id] = (cid < nt ? 0u : ctrav[cid]) + (cj < nt ? 0u : ctrav[cj]) + (count > max_leaf ? 1u : 0u);
         ctri[id] = 0;
         cid = id;
         b = m;
@@ -613,8 +614,18 @@ struct PlocLists {
 
 struct PlocClusters {
     rtq_aabb* box;
-    uint32_t *left, *right, *parent, *count, *tri;
+    uint32_t *left, *right, *parent, *count, *tri, *trav;
+    uint32_t n_tris, max_leaf;
 };
+
+// Triangles and binary traversal nodes below a cluster.
+__device__ __forceinline__ uint2 ploc_below(const PlocClusters& cl, uint32_t c) {
+    return make_uint2(cl.count[c], c < cl.n_tris ? 0u : cl.trav[c]);
+}
+__device__ __forceinline__ uint2 ploc_below_merged(const PlocClusters& cl, uint2 a, uint2 b) {
+    const uint32_t count = a.x + b.x;
+    return make_uint2(count, a.y + b.y + (count > cl.max_leaf ? 1u : 0u));
+}
 
 __device__ __forceinline__ uint64_t tile_word(uint64_t st, uint32_t merges, uint32_t stays) {
     return st | ((uint64_t)merges << 32) | stays;
@@ -646,9 +657,9 @@ __device__ __forceinline__ uint32_t block_exclusive_sum(uint32_t v, uint32_t* s_
 
 // Merge of clusters cid (box b) and cj (box bj) into cluster id, as
 // k_ploc_merge writes it; b becomes the merged box.
-// Merged cluster id of (cid, cj) with triangle count `count` (the sum of theirs).
+// `below`: what lies below it (ploc_below_merged).
 __device__ __forceinline__ void ploc_merge_store(const PlocClusters& cl, uint32_t id, uint32_t cid, uint32_t cj,
-                                                 uint32_t count, Box6& b, const Box6& bj) {
+                                                 uint2 below, Box6& b, const Box6& bj) {
     Box6 m;
     rtq_aabb a{};
 #pragma unroll
@@ -663,7 +674,8 @@ __device__ __forceinline__ void ploc_merge_store(const PlocClusters& cl, uint32_
     cl.right[id] = cj;
     cl.parent[cid] = id;
     cl.parent[cj] = id;
-    cl.count[id] = count;
+    cl.count[id] = below.x;
+    cl.trav[id] = below.y;
     cl.tri[id] = 0;
     b = m;
 }
@@ -672,8 +684,8 @@ __device__ __forceinline__ void ploc_merge_write(const PlocClusters& cl, uint32_
                                                  Box6& b, const Box6& bj) {
     // the counts are read before any store: the arrays may alias as far as
     // the compiler knows, and a load after a store waits for the store
-    const uint32_t count = cl.count[cid] + cl.count[cj];
-    ploc_merge_store(cl, id, cid, cj, count, b, bj);
+    const uint2 below = ploc_below_merged(cl, ploc_below(cl, cid), ploc_below(cl, cj));
+    ploc_merge_store(cl, id, cid, cj, below, b, bj);
 }
 
 struct PlocPassArgs {
@@ -876,12 +888,12 @@ __device__ __forceinline__ uint32_t nearest_by_lanes(const Box6* w, int i, int q
     return arg;
 }
 
-// The tail's list in LDS, with its triangle counts (no global loads between the
-// passes' barriers) and nearest neighbours.
+// The tail's list in LDS, with its triangle and node counts (no global loads
+// between the passes' barriers) and nearest neighbours.
 struct TailLists {
     Box6 list[kTailMax + 2 * kRefRadius];   // kRefRadius far boxes, the list's boxes, kRefRadius far boxes
     uint32_t c[kTailMax];
-    uint32_t n[kTailMax];
+    uint2 n[kTailMax];
     uint16_t nn[kTailMax];
     uint32_t w[kTailThreads / 64];
 };
@@ -907,7 +919,8 @@ __device__ __forceinline__ uint32_t tail_merge(TailLists& L, int tid, uint32_t m
         back[k] = L.nn[j[k]];
     }
     Box6 ob[K], pb[K];
-    uint32_t oc[K], on[K], pc[K], pn[K], opos[K];
+    uint32_t oc[K], pc[K], opos[K];
+    uint2 on[K], pn[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const uint32_t i = min((uint32_t)(K * tid + k), m - 1);
@@ -945,7 +958,7 @@ __device__ __forceinline__ uint32_t tail_merge(TailLists& L, int tid, uint32_t m
         opos[k] = (f[k] & 0xFFFFu) ? run & 0xFFFFu : kNone;
         if (f[k] >> 16) {
             const uint32_t id = n_total + (run >> 16);
-            on[k] += pn[k];
+            on[k] = ploc_below_merged(cl, on[k], pn[k]);
             ploc_merge_store(cl, id, oc[k], pc[k], on[k], ob[k], pb[k]);
             oc[k] = id;
         }
@@ -1002,7 +1015,7 @@ __global__ __launch_bounds__(kTailThreads) void k_ploc_tail(uint32_t* __restrict
         s_box[q] = lists.b[cur][q];
         const uint32_t c = lists.c[cur][q];
         L.c[q] = c;
-        L.n[q] = cl.count[c];
+        L.n[q] = ploc_below(cl, c);
     }
     if (tid < kRefRadius) {
         L.list[tid] = far_box();
@@ -1049,38 +1062,26 @@ __global__ __launch_bounds__(kTailThreads) void k_ploc_tail(uint32_t* __restrict
     if (tid == 0) {
         state[0] = m;
         state[1] = n_total;
+        state[3] = L.n[0].y;   // the root's, once one cluster is left
         *log_count = passes;
     }
 }
 
-__device__ __forceinline__ void place_one(uint32_t p, const uint32_t* __restrict__ cleft,
-                                          const uint32_t* __restrict__ cright, const uint32_t* __restrict__ ccount,
-                                          uint32_t* __restrict__ pos, uint32_t* __restrict__ fl,
-                                          uint32_t* __restrict__ dep) {
-    const uint32_t l = cleft[p], r = cright[p];
-    const uint32_t pp = pos[p], pf = fl[p], pd = dep[p];
-    const uint32_t lc = ccount[l];
-    pos[l] = pp + 1;
-    pos[r] = pp + 2 * lc;
-    fl[l] = pf;
-    fl[r] = pf + lc;
-    dep[l] = pd + 1;
-    dep[r] = pd + 1;
-}
-
-// Top-down pre-order placement for the clusters created in one PLOC pass
-// (their parents were created in later passes, so are already placed):
-// left child right after the parent, right child after the left subtree
-// (scene.cpp:189-201); fl = rank of the subtree's first leaf.
-__global__ __launch_bounds__(kThreads) void k_place_pass(uint32_t first, uint32_t count,
+// Clusters of one PLOC pass give their children's places (their own are known:
+// their parents were created in later passes).
+__global__ __launch_bounds__(kThreads) void k_place_pass(uint32_t first, uint32_t count, uint32_t nt,
                                                          const uint32_t* __restrict__ cleft,
                                                          const uint32_t* __restrict__ cright,
                                                          const uint32_t* __restrict__ ccount,
-                                                         uint32_t* __restrict__ pos,
-                                                         uint32_t* __restrict__ fl,
-                                                         uint32_t* __restrict__ dep) {
+                                                         const uint32_t* __restrict__ ctrav,
+                                                         uint4* __restrict__ placed) {
     const uint32_t k = blockIdx.x * kThreads + threadIdx.x;
-    if (k < count) place_one(first + k, cleft, cright, ccount, pos, fl, dep);
+    if (k >= count) return;
+    const uint32_t l = cleft[first + k], r = cright[first + k];
+    const Place p = place_of(placed[first + k]);
+    const uint32_t lc = ccount[l], lt = l < nt ? 0u : ctrav[l];
+    placed[l] = left_place(p);
+    placed[r] = right_place(p, lc, lt);
 }
 
 // The middle subtrees' clusters (from c_mid on), level by level from the root,
@@ -1090,61 +1091,64 @@ __global__ __launch_bounds__(kThreads) void k_place_pass(uint32_t first, uint32_
 // of `list`; the order within a level is free, no result depends on it.
 constexpr uint32_t kFront = 256;
 
-__global__ __launch_bounds__(kSubThreads) void k_place_subtrees(uint2* roots, uint32_t c_mid,
+__global__ __launch_bounds__(kSubThreads) void k_place_subtrees(uint2* roots, uint32_t c_mid, uint32_t nt,
                                                                 const uint32_t* __restrict__ cleft,
                                                                 const uint32_t* __restrict__ cright,
-                                                                const uint32_t* __restrict__ ccount, uint32_t* pos,
-                                                                uint32_t* fl, uint32_t* dep, uint32_t* list_base) {
-    __shared__ uint4 s_front[2][kFront];
+                                                                const uint32_t* __restrict__ ccount,
+                                                                const uint32_t* __restrict__ ctrav, uint4* placed,
+                                                                uint32_t* list_base) {
+    __shared__ uint32_t s_id[2][kFront];
+    __shared__ uint4 s_at[2][kFront];
     if (blockIdx.x >= roots[0].x) return;
     const uint32_t lane = threadIdx.x;
     const uint32_t root = roots[1 + blockIdx.x].x;
-    const uint32_t root_fl = fl[root];
-    uint32_t* const list = list_base + root_fl;
+    const uint4 at = placed[root];
+    uint32_t* const list = list_base + at.y;
     if (lane == 0) {
-        s_front[0][0] = make_uint4(root, pos[root], root_fl, dep[root]);
+        s_id[0][0] = root;
+        s_at[0][0] = at;
         list[0] = root | kLevelStart;
     }
     __syncthreads();
     uint32_t begin = 0, end = 1;
     for (uint32_t k = 0; begin < end; ++k) {
-        const uint4* const front = s_front[k & 1u];
-        uint4* const next = s_front[~k & 1u];
+        const uint32_t cur = k & 1u, nxt = cur ^ 1u;
         uint32_t n_next = 0;
         for (uint32_t e0 = begin; e0 < end; e0 += kSubThreads) {
             const uint32_t e = e0 + lane;
-            uint4 f = make_uint4(0, 0, 0, 0);
-            uint32_t l = 0, r = 0, lc = 0;
+            uint32_t l = 0, r = 0;
+            uint4 lp{}, rp{};
             if (e < end) {
+                uint32_t c;
+                Place p;
                 if (e - begin < kFront) {
-                    f = front[e - begin];
+                    c = s_id[cur][e - begin];
+                    p = place_of(s_at[cur][e - begin]);
                 } else {
-                    f.x = list[e] & ~kLevelStart;
-                    f.y = pos[f.x];
-                    f.z = fl[f.x];
-                    f.w = dep[f.x];
+                    c = list[e] & ~kLevelStart;
+                    p = place_of(placed[c]);
                 }
-                l = cleft[f.x];
-                r = cright[f.x];
-                lc = ccount[l];
-                pos[l] = f.y + 1;
-                pos[r] = f.y + 2 * lc;
-                fl[l] = f.z;
-                fl[r] = f.z + lc;
-                dep[l] = f.w + 1;
-                dep[r] = f.w + 1;
+                l = cleft[c];
+                r = cright[c];
+                lp = left_place(p);
+                rp = right_place(p, ccount[l], l < nt ? 0u : ctrav[l]);
+                placed[l] = lp;
+                placed[r] = rp;
             }
             // children of the middle passes to the next level
             const bool bl = l >= c_mid, br = r >= c_mid;
             const uint64_t ml = __ballot(bl), mr = __ballot(br);
             const uint64_t below = (1ull << lane) - 1u;
-            const auto put = [&](uint32_t i, uint32_t c, uint32_t p, uint32_t first) {
+            const auto put = [&](uint32_t i, uint32_t c, const uint4& v) {
                 list[end + i] = i == 0 ? c | kLevelStart : c;
-                if (i < kFront) next[i] = make_uint4(c, p, first, f.w + 1);
+                if (i < kFront) {
+                    s_id[nxt][i] = c;
+                    s_at[nxt][i] = v;
+                }
             };
-            if (bl) put(n_next + (uint32_t)__popcll(ml & below), l, f.y + 1, f.z);
+            if (bl) put(n_next + (uint32_t)__popcll(ml & below), l, lp);
             n_next += (uint32_t)__popcll(ml);
-            if (br) put(n_next + (uint32_t)__popcll(mr & below), r, f.y + 2 * lc, f.z + lc);
+            if (br) put(n_next + (uint32_t)__popcll(mr & below), r, rp);
             n_next += (uint32_t)__popcll(mr);
         }
         __syncthreads();
@@ -1155,25 +1159,26 @@ __global__ __launch_bounds__(kSubThreads) void k_place_subtrees(uint2* roots, ui
 }
 
 // The passes [k0, k1) at the top of the tree in one workgroup, last pass
-// first, with the placement state (position, first leaf, depth) of their
-// clusters [c_lo, nc) in LDS: a pass reads and writes LDS only, a barrier
-// between passes.  Children from earlier passes get their state in global
-// memory, and those from c_mid on are the roots of the middle subtrees, listed
-// in roots; the clusters of the range write their state back at the end.  Each
-// thread keeps the child ids and left-child triangle counts of its clusters
-// c_lo + t + kLdsThreads * s in registers.  1 <= nc - c_lo <= kLdsClusters.
+// first, with the places of their clusters [c_lo, nc) in LDS: a pass reads and
+// writes LDS only, a barrier between passes.  Children from earlier passes get
+// their places in global memory, and those from c_mid on are the roots of the
+// middle subtrees, listed in roots; the clusters of the range write theirs back
+// at the end.  Each thread keeps the child ids and the left child's counts of
+// its clusters c_lo + t + kLdsThreads * s in registers.  1 <= nc - c_lo <=
+// kLdsClusters.
 __global__ __launch_bounds__(kLdsThreads) void k_place_lds(const uint2* __restrict__ passes, uint32_t k0, uint32_t k1,
-                                                           uint32_t c_lo, uint32_t nc, uint32_t c_mid,
+                                                           uint32_t c_lo, uint32_t nc, uint32_t c_mid, uint32_t nt,
                                                            const uint32_t* __restrict__ cleft,
                                                            const uint32_t* __restrict__ cright,
                                                            const uint32_t* __restrict__ ccount,
-                                                           uint32_t* __restrict__ pos, uint32_t* __restrict__ fl,
-                                                           uint32_t* __restrict__ dep, uint2* __restrict__ roots) {
+                                                           const uint32_t* __restrict__ ctrav,
+                                                           uint4* __restrict__ placed, uint2* __restrict__ roots) {
     constexpr int kSlots = kLdsClusters / kLdsThreads;
-    __shared__ uint32_t s_pos[kLdsClusters], s_fl[kLdsClusters], s_dep[kLdsClusters], s_roots;
+    __shared__ uint4 s_at[kLdsClusters];
+    __shared__ uint32_t s_roots;
     const uint32_t t = threadIdx.x;
     const uint32_t R = nc - c_lo;
-    uint32_t L[kSlots], Rc[kSlots], LC[kSlots];
+    uint32_t L[kSlots], Rc[kSlots], LC[kSlots], LT[kSlots];
 #pragma unroll
     for (int q = 0; q < kSlots; ++q) {
         const uint32_t idx = t + kLdsThreads * q;
@@ -1181,11 +1186,14 @@ __global__ __launch_bounds__(kLdsThreads) void k_place_lds(const uint2* __restri
         Rc[q] = idx < R ? cright[c_lo + idx] : 0u;
     }
 #pragma unroll
-    for (int q = 0; q < kSlots; ++q) LC[q] = L[q] < nc && t + kLdsThreads * q < R ? ccount[L[q]] : 0u;
+    for (int q = 0; q < kSlots; ++q) {
+        // a scene of one triangle has no child
+        const bool in = L[q] < nc && t + kLdsThreads * q < R;
+        LC[q] = in ? ccount[L[q]] : 0u;
+        LT[q] = in && L[q] >= nt ? ctrav[L[q]] : 0u;
+    }
     if (t == 0) {  // the root, the last cluster
-        s_pos[R - 1] = 0;
-        s_fl[R - 1] = 0;
-        s_dep[R - 1] = 0;
+        s_at[R - 1] = make_uint4(0, 0, 0, 0);
         s_roots = 0;
     }
     __syncthreads();
@@ -1195,19 +1203,13 @@ __global__ __launch_bounds__(kLdsThreads) void k_place_lds(const uint2* __restri
         for (int q = 0; q < kSlots; ++q) {
             const uint32_t idx = t + kLdsThreads * q, c = c_lo + idx;
             if (idx >= R || c < p.x || c >= p.x + p.y) continue;
-            const uint32_t pp = s_pos[idx], pf = s_fl[idx], pd = s_dep[idx];
-            const uint32_t l = L[q], r = Rc[q], lc = LC[q];
-            // left child right after the parent, right child after the left subtree
-            if (l >= c_lo) {
-                s_pos[l - c_lo] = pp + 1; s_fl[l - c_lo] = pf; s_dep[l - c_lo] = pd + 1;
-            } else {
-                pos[l] = pp + 1; fl[l] = pf; dep[l] = pd + 1;
-            }
-            if (r >= c_lo) {
-                s_pos[r - c_lo] = pp + 2 * lc; s_fl[r - c_lo] = pf + lc; s_dep[r - c_lo] = pd + 1;
-            } else {
-                pos[r] = pp + 2 * lc; fl[r] = pf + lc; dep[r] = pd + 1;
-            }
+            const Place at = place_of(s_at[idx]);
+            const uint32_t l = L[q], r = Rc[q];
+            const uint4 lp = left_place(at), rp = right_place(at, LC[q], LT[q]);
+            if (l >= c_lo) s_at[l - c_lo] = lp;
+            else placed[l] = lp;
+            if (r >= c_lo) s_at[r - c_lo] = rp;
+            else placed[r] = rp;
         }
         __syncthreads();
     }
@@ -1215,11 +1217,7 @@ __global__ __launch_bounds__(kLdsThreads) void k_place_lds(const uint2* __restri
     for (int q = 0; q < kSlots; ++q) {
         const uint32_t idx = t + kLdsThreads * q;
         const bool in = idx < R;
-        if (in) {
-            pos[c_lo + idx] = s_pos[idx];
-            fl[c_lo + idx] = s_fl[idx];
-            dep[c_lo + idx] = s_dep[idx];
-        }
+        if (in) placed[c_lo + idx] = s_at[idx];
         const bool bl = in && L[q] >= c_mid && L[q] < c_lo, br = in && Rc[q] >= c_mid && Rc[q] < c_lo;
         const uint64_t ml = __ballot(bl), mr = __ballot(br);
         uint32_t at = 0;
@@ -1237,19 +1235,19 @@ __global__ __launch_bounds__(kLdsThreads) void k_place_lds(const uint2* __restri
 // leaf in block_depth[blockIdx.x] (k_max_u32 takes the maximum: atomics of
 // every wave on one word would serialise, tens of thousands of them).
 __global__ __launch_bounds__(kThreads) void k_write_leaves(
-    uint32_t n_clusters, const uint32_t* __restrict__ ctri, const uint32_t* __restrict__ cleft,
-    const uint32_t* __restrict__ fl, const uint32_t* __restrict__ dep, const float4* __restrict__ tri_world,
-    float4* __restrict__ tris, uint32_t* __restrict__ block_depth) {
+    uint32_t n, const uint32_t* __restrict__ ctri, const uint4* __restrict__ placed,
+    const float4* __restrict__ tri_world, float4* __restrict__ tris, uint32_t* __restrict__ block_depth) {
     __shared__ uint32_t s_max[kThreads / 64];
     const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
     uint32_t depth = 0;
-    if (c < n_clusters && cleft[c] == kNone) {
+    if (c < n) {   // the clusters of one triangle
         const uint32_t t = ctri[c];
-        const uint64_t dst = 3ull * fl[c];
+        const Place p = place_of(placed[c]);
+        const uint64_t dst = 3ull * p.first;
         tris[dst + 0] = tri_world[3ull * t + 0];
         tris[dst + 1] = tri_world[3ull * t + 1];
         tris[dst + 2] = tri_world[3ull * t + 2];
-        depth = dep[c];
+        depth = p.depth;
     }
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) depth = max(depth, (uint32_t)__shfl_xor(depth, d, 64));
@@ -1282,7 +1280,7 @@ __global__ __launch_bounds__(1024) void k_max_u32(const uint32_t* __restrict__ v
 // position, children as positions, leaves with their triangle.
 __global__ __launch_bounds__(kThreads) void k_write_ref(
     uint32_t n_clusters, const rtq_aabb* __restrict__ cbox, const uint32_t* __restrict__ ctri,
-    const uint32_t* __restrict__ cleft, const uint32_t* __restrict__ cright, const uint32_t* __restrict__ pos,
+    const uint32_t* __restrict__ cleft, const uint32_t* __restrict__ cright, const uint4* __restrict__ placed,
     rtq_bvh_node* __restrict__ ref) {
     const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
     if (c >= n_clusters) return;
@@ -1292,71 +1290,50 @@ __global__ __launch_bounds__(kThreads) void k_write_ref(
     nd.box.pad1_ = 0.0f;
     const bool leaf = cleft[c] == kNone;
     nd.triangle_id = leaf ? ctri[c] : 0u;
-    nd.left_child = leaf ? 0u : pos[cleft[c]];
-    nd.right_child = leaf ? 0u : pos[cright[c]];
+    nd.left_child = leaf ? 0u : placed[cleft[c]].x;
+    nd.right_child = leaf ? 0u : placed[cright[c]].x;
     nd.pad_ = 0u;
-    ref[pos[c]] = nd;
+    ref[placed[c].x] = nd;
 }
 
-__device__ __forceinline__ bool is_trav_node(uint32_t c, uint32_t root, uint32_t max_leaf,
-                                             const uint32_t* cleft, const uint32_t* ccount) {
-    return cleft[c] != kNone && (ccount[c] > max_leaf || c == root);
-}
-
-__global__ __launch_bounds__(kThreads) void k_mark_trav(uint32_t n_clusters, uint32_t root, uint32_t max_leaf,
-                                                        const uint32_t* __restrict__ cleft,
-                                                        const uint32_t* __restrict__ ccount,
-                                                        const uint32_t* __restrict__ pos,
-                                                        uint32_t* __restrict__ flag) {
-    const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
-    if (c >= n_clusters) return;
-    flag[pos[c]] = is_trav_node(c, root, max_leaf, cleft, ccount) ? 1u : 0u;
-}
-
-// Traversal node (64 B): child boxes widened outward by `pad`, interleaved as
+// Traversal node (64 B): child boxes widened outward by the box margin, interleaved as
 //   [c0.lo.x c0.hi.x c0.lo.y c0.hi.y] [c0.lo.z c0.hi.z c1.lo.x c1.hi.x]
 //   [c1.lo.y c1.hi.y c1.lo.z c1.hi.z] [ref0 ref1 order 0]
 // where `order` holds the learned child-order bits (zero until a model is applied).
-__device__ __forceinline__ void child_desc(uint32_t ch, uint32_t root, uint32_t max_leaf,
-                                           const rtq_aabb* cbox, const uint32_t* cleft,
-                                           const uint32_t* ccount, const uint32_t* pos,
-                                           const uint32_t* fl, const uint32_t* bidx, float pad,
-                                           float* lo, float* hi, uint32_t* ref) {
-    const rtq_aabb a = cbox[ch];
-    for (int k = 0; k < 3; ++k) { lo[k] = a.min[k] - pad; hi[k] = a.max[k] + pad; }
-    if (is_trav_node(ch, root, max_leaf, cleft, ccount)) *ref = bidx[pos[ch]];
-    else *ref = leaf_ref(fl[ch], ccount[ch]);
-}
-
+// One thread per merged cluster; what a child needs besides its box follows from
+// the node's own place and the counts below the children.  2,095,104 triangles:
+// 150 us when a child's index came from a scan over marks in pre-order, 61 us
+// with the counts that PLOC's merges keep (they cost its passes nothing).
 __global__ __launch_bounds__(kThreads) void k_write_trav(
-    uint32_t n_clusters, uint32_t root, uint32_t max_leaf, float pad, const rtq_aabb* __restrict__ cbox,
-    const uint32_t* __restrict__ cleft, const uint32_t* __restrict__ cright,
-    const uint32_t* __restrict__ ccount, const uint32_t* __restrict__ pos, const uint32_t* __restrict__ fl,
-    const uint32_t* __restrict__ bidx, const uint32_t* __restrict__ dep, float4* __restrict__ nodes,
-    uint4* __restrict__ aux) {
-    const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
-    if (c >= n_clusters) return;
-    if (!is_trav_node(c, root, max_leaf, cleft, ccount)) return;
-    float l0[3], h0[3], l1[3], h1[3];
-    uint32_t r0, r1;
-    child_desc(cleft[c], root, max_leaf, cbox, cleft, ccount, pos, fl, bidx, pad, l0, h0, &r0);
-    child_desc(cright[c], root, max_leaf, cbox, cleft, ccount, pos, fl, bidx, pad, l1, h1, &r1);
-    const uint32_t idx = bidx[pos[c]];
-    float4* o = nodes + 4ull * idx;
-    o[0] = make_float4(l0[0], h0[0], l0[1], h0[1]);
-    o[1] = make_float4(l0[2], h0[2], l1[0], h1[0]);
-    o[2] = make_float4(l1[1], h1[1], l1[2], h1[2]);
+    uint32_t nt, uint32_t nc, uint32_t max_leaf, const rtq_aabb* __restrict__ bounds,
+    const rtq_aabb* __restrict__ cbox, const uint32_t* __restrict__ cleft, const uint32_t* __restrict__ cright,
+    const uint32_t* __restrict__ ccount, const uint32_t* __restrict__ ctrav, const uint4* __restrict__ placed,
+    float4* __restrict__ nodes, uint4* __restrict__ aux) {
+    const uint32_t c = nt + blockIdx.x * kThreads + threadIdx.x;
+    if (c >= nc || !(ccount[c] > max_leaf || c == nc - 1)) return;
+    const uint32_t l = cleft[c], r = cright[c];
+    const Place p = place_of(placed[c]);
+    const rtq_aabb bl = cbox[l], br = cbox[r];
+    const uint32_t lc = ccount[l], rc = ccount[r], lt = l < nt ? 0u : ctrav[l];
+    const float pad = box_pad_of(bounds[0]);
+    const uint32_t middle = p.first + lc;
+    const uint32_t r0 = l >= nt && lc > max_leaf ? p.trav + 1 : leaf_ref(p.first, lc);
+    const uint32_t r1 = r >= nt && rc > max_leaf ? p.trav + 1 + lt : leaf_ref(middle, rc);
+    float4* o = nodes + 4ull * p.trav;
+    o[0] = make_float4(bl.min[0] - pad, bl.max[0] + pad, bl.min[1] - pad, bl.max[1] + pad);
+    o[1] = make_float4(bl.min[2] - pad, bl.max[2] + pad, br.min[0] - pad, br.max[0] + pad);
+    o[2] = make_float4(br.min[1] - pad, br.max[1] + pad, br.min[2] - pad, br.max[2] + pad);
     // .z holds the learned child-order bits (none until an order model is applied)
     o[3] = make_float4(__uint_as_float(r0), __uint_as_float(r1), 0.0f, 0.0f);
     // leaf-order ranges of the children, [A, B) and [B, C), and the binary depth
-    const uint32_t a0 = fl[cleft[c]], b0 = fl[cright[c]];
-    aux[idx] = make_uint4(a0, b0, b0 + ccount[cright[c]], dep[c]);
+    aux[p.trav] = make_uint4(p.first, middle, middle + rc, p.depth);
 }
 
 // Single-triangle scene: one node whose two children are the same leaf.
-__global__ void k_write_single(const rtq_aabb* __restrict__ cbox, float pad, float4* __restrict__ nodes,
-                               uint4* __restrict__ aux) {
+__global__ void k_write_single(const rtq_aabb* __restrict__ bounds, const rtq_aabb* __restrict__ cbox,
+                               float4* __restrict__ nodes, uint4* __restrict__ aux) {
     const rtq_aabb a = cbox[0];
+    const float pad = box_pad_of(bounds[0]);
     float lo[3], hi[3];
     for (int k = 0; k < 3; ++k) { lo[k] = a.min[k] - pad; hi[k] = a.max[k] + pad; }
     const uint32_t r = leaf_ref(0, 1);
@@ -1394,8 +1371,10 @@ rtq_status compute_bounds(rtq_ctx* ctx, Scene* s, uint32_t pad_origin, rtq_aabb*
 // active list starts in (c0, b0); c1, b1 are the other buffers.  A batch's
 // passes all take the grid of its first pass; 16 passes per batch bring a
 // 2M-triangle terrain (61 passes) to the tail in two host round trips.
+// root_trav: the traversal nodes in the whole tree (Scene::ctrav of the root).
 rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint32_t* c0, uint32_t* c1,
-                      Box6* b0, Box6* b1, std::vector<std::pair<uint32_t, uint32_t>>& passes, hipStream_t st) {
+                      Box6* b0, Box6* b1, std::vector<std::pair<uint32_t, uint32_t>>& passes, uint32_t* root_trav,
+                      hipStream_t st) {
     constexpr uint32_t kPlocBatch = 16;
     const uint32_t n = s->n_tris;
     const uint32_t T = kPassThreads - 2 * radius;
@@ -1418,7 +1397,8 @@ rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
     RTQ_HIP(ctx, hipMemcpyAsync(state, h_state0, sizeof h_state0, hipMemcpyHostToDevice, st));
     RTQ_HIP(ctx, hipMemsetAsync(err, 0, 2 * sizeof(uint32_t), st));
     PlocLists lists{{c0, c1}, {b0, b1}};
-    PlocClusters cl{s->cbox, s->cleft, s->cright, s->cparent, s->ccount, s->ctri};
+    PlocClusters cl{s->cbox, s->cleft,  s->cright, s->cparent, s->ccount,
+                    s->ctri, s->ctrav, n,         s->params.max_leaf_size};
     uint32_t iter = n, n_total = n;
     std::vector<uint4> h_tail;
     while (iter > 1) {
@@ -1477,6 +1457,7 @@ rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
             return fail(ctx, RTQ_EINTERNAL, "PLOC made no progress at %u clusters", iter);
         iter = h_state[0];
         n_total = h_state[1];
+        *root_trav = h_state[3];
     }
     if (n_total != 2 * n - 1) return fail(ctx, RTQ_EINTERNAL, "PLOC produced %u clusters, expected %u", n_total, 2 * n - 1);
     return RTQ_OK;
@@ -1489,7 +1470,7 @@ rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
 // cluster and change nothing).
 rtq_status ploc_split(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint32_t* c_in, uint32_t* c_out,
                       Box6* b_in, Box6* b_out, std::vector<std::pair<uint32_t, uint32_t>>& pass_ranges,
-                      hipStream_t st) {
+                      uint32_t* root_trav, hipStream_t st) {
     constexpr uint32_t kPlocBatch = 8;
     const uint32_t n = s->n_tris;
     uint32_t *nn = nullptr, *state = nullptr;
@@ -1518,7 +1499,7 @@ rtq_status ploc_split(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
             if (rs != RTQ_OK) return rs;
             hipLaunchKernelGGL(k_ploc_merge, dim3(blocks_for(bound)), dim3(kThreads), 0, st, state, nn, flags, offs,
                                c_in, b_in, c_out, b_out, s->cbox, s->cleft, s->cright, s->cparent, s->ccount,
-                               s->ctri);
+                               s->ctri, s->ctrav, n, s->params.max_leaf_size);
             RTQ_HIP(ctx, hipGetLastError());
             hipLaunchKernelGGL(k_ploc_advance, dim3(1), dim3(1), 0, st, tot, state, pass_log, k);
             RTQ_HIP(ctx, hipGetLastError());
@@ -1542,6 +1523,11 @@ rtq_status ploc_split(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
     }
     if (n_total != 2 * n - 1)
         return fail(ctx, RTQ_EINTERNAL, "PLOC produced %u clusters, expected %u", n_total, 2 * n - 1);
+    if (n > 1) {
+        HostReads rd(ctx, st);
+        RTQ_HIP(ctx, rd.add(root_trav, s->ctrav + (n_total - 1), sizeof(uint32_t)));
+        RTQ_HIP(ctx, rd.wait());
+    }
     return RTQ_OK;
 }
 
@@ -1582,36 +1568,27 @@ private:
 };
 
 // refit: the tree is the one the last build wrote the layouts for, with new
-// boxes: its pre-order placement is kept and the 8-wide nodes keep their
-// children.  flag_dev (optional): one more device word to read back with the
-// layout's own host read, into *flag_host.
+// boxes: its placement is kept and the 8-wide nodes keep their children.
+// d_bounds: the scene's box and cube, after a refit the root cluster's box.
+// flag_dev (optional): one more device word to read back with the layout's own
+// host read, into *flag_host; done (optional): recorded after the last launch.
 rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipStream_t st, bool refit,
-                         const uint32_t* flag_dev = nullptr, uint32_t* flag_host = nullptr) {
+                         const uint32_t* flag_dev = nullptr, uint32_t* flag_host = nullptr,
+                         hipEvent_t done = nullptr) {
     const uint32_t n = s->n_tris;
     const uint32_t nc = s->n_clusters;
     Temps tmp(ctx);
-    uint32_t *maxd = nullptr, *flag = nullptr, *bidx = nullptr, *ntrav = nullptr;
-    // pre-order positions, first leaf ranks and depths stay with the scene:
-    // the reference node array is written from them on demand
-    // (ensure_ref_nodes), and a refit keeps them
-    if (!s->preorder) RTQ_HIP(ctx, dev_alloc(&s->preorder, nc));
-    if (!s->first_leaf) RTQ_HIP(ctx, dev_alloc(&s->first_leaf, nc));
-    if (!s->node_depth) RTQ_HIP(ctx, dev_alloc(&s->node_depth, nc));
+    // the places stay with the scene: the reference node array is written from
+    // them on demand (ensure_ref_nodes), and a refit keeps them
+    if (!s->placed) RTQ_HIP(ctx, dev_alloc(&s->placed, nc));
     if (!s->sub_roots) RTQ_HIP(ctx, dev_alloc(&s->sub_roots, kLdsClusters + 2));
     if (!s->sub_list) RTQ_HIP(ctx, dev_alloc(&s->sub_list, n));
-    // so is every cluster's traversal node index: a refit needs no new marks
-    if (!s->trav_index) RTQ_HIP(ctx, dev_alloc(&s->trav_index, nc));
-    uint32_t* const pos = s->preorder;
-    uint32_t* const fl = s->first_leaf;
-    uint32_t* const dep = s->node_depth;
-    bidx = s->trav_index;
+    if (!s->nodes) RTQ_HIP(ctx, take(s->kept_nodes, &s->nodes, 4ull * s->n_trav));
+    if (!s->node_aux) RTQ_HIP(ctx, take(s->kept_aux, &s->node_aux, s->n_trav));
     s->ref_ready = false;
-    RTQ_HIP(ctx, tmp.get(&maxd, 2));
-    uint32_t* bdep = nullptr;
-    RTQ_HIP(ctx, tmp.get(&bdep, blocks_for(nc)));
-    RTQ_HIP(ctx, tmp.get(&flag, nc));
-    RTQ_HIP(ctx, tmp.get(&ntrav, 1));
-    const uint32_t root = nc - 1;
+    uint32_t *maxd = nullptr, *bdep = nullptr;
+    RTQ_HIP(ctx, tmp.get(&maxd, 1));
+    RTQ_HIP(ctx, tmp.get(&bdep, blocks_for(n)));
     float* wcost = nullptr;
     uint32_t* wchoice = nullptr;
     SideWork side(ctx);
@@ -1631,7 +1608,7 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipSt
         const uint32_t c_mid = s->sub_from < s->lds_from ? s->passes[s->sub_from].first : c_lo;
         if (cost) RTQ_HIP(ctx, side.fork(st));
         hipLaunchKernelGGL(k_place_lds, dim3(1), dim3(kLdsThreads), 0, st, s->d_passes, s->lds_from, n_passes, c_lo,
-                           nc, c_mid, s->cleft, s->cright, s->ccount, pos, fl, dep, s->sub_roots);
+                           nc, c_mid, n, s->cleft, s->cright, s->ccount, s->ctrav, s->placed, s->sub_roots);
         RTQ_HIP(ctx, hipGetLastError());
         if (cost) {
             rs = wide_cost_bottom(ctx, s, wcost, wchoice, ctx->side);
@@ -1639,7 +1616,7 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipSt
         }
         if (c_mid < c_lo) {
             hipLaunchKernelGGL(k_place_subtrees, dim3(nc - c_lo + 1), dim3(kSubThreads), 0, st, s->sub_roots, c_mid,
-                               s->cleft, s->cright, s->ccount, pos, fl, dep, s->sub_list);
+                               n, s->cleft, s->cright, s->ccount, s->ctrav, s->placed, s->sub_list);
             RTQ_HIP(ctx, hipGetLastError());
         }
         if (cost) {
@@ -1650,70 +1627,45 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipSt
         for (uint32_t k = s->sub_from; k > 0; --k) {
             const auto& pr = s->passes[k - 1];
             hipLaunchKernelGGL(k_place_pass, dim3(blocks_for(pr.second)), dim3(kThreads), 0, st, pr.first, pr.second,
-                               s->cleft, s->cright, s->ccount, pos, fl, dep);
+                               n, s->cleft, s->cright, s->ccount, s->ctrav, s->placed);
             RTQ_HIP(ctx, hipGetLastError());
         }
     }
-    hipLaunchKernelGGL(k_write_leaves, dim3(blocks_for(nc)), dim3(kThreads), 0, st, nc, s->ctri, s->cleft, fl,
-                       dep, s->tri_world, s->tris, bdep);
+    hipLaunchKernelGGL(k_write_leaves, dim3(blocks_for(n)), dim3(kThreads), 0, st, n, s->ctri, s->placed, s->tri_world,
+                       s->tris, bdep);
     RTQ_HIP(ctx, hipGetLastError());
-    // the depth and the traversal node indices depend on the topology only:
-    // a refit keeps them
-    if (!refit) {
-        hipLaunchKernelGGL(k_max_u32, dim3(1), dim3(1024), 0, st, bdep, blocks_for(nc), maxd);
-        RTQ_HIP(ctx, hipGetLastError());
-        if (n > 1) {
-            hipLaunchKernelGGL(k_mark_trav, dim3(blocks_for(nc)), dim3(kThreads), 0, st, nc, root,
-                               s->params.max_leaf_size, s->cleft, s->ccount, pos, flag);
-            RTQ_HIP(ctx, hipGetLastError());
-            rs = scan_u32(ctx, flag, bidx, nc, ntrav, st);
-            if (rs != RTQ_OK) return rs;
-        }
-    }
-
-    // one host read: scene bounds (box pad), and after a build the tree depth
-    // and the traversal node count
-    rtq_aabb h_bounds[2];
-    uint32_t h_depth = s->depth, h_ntrav = refit ? s->n_trav : 1u;
-    HostReads rd(ctx, st);
-    RTQ_HIP(ctx, rd.add(h_bounds, d_bounds, refit ? sizeof(rtq_aabb) : sizeof h_bounds));   // a refit: the root box
-    if (!refit) RTQ_HIP(ctx, rd.add(&h_depth, maxd, sizeof h_depth));
-    if (!refit && n > 1) RTQ_HIP(ctx, rd.add(&h_ntrav, ntrav, sizeof h_ntrav));
-    if (flag_dev) RTQ_HIP(ctx, rd.add(flag_host, flag_dev, sizeof(uint32_t)));
-    RTQ_HIP(ctx, rd.wait());
-    float extent = 0.0f;
-    for (int k = 0; k < 3; ++k)
-        extent = std::max(extent, std::max(std::fabs(h_bounds[0].min[k]), std::fabs(h_bounds[0].max[k])));
-    s->box_pad = std::max(std::ldexp(extent, -18), 1e-30f);
-    s->depth = h_depth;
-
-    const uint32_t max_leaf = s->params.max_leaf_size;
-    if (s->nodes && h_ntrav != s->n_trav)
-        return fail(ctx, RTQ_EINTERNAL, "refit: %u traversal nodes, the tree has %u", h_ntrav, s->n_trav);
-    s->n_trav = h_ntrav;
-    if (!s->nodes) RTQ_HIP(ctx, take(s->kept_nodes, &s->nodes, 4ull * h_ntrav));
-    if (!s->node_aux) RTQ_HIP(ctx, take(s->kept_aux, &s->node_aux, h_ntrav));
-    if (n == 1) {
-        hipLaunchKernelGGL(k_write_single, dim3(1), dim3(1), 0, st, s->cbox, s->box_pad, s->nodes, s->node_aux);
-        RTQ_HIP(ctx, hipGetLastError());
-    } else {
-        hipLaunchKernelGGL(k_write_trav, dim3(blocks_for(nc)), dim3(kThreads), 0, st, nc, root, max_leaf,
-                           s->box_pad, s->cbox, s->cleft, s->cright, s->ccount, pos, fl, bidx, dep, s->nodes,
-                           s->node_aux);
+    if (!refit) {   // the depth depends on the topology only: a refit keeps it
+        hipLaunchKernelGGL(k_max_u32, dim3(1), dim3(1024), 0, st, bdep, blocks_for(n), maxd);
         RTQ_HIP(ctx, hipGetLastError());
     }
+    if (n == 1)
+        hipLaunchKernelGGL(k_write_single, dim3(1), dim3(1), 0, st, d_bounds, s->cbox, s->nodes, s->node_aux);
+    else
+        hipLaunchKernelGGL(k_write_trav, dim3(blocks_for(nc - n)), dim3(kThreads), 0, st, n, nc,
+                           s->params.max_leaf_size, d_bounds, s->cbox, s->cleft, s->cright, s->ccount, s->ctrav,
+                           s->placed, s->nodes, s->node_aux);
+    RTQ_HIP(ctx, hipGetLastError());
+    rs = write_top(ctx, s, st);
+    if (rs != RTQ_OK) return rs;
     if (s->params.node_width == 8) {
         if (refit) {
             rs = refit_wide(ctx, s, st);
         } else {
             RTQ_HIP(ctx, side.join(st));
-            rs = build_wide(ctx, s, wchoice, fl, pos, n == 1 ? nullptr : bidx, st);
+            rs = build_wide(ctx, s, wchoice, d_bounds, st);
         }
         if (rs != RTQ_OK) return rs;
     }
-    rs = write_top(ctx, s, st);
-    if (rs != RTQ_OK) return rs;
-    RTQ_HIP(ctx, hipStreamSynchronize(st));
+    if (done) RTQ_HIP(ctx, hipEventRecord(done, st));
+    // one host read: the scene's box (for the box margin) and after a build the
+    // tree depth
+    rtq_aabb h_bounds;
+    HostReads rd(ctx, st);
+    RTQ_HIP(ctx, rd.add(&h_bounds, d_bounds, sizeof h_bounds));
+    if (!refit) RTQ_HIP(ctx, rd.add(&s->depth, maxd, sizeof s->depth));
+    if (flag_dev) RTQ_HIP(ctx, rd.add(flag_host, flag_dev, sizeof(uint32_t)));
+    RTQ_HIP(ctx, rd.wait());
+    s->box_pad = box_pad_of(h_bounds);
     return RTQ_OK;
 }
 
@@ -1722,12 +1674,12 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipSt
 rtq_status ensure_ref_nodes(rtq_ctx* ctx, Scene* s, hipStream_t st) {
     if (s->ref_ready) return RTQ_OK;
     const uint32_t nc = s->n_clusters;
-    if (!s->built || !s->preorder || nc == 0)
+    if (!s->built || !s->placed || nc == 0)
         return fail(ctx, RTQ_EINTERNAL, "reference nodes: scene has no placed tree");
     if (!s->ref_nodes) RTQ_HIP(ctx, dev_alloc(&s->ref_nodes, nc));
     if (!s->ref_nodes) return fail(ctx, RTQ_ENOMEM, "reference nodes: allocation failed");
     hipLaunchKernelGGL(k_write_ref, dim3(blocks_for(nc)), dim3(kThreads), 0, st, nc, s->cbox, s->ctri, s->cleft,
-                       s->cright, s->preorder, s->ref_nodes);
+                       s->cright, s->placed, s->ref_nodes);
     RTQ_HIP(ctx, hipGetLastError());
     s->ref_ready = true;
     return RTQ_OK;
@@ -1744,14 +1696,13 @@ rtq_status build_scene(rtq_ctx* ctx, Scene* s, const rtq_build_params& prm) {
     s->n_clusters = nc;
     // size the context's scratch for this build's temporaries up front, so a
     // first build does not allocate them one by one.  Alive together, per
-    // triangle: sort keys and values and the PLOC lists 64 B, the traversal
-    // node marks and indices 16 B; with 8-wide nodes also the collapse cost
-    // table 36 B and the collapse's two level lists 8 B per binary traversal
-    // node (one per triangle with leaves of one triangle); the fused PLOC
-    // passes' tile status words (16 passes x 8 B per tile of 480), each
-    // placement workgroup's deepest leaf and the collapse's tile status
-    // words, under n / 2 B; 1 MiB for scans and 256-B rounding
-    const size_t per_tri = prm.node_width == 8 ? 64 + 16 + 36 + 8 : 64 + 16;
+    // triangle: sort keys and values and the PLOC lists 64 B; with 8-wide nodes
+    // also the collapse cost table 36 B and the collapse's two level lists 8 B
+    // per binary traversal node (one per triangle with leaves of one triangle);
+    // the fused PLOC passes' tile status words (16 passes x 8 B per tile of 480),
+    // each leaf workgroup's deepest leaf and the collapse's tile status words,
+    // under n / 2 B; 1 MiB for scans and 256-B rounding
+    const size_t per_tri = prm.node_width == 8 ? 64 + 36 + 8 : 64;
     ctx->arena.peak = std::max<size_t>(ctx->arena.peak, per_tri * n + n / 2 + ((size_t)1 << 20));
     rtq_status rs = arena_reserve(ctx);
     if (rs != RTQ_OK) return rs;
@@ -1772,6 +1723,7 @@ rtq_status build_scene(rtq_ctx* ctx, Scene* s, const rtq_build_params& prm) {
     if (!s->cright) RTQ_HIP(ctx, dev_alloc(&s->cright, nc));
     if (!s->cparent) RTQ_HIP(ctx, dev_alloc(&s->cparent, nc));
     if (!s->ccount) RTQ_HIP(ctx, dev_alloc(&s->ccount, nc));
+    if (!s->ctrav) RTQ_HIP(ctx, dev_alloc(&s->ctrav, nc));
     if (!s->sorted_idx) RTQ_HIP(ctx, dev_alloc(&s->sorted_idx, n));
     if (!s->sorted_codes) RTQ_HIP(ctx, dev_alloc(&s->sorted_codes, n));
     if (!s->tris) RTQ_HIP(ctx, dev_alloc(&s->tris, 3ull * n));
@@ -1808,10 +1760,12 @@ rtq_status build_scene(rtq_ctx* ctx, Scene* s, const rtq_build_params& prm) {
                        s->sorted_idx, n, s->cbox, s->ctri, s->ccount, c_in, b_in);
     RTQ_HIP(ctx, hipGetLastError());
     std::vector<std::pair<uint32_t, uint32_t>> pass_ranges;
+    uint32_t root_trav = 0;
     rs = (prm.flags & RTQ_BUILD_PLOC_SPLIT)
-             ? ploc_split(ctx, s, prm.search_radius, tmp, c_in, c_out, b_in, b_out, pass_ranges, st)
-             : ploc_fused(ctx, s, prm.search_radius, tmp, c_in, c_out, b_in, b_out, pass_ranges, st);
+             ? ploc_split(ctx, s, prm.search_radius, tmp, c_in, c_out, b_in, b_out, pass_ranges, &root_trav, st)
+             : ploc_fused(ctx, s, prm.search_radius, tmp, c_in, c_out, b_in, b_out, pass_ranges, &root_trav, st);
     if (rs != RTQ_OK) return rs;
+    s->n_trav = std::max(root_trav, 1u);   // the root always has a node
     s->ploc_passes = (uint32_t)pass_ranges.size();
     s->passes = pass_ranges;
     // device copy of the pass ranges for the single-workgroup launches of the
@@ -1832,11 +1786,9 @@ rtq_status build_scene(rtq_ctx* ctx, Scene* s, const rtq_build_params& prm) {
 
     // 3-4. node arrays of every layout
     uint32_t h_sort_err = 0;
-    rs = write_layouts(ctx, s, d_bounds, st, false, sort_err, &h_sort_err);
+    rs = write_layouts(ctx, s, d_bounds, st, false, sort_err, &h_sort_err, ev1);
     if (rs != RTQ_OK) return rs;
     if (h_sort_err) return fail(ctx, RTQ_EINTERNAL, "build: a radix sort pass's look-back gave up");
-    RTQ_HIP(ctx, hipEventRecord(ev1, st));
-    RTQ_HIP(ctx, hipEventSynchronize(ev1));
     float ms = 0.0f;
     RTQ_HIP(ctx, hipEventElapsedTime(&ms, ev0, ev1));
     s->build_ms = ms;
@@ -1851,17 +1803,10 @@ rtq_status write_top(rtq_ctx* ctx, Scene* s, hipStream_t st) {
     if (kTopNodes == 0) return RTQ_OK;
     // the set depends on the topology only, so a refit or an order update
     // rewrites the same buffer with the same node count
-    // one float4 past the nodes holds the node count
-    if (!s->top) RTQ_HIP(ctx, dev_alloc(&s->top, 4ull * kTopNodes + 1));
-    uint32_t* d_n = reinterpret_cast<uint32_t*>(s->top + 4ull * kTopNodes);
-    hipLaunchKernelGGL(k_top_nodes, dim3(1), dim3(64), 0, st, s->nodes, s->top, d_n);
-    hipError_t e = hipGetLastError();
-    uint32_t n = 0;
-    HostReads rd(ctx, st);
-    if (e == hipSuccess) e = rd.add(&n, d_n, sizeof n);
-    if (e == hipSuccess) e = rd.wait();
-    if (e != hipSuccess) return hip_fail(ctx, e, "write_top");
-    s->n_top = n;
+    if (!s->top) RTQ_HIP(ctx, dev_alloc(&s->top, 4ull * kTopNodes));
+    hipLaunchKernelGGL(k_top_nodes, dim3(1), dim3(64), 0, st, s->nodes, s->top);
+    RTQ_HIP(ctx, hipGetLastError());
+    s->n_top = std::min(kTopNodes, s->n_trav);   // every traversal node can be reached from the root
     return RTQ_OK;
 }
 
@@ -1888,7 +1833,7 @@ rtq_status refit_scene(rtq_ctx* ctx, Scene* s) {
     if (s->sub_from < s->lds_from) {
         const uint32_t blocks = s->n_clusters - s->passes[s->lds_from].first + 1;
         hipLaunchKernelGGL(k_refit_subtrees, dim3(blocks), dim3(kSubThreads), 0, st, s->sub_roots, s->sub_list,
-                           s->first_leaf, s->cleft, s->cright, s->cbox);
+                           s->placed, s->cleft, s->cright, s->cbox);
         RTQ_HIP(ctx, hipGetLastError());
     }
     if (s->lds_from < n_passes) {

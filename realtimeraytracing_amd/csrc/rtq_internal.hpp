@@ -55,12 +55,10 @@ struct Scene {
     uint32_t* sorted_codes = nullptr;   // N
     rtq_bvh_node* ref_nodes = nullptr;  // 2N - 1 pre-order nodes (reference layout), written on demand
     bool ref_ready = false;             // ref_nodes matches the current tree and boxes
-    uint32_t* preorder = nullptr;       // pre-order position of every cluster (2N - 1)
-    uint32_t* first_leaf = nullptr;     // rank of the first leaf below every cluster (2N - 1)
-    uint32_t* node_depth = nullptr;     // depth of every cluster (2N - 1)
+    uint32_t* ctrav = nullptr;          // binary traversal nodes in each merged cluster's subtree, itself included
+    uint4* placed = nullptr;            // every cluster's place in the tree (Place, 2N - 1)
     uint2* sub_roots = nullptr;         // .x = number of middle subtrees, then each one's (root, listed clusters)
     uint32_t* sub_list = nullptr;       // N: each one's clusters level by level, from its first leaf's rank on
-    uint32_t* trav_index = nullptr;     // binary traversal node of every cluster (2N - 1), kNone if none
     float4* nodes = nullptr;            // traversal nodes, 4 float4 (64 B) each
     uint4* node_aux = nullptr;          // per traversal node: child leaf ranges [A,B) [B,C), depth
     bool ordered = false;               // learned child-order words stored in the nodes
@@ -333,13 +331,36 @@ rtq_status noalloc_setup(rtq_ctx* ctx);
 rtq_status trace_noalloc(rtq_ctx* ctx, const Scene* s, const rtq_ray* rays, uint64_t n, uint32_t flags,
                          rtq_hit* hits, hipStream_t st);
 void scratch_free(TraceScratch* sc);
-// Compressed 8-wide nodes from the cluster arrays (fl: first leaf rank per cluster).
-// pos, bidx: pre-order position of every cluster and binary traversal index
-// of every position (null for a one-triangle scene, which has no binary node).
+// A cluster's place in the tree, one 16-B word of Scene::placed: pre-order
+// position, rank of the first leaf below it, depth, and the index of its binary
+// traversal node, the number of those before it in pre-order (only if it has
+// one: merged, and the root or of more than max_leaf_size triangles).
+struct Place {
+    uint32_t pos, first, depth, trav;
+};
+__device__ __forceinline__ Place place_of(uint4 v) { return {v.x, v.y, v.z, v.w}; }
+// The places of the children of a cluster placed at p: the left child right
+// after it, the right one after the left subtree of lc triangles and lt
+// traversal nodes (scene.cpp:189-201).
+__device__ __forceinline__ uint4 left_place(const Place& p) {
+    return make_uint4(p.pos + 1, p.first, p.depth + 1, p.trav + 1);
+}
+__device__ __forceinline__ uint4 right_place(const Place& p, uint32_t lc, uint32_t lt) {
+    return make_uint4(p.pos + 2 * lc, p.first + lc, p.depth + 1, p.trav + 1 + lt);
+}
+
+// Margin of every stored box: the largest coordinate magnitude of the scene
+// bounds times 2^-18.
+__host__ __device__ __forceinline__ float box_pad_of(const rtq_aabb& b) {
+    float e = 0.0f;
+    for (int k = 0; k < 3; ++k) e = fmaxf(e, fmaxf(fabsf(b.min[k]), fabsf(b.max[k])));
+    return fmaxf(e * 0x1p-18f, 1e-30f);
+}
+
+// Compressed 8-wide nodes from the cluster arrays.  bounds: the scene's (device).
 // choice: the collapse's cost-table decisions (wide_cost_top), null for a
 // one-triangle scene.
-rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const uint32_t* fl, const uint32_t* pos,
-                      const uint32_t* bidx, hipStream_t st);
+rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const rtq_aabb* bounds, hipStream_t st);
 // Clusters created by the passes from Scene::lds_from on: at most this many
 // (their placement state, 12 B each, and cost rows, 32 B each, in LDS).
 constexpr uint32_t kLdsClusters = 4096;
@@ -363,8 +384,8 @@ constexpr int kSubThreads = 64;
 // binary layout's placement.
 rtq_status wide_cost_bottom(rtq_ctx* ctx, const Scene* s, float* cost, uint32_t* choice, hipStream_t st);
 rtq_status wide_cost_top(rtq_ctx* ctx, const Scene* s, float* cost, uint32_t* choice, hipStream_t st);
-// New boxes for the kept 8-wide nodes after a refit (the cluster boxes and
-// box pad already refitted): one launch over the nodes, child refs kept.
+// New boxes for the kept 8-wide nodes after a refit (the cluster boxes already
+// refitted): one launch over the nodes, child refs kept.
 rtq_status refit_wide(rtq_ctx* ctx, Scene* s, hipStream_t st);
 // Learned first-child tables of the 8-wide nodes from the binary nodes' order
 // words (learned.hip); clear = zero them.

@@ -118,7 +118,7 @@ __global__ __launch_bounds__(kThreads) void k_dp_pass(uint32_t first, uint32_t c
 // level first.
 __global__ __launch_bounds__(kSubThreads) void k_dp_subtrees(const uint2* __restrict__ roots,
                                                              const uint32_t* __restrict__ list,
-                                                             const uint32_t* __restrict__ fl, uint32_t nt,
+                                                             const uint4* __restrict__ placed, uint32_t nt,
                                                              uint32_t max_leaf, const uint32_t* __restrict__ cleft,
                                                              const uint32_t* __restrict__ cright,
                                                              const uint32_t* __restrict__ ccount,
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(kSubThreads) void k_dp_subtrees(const uint2* __rest
                                                              uint32_t* __restrict__ choice) {
     if (blockIdx.x >= roots[0].x) return;
     const uint2 root = roots[1 + blockIdx.x];
-    levels_up(list + fl[root.x], root.y,
+    levels_up(list + placed[root.x].y, root.y,
               [&](uint32_t c) { dp_cluster(c, nt, max_leaf, cleft, cright, ccount, cbox, cost, choice); });
 }
 
@@ -314,7 +314,7 @@ struct LevelArgs {
     uint32_t* err;
     uint32_t max_leaf;
     uint32_t nt;
-    float pad;
+    const rtq_aabb* bounds;    // the scene's, for the box margin
     const uint32_t* items;     // this level's node clusters
     uint32_t* next_items;      // the next level's
     const uint32_t* cleft;
@@ -322,9 +322,7 @@ struct LevelArgs {
     const uint32_t* ccount;
     const rtq_aabb* cbox;
     const uint32_t* choice;
-    const uint32_t* fl;
-    const uint32_t* pos;
-    const uint32_t* bidx;
+    const uint4* placed;
     float4* nodes;
     uint32_t* wide_trav;
     uint32_t* kids;            // 8 child clusters per node (kNone past the last)
@@ -370,7 +368,7 @@ __global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
     const uint32_t slot = has ? __popc(mask & below) : n + __popc(~mask & below);
     const uint32_t cnt = has ? a.ccount[c] : 0u;
     const rtq_aabb box = a.cbox[c];
-    const uint32_t first = has ? a.fl[c] : 0u;
+    const uint32_t first = has ? a.placed[c].y : 0u;
     const bool expand = has && c >= a.nt && cnt > a.max_leaf;   // an 8-wide node of the next level
     // exclusive sum of the expandable children over the workgroup
     const uint64_t em = __ballot(expand);
@@ -452,7 +450,7 @@ __global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
     }
 
     uint32_t* const img = s_img + (tid / kWidth) * kImageWords;
-    wide_boxes(live, has, slot, n, box, a.pad, img);
+    wide_boxes(live, has, slot, n, box, box_pad_of(a.bounds[0]), img);
     // an empty slot's box is inverted (wide_boxes); should a far ray still enter
     // it, its ref is the leaf of traversal triangle 0 alone: a real triangle, so
     // whatever that test reports is a genuine hit
@@ -473,8 +471,9 @@ __global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
         img[24 + slot] = 0;
         // the node's child clusters, for a refit
         a.kids[8ull * (level_base + k) + slot] = has ? c : kNone;
-        // the binary traversal node of this node's root cluster (learned order)
-        if (slot == 0) a.wide_trav[level_base + k] = a.bidx ? a.bidx[a.pos[c0]] : kNone;
+        // the binary traversal node of this node's root cluster (learned order;
+        // a scene of one triangle has none)
+        if (slot == 0) a.wide_trav[level_base + k] = c0 >= a.nt ? a.placed[c0].w : kNone;
     }
     wave_lds_fence();
     if (live)
@@ -485,7 +484,7 @@ __global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
 // clusters (kids, kNone past the last) quantised again from their refitted
 // boxes; child refs stay, learned tables are cleared.
 __global__ __launch_bounds__(kThreads) void k_wide_refit(uint32_t n_wide, const uint32_t* __restrict__ kids,
-                                                         const rtq_aabb* __restrict__ cbox, float pad,
+                                                         const rtq_aabb* __restrict__ cbox, uint32_t root,
                                                          float4* __restrict__ nodes) {
     __shared__ __align__(16) uint32_t s_img[kThreads / kWidth * kImageWords];
     const uint32_t tid = threadIdx.x, slot = tid % kWidth;
@@ -497,7 +496,7 @@ __global__ __launch_bounds__(kThreads) void k_wide_refit(uint32_t n_wide, const 
     const uint32_t n = __popc((uint32_t)(__ballot(has) >> group) & 0xFFu);
     const rtq_aabb box = cbox[has ? c : 0u];
     uint32_t* const img = s_img + (tid / kWidth) * kImageWords;
-    wide_boxes(live, has, slot, n, box, pad, img);
+    wide_boxes(live, has, slot, n, box, box_pad_of(cbox[root]), img);
     if (live) img[24 + slot] = 0;
     wave_lds_fence();
     if (live && (slot < 4 || slot == 6))
@@ -524,7 +523,7 @@ rtq_status wide_cost_top(rtq_ctx* ctx, const Scene* s, float* cost, uint32_t* ch
     const uint32_t nt = s->n_tris, max_leaf = s->params.max_leaf_size, c_lo = s->passes[s->lds_from].first;
     if (s->sub_from < s->lds_from) {
         hipLaunchKernelGGL(k_dp_subtrees, dim3(s->n_clusters - c_lo + 1), dim3(kSubThreads), 0, st, s->sub_roots,
-                           s->sub_list, s->first_leaf, nt, max_leaf, s->cleft, s->cright, s->ccount, s->cbox, cost,
+                           s->sub_list, s->placed, nt, max_leaf, s->cleft, s->cright, s->ccount, s->cbox, cost,
                            choice);
         RTQ_HIP(ctx, hipGetLastError());
     }
@@ -536,10 +535,8 @@ rtq_status wide_cost_top(rtq_ctx* ctx, const Scene* s, float* cost, uint32_t* ch
 }
 
 // Builds s->wide (s->n_wide nodes, s->wide_depth levels) from the cluster
-// arrays and the cost table's choices; fl = first leaf rank of every cluster
-// (device).
-rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const uint32_t* fl, const uint32_t* pos,
-                      const uint32_t* bidx, hipStream_t st) {
+// arrays and the cost table's choices.
+rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const rtq_aabb* bounds, hipStream_t st) {
     const uint32_t nc = s->n_clusters;
     const uint32_t root = nc - 1;
     const uint32_t cap = std::max<uint32_t>(s->n_trav, 1);  // wide nodes are a subset of the binary ones
@@ -549,8 +546,9 @@ rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const uint
     RTQ_HIP(ctx, tmp.get(&items, cap));
     RTQ_HIP(ctx, tmp.get(&next, cap));
     // tile status words of every level's scan: a level of c nodes takes
-    // ceil(c / kLevelNodes) of them, and there are at most depth + 1 levels
-    const uint32_t n_status = cap / kLevelNodes + s->depth + 2;
+    // ceil(c / kLevelNodes) of them, and there are at most depth + 1 levels,
+    // the depth no more than the PLOC passes
+    const uint32_t n_status = cap / kLevelNodes + s->ploc_passes + 2;
     uint64_t* status = nullptr;
     // and before them two sets of tile counters: a level clears the next one's
     constexpr uint32_t kTickets = 2 * kTicketWords / 2;
@@ -582,15 +580,13 @@ rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const uint
     la.err = err;
     la.max_leaf = s->params.max_leaf_size;
     la.nt = s->n_tris;
-    la.pad = s->box_pad;
+    la.bounds = bounds;
     la.cleft = s->cleft;
     la.cright = s->cright;
     la.ccount = s->ccount;
     la.cbox = s->cbox;
     la.choice = choice;
-    la.fl = fl;
-    la.pos = pos;
-    la.bidx = bidx;
+    la.placed = s->placed;
     la.nodes = s->wide;
     la.wide_trav = s->wide_trav;
     la.kids = s->wide_kids;
@@ -639,7 +635,7 @@ rtq_status refit_wide(rtq_ctx* ctx, Scene* s, hipStream_t st) {
     if (!s->wide || !s->wide_kids) return fail(ctx, RTQ_EINTERNAL, "refit: the scene has no 8-wide nodes");
     if (s->n_wide == 0) return RTQ_OK;
     hipLaunchKernelGGL(k_wide_refit, dim3(blocks_for(8ull * s->n_wide)), dim3(kThreads), 0, st, s->n_wide, s->wide_kids,
-                       s->cbox, s->box_pad, s->wide);
+                       s->cbox, s->n_clusters - 1, s->wide);
     RTQ_HIP(ctx, hipGetLastError());
     s->wide_ordered = false;   // the tables were cleared
     return RTQ_OK;

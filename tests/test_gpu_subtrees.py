@@ -1,7 +1,8 @@
 """Placement and refit of trees whose passes run in one workgroup's LDS, as
 subtrees below them and in launches of their own: positions and children of
-every node against a walk of the exported clusters, and after new vertices every
-box against its children's."""
+every node against a walk of the exported clusters, the binary traversal nodes
+against that walk's marks in pre-order, and after new vertices every box against
+its children's."""
 import numpy as np
 import pytest
 
@@ -19,17 +20,33 @@ def test_placement_and_refit(rtq_ctx, n, width):
         cl, ref = sc.export_clusters(), sc.export_ref()
         left, right = cl["left"].astype(np.int64), cl["right"].astype(np.int64)
         nc = 2 * n - 1
-        count, pos = np.ones(nc, np.int64), np.zeros(nc, np.int64)
+        count, pos, first, depth = (np.full(nc, v, np.int64) for v in (1, 0, 0, 0))
         for c in range(n, nc):
             count[c] = count[left[c]] + count[right[c]]
         for c in range(nc - 1, n - 1, -1):
             pos[left[c]] = pos[c] + 1
             pos[right[c]] = pos[c] + 2 * count[left[c]]
+            first[left[c]], first[right[c]] = first[c], first[c] + count[left[c]]
+            depth[left[c]] = depth[right[c]] = depth[c] + 1
         assert np.array_equal(np.sort(pos), np.arange(nc))
         inner = np.arange(n, nc)
         assert np.array_equal(ref["left_child"][pos[inner]], pos[left[inner]])
         assert np.array_equal(ref["right_child"][pos[inner]], pos[right[inner]])
         assert np.array_equal(ref["triangle_id"][pos[:n]], cl["triangle_id"][:n])
+
+        # the traversal nodes: clusters of more than 4 triangles and the root, in pre-order
+        has = inner[(count[inner] > 4) | (inner == nc - 1)]
+        has = has[np.argsort(pos[has])]
+        index = np.full(nc, -1, np.int64)
+        index[has] = np.arange(len(has))
+        nodes, ranges = sc.export_trav()
+        middle = first[has] + count[left[has]]
+        assert np.array_equal(ranges, np.stack([first[has], middle, first[has] + count[has], depth[has]], axis=1))
+        refs = nodes.view(np.uint32)[:, 12:14]
+        for k, child in enumerate((left[has], right[has])):
+            leaf = 0x80000000 | first[child] << 3 | (count[child] - 1)
+            assert np.array_equal(refs[:, k], np.where(index[child] >= 0, index[child], leaf))
+        assert sc.info().depth == depth.max()
 
         moved = tris.copy()
         for k in ("p0", "p1", "p2"):
