@@ -104,12 +104,11 @@ __global__ __launch_bounds__(kSubThreads) void k_refit_subtrees(const uint2* __r
               [&](uint32_t c) { cbox[c] = merged_box(cbox[cleft[c]], cbox[cright[c]]); });
 }
 
-// The passes [k0, k1) at the top of the tree in one workgroup, in build order,
+// The passes at the top of the tree in one workgroup, in build order,
 // with the boxes of their clusters [c_lo, nc) in LDS (a child from an earlier
 // pass gives its box from global memory); a barrier between passes, and the
 // range's boxes written back at the end.  nc - c_lo <= kLdsClusters.
-__global__ __launch_bounds__(kLdsThreads) void k_refit_merge_lds(const uint2* __restrict__ passes, uint32_t k0,
-                                                                 uint32_t k1, uint32_t c_lo, uint32_t nc,
+__global__ __launch_bounds__(kLdsThreads) void k_refit_merge_lds(TopPasses passes, uint32_t c_lo, uint32_t nc,
                                                                  const uint32_t* __restrict__ cleft,
                                                                  const uint32_t* __restrict__ cright,
                                                                  rtq_aabb* __restrict__ cbox) {
@@ -124,7 +123,7 @@ __global__ __launch_bounds__(kLdsThreads) void k_refit_merge_lds(const uint2* __
         L[q] = idx < R ? cleft[c_lo + idx] : 0u;
         Rc[q] = idx < R ? cright[c_lo + idx] : 0u;
     }
-    for (uint32_t k = k0; k < k1; ++k) {
+    for (uint32_t k = 0; k < passes.n; ++k) {
         const uint2 p = passes[k];
 #pragma unroll
         for (int q = 0; q < kSlots; ++q) {
@@ -155,7 +154,26 @@ __global__ __launch_bounds__(kLdsThreads) void k_refit_merge_lds(const uint2* __
 // before right) order with a wave prefix sum, which is the order a FIFO
 // breadth-first walk appends them; children past kTopNodes keep their refs.
 static_assert(kTopNodes <= 64, "one lane per top-of-tree slot");
-__global__ __launch_bounds__(64) void k_top_nodes(const float4* __restrict__ nodes, float4* __restrict__ top) {
+// A second workgroup, if launched, takes the maximum of block_depth.
+constexpr int kTopThreads = 1024;
+__global__ __launch_bounds__(kTopThreads) void k_top_nodes(const float4* __restrict__ nodes, float4* __restrict__ top,
+                                                           const uint32_t* __restrict__ block_depth, uint32_t n_blocks,
+                                                           uint32_t* __restrict__ depth) {
+    if (blockIdx.x == 1) {
+        __shared__ uint32_t s_max[kTopThreads / 64];
+        uint32_t m = 0;
+        for (uint32_t i = threadIdx.x; i < n_blocks; i += kTopThreads) m = max(m, block_depth[i]);
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) m = max(m, (uint32_t)__shfl_xor(m, d, 64));
+        if ((threadIdx.x & 63) == 0) s_max[threadIdx.x / 64] = m;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (uint32_t w = 1; w < kTopThreads / 64; ++w) m = max(m, s_max[w]);
+            *depth = m;
+        }
+        return;
+    }
+    if (threadIdx.x >= 64) return;
     __shared__ uint32_t s_q[64];
     const uint32_t lane = threadIdx.x;
     uint32_t node = 0;                 // node index of slot `lane` once its level is reached
@@ -238,7 +256,7 @@ __global__ __launch_bounds__(kThreads) void k_bounds_partial(const rtq_triangle*
 }
 
 // Reduces the partial boxes, then (one thread) the circumscribed cube of
-// bvh.cpp:253-303.  out[0] = scene box, out[1] = cube.
+// bvh.cpp:253-303.  out[0] = scene box, out[1] = cube, one word zero after them.
 __global__ __launch_bounds__(kThreads) void k_bounds_final(const float* __restrict__ partial, uint32_t nb,
                                                            uint32_t n, uint32_t pad_origin,
                                                            rtq_aabb* __restrict__ out) {
@@ -293,6 +311,7 @@ __global__ __launch_bounds__(kThreads) void k_bounds_final(const float* __restri
         delta = (max_dist - dist_y) / 2.0f; c.max[1] += delta; c.min[1] -= delta;
     }
     out[1] = c;
+    *reinterpret_cast<uint32_t*>(out + 2) = 0;
 }
 
 // ------------------------------------------------------------- Morton codes
@@ -425,28 +444,26 @@ __device__ __forceinline__ uint32_t nearest_in_window(const Box6* w, int i, int 
     return arg;
 }
 
-__global__ __launch_bounds__(kThreads) void k_cluster_init(uint32_t n, uint32_t* __restrict__ cparent,
-                                                           uint32_t* __restrict__ cleft,
-                                                           uint32_t* __restrict__ cright,
-                                                           uint32_t* __restrict__ ctri) {
-    const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
-    if (c >= 2 * n - 1) return;
-    cparent[c] = kNone;
-    cleft[c] = kNone;
-    cright[c] = kNone;
-    ctri[c] = 0;
-}
+// plocPreprocessing, bvh.cpp:26-46: the clusters of one triangle each (the merges
+// write everything of the others but the root's parent), the list they start as
+// and, unless null, the fused passes' state (kPlocHeadWords words).
+constexpr uint32_t kPlocBatch = 16;
+constexpr uint32_t kPlocHeadWords = 16 + 4 * kPlocBatch;   // state (8), errors and tail pass count (8), pass log
 
-// plocPreprocessing, bvh.cpp:26-46.
 __global__ __launch_bounds__(kThreads) void k_leaf_init(const rtq_triangle* __restrict__ tris,
                                                         const DevModel* __restrict__ models,
                                                         const uint32_t* __restrict__ sorted_idx,
                                                         uint32_t n, rtq_aabb* __restrict__ cbox,
                                                         uint32_t* __restrict__ ctri,
                                                         uint32_t* __restrict__ ccount,
+                                                        uint32_t* __restrict__ cleft,
+                                                        uint32_t* __restrict__ cright,
+                                                        uint32_t* __restrict__ cparent,
                                                         uint32_t* __restrict__ c_in,
-                                                        Box6* __restrict__ b_in) {
+                                                        Box6* __restrict__ b_in, uint32_t* __restrict__ state) {
     const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+    if (i == 0) cparent[2 * n - 2] = kNone;
+    if (state && i < 16) state[i] = i < 2 ? n : 0u;
     if (i >= n) return;
     // in range even after a failed sort (which fails the build)
     const uint32_t ti = min(sorted_idx[i], n - 1);
@@ -458,6 +475,8 @@ __global__ __launch_bounds__(kThreads) void k_leaf_init(const rtq_triangle* __re
     cbox[i] = a;
     ctri[i] = ti;
     ccount[i] = 1;
+    cleft[i] = kNone;
+    cright[i] = kNone;
     c_in[i] = i;
     b_in[i] = b;
 }
@@ -1158,7 +1177,7 @@ __global__ __launch_bounds__(kSubThreads) void k_place_subtrees(uint2* roots, ui
     if (lane == 0) roots[1 + blockIdx.x].y = end;
 }
 
-// The passes [k0, k1) at the top of the tree in one workgroup, last pass
+// The passes at the top of the tree in one workgroup, last pass
 // first, with the places of their clusters [c_lo, nc) in LDS: a pass reads and
 // writes LDS only, a barrier between passes.  Children from earlier passes get
 // their places in global memory, and those from c_mid on are the roots of the
@@ -1166,8 +1185,8 @@ __global__ __launch_bounds__(kSubThreads) void k_place_subtrees(uint2* roots, ui
 // at the end.  Each thread keeps the child ids and the left child's counts of
 // its clusters c_lo + t + kLdsThreads * s in registers.  1 <= nc - c_lo <=
 // kLdsClusters.
-__global__ __launch_bounds__(kLdsThreads) void k_place_lds(const uint2* __restrict__ passes, uint32_t k0, uint32_t k1,
-                                                           uint32_t c_lo, uint32_t nc, uint32_t c_mid, uint32_t nt,
+__global__ __launch_bounds__(kLdsThreads) void k_place_lds(TopPasses passes, uint32_t c_lo, uint32_t nc,
+                                                           uint32_t c_mid, uint32_t nt,
                                                            const uint32_t* __restrict__ cleft,
                                                            const uint32_t* __restrict__ cright,
                                                            const uint32_t* __restrict__ ccount,
@@ -1197,7 +1216,7 @@ __global__ __launch_bounds__(kLdsThreads) void k_place_lds(const uint2* __restri
         s_roots = 0;
     }
     __syncthreads();
-    for (uint32_t k = k1; k > k0; --k) {
+    for (uint32_t k = passes.n; k > 0; --k) {
         const uint2 p = passes[k - 1];
 #pragma unroll
         for (int q = 0; q < kSlots; ++q) {
@@ -1232,11 +1251,11 @@ __global__ __launch_bounds__(kLdsThreads) void k_place_lds(const uint2* __restri
 }
 
 // Leaf-ordered traversal triangles, and the depth of each workgroup's deepest
-// leaf in block_depth[blockIdx.x] (k_max_u32 takes the maximum: atomics of
+// leaf in block_depth[blockIdx.x] (k_top_nodes takes the maximum: atomics of
 // every wave on one word would serialise, tens of thousands of them).
-__global__ __launch_bounds__(kThreads) void k_write_leaves(
-    uint32_t n, const uint32_t* __restrict__ ctri, const uint4* __restrict__ placed,
-    const float4* __restrict__ tri_world, float4* __restrict__ tris, uint32_t* __restrict__ block_depth) {
+__device__ __forceinline__ void write_leaves(uint32_t n, const uint32_t* __restrict__ ctri,
+                                             const uint4* __restrict__ placed, const float4* __restrict__ tri_world,
+                                             float4* __restrict__ tris, uint32_t* __restrict__ block_depth) {
     __shared__ uint32_t s_max[kThreads / 64];
     const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
     uint32_t depth = 0;
@@ -1257,22 +1276,6 @@ __global__ __launch_bounds__(kThreads) void k_write_leaves(
         uint32_t m = 0;
         for (uint32_t w = 0; w < kThreads / 64; ++w) m = max(m, s_max[w]);
         block_depth[blockIdx.x] = m;
-    }
-}
-
-// out[0] = max of v[0..n) (one workgroup of 1024 lanes).
-__global__ __launch_bounds__(1024) void k_max_u32(const uint32_t* __restrict__ v, uint32_t n,
-                                                  uint32_t* __restrict__ out) {
-    __shared__ uint32_t s_max[16];
-    uint32_t m = 0;
-    for (uint32_t i = threadIdx.x; i < n; i += 1024) m = max(m, v[i]);
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) m = max(m, (uint32_t)__shfl_xor(m, d, 64));
-    if ((threadIdx.x & 63) == 0) s_max[threadIdx.x / 64] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (uint32_t w = 1; w < 16; ++w) m = max(m, s_max[w]);
-        out[0] = m;
     }
 }
 
@@ -1300,22 +1303,21 @@ __global__ __launch_bounds__(kThreads) void k_write_ref(
 //   [c0.lo.x c0.hi.x c0.lo.y c0.hi.y] [c0.lo.z c0.hi.z c1.lo.x c1.hi.x]
 //   [c1.lo.y c1.hi.y c1.lo.z c1.hi.z] [ref0 ref1 order 0]
 // where `order` holds the learned child-order bits (zero until a model is applied).
-// One thread per merged cluster; what a child needs besides its box follows from
-// the node's own place and the counts below the children.  2,095,104 triangles:
-// 150 us when a child's index came from a scan over marks in pre-order, 61 us
-// with the counts that PLOC's merges keep (they cost its passes nothing).
-__global__ __launch_bounds__(kThreads) void k_write_trav(
-    uint32_t nt, uint32_t nc, uint32_t max_leaf, const rtq_aabb* __restrict__ bounds,
-    const rtq_aabb* __restrict__ cbox, const uint32_t* __restrict__ cleft, const uint32_t* __restrict__ cright,
-    const uint32_t* __restrict__ ccount, const uint32_t* __restrict__ ctrav, const uint4* __restrict__ placed,
-    float4* __restrict__ nodes, uint4* __restrict__ aux) {
-    const uint32_t c = nt + blockIdx.x * kThreads + threadIdx.x;
-    if (c >= nc || !(ccount[c] > max_leaf || c == nc - 1)) return;
+// One thread per merged cluster c; what a child needs besides its box follows
+// from the node's own place and the counts below the children.  2,095,104
+// triangles: 150 us when a child's index came from a scan over marks in
+// pre-order, 61 us with the counts that PLOC's merges keep (they cost its passes
+// nothing).
+__device__ __forceinline__ void write_trav(uint32_t c, uint32_t nt, uint32_t nc, uint32_t max_leaf, float pad,
+                                           const rtq_aabb* __restrict__ cbox, const uint32_t* __restrict__ cleft,
+                                           const uint32_t* __restrict__ cright, const uint32_t* __restrict__ ccount,
+                                           const uint32_t* __restrict__ ctrav, const uint4* __restrict__ placed,
+                                           float4* __restrict__ nodes, uint4* __restrict__ aux) {
+    if (!(ccount[c] > max_leaf || c == nc - 1)) return;
     const uint32_t l = cleft[c], r = cright[c];
     const Place p = place_of(placed[c]);
     const rtq_aabb bl = cbox[l], br = cbox[r];
     const uint32_t lc = ccount[l], rc = ccount[r], lt = l < nt ? 0u : ctrav[l];
-    const float pad = box_pad_of(bounds[0]);
     const uint32_t middle = p.first + lc;
     const uint32_t r0 = l >= nt && lc > max_leaf ? p.trav + 1 : leaf_ref(p.first, lc);
     const uint32_t r1 = r >= nt && rc > max_leaf ? p.trav + 1 + lt : leaf_ref(middle, rc);
@@ -1330,10 +1332,8 @@ __global__ __launch_bounds__(kThreads) void k_write_trav(
 }
 
 // Single-triangle scene: one node whose two children are the same leaf.
-__global__ void k_write_single(const rtq_aabb* __restrict__ bounds, const rtq_aabb* __restrict__ cbox,
-                               float4* __restrict__ nodes, uint4* __restrict__ aux) {
-    const rtq_aabb a = cbox[0];
-    const float pad = box_pad_of(bounds[0]);
+__device__ __forceinline__ void write_single(const rtq_aabb& a, float pad, float4* __restrict__ nodes,
+                                             uint4* __restrict__ aux) {
     float lo[3], hi[3];
     for (int k = 0; k < 3; ++k) { lo[k] = a.min[k] - pad; hi[k] = a.max[k] + pad; }
     const uint32_t r = leaf_ref(0, 1);
@@ -1344,17 +1344,40 @@ __global__ void k_write_single(const rtq_aabb* __restrict__ bounds, const rtq_aa
     aux[0] = make_uint4(0u, 1u, 1u, 0u);
 }
 
+// The traversal triangles (the first leaf_blocks workgroups) and the binary
+// traversal nodes (the others) in one launch: neither reads what the other
+// writes.
+__global__ __launch_bounds__(kThreads) void k_write_layout(
+    uint32_t leaf_blocks, uint32_t nt, uint32_t nc, uint32_t max_leaf, const rtq_aabb* __restrict__ bounds,
+    const uint32_t* __restrict__ ctri, const float4* __restrict__ tri_world, const rtq_aabb* __restrict__ cbox,
+    const uint32_t* __restrict__ cleft, const uint32_t* __restrict__ cright, const uint32_t* __restrict__ ccount,
+    const uint32_t* __restrict__ ctrav, const uint4* __restrict__ placed, float4* __restrict__ tris,
+    uint32_t* __restrict__ block_depth, float4* __restrict__ nodes, uint4* __restrict__ aux) {
+    if (blockIdx.x < leaf_blocks) {
+        write_leaves(nt, ctri, placed, tri_world, tris, block_depth);
+        return;
+    }
+    const uint32_t i = (blockIdx.x - leaf_blocks) * kThreads + threadIdx.x;
+    const float pad = box_pad_of(bounds[0]);
+    if (nc == 1) {
+        if (i == 0) write_single(cbox[0], pad, nodes, aux);
+    } else if (nt + i < nc) {
+        write_trav(nt + i, nt, nc, max_leaf, pad, cbox, cleft, cright, ccount, ctrav, placed, nodes, aux);
+    }
+}
+
 inline uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + kThreads - 1) / kThreads); }
 
 // Shared front half of the build and of rtq_morton_codes: scene box + cube.
-// d_bounds holds 2 boxes followed by 6 floats per partial block (at most
-// kBoundsPartials): kBoundsBoxes boxes of 32 B.
+// d_bounds holds 2 boxes, the words that a build reads back with them (8, the
+// first one zeroed here: the sort's errors, then the depth), and 6 floats per
+// partial block (at most kBoundsPartials): kBoundsBoxes boxes of 32 B.
 constexpr uint32_t kBoundsPartials = 1024;
-constexpr uint32_t kBoundsBoxes = 2 + (6 * kBoundsPartials + 7) / 8;
+constexpr uint32_t kBoundsBoxes = 3 + (6 * kBoundsPartials + 7) / 8;
 rtq_status compute_bounds(rtq_ctx* ctx, Scene* s, uint32_t pad_origin, rtq_aabb* d_bounds,
                           hipStream_t st) {
     const uint32_t nb = std::min<uint32_t>(blocks_for(s->n_tris), kBoundsPartials);
-    float* partial = reinterpret_cast<float*>(d_bounds + 2);
+    float* partial = reinterpret_cast<float*>(d_bounds + 3);
     hipLaunchKernelGGL(k_bounds_partial, dim3(nb), dim3(kThreads), 0, st, s->tris_ref, s->models,
                        s->n_tris, partial);
     RTQ_HIP(ctx, hipGetLastError());
@@ -1368,34 +1391,26 @@ rtq_status compute_bounds(rtq_ctx* ctx, Scene* s, uint32_t pad_origin, rtq_aabb*
 // PLOC with fused passes: batches of kPlocBatch k_ploc_pass launches (each a
 // no-op once at most kTailMax clusters are left) and one k_ploc_tail launch
 // (a no-op until then), then one read of the state and the pass logs.  The
-// active list starts in (c0, b0); c1, b1 are the other buffers.  A batch's
+// active list starts in (c0, b0); c1, b1 are the other buffers.  state: the
+// kPlocHeadWords words that k_leaf_init set, then room for the tail's log.  A batch's
 // passes all take the grid of its first pass; 16 passes per batch bring a
 // 2M-triangle terrain (61 passes) to the tail in two host round trips.
 // root_trav: the traversal nodes in the whole tree (Scene::ctrav of the root).
-rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint32_t* c0, uint32_t* c1,
+rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint32_t* state, uint32_t* c0, uint32_t* c1,
                       Box6* b0, Box6* b1, std::vector<std::pair<uint32_t, uint32_t>>& passes, uint32_t* root_trav,
                       hipStream_t st) {
-    constexpr uint32_t kPlocBatch = 16;
     const uint32_t n = s->n_tris;
     const uint32_t T = kPassThreads - 2 * radius;
     const uint32_t max_tiles = (n + T - 1) / T;
     // ctl: kPlocBatch tile counters, then kPlocBatch x max_tiles status words
     constexpr size_t kCtrWords = (size_t)kPlocBatch * kTicketWords;
     const size_t ctl_words = kCtrWords + (size_t)kPlocBatch * max_tiles * 2;
-    uint32_t *ctl = nullptr, *state = nullptr, *err = nullptr, *tail_count = nullptr;
-    uint4 *log = nullptr, *tail_log = nullptr;
-    RTQ_HIP(ctx, tmp.get(&ctl, ctl_words));
-    // state (8 words), error and tail pass count (8), pass log: one block,
-    // read back with one copy per batch
-    constexpr uint32_t kHeadWords = 16 + 4 * kPlocBatch;
-    RTQ_HIP(ctx, tmp.get(&state, kHeadWords));
-    err = state + 8;
-    log = reinterpret_cast<uint4*>(state + 16);
-    RTQ_HIP(ctx, tmp.get(&tail_log, kTailMax));
-    tail_count = err + 1;
-    const uint32_t h_state0[8] = {n, n, 0u, 0u, 0u, 0u, 0u, 0u};
-    RTQ_HIP(ctx, hipMemcpyAsync(state, h_state0, sizeof h_state0, hipMemcpyHostToDevice, st));
-    RTQ_HIP(ctx, hipMemsetAsync(err, 0, 2 * sizeof(uint32_t), st));
+    uint32_t* ctl = nullptr;
+    if (n > kTailMax) RTQ_HIP(ctx, tmp.get(&ctl, ctl_words));
+    uint32_t* const err = state + 8;
+    uint32_t* const tail_count = err + 1;
+    uint4* const log = reinterpret_cast<uint4*>(state + 16);
+    uint4* const tail_log = reinterpret_cast<uint4*>(state + kPlocHeadWords);
     PlocLists lists{{c0, c1}, {b0, b1}};
     PlocClusters cl{s->cbox, s->cleft,  s->cright, s->cparent, s->ccount,
                     s->ctri, s->ctrav, n,         s->params.max_leaf_size};
@@ -1421,11 +1436,9 @@ rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
         // the head block and the first tail log entries in one read (entries
         // past the tail's pass count are not used)
         constexpr uint32_t kTailPeek = 128;
-        uint32_t h_head[kHeadWords];
-        uint4 h_peek[kTailPeek];
+        uint32_t h_head[kPlocHeadWords + 4 * kTailPeek];
         HostReads rd(ctx, st);
         RTQ_HIP(ctx, rd.add(h_head, state, sizeof h_head));
-        RTQ_HIP(ctx, rd.add(h_peek, tail_log, sizeof h_peek));
         RTQ_HIP(ctx, rd.wait());
         const uint32_t* h_state = h_head;
         const uint32_t* h_err = h_head + 8;
@@ -1446,7 +1459,7 @@ rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
         if (nt) {
             h_tail.resize(nt);
             if (nt <= kTailPeek) {
-                memcpy(h_tail.data(), h_peek, sizeof(uint4) * nt);
+                memcpy(h_tail.data(), h_head + kPlocHeadWords, sizeof(uint4) * nt);
             } else {
                 RTQ_HIP(ctx, rd.add(h_tail.data(), tail_log, sizeof(uint4) * nt));
                 RTQ_HIP(ctx, rd.wait());
@@ -1569,12 +1582,9 @@ private:
 
 // refit: the tree is the one the last build wrote the layouts for, with new
 // boxes: its placement is kept and the 8-wide nodes keep their children.
-// d_bounds: the scene's box and cube, after a refit the root cluster's box.
-// flag_dev (optional): one more device word to read back with the layout's own
-// host read, into *flag_host; done (optional): recorded after the last launch.
-rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipStream_t st, bool refit,
-                         const uint32_t* flag_dev = nullptr, uint32_t* flag_host = nullptr,
-                         hipEvent_t done = nullptr) {
+// d_bounds: the scene's box, cube and words (compute_bounds), after a refit the
+// root cluster's box.
+rtq_status write_layouts(rtq_ctx* ctx, Scene* s, rtq_aabb* d_bounds, hipStream_t st, bool refit) {
     const uint32_t n = s->n_tris;
     const uint32_t nc = s->n_clusters;
     Temps tmp(ctx);
@@ -1586,8 +1596,7 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipSt
     if (!s->nodes) RTQ_HIP(ctx, take(s->kept_nodes, &s->nodes, 4ull * s->n_trav));
     if (!s->node_aux) RTQ_HIP(ctx, take(s->kept_aux, &s->node_aux, s->n_trav));
     s->ref_ready = false;
-    uint32_t *maxd = nullptr, *bdep = nullptr;
-    RTQ_HIP(ctx, tmp.get(&maxd, 1));
+    uint32_t* bdep = nullptr;
     RTQ_HIP(ctx, tmp.get(&bdep, blocks_for(n)));
     float* wcost = nullptr;
     uint32_t* wchoice = nullptr;
@@ -1607,8 +1616,8 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipSt
         const uint32_t c_lo = n_passes ? s->passes[s->lds_from].first : nc - 1;
         const uint32_t c_mid = s->sub_from < s->lds_from ? s->passes[s->sub_from].first : c_lo;
         if (cost) RTQ_HIP(ctx, side.fork(st));
-        hipLaunchKernelGGL(k_place_lds, dim3(1), dim3(kLdsThreads), 0, st, s->d_passes, s->lds_from, n_passes, c_lo,
-                           nc, c_mid, n, s->cleft, s->cright, s->ccount, s->ctrav, s->placed, s->sub_roots);
+        hipLaunchKernelGGL(k_place_lds, dim3(1), dim3(kLdsThreads), 0, st, top_passes(s), c_lo, nc, c_mid, n,
+                           s->cleft, s->cright, s->ccount, s->ctrav, s->placed, s->sub_roots);
         RTQ_HIP(ctx, hipGetLastError());
         if (cost) {
             rs = wide_cost_bottom(ctx, s, wcost, wchoice, ctx->side);
@@ -1631,21 +1640,13 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipSt
             RTQ_HIP(ctx, hipGetLastError());
         }
     }
-    hipLaunchKernelGGL(k_write_leaves, dim3(blocks_for(n)), dim3(kThreads), 0, st, n, s->ctri, s->placed, s->tri_world,
-                       s->tris, bdep);
+    const uint32_t leaf_blocks = blocks_for(n);
+    hipLaunchKernelGGL(k_write_layout, dim3(leaf_blocks + blocks_for(std::max(nc - n, 1u))), dim3(kThreads), 0, st,
+                       leaf_blocks, n, nc, s->params.max_leaf_size, d_bounds, s->ctri, s->tri_world, s->cbox, s->cleft,
+                       s->cright, s->ccount, s->ctrav, s->placed, s->tris, bdep, s->nodes, s->node_aux);
     RTQ_HIP(ctx, hipGetLastError());
-    if (!refit) {   // the depth depends on the topology only: a refit keeps it
-        hipLaunchKernelGGL(k_max_u32, dim3(1), dim3(1024), 0, st, bdep, blocks_for(n), maxd);
-        RTQ_HIP(ctx, hipGetLastError());
-    }
-    if (n == 1)
-        hipLaunchKernelGGL(k_write_single, dim3(1), dim3(1), 0, st, d_bounds, s->cbox, s->nodes, s->node_aux);
-    else
-        hipLaunchKernelGGL(k_write_trav, dim3(blocks_for(nc - n)), dim3(kThreads), 0, st, n, nc,
-                           s->params.max_leaf_size, d_bounds, s->cbox, s->cleft, s->cright, s->ccount, s->ctrav,
-                           s->placed, s->nodes, s->node_aux);
-    RTQ_HIP(ctx, hipGetLastError());
-    rs = write_top(ctx, s, st);
+    // the depth depends on the topology only: a refit keeps it
+    rs = write_top(ctx, s, bdep, leaf_blocks, refit ? nullptr : reinterpret_cast<uint32_t*>(d_bounds + 2) + 1, st);
     if (rs != RTQ_OK) return rs;
     if (s->params.node_width == 8) {
         if (refit) {
@@ -1656,16 +1657,19 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipSt
         }
         if (rs != RTQ_OK) return rs;
     }
-    if (done) RTQ_HIP(ctx, hipEventRecord(done, st));
+    if (!refit) RTQ_HIP(ctx, hipEventRecord(ctx->build_end, st));
     // one host read: the scene's box (for the box margin) and after a build the
-    // tree depth
-    rtq_aabb h_bounds;
+    // sort's errors and the tree depth
+    struct {
+        rtq_aabb box, cube;
+        uint32_t sort_err, depth;
+    } h{};
     HostReads rd(ctx, st);
-    RTQ_HIP(ctx, rd.add(&h_bounds, d_bounds, sizeof h_bounds));
-    if (!refit) RTQ_HIP(ctx, rd.add(&s->depth, maxd, sizeof s->depth));
-    if (flag_dev) RTQ_HIP(ctx, rd.add(flag_host, flag_dev, sizeof(uint32_t)));
+    RTQ_HIP(ctx, rd.add(&h, d_bounds, refit ? sizeof h.box : sizeof h));
     RTQ_HIP(ctx, rd.wait());
-    s->box_pad = box_pad_of(h_bounds);
+    if (h.sort_err) return fail(ctx, RTQ_EINTERNAL, "build: a radix sort pass's look-back gave up");
+    if (!refit) s->depth = h.depth;
+    s->box_pad = box_pad_of(h.box);
     return RTQ_OK;
 }
 
@@ -1683,6 +1687,15 @@ rtq_status ensure_ref_nodes(rtq_ctx* ctx, Scene* s, hipStream_t st) {
     RTQ_HIP(ctx, hipGetLastError());
     s->ref_ready = true;
     return RTQ_OK;
+}
+
+TopPasses top_passes(const Scene* s) {
+    TopPasses t{};
+    t.n = (uint32_t)s->passes.size() - s->lds_from;
+    for (uint32_t k = 0; k < std::min(t.n, kInlinePasses); ++k)
+        t.inline_passes[k] = make_uint2(s->passes[s->lds_from + k].first, s->passes[s->lds_from + k].second);
+    t.rest = s->d_passes;
+    return t;
 }
 
 rtq_status build_scene(rtq_ctx* ctx, Scene* s, const rtq_build_params& prm) {
@@ -1707,14 +1720,7 @@ rtq_status build_scene(rtq_ctx* ctx, Scene* s, const rtq_build_params& prm) {
     rtq_status rs = arena_reserve(ctx);
     if (rs != RTQ_OK) return rs;
 
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    RTQ_HIP(ctx, hipEventCreate(&ev0));
-    RTQ_HIP(ctx, hipEventCreate(&ev1));
-    struct EvGuard {
-        hipEvent_t a, b;
-        ~EvGuard() { (void)hipEventDestroy(a); (void)hipEventDestroy(b); }
-    } evg{ev0, ev1};
-    RTQ_HIP(ctx, hipEventRecord(ev0, st));
+    RTQ_HIP(ctx, hipEventRecord(ctx->build_begin, st));
 
     // persistent products, sized by the triangle count: a rebuild rewrites them
     if (!s->cbox) RTQ_HIP(ctx, dev_alloc(&s->cbox, nc));
@@ -1739,9 +1745,6 @@ rtq_status build_scene(rtq_ctx* ctx, Scene* s, const rtq_build_params& prm) {
     RTQ_HIP(ctx, tmp.get(&c_out, n));
     RTQ_HIP(ctx, tmp.get(&b_in, n));
     RTQ_HIP(ctx, tmp.get(&b_out, n));
-    uint32_t* sort_err = nullptr;
-    RTQ_HIP(ctx, tmp.get(&sort_err, 1));
-    RTQ_HIP(ctx, hipMemsetAsync(sort_err, 0, sizeof(uint32_t), st));
 
     // 1. bounds, cube, Morton codes, sort
     rs = compute_bounds(ctx, s, prm.flags & RTQ_BUILD_REF_PADDED_BOUNDS, d_bounds, st);
@@ -1749,48 +1752,46 @@ rtq_status build_scene(rtq_ctx* ctx, Scene* s, const rtq_build_params& prm) {
     hipLaunchKernelGGL(k_morton, dim3(blocks_for(n)), dim3(kThreads), 0, st, s->tris_ref, s->models, n,
                        d_bounds, s->sorted_codes, s->sorted_idx);
     RTQ_HIP(ctx, hipGetLastError());
-    rs = radix_sort_pairs(ctx, s->sorted_codes, s->sorted_idx, tk, tv, n, 30, sort_err, st);
+    rs = radix_sort_pairs(ctx, s->sorted_codes, s->sorted_idx, tk, tv, n, 30,
+                          reinterpret_cast<uint32_t*>(d_bounds + 2), st);
     if (rs != RTQ_OK) return rs;
 
     // 2. PLOC
-    hipLaunchKernelGGL(k_cluster_init, dim3(blocks_for(nc)), dim3(kThreads), 0, st, n, s->cparent,
-                       s->cleft, s->cright, s->ctri);
-    RTQ_HIP(ctx, hipGetLastError());
+    uint32_t* head = nullptr;
+    RTQ_HIP(ctx, tmp.get(&head, kPlocHeadWords + 4 * kTailMax));
     hipLaunchKernelGGL(k_leaf_init, dim3(blocks_for(n)), dim3(kThreads), 0, st, s->tris_ref, s->models,
-                       s->sorted_idx, n, s->cbox, s->ctri, s->ccount, c_in, b_in);
+                       s->sorted_idx, n, s->cbox, s->ctri, s->ccount, s->cleft, s->cright, s->cparent, c_in, b_in,
+                       head);
     RTQ_HIP(ctx, hipGetLastError());
     std::vector<std::pair<uint32_t, uint32_t>> pass_ranges;
     uint32_t root_trav = 0;
     rs = (prm.flags & RTQ_BUILD_PLOC_SPLIT)
              ? ploc_split(ctx, s, prm.search_radius, tmp, c_in, c_out, b_in, b_out, pass_ranges, &root_trav, st)
-             : ploc_fused(ctx, s, prm.search_radius, tmp, c_in, c_out, b_in, b_out, pass_ranges, &root_trav, st);
+             : ploc_fused(ctx, s, prm.search_radius, tmp, head, c_in, c_out, b_in, b_out, pass_ranges, &root_trav, st);
     if (rs != RTQ_OK) return rs;
     s->n_trav = std::max(root_trav, 1u);   // the root always has a node
     s->ploc_passes = (uint32_t)pass_ranges.size();
     s->passes = pass_ranges;
-    // device copy of the pass ranges for the single-workgroup launches of the
-    // top passes (placement, collapse costs, refit merges): the passes from
-    // lds_from on create at most kLdsClusters clusters in all
+    // the passes of the single-workgroup launches (placement, collapse costs,
+    // refit merges): those from lds_from on create at most kLdsClusters clusters
     s->lds_from = s->ploc_passes;
     while (s->lds_from > 0 && nc - s->passes[s->lds_from - 1].first <= kLdsClusters) --s->lds_from;
     s->sub_from = s->lds_from;
     while (s->sub_from > 0 && s->passes[s->sub_from - 1].second <= kSubPass) --s->sub_from;
-    if (s->ploc_passes > 0) {
-        s->h_passes.resize(s->ploc_passes);
-        for (uint32_t k = 0; k < s->ploc_passes; ++k)
-            s->h_passes[k] = make_uint2(s->passes[k].first, s->passes[k].second);
-        RTQ_HIP(ctx, take(s->kept_passes, &s->d_passes, s->ploc_passes));
-        RTQ_HIP(ctx, hipMemcpyAsync(s->d_passes, s->h_passes.data(), sizeof(uint2) * s->ploc_passes,
-                                    hipMemcpyHostToDevice, st));
+    if (s->ploc_passes - s->lds_from > kInlinePasses) {
+        const uint32_t from = s->lds_from + kInlinePasses, rest = s->ploc_passes - from;
+        s->h_passes.resize(rest);
+        for (uint32_t k = 0; k < rest; ++k)
+            s->h_passes[k] = make_uint2(s->passes[from + k].first, s->passes[from + k].second);
+        RTQ_HIP(ctx, take(s->kept_passes, &s->d_passes, rest));
+        RTQ_HIP(ctx, hipMemcpyAsync(s->d_passes, s->h_passes.data(), sizeof(uint2) * rest, hipMemcpyHostToDevice, st));
     }
 
     // 3-4. node arrays of every layout
-    uint32_t h_sort_err = 0;
-    rs = write_layouts(ctx, s, d_bounds, st, false, sort_err, &h_sort_err, ev1);
+    rs = write_layouts(ctx, s, d_bounds, st, false);
     if (rs != RTQ_OK) return rs;
-    if (h_sort_err) return fail(ctx, RTQ_EINTERNAL, "build: a radix sort pass's look-back gave up");
     float ms = 0.0f;
-    RTQ_HIP(ctx, hipEventElapsedTime(&ms, ev0, ev1));
+    RTQ_HIP(ctx, hipEventElapsedTime(&ms, ctx->build_begin, ctx->build_end));
     s->build_ms = ms;
     s->built = true;
     s->generation = ++ctx->builds;
@@ -1799,12 +1800,14 @@ rtq_status build_scene(rtq_ctx* ctx, Scene* s, const rtq_build_params& prm) {
     return RTQ_OK;
 }
 
-rtq_status write_top(rtq_ctx* ctx, Scene* s, hipStream_t st) {
-    if (kTopNodes == 0) return RTQ_OK;
+rtq_status write_top(rtq_ctx* ctx, Scene* s, const uint32_t* block_depth, uint32_t n_blocks, uint32_t* depth,
+                     hipStream_t st) {
+    if (kTopNodes == 0 && !depth) return RTQ_OK;
     // the set depends on the topology only, so a refit or an order update
     // rewrites the same buffer with the same node count
-    if (!s->top) RTQ_HIP(ctx, dev_alloc(&s->top, 4ull * kTopNodes));
-    hipLaunchKernelGGL(k_top_nodes, dim3(1), dim3(64), 0, st, s->nodes, s->top);
+    if (!s->top) RTQ_HIP(ctx, dev_alloc(&s->top, 4ull * std::max(kTopNodes, 1u)));
+    hipLaunchKernelGGL(k_top_nodes, dim3(depth ? 2 : 1), dim3(kTopThreads), 0, st, s->nodes, s->top, block_depth,
+                       n_blocks, depth);
     RTQ_HIP(ctx, hipGetLastError());
     s->n_top = std::min(kTopNodes, s->n_trav);   // every traversal node can be reached from the root
     return RTQ_OK;
@@ -1837,7 +1840,7 @@ rtq_status refit_scene(rtq_ctx* ctx, Scene* s) {
         RTQ_HIP(ctx, hipGetLastError());
     }
     if (s->lds_from < n_passes) {
-        hipLaunchKernelGGL(k_refit_merge_lds, dim3(1), dim3(kLdsThreads), 0, st, s->d_passes, s->lds_from, n_passes,
+        hipLaunchKernelGGL(k_refit_merge_lds, dim3(1), dim3(kLdsThreads), 0, st, top_passes(s),
                            s->passes[s->lds_from].first, s->n_clusters, s->cleft, s->cright, s->cbox);
         RTQ_HIP(ctx, hipGetLastError());
     }

@@ -961,7 +961,7 @@ rtq_status rtq_order_apply(rtq_ctx* ctx, uint32_t scene_id, const float* params_
     }
     RTQ_HIP(ctx, hipGetLastError());
     // the LDS copy of the top of the tree carries the order words too
-    rtq_status rs = write_top(ctx, s, st);
+    rtq_status rs = write_top(ctx, s, nullptr, 0, nullptr, st);
     if (rs != RTQ_OK) return rs;
     // the 8-wide nodes' first-child tables follow the binary decisions
     rs = write_wide_order(ctx, s, params_dev == nullptr, st);

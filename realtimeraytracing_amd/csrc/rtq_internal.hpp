@@ -78,11 +78,12 @@ struct Scene {
     uint32_t ploc_passes = 0;
     // (first cluster id, count) of the merges of each PLOC pass, in build order
     std::vector<std::pair<uint32_t, uint32_t>> passes;
-    // the same on the device (and its host staging copy); the clusters of the
-    // passes from lds_from on fit in one workgroup's LDS together
-    // (kLdsClusters): placement, collapse costs and refit merges run those
-    // passes in one launch, the passes [sub_from, lds_from) as subtrees below
-    // them in another, and each pass before sub_from in its own
+    // The clusters of the passes from lds_from on fit in one workgroup's LDS
+    // together (kLdsClusters): placement, collapse costs and refit merges run
+    // those passes in one launch, the passes [sub_from, lds_from) as subtrees
+    // below them in another, and each pass before sub_from in its own.
+    // d_passes: the passes from lds_from on that do not fit in a kernel's
+    // arguments (TopPasses), h_passes their staging copy
     uint2* d_passes = nullptr;
     std::vector<uint2> h_passes;
     uint32_t lds_from = 0;
@@ -137,6 +138,7 @@ struct rtq_ctx {
     // main stream's, forked and joined with the two events
     hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
+    hipEvent_t build_begin = nullptr, build_end = nullptr;   // a build's device time
     // pinned host memory (rtq::kPinnedBytes) for the build's small device-to-
     // host reads (rtq::HostReads)
     void* pinned = nullptr;
@@ -365,6 +367,19 @@ rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const rtq_
 // (their placement state, 12 B each, and cost rows, 32 B each, in LDS).
 constexpr uint32_t kLdsClusters = 4096;
 constexpr int kLdsThreads = 1024;   // 4 clusters per thread
+// Those passes, (first cluster, merges) in build order, as a kernel argument:
+// the first kInlinePasses by value (a 2M-triangle terrain has 33 of them), so
+// that a build uploads a table only for a tree with more.
+constexpr uint32_t kInlinePasses = 64;
+struct TopPasses {
+    uint32_t n;
+    uint2 inline_passes[kInlinePasses];
+    const uint2* rest;
+    __device__ __forceinline__ uint2 operator[](uint32_t k) const {
+        return k < kInlinePasses ? inline_passes[k] : rest[k - kInlinePasses];
+    }
+};
+TopPasses top_passes(const Scene* s);
 
 // Middle subtrees: the clusters of the passes [sub_from, lds_from), hanging from
 // the top ones.  A pass of up to kSubPass merges is shorter than its launch, and
@@ -393,8 +408,10 @@ rtq_status write_wide_order(rtq_ctx* ctx, Scene* s, bool clear, hipStream_t st);
 // New boxes for the kept topology after rtq_scene_update (build.hip).
 rtq_status refit_scene(rtq_ctx* ctx, Scene* s);
 // (Re)writes s->top from s->nodes: after the traversal nodes or their order
-// words change (build.hip).
-rtq_status write_top(rtq_ctx* ctx, Scene* s, hipStream_t st);
+// words change (build.hip).  depth, unless null: a device word for the maximum
+// of block_depth's n_blocks words.
+rtq_status write_top(rtq_ctx* ctx, Scene* s, const uint32_t* block_depth, uint32_t n_blocks, uint32_t* depth,
+                     hipStream_t st);
 // Writes s->ref_nodes (the reference's pre-order BVH_NodeGPU array) from the
 // cluster arrays when the build or refit since the last call changed them;
 // queued on st (build.hip).

@@ -130,13 +130,12 @@ __global__ __launch_bounds__(kSubThreads) void k_dp_subtrees(const uint2* __rest
               [&](uint32_t c) { dp_cluster(c, nt, max_leaf, cleft, cright, ccount, cbox, cost, choice); });
 }
 
-// Passes [k0, k1) at the top of the tree in one workgroup, bottom-up, with
+// The passes at the top of the tree in one workgroup, bottom-up, with
 // the cost rows of their clusters [c_lo, nc) in LDS (a child from an earlier
 // pass gives its row from global memory); a barrier between passes.  Each
 // thread keeps the child ids, box area and triangle count of its clusters
 // c_lo + t + kLdsThreads * s in registers.  nc - c_lo <= kLdsClusters.
-__global__ __launch_bounds__(kLdsThreads) void k_dp_lds(const uint2* __restrict__ passes, uint32_t k0, uint32_t k1,
-                                                        uint32_t c_lo, uint32_t nc, uint32_t nt, uint32_t max_leaf,
+__global__ __launch_bounds__(kLdsThreads) void k_dp_lds(TopPasses passes, uint32_t c_lo, uint32_t nc, uint32_t nt, uint32_t max_leaf,
                                                         const uint32_t* __restrict__ cleft,
                                                         const uint32_t* __restrict__ cright,
                                                         const uint32_t* __restrict__ ccount,
@@ -157,7 +156,7 @@ __global__ __launch_bounds__(kLdsThreads) void k_dp_lds(const uint2* __restrict_
         N[q] = in ? ccount[c_lo + idx] : 0u;
         A[q] = in ? box_area(cbox[c_lo + idx]) : 0.0f;
     }
-    for (uint32_t k = k0; k < k1; ++k) {
+    for (uint32_t k = 0; k < passes.n; ++k) {
         const uint2 p = passes[k];
 #pragma unroll
         for (int q = 0; q < kSlots; ++q) {
@@ -305,13 +304,12 @@ constexpr uint32_t kLvSpinLimit = 1u << 24;
 enum : uint32_t { kWideErrOverflow = 1, kWideErrScan = 2 };
 
 struct LevelArgs {
-    uint32_t* lv;              // this level's words: count, first node, first status word, unused
+    uint32_t* lv;              // this level's words: count, first node, first status word, errors; then the next one's
     uint32_t* tickets;         // tile counters of this level, zero before it
     uint32_t* next_tickets;    // of the next one
     uint64_t* status;          // tile status words, n_status of them, zero before the first level
     uint32_t n_status;
     uint32_t cap;              // node capacity
-    uint32_t* err;
     uint32_t max_leaf;
     uint32_t nt;
     const rtq_aabb* bounds;    // the scene's, for the box margin
@@ -431,7 +429,7 @@ __global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
         if (lane == 0) {
             s_excl = excl;
             s_bad = failed ? 1u : 0u;
-            if (failed) atomicOr(a.err, kWideErrScan);
+            if (failed) atomicOr(a.lv + 3, kWideErrScan);
         }
     }
     __syncthreads();
@@ -441,7 +439,7 @@ __global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
     if (tile == tiles - 1 && tid == 0) {
         uint32_t next_count = excl + total;
         if ((uint64_t)next_base + next_count > a.cap) {
-            atomicOr(a.err, kWideErrOverflow);   // more wide nodes than binary ones: a broken invariant
+            atomicOr(a.lv + 3, kWideErrOverflow);   // more wide nodes than binary ones: a broken invariant
             next_count = 0;
         }
         a.lv[4] = next_count;
@@ -461,7 +459,7 @@ __global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
         if ((uint64_t)next_base + to < a.cap) {
             a.next_items[to] = c;
         } else {
-            atomicOr(a.err, kWideErrOverflow);
+            atomicOr(a.lv + 3, kWideErrOverflow);
         }
     } else if (has) {
         ref = leaf_ref(first, cnt);
@@ -503,7 +501,15 @@ __global__ __launch_bounds__(kThreads) void k_wide_refit(uint32_t n_wide, const 
         nodes[8ull * k + slot] = image_part(img, slot);
 }
 
-__global__ void k_set_u32(uint32_t* p, uint32_t v) { *p = v; }
+// Before the first level: n_clear words zero from `clear` on (the tile counters
+// and status words, then the levels' words), the first level's one node, and
+// that node's cluster.
+__global__ __launch_bounds__(kThreads) void k_level_init(uint32_t* __restrict__ clear, uint32_t n_clear, uint32_t lv,
+                                                         uint32_t* __restrict__ items, uint32_t root) {
+    const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+    if (i < n_clear) clear[i] = i == lv ? 1u : 0u;
+    if (i == 0) items[0] = root;
+}
 
 inline uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + kThreads - 1) / kThreads); }
 
@@ -527,9 +533,8 @@ rtq_status wide_cost_top(rtq_ctx* ctx, const Scene* s, float* cost, uint32_t* ch
                            choice);
         RTQ_HIP(ctx, hipGetLastError());
     }
-    hipLaunchKernelGGL(k_dp_lds, dim3(1), dim3(kLdsThreads), 0, st, s->d_passes, s->lds_from,
-                       (uint32_t)s->passes.size(), c_lo, s->n_clusters, nt, max_leaf, s->cleft, s->cright, s->ccount,
-                       s->cbox, cost, choice);
+    hipLaunchKernelGGL(k_dp_lds, dim3(1), dim3(kLdsThreads), 0, st, top_passes(s), c_lo, s->n_clusters, nt,
+                       max_leaf, s->cleft, s->cright, s->ccount, s->cbox, cost, choice);
     RTQ_HIP(ctx, hipGetLastError());
     return RTQ_OK;
 }
@@ -548,36 +553,29 @@ rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const rtq_
     // tile status words of every level's scan: a level of c nodes takes
     // ceil(c / kLevelNodes) of them, and there are at most depth + 1 levels,
     // the depth no more than the PLOC passes
-    const uint32_t n_status = cap / kLevelNodes + s->ploc_passes + 2;
-    uint64_t* status = nullptr;
-    // and before them two sets of tile counters: a level clears the next one's
-    constexpr uint32_t kTickets = 2 * kTicketWords / 2;
-    RTQ_HIP(ctx, tmp.get(&status, (size_t)kTickets + n_status));
-    RTQ_HIP(ctx, hipMemsetAsync(status, 0, sizeof(uint64_t) * (kTickets + n_status), st));
-    uint32_t* const tickets = reinterpret_cast<uint32_t*>(status);
-    status += kTickets;
+    const uint32_t max_levels = s->ploc_passes + 1;
+    const uint32_t n_status = cap / kLevelNodes + max_levels + 1;
+    // two sets of tile counters (a level clears the next one's), the status
+    // words, and each level's words (and those of the one after the last)
+    constexpr uint32_t kTickets = 2 * kTicketWords, kLvWords = 4;
+    const uint32_t lv0 = kTickets + 2 * n_status;
+    const uint32_t n_words = lv0 + kLvWords * (max_levels + 1);
+    uint32_t* words = nullptr;
+    RTQ_HIP(ctx, tmp.get(&words, n_words));
+    uint32_t* const tickets = words;
+    uint32_t* const lvl = words + lv0;
     // a refit writes the same buffer again (its size depends on the topology only)
     if (!s->wide) RTQ_HIP(ctx, take(s->kept_wide, &s->wide, 8ull * cap));
     if (!s->wide_trav) RTQ_HIP(ctx, take(s->kept_wide_trav, &s->wide_trav, cap));
     if (!s->wide_kids) RTQ_HIP(ctx, take(s->kept_wide_kids, &s->wide_kids, 8ull * cap));
     s->wide_ordered = false;   // the nodes are rewritten with empty tables
-    hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, st, items, root);
+    hipLaunchKernelGGL(k_level_init, dim3(blocks_for(n_words)), dim3(kThreads), 0, st, words, n_words, lv0, items,
+                       root);
     RTQ_HIP(ctx, hipGetLastError());
-    // levels top-down, one launch each, kLevelsPerRead of them between host
-    // reads: a level's words (count, first node, first status word)
-    // stay on the device, its launch covers an upper bound of its count (8
-    // children per node, at most cap nodes)
-    constexpr uint32_t kLevelsPerRead = 6;
-    static_assert(kLevelsPerRead % 2 == 0, "the levels of a group start with the first set of tile counters");
-    constexpr uint32_t kLvWords = 4 * (kLevelsPerRead + 1);
-    uint32_t* lvl = nullptr;
-    RTQ_HIP(ctx, tmp.get(&lvl, kLvWords + 1));
-    uint32_t* err = lvl + kLvWords;
     LevelArgs la{};
-    la.status = status;
+    la.status = reinterpret_cast<uint64_t*>(words + kTickets);
     la.n_status = n_status;
     la.cap = cap;
-    la.err = err;
     la.max_leaf = s->params.max_leaf_size;
     la.nt = s->n_tris;
     la.bounds = bounds;
@@ -590,17 +588,21 @@ rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const rtq_
     la.nodes = s->wide;
     la.wide_trav = s->wide_trav;
     la.kids = s->wide_kids;
-    uint32_t level_items = 1, level_base = 0, level_status = 0, levels = 0, n_wide = 0;
-    while (level_items > 0) {
-        // the group's first level; the others (and the error word) zero until written
-        uint32_t h_head[kLvWords + 1] = {};
-        h_head[0] = level_items;
-        h_head[1] = level_base;
-        h_head[2] = level_status;
-        RTQ_HIP(ctx, hipMemcpyAsync(lvl, h_head, sizeof h_head, hipMemcpyHostToDevice, st));
-        uint64_t ub = level_items;
-        for (uint32_t g = 0; g < kLevelsPerRead; ++g) {
-            la.lv = lvl + 4 * g;
+    // levels top-down, one launch each, several between host reads: a level's
+    // words (count, first node, first status word, errors) stay on the device,
+    // its launch covers an upper bound of its count (8 children per node, at
+    // most cap nodes).  The first group is as long as a tree of so many nodes
+    // is likely to be deep (an empty level costs less than a host read).
+    constexpr uint32_t kMaxGroup = 16;
+    uint32_t group = 2;
+    while (group < kMaxGroup && (1ull << (2 * (group - 2))) < cap) ++group;
+    uint32_t done = 0, levels = 0, n_wide = 0;
+    uint64_t ub = 1;
+    for (bool more = true; more;) {
+        if (done >= max_levels) return fail(ctx, RTQ_EINTERNAL, "wide collapse: more levels than PLOC passes");
+        const uint32_t g0 = done, g1 = std::min(done + group, max_levels);
+        for (uint32_t g = g0; g < g1; ++g) {
+            la.lv = lvl + kLvWords * g;
             la.items = items;
             la.next_items = next;
             la.tickets = tickets + (g & 1u) * kTicketWords;
@@ -611,20 +613,23 @@ rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const rtq_
             std::swap(items, next);
             ub = std::min<uint64_t>(8 * ub, cap);
         }
-        uint32_t h_lvl[kLvWords + 1];
+        uint32_t h_lv[kLvWords * (kMaxGroup + 1)];
         HostReads rd(ctx, st);
-        RTQ_HIP(ctx, rd.add(h_lvl, lvl, sizeof h_lvl));
+        RTQ_HIP(ctx, rd.add(h_lv, lvl + kLvWords * g0, sizeof(uint32_t) * kLvWords * (g1 - g0 + 1)));
         RTQ_HIP(ctx, rd.wait());
-        if (h_lvl[kLvWords] & kWideErrScan) return fail(ctx, RTQ_EINTERNAL, "wide collapse: a level scan gave up");
-        if (h_lvl[kLvWords]) return fail(ctx, RTQ_EINTERNAL, "wide collapse overflow");
-        for (uint32_t g = 0; g < kLevelsPerRead; ++g)
-            if (h_lvl[4 * g] > 0) {
-                ++levels;
-                n_wide = h_lvl[4 * g + 1] + h_lvl[4 * g];
-            }
-        level_items = h_lvl[4 * kLevelsPerRead];
-        level_base = h_lvl[4 * kLevelsPerRead + 1];
-        level_status = h_lvl[4 * kLevelsPerRead + 2];
+        uint32_t err = 0;
+        for (uint32_t g = 0; g < g1 - g0; ++g) {
+            const uint32_t* const w = h_lv + kLvWords * g;
+            err |= w[3];
+            if (w[0] == 0) continue;
+            ++levels;
+            n_wide = w[1] + w[0];
+        }
+        if (err & kWideErrScan) return fail(ctx, RTQ_EINTERNAL, "wide collapse: a level scan gave up");
+        if (err) return fail(ctx, RTQ_EINTERNAL, "wide collapse overflow");
+        more = h_lv[kLvWords * (g1 - g0)] > 0;
+        done = g1;
+        group = 4;
     }
     s->n_wide = n_wide;
     s->wide_depth = levels;
