@@ -125,6 +125,9 @@ __device__ __forceinline__ void child_hits(float4 n0, float4 n1, float4 n2, cons
 constexpr uint32_t kLogStack = 96;
 constexpr uint32_t kLogRecords = 32;       // samples of a ray kept until its wave ends
 constexpr uint32_t kLogBudget = 1u << 14;  // node visits + triangle tests per sub-traversal
+// Lanes of a ray that prices 2 or 3 levels at a time: 2 + 4 or 2 + 4 + 8 of
+// them, rounded up to a power of two.
+constexpr uint32_t log_lanes(int ahead) { return ahead == 2 ? 8 : 16; }
 
 struct LogRay {
     float o[3], inv[3], tmin, tmax;
@@ -204,33 +207,63 @@ __device__ void emit(float* __restrict__ out, uint32_t cap, uint32_t slot, const
     o[kIn + 1] = weight;
 }
 
+// The first node from `ref` down that has both children hit over the ray's
+// interval, following the only hit child to it; its child refs.  kNone: a leaf
+// or a node without a hit child comes first.
+__device__ uint32_t next_decision(const float4* __restrict__ nodes, const LogRay& R, uint32_t ref, uint32_t& r0,
+                                  uint32_t& r1) {
+    while (!(ref & kLeafBit)) {
+        const float4* nd = nodes + 4ull * ref;
+        const float4 n3 = nd[3];
+        bool h0, h1;
+        float tn0, tn1;
+        child_hits(nd[0], nd[1], nd[2], R.o, R.inv, R.tmin, R.tmax, h0, h1, tn0, tn1);
+        r0 = __float_as_uint(n3.x);
+        r1 = __float_as_uint(n3.y);
+        if (h0 && h1) return ref;
+        if (!(h0 || h1)) break;
+        ref = h0 ? r0 : r1;
+    }
+    return kNone;
+}
+
 // Samples of one ray every `stride`: from the root, each node whose two
 // children are both hit is priced in both visit orders with sub-traversals
 // (node visits + triangle tests until the closest hit is certain, or until an
 // occluder is found for any-hit rays); label = the cheaper child first, weight
 // log2(1 + cost difference), no sample on a tie.  The walk continues into the
 // cheaper child and stops where no hit lies below it.
-// A pair of lanes per ray: the even one prices child 0 first, the odd one
-// child 1 first.  A launch lasts as long as its longest walks, so a wave takes
-// only `per_wave` rays, and its stacks lie in LDS, `levels` entries per lane.  A
-// ray's samples wait in registers' scratch, so that a wave takes their slots
-// with one atomic at its end: atomics of every sample on one word serialise.
-// 25,000 any-hit rays on 300,000 occluded triangles: 1.04 ms (closest hit
-// 1.60), 2.64 (5.15) with a lane per ray and full waves; 200,000 rays 2.53
-// against 3.26 ms.
+// Two lanes price a node: the even one child 0 first, the odd one child 1
+// first.  A ray has the pairs of AHEAD levels of such nodes, the 1, 2 or 4 that
+// the walk can come to: they are priced together, which takes about as long as
+// the first level alone, and the ones off the walk's way are dropped.  The
+// stacks lie in LDS, `levels` entries per lane.  A ray's samples wait in
+// registers' scratch, so that a wave takes their slots with one atomic at its
+// end: atomics of every sample on one word serialise.
+// The chains of dependent node loads of a ray's walks bound it.  300,000
+// occluded triangles, any-hit rays (closest-hit), with 1, 2 and 3 levels at a
+// time: 6,250 rays 0.63 (1.11), 0.51 (0.95), 0.35 (0.65) ms; 25,000 rays 0.88
+// (1.48), 0.58 (0.99), 0.58 (0.95); 200,000 rays 2.53 (4.97), 2.36 (4.03), 2.90
+// (4.78).
+template <int AHEAD>
 __global__ __launch_bounds__(64) void k_order_log(const float4* __restrict__ nodes, const uint4* __restrict__ aux,
                                                   const float4* __restrict__ tris, const rtq_ray* __restrict__ rays,
-                                                  uint32_t n, uint32_t stride, uint32_t per_wave, uint32_t levels,
-                                                  uint32_t any, float* __restrict__ out, uint32_t cap,
+                                                  uint32_t n, uint32_t stride, uint32_t any, float* __restrict__ out, uint32_t cap,
                                                   uint32_t* __restrict__ count) {
     extern __shared__ uint32_t s_log[];
-    const uint32_t lane = threadIdx.x, lanes = 2 * per_wave;
-    const bool second = lane & 1u;          // prices child 1 first
-    uint32_t* const stack = s_log + lane;   // [levels][lanes]
-    uint2 rec[kLogRecords];                 // node | child 0 first << 31, weight (even lanes)
-    const uint64_t r = ((uint64_t)blockIdx.x * per_wave + lane / 2) * stride;
+    constexpr uint32_t kGroup = log_lanes(AHEAD), kRays = 64 / kGroup;
+    const uint32_t lane = threadIdx.x;
+    const uint32_t sub = lane % kGroup, lead = lane - sub;
+    // the lane's level and the choices down to it: the child taken at each
+    // level before it, then the child it prices first (0 as the level: idle)
+    const uint32_t level = sub < 2 ? 1u : sub < 6 ? 2u : AHEAD > 2 && sub < 14 ? 3u : 0u;
+    const uint32_t way = sub - (level == 2 ? 2u : level == 3 ? 6u : 0u);
+    const bool second = way & 1u;           // prices child 1 first
+    uint32_t* const stack = s_log + lane;   // [levels][64]
+    uint2 rec[kLogRecords];                 // node | child 0 first << 31, weight (a ray's first lane)
+    const uint64_t r = ((uint64_t)blockIdx.x * kRays + lane / kGroup) * stride;
     uint32_t n_rec = 0, octant = 0;
-    if (lane < lanes && r < n) {
+    if (r < n) {
         const rtq_ray ray = rays[r];
         LogRay R;
         for (int k = 0; k < 3; ++k) {
@@ -263,73 +296,75 @@ __global__ __launch_bounds__(64) void k_order_log(const float4* __restrict__ nod
         // has been visited before such a node, so its interval is the ray's own.
         // (An empty interval or a zero direction hits nothing: no walk.)
         uint32_t cur = ray.tmin <= ray.tmax && dkz != 0.0f ? 0u : kLeafBit;
-        while (!(cur & kLeafBit)) {
-            const float4* nd = nodes + 4ull * cur;
-            const float4 n3 = nd[3];
-            bool h0, h1;
-            float tn0, tn1;
-            child_hits(nd[0], nd[1], nd[2], R.o, R.inv, R.tmin, R.tmax, h0, h1, tn0, tn1);
-            const uint32_t r0 = __float_as_uint(n3.x), r1 = __float_as_uint(n3.y);
-            if (!(h0 || h1)) break;
-            if (!(h0 && h1)) {
-                cur = h0 ? r0 : r1;
-                continue;
-            }
+        for (bool more = true; more;) {
+            uint32_t r0 = 0, r1 = 0;
+            uint32_t at = next_decision(nodes, R, cur, r0, r1);   // the node the lane prices
+            if (at == kNone) break;
+#pragma unroll
+            for (uint32_t l = 1; l < (uint32_t)AHEAD; ++l)
+                if (level > l && at != kNone)
+                    at = next_decision(nodes, R, (way >> (level - l)) & 1u ? r1 : r0, r0, r1);
             // the lane's first child, and for closest-hit rays the other one
             // with the interval the first left (an occluder below the first
             // child ends an any-hit ray there, and the other lane's walk gives
             // the other child's cost)
-            uint32_t cost, more = 0;
-            bool ok, ok2 = true;
-            float t = R.tmax;
-            const bool found = log_walk(nodes, tris, R, second ? r1 : r0, any, stack, lanes, t, cost, ok) != kNone;
-            if (!any) log_walk(nodes, tris, R, second ? r0 : r1, false, stack, lanes, t, more, ok2);
-            const int good = ok && ok2, other_good = __shfl_xor(good, 1);
-            const bool other_found = __shfl_xor((int)found, 1) != 0;
-            const uint32_t mine = cost + more, other = __shfl_xor(mine, 1);
-            if (!good || !other_good) break;
-            const uint32_t total = any && !found ? mine + other : mine;
-            const uint32_t other_total = any && !other_found ? other + mine : other;
-            const bool f0 = second ? other_found : found, f1 = second ? found : other_found;
-            const uint32_t cost01 = second ? other_total : total, cost10 = second ? total : other_total;
-            // with no hit below either child every order visits the same nodes
-            if (!f0 && !f1) break;
-            if (cost01 != cost10 && !second) {
-                const float diff = (float)(cost01 > cost10 ? cost01 - cost10 : cost10 - cost01);
-                const float weight = log2f(1.0f + diff);
-                if (n_rec < kLogRecords) {
-                    rec[n_rec++] = make_uint2(cur | (cost01 < cost10 ? kLeafBit : 0u), __float_as_uint(weight));
-                } else {   // a path of more levels than the records hold
-                    emit(out, cap, atomicAdd(count, 1u), nodes, aux, cur, octant, any, cost01 < cost10, weight);
-                }
+            uint32_t cost = 0, rest = 0;
+            bool found = false, ok = true, ok2 = true;
+            if (level > 0 && at != kNone) {
+                float t = R.tmax;
+                found = log_walk(nodes, tris, R, second ? r1 : r0, any, stack, 64, t, cost, ok) != kNone;
+                if (!any) log_walk(nodes, tris, R, second ? r0 : r1, false, stack, 64, t, rest, ok2);
             }
-            const bool go0 = cost01 <= cost10;
-            if (!(go0 ? f0 : f1)) break;
-            cur = go0 ? r0 : r1;
+            const uint32_t flags = (found ? 1u : 0u) | (ok && ok2 ? 2u : 0u);
+            cost += rest;
+            uint32_t choice = 0;   // the children taken so far in this round
+#pragma unroll
+            for (uint32_t l = 0; l < (uint32_t)AHEAD; ++l) {
+                const int from = (int)(lead + (2u << l) - 2u + 2u * choice);
+                const uint32_t node = __shfl(at, from, 64);
+                const uint32_t c0 = __shfl(cost, from, 64), c1 = __shfl(cost, from + 1, 64);
+                const uint32_t g0 = __shfl(flags, from, 64), g1 = __shfl(flags, from + 1, 64);
+                const uint32_t n0 = __shfl(r0, from, 64), n1 = __shfl(r1, from, 64);
+                const bool f0 = g0 & 1u, f1 = g1 & 1u;
+                // past the walk's end, a walk past its bounds, or no hit below
+                // either child (every order visits the same nodes)
+                if (!more || node == kNone || !(g0 & g1 & 2u) || !(f0 || f1)) {
+                    more = false;
+                    continue;
+                }
+                const uint32_t cost01 = any && !f0 ? c0 + c1 : c0, cost10 = any && !f1 ? c1 + c0 : c1;
+                if (cost01 != cost10 && sub == 0) {
+                    const float diff = (float)(cost01 > cost10 ? cost01 - cost10 : cost10 - cost01);
+                    const float weight = log2f(1.0f + diff);
+                    if (n_rec < kLogRecords) {
+                        rec[n_rec++] = make_uint2(node | (cost01 < cost10 ? kLeafBit : 0u), __float_as_uint(weight));
+                    } else {   // a path of more levels than the records hold
+                        emit(out, cap, atomicAdd(count, 1u), nodes, aux, node, octant, any, cost01 < cost10, weight);
+                    }
+                }
+                const bool go0 = cost01 <= cost10;
+                more = go0 ? f0 : f1;
+                cur = go0 ? n0 : n1;
+                choice = 2 * choice + (go0 ? 0u : 1u);
+            }
         }
     }
-    // the wave's slots, then each ray's samples by its two lanes in turn
-    uint32_t incl = n_rec;   // in the even lanes; 0 in the odd ones
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = __shfl_up(incl, d, 64);
-        if (lane >= (uint32_t)d) incl += o;
-    }
-    const uint32_t all = __shfl(incl, 63, 64);
+    // the wave's slots, then each ray's samples by its first two lanes in turn
+    const uint32_t incl = wave_inclusive_sum(n_rec);
+    const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
     if (all == 0) return;
     uint32_t base = 0;
     if (lane == 0) base = atomicAdd(count, all);
-    base = __shfl(base, 0, 64) + __shfl(incl - n_rec, (int)(lane & ~1u), 64);
+    base = __shfl(base, 0, 64) + __shfl(incl - n_rec, (int)lead, 64);
+    const uint32_t have = __shfl(n_rec, (int)lead, 64);
     for (uint32_t k = 0; k < kLogRecords; k += 2) {
         if (__ballot(k < n_rec) == 0) break;
-        // the even lane's records k and k + 1, one for each lane of the pair
+        // the first lane's records k and k + 1, one for each lane of the pair
         const uint2 a0 = rec[k], a1 = rec[k + 1];
-        const uint32_t sx = __shfl(second ? a0.x : a1.x, (int)(lane & ~1u), 64);
-        const uint32_t sy = __shfl(second ? a0.y : a1.y, (int)(lane & ~1u), 64);
-        const uint32_t have = __shfl(n_rec, (int)(lane & ~1u), 64);
-        const uint2 s = second ? make_uint2(sx, sy) : a0;
-        if (k + second < have)
-            emit(out, cap, base + k + second, nodes, aux, s.x & ~kLeafBit, octant, any, (s.x & kLeafBit) != 0,
+        const uint32_t sx = __shfl(a1.x, (int)lead, 64), sy = __shfl(a1.y, (int)lead, 64);
+        const uint2 s = sub == 1 ? make_uint2(sx, sy) : a0;
+        if (sub < 2 && k + sub < have)
+            emit(out, cap, base + k + sub, nodes, aux, s.x & ~kLeafBit, octant, any, (s.x & kLeafBit) != 0,
                  __uint_as_float(s.y));
     }
 }
@@ -802,15 +837,15 @@ rtq_status rtq_order_log(rtq_ctx* ctx, uint32_t scene_id, const rtq_ray* rays_de
     hipError_t e = hipMemsetAsync(cnt, 0, sizeof(uint32_t), st);
     const uint64_t threads = (n_rays + stride - 1) / stride;
     if (e == hipSuccess && threads > 0) {
-        // four waves per SIMD, of at least 4 rays (25,000 rays on 300,000
-        // occluded triangles: 1.22 ms with one wave per SIMD, 1.04 with four,
-        // 1.18 with eight), then full ones
-        const uint64_t simds = 4 * (uint64_t)std::max(ctx->n_cu, 1);
-        const uint32_t per_wave = (uint32_t)std::min<uint64_t>(32, std::max<uint64_t>(4, threads / (4 * simds)));
+        // three levels at a time (16 lanes per ray) while the waves fit the
+        // chip at four per SIMD, else two (8 lanes): the times are at k_order_log
+        const int ahead = threads <= 4 * 4 * 4 * (uint64_t)std::max(ctx->n_cu, 1) ? 3 : 2;
+        const uint32_t per_wave = 64 / log_lanes(ahead);
         const uint32_t levels = std::min<uint32_t>(kLogStack, s->depth + 1);
-        hipLaunchKernelGGL(k_order_log, dim3((uint32_t)((threads + per_wave - 1) / per_wave)), dim3(64),
-                           sizeof(uint32_t) * levels * 2 * per_wave, st, s->nodes, s->node_aux, s->tris, rays_dev,
-                           (uint32_t)n_rays, stride, per_wave, levels, (flags & RTQ_TRACE_ANY) ? 1u : 0u, samples_dev,
+        hipLaunchKernelGGL(ahead == 3 ? &k_order_log<3> : &k_order_log<2>,
+                           dim3((uint32_t)((threads + per_wave - 1) / per_wave)), dim3(64),
+                           sizeof(uint32_t) * levels * 64, st, s->nodes, s->node_aux, s->tris, rays_dev,
+                           (uint32_t)n_rays, stride, (flags & RTQ_TRACE_ANY) ? 1u : 0u, samples_dev,
                            (uint32_t)capacity, cnt);
         e = hipGetLastError();
     }

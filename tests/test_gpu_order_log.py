@@ -55,3 +55,18 @@ def test_full_store(scene, torch_mod):
     assert len(kept) == room
     rows = {r.tobytes() for r in every}
     assert all(r.tobytes() in rows for r in kept)
+
+
+@pytest.mark.parametrize("any_hit", [True, False])
+def test_many_rays_give_the_samples_of_fewer(scene, torch_mod, any_hit):
+    """Past the ray count where a ray gets fewer lanes the samples stay the same."""
+    n = 33_003
+    rays = scenes.random_rays(n, 14, (0, 0, 0), (1, 1, 1))
+    rays["tmax"][::7] = 0.3
+    rays["d"][5::501] = 0.0
+    got = log(scene, torch_mod, devmem.to_device(rays), n, any_hit, 1, 24 * n)
+    parts = [log(scene, torch_mod, devmem.to_device(rays[i:i + 5000]), len(rays[i:i + 5000]), any_hit, 1, 24 * 5000)
+             for i in range(0, n, 5000)]
+    want = np.concatenate(parts)
+    assert len(got) == len(want) < 24 * n
+    assert np.array_equal(as_sorted(got).view(np.uint32), as_sorted(want).view(np.uint32))
