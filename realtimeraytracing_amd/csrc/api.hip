@@ -390,7 +390,7 @@ rtq_status rtq_create(rtq_ctx** out, int hip_device) {
         hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&ctx->join, hipEventDisableTiming) != hipSuccess ||
         hipEventCreate(&ctx->build_begin) != hipSuccess || hipEventCreate(&ctx->build_end) != hipSuccess ||
-        hipHostMalloc(&ctx->pinned, kPinnedBytes, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(&ctx->pinned, kPinnedBytes + kHostRays * (sizeof(rtq_ray) + sizeof(rtq_hit)), hipHostMallocDefault) != hipSuccess ||
         scratch_alloc(ctx, &ctx->scratch) != RTQ_OK || noalloc_setup(ctx) != RTQ_OK) {
         scratch_free(&ctx->scratch);
         if (ctx->pinned) (void)hipHostFree(ctx->pinned);
@@ -850,13 +850,39 @@ rtq_status rtq_trace_host(rtq_ctx* ctx, uint32_t scene_id, const rtq_ray* rays, 
     if (n_rays == 0) return RTQ_OK;
     if (!rays || !hits) return fail(ctx, RTQ_EINVAL, "trace_host: null pointer");
     RTQ_HIP(ctx, hipSetDevice(ctx->device));
+    if (n_rays <= kHostRays) {
+        rtq_ray* const hr = reinterpret_cast<rtq_ray*>(static_cast<char*>(ctx->pinned) + kPinnedBytes);
+        rtq_hit* const hh = reinterpret_cast<rtq_hit*>(hr + kHostRays);
+        std::memcpy(hr, rays, sizeof(rtq_ray) * n_rays);
+        const rtq_status s = trace_common(ctx, scene_id, hr, n_rays, flags, hh, nullptr, nullptr, false, ctx->stream);
+        if (s != RTQ_OK) return s;
+        RTQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        std::memcpy(hits, hh, sizeof(rtq_hit) * n_rays);
+        return RTQ_OK;
+    }
     rtq_ray* dr = nullptr;
     rtq_hit* dh = nullptr;
-    RTQ_HIP(ctx, dev_alloc(&dr, n_rays));
-    hipError_t e = dev_alloc(&dh, n_rays);
-    if (e != hipSuccess) { (void)hipFree(dr); return hip_fail(ctx, e, "trace_host alloc"); }
+    Temps tmp(ctx);
+    struct Own {   // buffers past the scratch's limit
+        void *r = nullptr, *h = nullptr;
+        ~Own() {
+            if (r) (void)hipFree(r);
+            if (h) (void)hipFree(h);
+        }
+    } own;
+    if (n_rays <= kArenaRays) {
+        const rtq_status ra = arena_reserve(ctx);
+        if (ra != RTQ_OK) return ra;
+        RTQ_HIP(ctx, tmp.get(&dr, n_rays));
+        RTQ_HIP(ctx, tmp.get(&dh, n_rays));
+    } else {
+        RTQ_HIP(ctx, dev_alloc(&dr, n_rays));
+        own.r = dr;
+        RTQ_HIP(ctx, dev_alloc(&dh, n_rays));
+        own.h = dh;
+    }
     rtq_status s = RTQ_OK;
-    e = hipMemcpyAsync(dr, rays, sizeof(rtq_ray) * n_rays, hipMemcpyHostToDevice, ctx->stream);
+    hipError_t e = hipMemcpyAsync(dr, rays, sizeof(rtq_ray) * n_rays, hipMemcpyHostToDevice, ctx->stream);
     if (e != hipSuccess) s = hip_fail(ctx, e, "trace_host copy-in");
     if (s == RTQ_OK) s = trace_common(ctx, scene_id, dr, n_rays, flags, dh, nullptr, nullptr, false, ctx->stream);
     if (s == RTQ_OK) {
@@ -865,8 +891,6 @@ rtq_status rtq_trace_host(rtq_ctx* ctx, uint32_t scene_id, const rtq_ray* rays, 
     }
     e = hipStreamSynchronize(ctx->stream);
     if (s == RTQ_OK && e != hipSuccess) s = hip_fail(ctx, e, "trace_host sync");
-    (void)hipFree(dr);
-    (void)hipFree(dh);
     return s;
 }
 

@@ -139,8 +139,8 @@ struct rtq_ctx {
     hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
     hipEvent_t build_begin = nullptr, build_end = nullptr;   // a build's device time
-    // pinned host memory (rtq::kPinnedBytes) for the build's small device-to-
-    // host reads (rtq::HostReads)
+    // pinned host memory: rtq::kPinnedBytes for the build's small device-to-host
+    // reads (rtq::HostReads), then rtq::kHostRays rays and hits of rtq_trace_host
     void* pinned = nullptr;
     std::string err;
     std::map<uint32_t, rtq::Scene*> scenes;
@@ -168,6 +168,14 @@ struct rtq_ctx {
 
 namespace rtq {
 constexpr size_t kPinnedBytes = 128 << 10;
+// rtq_trace_host: up to kHostRays rays are read, and their hits written, by the
+// kernel in pinned host memory; up to kArenaRays in the context's scratch, more
+// in buffers of the call's own (so that one large call does not grow the scratch
+// for good).  1,021 rays on 960 triangles: 64 us with two allocations and two
+// copies, 48 in pinned memory.  2,000 triangles: 8,192 rays 78 us in pinned
+// memory and 98 in the scratch, 32,768 142 and 163, 65,536 246 and 232; 65,537
+// 249 us in the scratch, 287 with allocations.
+constexpr uint64_t kHostRays = 32768, kArenaRays = 262144;
 
 // Device-to-host reads staged through the context's pinned buffer (a copy to
 // pageable memory is staged and waited for one by one): add() queues a copy
