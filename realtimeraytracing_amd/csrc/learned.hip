@@ -397,52 +397,78 @@ struct GradLds {
     float d1[kTB * kLdH];   // gradients of the layers' inputs to ReLU [sample][unit]
     float d2[kTB * kLdH];
     float w2[kH * kLdH];    // [in][out]
-    float y[kTB], w[kTB], dz[kTB], loss[kTB];
+    float y[kTB], w[kTB], z[kTB], dz[kTB], loss[kTB], w3[kH];
 };
 static_assert(sizeof(GradLds) <= 160 * 1024, "one workgroup per CU");
 
-// Forward + backward of up to 64 samples: sample i of the step is
-// samples[(start + i) * mul % n]; writes the block's gradient sums and its sum
-// of weighted losses.  Loss of a sample: weight * BCE(sigmoid(z), label).
-// Every layer's product is 16 tiles of 16 x 16, one per wave, on the FP32
-// matrix instruction.  A training step has few blocks (16 at the default batch
-// of 1,024), so its time is one block's chain of phases: 98.6 us a step with a
-// block in one wave (a sample or a column per lane, each product a loop over
-// LDS), 11.5 us now.
+// The order of an epoch: position i of a step holds sample (base + i * mul) % n,
+// base < n, mul < n < 2^31 and i < 2^16.  i * mul is exact in a double, its
+// quotient by n wrong by one at most (a 64-bit remainder is 1,000 cycles).
+struct SampleOrder {
+    uint32_t n, base, mul;
+    double inv_n;
+    __device__ __forceinline__ uint32_t operator[](uint32_t i) const {
+        const uint64_t x = (uint64_t)i * mul;
+        const uint32_t q = (uint32_t)((double)x * inv_n);
+        int64_t r = (int64_t)(x - (uint64_t)q * n);
+        r += r < 0 ? (int64_t)n : 0;
+        r -= r >= (int64_t)n ? (int64_t)n : 0;
+        r += base;
+        return (uint32_t)(r >= (int64_t)n ? r - n : r);
+    }
+};
+
+// Forward + backward of up to 64 samples at the order's positions from 64 times
+// the block on; writes the block's gradient sums and its sum of weighted losses.
+// Loss of a sample: weight * BCE(sigmoid(z), label).  Every layer's product is
+// 16 tiles of 16 x 16, one per wave, on the FP32 matrix instruction.
+// A training step has few blocks (16 at the default batch of 1,024), so its time
+// is one block's chain of phases, bound by its CU's matrix and LDS rate: PARTS
+// workgroups share a block.  Each goes forward alone and takes 64 / PARTS of the
+// columns backward, so the sums are the same.  98.6 us a step with a block in one
+// wave (a sample or a column per lane, each product a loop over LDS), 11.5 with
+// one workgroup per block, 8.7 with four and every load issued at the start.
+template <int PARTS>
 __global__ __launch_bounds__(kGradThreads) void k_mlp_grad(const float* __restrict__ P,
-                                                           const float* __restrict__ samples, uint32_t n,
-                                                           uint64_t start, uint32_t count, uint64_t mul,
-                                                           float* __restrict__ partial,
+                                                           const float* __restrict__ samples, SampleOrder order,
+                                                           uint32_t count, float* __restrict__ partial,
                                                            float* __restrict__ loss_part) {
+    constexpr int kTiles = 4 / PARTS;     // column tiles of a workgroup going backward
+    const uint32_t block = blockIdx.x / PARTS, part = blockIdx.x % PARTS;
     __shared__ GradLds L;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c = lane & 15, g = lane >> 4;          // operand column and k group
     const int mt = 16 * (wave >> 2), nt = 16 * (wave & 3);   // the wave's tile
-    // layer 1's weights straight into operand registers, layer 2's to LDS
-    float w1[kIn / 4];
+    // every load of the block at once: the samples' rows (16 threads each), layer
+    // 1's weights straight into operand registers, layer 2's for LDS
+    const int s = tid >> 4;
+    const bool valid = block * kTB + s < count;
+    const float* row = samples + (size_t)(valid ? order[block * kTB + s] : 0u) * kSample;
+    float v[3], w1[kIn / 4], w2[kH * kH / kGradThreads];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const int k = (tid & 15) + 16 * r;
+        v[r] = valid && k < kSample ? row[k] : 0.0f;
+    }
+#pragma unroll
+    for (int r = 0; r < kH * kH / kGradThreads; ++r) w2[r] = P[kW2 + tid + r * kGradThreads];
 #pragma unroll
     for (int t = 0; t < kIn / 4; ++t) w1[t] = P[kW1 + (4 * t + g) * kH + nt + c];
     const float b1 = P[kB1 + nt + c], b2 = P[kB2 + nt + c], w3 = P[kW3 + nt + c];
+    const float b3 = c == 0 ? P[kB3] : 0.0f;
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const int k = (tid & 15) + 16 * r;
+        if (k < kIn) L.x[s * kLdX + k] = v[r];
+        if (k == kIn) L.y[s] = v[r];
+        if (k == kIn + 1) L.w[s] = v[r];
+    }
 #pragma unroll
     for (int r = 0; r < kH * kH / kGradThreads; ++r) {
         const int i = tid + r * kGradThreads;
-        L.w2[(i / kH) * kLdH + i % kH] = P[kW2 + i];
+        L.w2[(i / kH) * kLdH + i % kH] = w2[r];
     }
-    // 16 threads per sample
-    {
-        const int s = tid >> 4;
-        const uint32_t local = blockIdx.x * kTB + s;
-        const bool valid = local < count;
-        const float* row = samples + (valid ? ((start + local) * mul) % n : 0) * kSample;
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {
-            const int k = (tid & 15) + 16 * r;
-            const float v = valid && k < kSample ? row[k] : 0.0f;
-            if (k < kIn) L.x[s * kLdX + k] = v;
-            if (k == kIn) L.y[s] = v;
-            if (k == kIn + 1) L.w[s] = v;
-        }
-    }
+    if (wave < 4 && g == 0) L.w3[nt + c] = w3;
     __syncthreads();
     float h1[4], h2[4];   // the wave's tile of both layers
     {
@@ -468,17 +494,21 @@ __global__ __launch_bounds__(kGradThreads) void k_mlp_grad(const float* __restri
         }
     }
     __syncthreads();
-    if (tid < kTB) {   // output layer and loss, one sample per lane
-        float z = P[kB3];
-#pragma unroll 8
-        for (int j = 0; j < kH; ++j) z = fmaf(L.h2[tid * kLdH + j], P[kW3 + j], z);
-        // BCE with logits: max(z, 0) - z y + log(1 + e^-|z|); dL/dz = w (sigmoid(z) - y)
-        const float y = L.y[tid], w = L.w[tid];
-        const float p = 1.0f / (1.0f + expf(-z));
-        const float loss = w * ((fmaxf(z, 0.0f) - z * y) + log1pf(expf(-fabsf(z))));
-        const bool valid = blockIdx.x * kTB + tid < count;
-        L.dz[tid] = valid ? w * (p - y) : 0.0f;
-        L.loss[tid] = valid ? loss : 0.0f;
+    if (wave < 4) {   // output layer (in a tile's first column) of the wave's 16 samples
+        const int m0 = 16 * wave;
+        f32x4 acc = {b3, b3, b3, b3};
+#pragma unroll
+        for (int t = 0; t < kH / 4; ++t)
+            acc = mfma_step(L.h2[(m0 + c) * kLdH + 4 * t + g], c == 0 ? L.w3[4 * t + g] : 0.0f, acc);
+        if (c == 0)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) L.z[m0 + 4 * g + r] = acc[r];
+        wave_lds_fence();
+        if (lane < 16) {   // dL/dz = w (sigmoid(z) - y)
+            const int m = m0 + lane;
+            const float p = 1.0f / (1.0f + expf(-L.z[m]));
+            L.dz[m] = block * kTB + m < count ? L.w[m] * (p - L.y[m]) : 0.0f;
+        }
     }
     __syncthreads();
     // dH2 = dz * w3 * (h2 > 0)
@@ -488,51 +518,89 @@ __global__ __launch_bounds__(kGradThreads) void k_mlp_grad(const float* __restri
         L.d2[m * kLdH + nt + c] = h2[r] > 0.0f ? L.dz[m] * w3 : 0.0f;
     }
     __syncthreads();
-    float* out = partial + (size_t)blockIdx.x * kNP;
-    {   // dH1 = (dH2 W2^T) * (h1 > 0)
+    // backward: the part's columns, a tile of each product per wave
+    float* out = partial + (size_t)block * kNP;
+    const int col = 16 * kTiles * (int)part;              // the first of them
+    const int bt = 16 * (wave / kTiles % 4), bn = col + 16 * (wave % kTiles);
+    if (wave < 4 * kTiles) {   // dH1 = (dH2 W2^T) * (h1 > 0)
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int t = 0; t < kH / 4; ++t)
-            acc = mfma_step(L.d2[(mt + c) * kLdH + 4 * t + g], L.w2[(nt + c) * kLdH + 4 * t + g], acc);
+            acc = mfma_step(L.d2[(bt + c) * kLdH + 4 * t + g], L.w2[(bn + c) * kLdH + 4 * t + g], acc);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) L.d1[(mt + 4 * g + r) * kLdH + nt + c] = h1[r] > 0.0f ? acc[r] : 0.0f;
+        for (int r = 0; r < 4; ++r) {
+            const int m = bt + 4 * g + r;
+            L.d1[m * kLdH + bn + c] = L.h1[m * kLdH + bn + c] > 0.0f ? acc[r] : 0.0f;
+        }
     }
-    {   // dW2[k][j] = sum_s h1[s][k] dh2[s][j]
+    // dW2[k][j] = sum_s h1[s][k] dh2[s][j], by other waves where there are any
+    if (PARTS == 1 || (wave >= 4 && wave < 8)) {
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int t = 0; t < kTB / 4; ++t)
-            acc = mfma_step(L.h1[(4 * t + g) * kLdH + mt + c], L.d2[(4 * t + g) * kLdH + nt + c], acc);
+            acc = mfma_step(L.h1[(4 * t + g) * kLdH + bt + c], L.d2[(4 * t + g) * kLdH + bn + c], acc);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) out[kW2 + (mt + 4 * g + r) * kH + nt + c] = acc[r];
+        for (int r = 0; r < 4; ++r) out[kW2 + (bt + 4 * g + r) * kH + bn + c] = acc[r];
     }
+    const int j = col + lane;                             // a column per lane
+    const bool mine = lane < 16 * kTiles;
+    // the sums that need no dH1 beside it, or after it with the others
+    const auto column_sums = [&](int w) {
+        if (w == 0 && mine) {          // dw3[j] = sum_s h2[s][j] dz[s]
+            float acc = 0.0f;
+#pragma unroll 8
+            for (int s = 0; s < kTB; ++s) acc = fmaf(L.h2[s * kLdH + j], L.dz[s], acc);
+            out[kW3 + j] = acc;
+        } else if (w == 1 && mine) {   // db2[j] = sum_s dh2[s][j]
+            float acc = 0.0f;
+#pragma unroll 8
+            for (int s = 0; s < kTB; ++s) acc += L.d2[s * kLdH + j];
+            out[kB2 + j] = acc;
+        } else if (w == 2 && part == 0) {   // db3 = sum of dz (lane 0) and the block's loss (lane 1)
+            // BCE with logits: max(z, 0) - z y + log(1 + e^-|z|)
+            const float z = L.z[lane];
+            const float loss = L.w[lane] * ((fmaxf(z, 0.0f) - z * L.y[lane]) + log1pf(expf(-fabsf(z))));
+            L.loss[lane] = block * kTB + lane < count ? loss : 0.0f;
+            wave_lds_fence();
+            const float* sum = lane == 0 ? L.dz : L.loss;
+            float acc = 0.0f;
+            if (lane < 2)
+#pragma unroll 8
+                for (int s = 0; s < kTB; ++s) acc += sum[s];
+            if (lane == 0) out[kB3] = acc;
+            if (lane == 1) loss_part[block] = acc;
+        }
+    };
+    if (PARTS > 1) column_sums(wave - 8);
     __syncthreads();
-    if (wave < 8) {   // dW1[k][j] = sum_s x[s][k] dh1[s][j]
+    if (wave < 2 * kTiles) {   // dW1[k][j] = sum_s x[s][k] dh1[s][j]
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int t = 0; t < kTB / 4; ++t)
-            acc = mfma_step(L.x[(4 * t + g) * kLdX + mt + c], L.d1[(4 * t + g) * kLdH + nt + c], acc);
+            acc = mfma_step(L.x[(4 * t + g) * kLdX + bt + c], L.d1[(4 * t + g) * kLdH + bn + c], acc);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) out[kW1 + (mt + 4 * g + r) * kH + nt + c] = acc[r];
-    } else if (wave == 8) {   // dw3[j] = sum_s h2[s][j] dz[s]
+        for (int r = 0; r < 4; ++r) out[kW1 + (bt + 4 * g + r) * kH + bn + c] = acc[r];
+    } else if (wave == 11) {   // db1[j] = sum_s dh1[s][j]
         float acc = 0.0f;
+        if (mine)
 #pragma unroll 8
-        for (int s = 0; s < kTB; ++s) acc = fmaf(L.h2[s * kLdH + lane], L.dz[s], acc);
-        out[kW3 + lane] = acc;
-    } else if (wave < 11) {   // db2[j] = sum_s dh2[s][j] and db1[j] = sum_s dh1[s][j]
-        const float* d = wave == 9 ? L.d2 : L.d1;
-        float acc = 0.0f;
-#pragma unroll 8
-        for (int s = 0; s < kTB; ++s) acc += d[s * kLdH + lane];
-        out[(wave == 9 ? kB2 : kB1) + lane] = acc;
-    } else if (wave == 11) {   // db3 = sum of dz (lane 0) and the block's loss (lane 1)
-        const float* v = lane == 0 ? L.dz : L.loss;
-        float acc = 0.0f;
-        if (lane < 2)
-#pragma unroll 8
-            for (int s = 0; s < kTB; ++s) acc += v[s];
-        if (lane == 0) out[kB3] = acc;
-        if (lane == 1) loss_part[blockIdx.x] = acc;
+            for (int s = 0; s < kTB; ++s) acc += L.d1[s * kLdH + j];
+        if (mine) out[kB1 + j] = acc;
+    } else if (PARTS == 1) {
+        column_sums(wave - 8);
     }
+}
+
+// Workgroups per block of 64 samples: four while the chip has the CUs.
+int grad_parts(const rtq_ctx* ctx, uint32_t blocks) { return 4 * blocks <= (uint32_t)std::max(ctx->n_cu, 1) ? 4 : 1; }
+
+hipError_t queue_grad(const rtq_ctx* ctx, const float* params, const float* samples, const SampleOrder& order,
+                      uint32_t count, float* partial, float* loss_part, hipStream_t st) {
+    const uint32_t blocks = (count + kTB - 1) / kTB;
+    const int parts = grad_parts(ctx, blocks);
+    hipLaunchKernelGGL(parts == 4 ? &k_mlp_grad<4> : &k_mlp_grad<1>, dim3(blocks * parts), dim3(kGradThreads), 0, st,
+                       params, samples, order, count, partial, loss_part);
+    return hipGetLastError();
 }
 
 // The blocks' gradients of parameter j, summed in block order (deterministic)
@@ -870,9 +938,7 @@ rtq_status rtq_order_grad(rtq_ctx* ctx, const float* params_dev, const float* sa
     RTQ_HIP(ctx, dev_alloc(&partial, (size_t)blocks * kNP));
     hipError_t e = dev_alloc(&lp, blocks);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_mlp_grad, dim3(blocks), dim3(kGradThreads), 0, st, params_dev, samples_dev, n, 0ull, n, 1ull,
-                           partial, lp);
-        e = hipGetLastError();
+        e = queue_grad(ctx, params_dev, samples_dev, SampleOrder{n, 0u, 1u, 1.0 / n}, n, partial, lp, st);
     }
     if (e == hipSuccess) {
         hipLaunchKernelGGL(k_mlp_reduce, dim3(kParamBlocks), dim3(kParamThreads), 0, st, partial, blocks,
@@ -923,9 +989,8 @@ rtq_status rtq_order_train(rtq_ctx* ctx, const float* samples_dev, uint64_t n_sa
             const uint64_t start = (uint64_t)sidx * tp->batch;
             const uint32_t cnt = (uint32_t)std::min<uint64_t>(tp->batch, n - start);
             const uint32_t bl = (cnt + kTB - 1) / kTB;
-            hipLaunchKernelGGL(k_mlp_grad, dim3(bl), dim3(kGradThreads), 0, st, params_dev, samples_dev, n, start, cnt,
-                               mul, partial, lp + (size_t)sidx * blocks);
-            e = hipGetLastError();
+            const SampleOrder order{n, (uint32_t)(start * mul % n), (uint32_t)mul, 1.0 / n};
+            e = queue_grad(ctx, params_dev, samples_dev, order, cnt, partial, lp + (size_t)sidx * blocks, st);
             if (e != hipSuccess) break;
             const uint32_t tstep = ++*step;
             const float c1 = 1.0f - powf(tp->beta1, (float)tstep), c2 = 1.0f - powf(tp->beta2, (float)tstep);

@@ -445,6 +445,13 @@ __device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t x) {
     return x;
 }
 
+// Orders a wave's LDS writes before its later LDS reads.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // A middle subtree's list of clusters: each level's first one has this bit.
 constexpr uint32_t kLevelStart = 1u << 31;
 

@@ -288,13 +288,6 @@ __device__ __forceinline__ float4 image_part(const uint32_t* img, uint32_t i) {
     return make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w));
 }
 
-// Orders a wave's LDS writes before its later LDS reads.
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Tile status of the level scan: value in the low 32 bits, state on top.
 constexpr uint64_t kLvAgg = 1ull << 62;     // the tile's own count
 constexpr uint64_t kLvPre = 2ull << 62;     // the counts through the tile

@@ -47,3 +47,22 @@ def test_step_is_gradient_and_adam(rtq_ctx, torch_mod, n):
     assert np.allclose(vh, (f(1) - b2) * (mh / (f(1) - b1)) ** 2, rtol=1e-5, atol=1e-30)
     want = P - f(1e-2) * (mh / (f(1) - b1)) / (np.sqrt(vh / (f(1) - b2)) + f(1e-8))
     assert np.allclose(dP.cpu().numpy(), want, rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("n,batch", [(1, 64), (130, 128), (5001, 4096), (70_003, 16384)])
+def test_epoch_visits_every_sample_once(rtq_ctx, torch_mod, n, batch):
+    """An epoch in the order i * mul mod n, with four workgroups per block of
+    samples and with one, takes each sample once."""
+    torch = torch_mod
+    P, S = rand_params(3), rand_samples(n, n + 9)
+    dP, dS = dev(P, torch), dev(S, torch)
+    m, v = (torch.zeros(ORDER_PARAMS, dtype=torch.float32, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    # no learning: every step of the epoch has the same parameters, so the
+    # epoch's loss is the mean over all samples, each visited once
+    tp = TrainParams(1, batch, 0.0, 0.9, 0.999, 0, 3)
+    _, losses = rtq_ctx.order_train(dS.data_ptr(), n, tp, dP.data_ptr(), m.data_ptr(), v.data_ptr())
+    want, _ = oracle.mlp_grad(P, S)
+    rel = 2.0 ** -24 * (64 + n / 64) * 4
+    assert losses[0] == pytest.approx(want, rel=rel)
+    assert np.array_equal(dP.cpu().numpy(), P)
