@@ -146,7 +146,7 @@ inline uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + kThreads - 1) / 
 // 3 float4 per triangle, the original id in the w of the first.  ref: the
 // scene's own triangles; src the same, or an update's, which are copied there on
 // the way.  A workgroup's triangles come in, and its vertices go out, through
-// LDS, so that neighbouring lanes read and write neighbouring 16 B.  2,095,104
+// LDS, so that neighbouring lanes read and write neighbouring 16 B.  2,093,058
 // triangles: a copy and a second read 106 us, in one pass with each lane's 64 B
 // read and written by itself 91 us, 59 us so.
 __global__ __launch_bounds__(kThreads) void k_world(const uint4* src, const DevModel* __restrict__ models, uint32_t n,

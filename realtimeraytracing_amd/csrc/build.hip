@@ -1304,7 +1304,7 @@ __global__ __launch_bounds__(kThreads) void k_write_ref(
 //   [c1.lo.y c1.hi.y c1.lo.z c1.hi.z] [ref0 ref1 order 0]
 // where `order` holds the learned child-order bits (zero until a model is applied).
 // One thread per merged cluster c; what a child needs besides its box follows
-// from the node's own place and the counts below the children.  2,095,104
+// from the node's own place and the counts below the children.  2,093,058
 // triangles: 150 us when a child's index came from a scan over marks in
 // pre-order, 61 us with the counts that PLOC's merges keep (they cost its passes
 // nothing).

@@ -189,7 +189,7 @@ constexpr uint32_t kSortSpinLimit = 1u << 24;   // ~0.5 s of s_sleep(1) polls
 // counts) and adds its non-zero bins: 256 workgroups, since the additions to
 // one bin serialise.  Neighbouring triangles' codes share their high digits,
 // and the lanes that add to one bin serialise too: each bin has a word per
-// eighth of a wave (2,095,104 Morton codes: 22.0 us with one word, 10.6 now;
+// eighth of a wave (2,093,058 Morton codes: 22.0 us with one word, 10.6 now;
 // 5,000,000 random keys 15.1 and 15.6).
 __global__ __launch_bounds__(kSortThreads) void k_sort_hist(const uint32_t* __restrict__ keys, uint32_t n,
                                                             uint32_t n_digits, uint32_t* __restrict__ hist) {

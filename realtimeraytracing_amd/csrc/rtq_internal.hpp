@@ -393,7 +393,7 @@ TopPasses top_passes(const Scene* s);
 // the top ones.  A pass of up to kSubPass merges is shorter than its launch, and
 // a tree has twenty of them: a workgroup takes a subtree through all its levels.
 // Larger passes fill the chip by themselves and keep a launch each.  Rebuild of
-// 2,095,104 triangles (28 passes below the top ones, placed and costed by 56
+// 2,093,058 triangles (28 passes below the top ones, placed and costed by 56
 // launches): 2,161 us; with the middle ones as subtrees 2,097 us (18 launches),
 // with passes up to 8,192 / 32,768 / 131,072 merges in them 2,127 / 2,104 /
 // 2,128 us, with all 2,267 us: few workgroups then have the long subtrees.

@@ -329,7 +329,7 @@ struct LevelArgs {
 // upper bound of the level's count; workgroups past the count, and every
 // workgroup of an empty level, return at once.
 // The chain of dependent loads down to a slot's child bounds small levels, the
-// children's scattered boxes large ones.  2,095,104 triangles, 12 levels: 354 us
+// children's scattered boxes large ones.  2,093,058 triangles, 12 levels: 354 us
 // with one thread per node (its walk, boxes and quantisation one child after
 // another), 171 us now; a level of a few nodes 20 us and 6 us.
 __global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
