@@ -214,8 +214,10 @@ static hipError_t queue_world(rtq_ctx* ctx, Scene* s, const rtq_triangle* src) {
 // included) are not all finite and at most 2^28 in magnitude; both start at
 // kNone.  A float is finite with |x| <= 2^28 exactly when its bits without the
 // sign are at most those of 2^28 (0x4D800000): infinities and NaNs lie above.
+// any_bad (zero before): one if there is any.
 __global__ __launch_bounds__(kThreads) void k_check_tris(const uint4* __restrict__ tris, uint32_t n,
-                                                         uint32_t n_models, uint32_t* __restrict__ bad) {
+                                                         uint32_t n_models, uint32_t* __restrict__ bad,
+                                                         uint32_t* __restrict__ any_bad) {
     const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
     const uint4 p0 = tris[4ull * i], p1 = tris[4ull * i + 1], p2 = tris[4ull * i + 2], rest = tris[4ull * i + 3];
@@ -225,6 +227,7 @@ __global__ __launch_bounds__(kThreads) void k_check_tris(const uint4* __restrict
     const uint32_t m = max(mag(p0), max(mag(p1), mag(p2)));
     if (rest.x >= n_models) atomicMin(bad, i);
     if (m > 0x4D800000u) atomicMin(bad + 1, i);
+    if (rest.x >= n_models || m > 0x4D800000u) *any_bad = 1;
 }
 
 __device__ __forceinline__ uint64_t splitmix64(uint64_t z) {
@@ -390,7 +393,8 @@ rtq_status rtq_create(rtq_ctx** out, int hip_device) {
         hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&ctx->join, hipEventDisableTiming) != hipSuccess ||
         hipEventCreate(&ctx->build_begin) != hipSuccess || hipEventCreate(&ctx->build_end) != hipSuccess ||
-        hipHostMalloc(&ctx->pinned, kPinnedBytes + kHostRays * (sizeof(rtq_ray) + sizeof(rtq_hit)), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(&ctx->pinned, kPinnedBytes + kHostRays * (sizeof(rtq_ray) + sizeof(rtq_hit)) + 4 * kReportWords,
+                      hipHostMallocDefault) != hipSuccess ||
         scratch_alloc(ctx, &ctx->scratch) != RTQ_OK || noalloc_setup(ctx) != RTQ_OK) {
         scratch_free(&ctx->scratch);
         if (ctx->pinned) (void)hipHostFree(ctx->pinned);
@@ -473,9 +477,13 @@ static rtq_status check_models(rtq_ctx* ctx, const char* what, const rtq_mesh_mo
 static rtq_status check_tris_on_device(rtq_ctx* ctx, const char* what, const rtq_triangle* host,
                                        const rtq_triangle* dev, uint32_t n, uint32_t n_models, uint32_t* words,
                                        hipStream_t st) {
+    uint32_t* const any_bad = report(ctx);
+    *any_bad = 0;
     hipLaunchKernelGGL(k_check_tris, dim3(blocks_for(n)), dim3(kThreads), 0, st, reinterpret_cast<const uint4*>(dev),
-                       n, n_models, words);
+                       n, n_models, words, any_bad);
     RTQ_HIP(ctx, hipGetLastError());
+    RTQ_HIP(ctx, hipStreamSynchronize(st));
+    if (*static_cast<volatile uint32_t*>(any_bad) == 0) return RTQ_OK;
     uint32_t bad[2];
     HostReads rd(ctx, st);
     RTQ_HIP(ctx, rd.add(bad, words, sizeof bad));

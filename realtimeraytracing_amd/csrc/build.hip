@@ -154,11 +154,18 @@ __global__ __launch_bounds__(kLdsThreads) void k_refit_merge_lds(TopPasses passe
 // before right) order with a wave prefix sum, which is the order a FIFO
 // breadth-first walk appends them; children past kTopNodes keep their refs.
 static_assert(kTopNodes <= 64, "one lane per top-of-tree slot");
-// A second workgroup, if launched, takes the maximum of block_depth.
+// A second workgroup, if launched, writes the host's words: the scene's box, and
+// after a build (n_blocks > 0) the sort's error word (the one past the two boxes
+// of bounds) and the maximum of block_depth.
+struct BuildReport {
+    rtq_aabb box;
+    uint32_t sort_err, depth;
+};
 constexpr int kTopThreads = 1024;
 __global__ __launch_bounds__(kTopThreads) void k_top_nodes(const float4* __restrict__ nodes, float4* __restrict__ top,
                                                            const uint32_t* __restrict__ block_depth, uint32_t n_blocks,
-                                                           uint32_t* __restrict__ depth) {
+                                                           const rtq_aabb* __restrict__ bounds,
+                                                           BuildReport* __restrict__ host) {
     if (blockIdx.x == 1) {
         __shared__ uint32_t s_max[kTopThreads / 64];
         uint32_t m = 0;
@@ -169,7 +176,9 @@ __global__ __launch_bounds__(kTopThreads) void k_top_nodes(const float4* __restr
         __syncthreads();
         if (threadIdx.x == 0) {
             for (uint32_t w = 1; w < kTopThreads / 64; ++w) m = max(m, s_max[w]);
-            *depth = m;
+            host->box = bounds[0];
+            host->sort_err = n_blocks ? *reinterpret_cast<const uint32_t*>(bounds + 2) : 0u;
+            host->depth = m;
         }
         return;
     }
@@ -449,6 +458,9 @@ __device__ __forceinline__ uint32_t nearest_in_window(const Box6* w, int i, int 
 // and, unless null, the fused passes' state (kPlocHeadWords words).
 constexpr uint32_t kPlocBatch = 16;
 constexpr uint32_t kPlocHeadWords = 16 + 4 * kPlocBatch;   // state (8), errors and tail pass count (8), pass log
+constexpr uint32_t kTailPeek = 128;                        // tail log entries that reach the host with them
+constexpr uint32_t kPlocReportWords = kPlocHeadWords + 4 * kTailPeek;
+static_assert(kPlocReportWords <= kReportWords && kPlocReportWords <= 1024, "one word per thread of the tail");
 
 __global__ __launch_bounds__(kThreads) void k_leaf_init(const rtq_triangle* __restrict__ tris,
                                                         const DevModel* __restrict__ models,
@@ -1012,7 +1024,7 @@ __device__ __forceinline__ uint32_t tail_merge(TailLists& L, int tid, uint32_t m
 __global__ __launch_bounds__(kTailThreads) void k_ploc_tail(uint32_t* __restrict__ state, uint32_t radius,
                                                             uint32_t* __restrict__ err, uint4* __restrict__ log,
                                                             uint32_t* __restrict__ log_count, PlocLists lists,
-                                                            PlocClusters cl) {
+                                                            PlocClusters cl, uint32_t* __restrict__ host) {
     __shared__ TailLists L;
     __shared__ uint32_t s_hdr[4];
     Box6* const s_box = L.list + kRefRadius;
@@ -1027,7 +1039,18 @@ __global__ __launch_bounds__(kTailThreads) void k_ploc_tail(uint32_t* __restrict
         if (s_hdr[3]) *log_count = 0;
     }
     __syncthreads();
-    if (s_hdr[3]) return;
+    // at the end, the head words and the log's first entries for the host: once
+    // every wave's own stores and atomics are done, read past the vector cache
+    const auto tell = [&]() {
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (tid < (int)kPlocReportWords)
+            host[tid] = __hip_atomic_load(state + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    if (s_hdr[3]) {
+        tell();
+        return;
+    }
     uint32_t m = s_hdr[0], n_total = s_hdr[1];
     const uint32_t cur = s_hdr[2];
     for (uint32_t q = tid; q < m; q += kTailThreads) {
@@ -1084,6 +1107,7 @@ __global__ __launch_bounds__(kTailThreads) void k_ploc_tail(uint32_t* __restrict
         state[3] = L.n[0].y;   // the root's, once one cluster is left
         *log_count = passes;
     }
+    tell();
 }
 
 // Clusters of one PLOC pass give their children's places (their own are known:
@@ -1370,7 +1394,7 @@ inline uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + kThreads - 1) / 
 
 // Shared front half of the build and of rtq_morton_codes: scene box + cube.
 // d_bounds holds 2 boxes, the words that a build reads back with them (8, the
-// first one zeroed here: the sort's errors, then the depth), and 6 floats per
+// first one zeroed here: the sort's errors), and 6 floats per
 // partial block (at most kBoundsPartials): kBoundsBoxes boxes of 32 B.
 constexpr uint32_t kBoundsPartials = 1024;
 constexpr uint32_t kBoundsBoxes = 3 + (6 * kBoundsPartials + 7) / 8;
@@ -1431,15 +1455,13 @@ rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
         }
         // the state of the batch's last pass is in slot 0 (kPlocBatch is even)
         hipLaunchKernelGGL(k_ploc_tail, dim3(1), dim3(kTailThreads), 0, st, state, radius, err, tail_log, tail_count,
-                           lists, cl);
+                           lists, cl, report(ctx));
         RTQ_HIP(ctx, hipGetLastError());
-        // the head block and the first tail log entries in one read (entries
-        // past the tail's pass count are not used)
-        constexpr uint32_t kTailPeek = 128;
-        uint32_t h_head[kPlocHeadWords + 4 * kTailPeek];
-        HostReads rd(ctx, st);
-        RTQ_HIP(ctx, rd.add(h_head, state, sizeof h_head));
-        RTQ_HIP(ctx, rd.wait());
+        // the head block and the first tail log entries (those past the tail's
+        // pass count are not used)
+        RTQ_HIP(ctx, hipStreamSynchronize(st));
+        uint32_t h_head[kPlocReportWords];
+        std::memcpy(h_head, report(ctx), sizeof h_head);
         const uint32_t* h_state = h_head;
         const uint32_t* h_err = h_head + 8;
         uint4 h_log[kPlocBatch];
@@ -1461,6 +1483,7 @@ rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
             if (nt <= kTailPeek) {
                 memcpy(h_tail.data(), h_head + kPlocHeadWords, sizeof(uint4) * nt);
             } else {
+                HostReads rd(ctx, st);
                 RTQ_HIP(ctx, rd.add(h_tail.data(), tail_log, sizeof(uint4) * nt));
                 RTQ_HIP(ctx, rd.wait());
             }
@@ -1584,7 +1607,7 @@ private:
 // boxes: its placement is kept and the 8-wide nodes keep their children.
 // d_bounds: the scene's box, cube and words (compute_bounds), after a refit the
 // root cluster's box.
-rtq_status write_layouts(rtq_ctx* ctx, Scene* s, rtq_aabb* d_bounds, hipStream_t st, bool refit) {
+rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipStream_t st, bool refit) {
     const uint32_t n = s->n_tris;
     const uint32_t nc = s->n_clusters;
     Temps tmp(ctx);
@@ -1646,7 +1669,7 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, rtq_aabb* d_bounds, hipStream_t
                        s->cright, s->ccount, s->ctrav, s->placed, s->tris, bdep, s->nodes, s->node_aux);
     RTQ_HIP(ctx, hipGetLastError());
     // the depth depends on the topology only: a refit keeps it
-    rs = write_top(ctx, s, bdep, leaf_blocks, refit ? nullptr : reinterpret_cast<uint32_t*>(d_bounds + 2) + 1, st);
+    rs = write_top(ctx, s, bdep, refit ? 0u : leaf_blocks, d_bounds, st);
     if (rs != RTQ_OK) return rs;
     if (s->params.node_width == 8) {
         if (refit) {
@@ -1658,15 +1681,9 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, rtq_aabb* d_bounds, hipStream_t
         if (rs != RTQ_OK) return rs;
     }
     if (!refit) RTQ_HIP(ctx, hipEventRecord(ctx->build_end, st));
-    // one host read: the scene's box (for the box margin) and after a build the
-    // sort's errors and the tree depth
-    struct {
-        rtq_aabb box, cube;
-        uint32_t sort_err, depth;
-    } h{};
-    HostReads rd(ctx, st);
-    RTQ_HIP(ctx, rd.add(&h, d_bounds, refit ? sizeof h.box : sizeof h));
-    RTQ_HIP(ctx, rd.wait());
+    RTQ_HIP(ctx, hipStreamSynchronize(st));
+    BuildReport h;
+    std::memcpy(&h, report(ctx), sizeof h);
     if (h.sort_err) return fail(ctx, RTQ_EINTERNAL, "build: a radix sort pass's look-back gave up");
     if (!refit) s->depth = h.depth;
     s->box_pad = box_pad_of(h.box);
@@ -1800,14 +1817,14 @@ rtq_status build_scene(rtq_ctx* ctx, Scene* s, const rtq_build_params& prm) {
     return RTQ_OK;
 }
 
-rtq_status write_top(rtq_ctx* ctx, Scene* s, const uint32_t* block_depth, uint32_t n_blocks, uint32_t* depth,
+rtq_status write_top(rtq_ctx* ctx, Scene* s, const uint32_t* block_depth, uint32_t n_blocks, const rtq_aabb* bounds,
                      hipStream_t st) {
-    if (kTopNodes == 0 && !depth) return RTQ_OK;
+    if (kTopNodes == 0 && !bounds) return RTQ_OK;
     // the set depends on the topology only, so a refit or an order update
     // rewrites the same buffer with the same node count
     if (!s->top) RTQ_HIP(ctx, dev_alloc(&s->top, 4ull * std::max(kTopNodes, 1u)));
-    hipLaunchKernelGGL(k_top_nodes, dim3(depth ? 2 : 1), dim3(kTopThreads), 0, st, s->nodes, s->top, block_depth,
-                       n_blocks, depth);
+    hipLaunchKernelGGL(k_top_nodes, dim3(bounds ? 2 : 1), dim3(kTopThreads), 0, st, s->nodes, s->top, block_depth,
+                       n_blocks, bounds, reinterpret_cast<BuildReport*>(report(ctx)));
     RTQ_HIP(ctx, hipGetLastError());
     s->n_top = std::min(kTopNodes, s->n_trav);   // every traversal node can be reached from the root
     return RTQ_OK;

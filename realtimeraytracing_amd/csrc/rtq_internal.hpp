@@ -140,7 +140,8 @@ struct rtq_ctx {
     hipEvent_t fork = nullptr, join = nullptr;
     hipEvent_t build_begin = nullptr, build_end = nullptr;   // a build's device time
     // pinned host memory: rtq::kPinnedBytes for the build's small device-to-host
-    // reads (rtq::HostReads), then rtq::kHostRays rays and hits of rtq_trace_host
+    // reads (rtq::HostReads), then rtq::kHostRays rays and hits of rtq_trace_host,
+    // then rtq::kReportWords words that kernels write for the host (rtq::report)
     void* pinned = nullptr;
     std::string err;
     std::map<uint32_t, rtq::Scene*> scenes;
@@ -176,6 +177,14 @@ constexpr size_t kPinnedBytes = 128 << 10;
 // memory and 98 in the scratch, 32,768 142 and 163, 65,536 246 and 232; 65,537
 // 249 us in the scratch, 287 with allocations.
 constexpr uint64_t kHostRays = 32768, kArenaRays = 262144;
+
+// Words that a kernel writes for the host, which reads them after it has waited
+// for the stream: no copy launch (about 4 us) before the wait.
+constexpr uint32_t kReportWords = 1024;
+inline uint32_t* report(const rtq_ctx* ctx) {
+    return reinterpret_cast<uint32_t*>(static_cast<char*>(ctx->pinned) + kPinnedBytes +
+                                       kHostRays * (sizeof(rtq_ray) + sizeof(rtq_hit)));
+}
 
 // Device-to-host reads staged through the context's pinned buffer (a copy to
 // pageable memory is staged and waited for one by one): add() queues a copy
@@ -416,9 +425,9 @@ rtq_status write_wide_order(rtq_ctx* ctx, Scene* s, bool clear, hipStream_t st);
 // New boxes for the kept topology after rtq_scene_update (build.hip).
 rtq_status refit_scene(rtq_ctx* ctx, Scene* s);
 // (Re)writes s->top from s->nodes: after the traversal nodes or their order
-// words change (build.hip).  depth, unless null: a device word for the maximum
-// of block_depth's n_blocks words.
-rtq_status write_top(rtq_ctx* ctx, Scene* s, const uint32_t* block_depth, uint32_t n_blocks, uint32_t* depth,
+// words change (build.hip).  bounds, unless null: reported to the host (see
+// k_top_nodes) with the maximum of block_depth's n_blocks words.
+rtq_status write_top(rtq_ctx* ctx, Scene* s, const uint32_t* block_depth, uint32_t n_blocks, const rtq_aabb* bounds,
                      hipStream_t st);
 // Writes s->ref_nodes (the reference's pre-order BVH_NodeGPU array) from the
 // cluster arrays when the build or refit since the last call changed them;
