@@ -317,7 +317,7 @@ __global__ __launch_bounds__(64) void k_order_log(const float4* __restrict__ nod
             }
             const uint32_t flags = (found ? 1u : 0u) | (ok && ok2 ? 2u : 0u);
             cost += rest;
-            uint32_t choice = 0;   // the children taken so far in this round
+            uint32_t choice = 0;   // the children taken since these walks
 #pragma unroll
             for (uint32_t l = 0; l < (uint32_t)AHEAD; ++l) {
                 const int from = (int)(lead + (2u << l) - 2u + 2u * choice);
