@@ -56,9 +56,9 @@ def host_flags() -> list[str]:
     return ["-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-ffp-contract=off", "-Wall", f"-I{ROOT / 'include'}"]
 
 
-def _compile(src: str) -> Path:
-    obj = OBJ / (Path(src).stem + ".o")
-    flags = host_flags() if src.endswith(".cpp") else compile_flags()
+def _compile(src: str, tag: str = "", defines: tuple[str, ...] = ()) -> Path:
+    obj = OBJ / (Path(src).stem + tag + ".o")
+    flags = [*(host_flags() if src.endswith(".cpp") else compile_flags()), *defines]
     cmd = [hipcc(), *flags, "-c", str(CSRC / src), "-o", str(obj)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
@@ -110,6 +110,24 @@ def build_oracle(verbose: bool = False) -> Path:
     return out
 
 
+def build_impatient(verbose: bool = False) -> Path:
+    """librtq with look-backs that wait for no other workgroup (RTQ_TILE_PATIENCE
+    0), for the tests: after build_library, whose other objects it links."""
+    waiting = ["build.hip", "primitives.hip", "wide.hip"]
+    with concurrent.futures.ThreadPoolExecutor(max_workers=len(waiting)) as ex:
+        objs = list(ex.map(lambda s: _compile(s, "_impatient", ("-DRTQ_TILE_PATIENCE=0",)), waiting))
+    objs += [OBJ / (Path(s).stem + ".o") for s in SOURCES if s not in waiting]
+    out = ROOT / "tests" / "cpp" / "build" / "librtq_impatient.so"
+    out.parent.mkdir(exist_ok=True)
+    cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(out), *map(str, objs)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
+    if verbose:
+        print(f"built {out}")
+    return out
+
+
 def build_cpp_check(verbose: bool = False) -> Path:
     """The C++ wrapper check program run by the GPU tests (tests/cpp)."""
     src = ROOT / "tests" / "cpp" / "wrapper_check.cpp"
@@ -134,4 +152,5 @@ if __name__ == "__main__":
     build_probe(verbose=True)
     if "--with-oracle" in sys.argv:
         build_oracle(verbose=True)
+        build_impatient(verbose=True)
         build_cpp_check(verbose=True)

@@ -155,11 +155,10 @@ __global__ __launch_bounds__(kLdsThreads) void k_refit_merge_lds(TopPasses passe
 // breadth-first walk appends them; children past kTopNodes keep their refs.
 static_assert(kTopNodes <= 64, "one lane per top-of-tree slot");
 // A second workgroup, if launched, writes the host's words: the scene's box, and
-// after a build (n_blocks > 0) the sort's error word (the one past the two boxes
-// of bounds) and the maximum of block_depth.
+// after a build (n_blocks > 0) the maximum of block_depth.
 struct BuildReport {
     rtq_aabb box;
-    uint32_t sort_err, depth;
+    uint32_t depth;
 };
 constexpr int kTopThreads = 1024;
 __global__ __launch_bounds__(kTopThreads) void k_top_nodes(const float4* __restrict__ nodes, float4* __restrict__ top,
@@ -177,7 +176,6 @@ __global__ __launch_bounds__(kTopThreads) void k_top_nodes(const float4* __restr
         if (threadIdx.x == 0) {
             for (uint32_t w = 1; w < kTopThreads / 64; ++w) m = max(m, s_max[w]);
             host->box = bounds[0];
-            host->sort_err = n_blocks ? *reinterpret_cast<const uint32_t*>(bounds + 2) : 0u;
             host->depth = m;
         }
         return;
@@ -265,7 +263,7 @@ __global__ __launch_bounds__(kThreads) void k_bounds_partial(const rtq_triangle*
 }
 
 // Reduces the partial boxes, then (one thread) the circumscribed cube of
-// bvh.cpp:253-303.  out[0] = scene box, out[1] = cube, one word zero after them.
+// bvh.cpp:253-303.  out[0] = scene box, out[1] = cube.
 __global__ __launch_bounds__(kThreads) void k_bounds_final(const float* __restrict__ partial, uint32_t nb,
                                                            uint32_t n, uint32_t pad_origin,
                                                            rtq_aabb* __restrict__ out) {
@@ -320,7 +318,6 @@ __global__ __launch_bounds__(kThreads) void k_bounds_final(const float* __restri
         delta = (max_dist - dist_y) / 2.0f; c.max[1] += delta; c.min[1] -= delta;
     }
     out[1] = c;
-    *reinterpret_cast<uint32_t*>(out + 2) = 0;
 }
 
 // ------------------------------------------------------------- Morton codes
@@ -477,8 +474,7 @@ __global__ __launch_bounds__(kThreads) void k_leaf_init(const rtq_triangle* __re
     if (i == 0) cparent[2 * n - 2] = kNone;
     if (state && i < 16) state[i] = i < 2 ? n : 0u;
     if (i >= n) return;
-    // in range even after a failed sort (which fails the build)
-    const uint32_t ti = min(sorted_idx[i], n - 1);
+    const uint32_t ti = sorted_idx[i];
     const rtq_triangle t = tris[ti];
     Box6 b;
     tri_box(t, models[t.model_id], b.lo, b.hi);
@@ -610,14 +606,11 @@ __global__ void k_ploc_advance(const uint2* __restrict__ tot, uint32_t* __restri
 // stay flags of its positions, scans them inside the workgroup and gets the
 // counts before its tile by decoupled look-back over per-tile status words
 // (Merrill & Garland, "Single-pass Parallel Prefix Scan with Decoupled
-// Look-back", 2016).  Tiles are numbered in the order workgroups start (an
-// atomic counter), so every tile a workgroup waits on is already running, and
-// the wait is bounded (kSpinLimit) so a broken invariant ends in an error
-// flag instead of a hang.  A status word carries its counts, so it is stored
+// Look-back", 2016).  Tiles are numbered by take_tile; a tile that has published
+// nothing for long (kTilePatience) is counted by the wave that waits for it
+// (ploc_tile_counts).  A status word carries its counts, so it is stored
 // and loaded with relaxed device-scope atomics: acquire / release would add an
-// L2 write-back or invalidate per poll.  A tile whose wait gave up publishes
-// kTilePoison; a tile whose look-back reaches one poisons itself too and
-// neither writes its clusters.  Each position goes through the arithmetic of
+// L2 write-back or invalidate per poll.  Each position goes through the arithmetic of
 // k_ploc_nn, k_ploc_flags and k_ploc_merge, so the clusters are identical.
 //
 // Passes with at most kTailMax clusters (33 of the 61 passes of a 2M-triangle
@@ -632,11 +625,9 @@ constexpr int kTailThreads = 1024;
 constexpr uint32_t kTailMax = 4 * kTailThreads;   // 4 positions per tail thread
 constexpr uint64_t kTileAgg = 1ull << 62;         // tile status: own counts published
 constexpr uint64_t kTilePre = 2ull << 62;         // tile status: counts through this tile
-constexpr uint64_t kTilePoison = 3ull << 62;      // tile status: a wait at or before it gave up
 constexpr uint64_t kTileState = 3ull << 62;
-constexpr uint32_t kSpinLimit = 1u << 24;         // ~0.5 s of s_sleep(1) polls
 
-enum : uint32_t { kPlocErrSpin = 1, kPlocErrNoNeighbour = 2, kPlocErrBound = 4, kPlocErrNoMerge = 8 };
+enum : uint32_t { kPlocErrNoNeighbour = 1, kPlocErrBound = 2, kPlocErrNoMerge = 4 };
 
 struct PlocLists {
     uint32_t* c[2];
@@ -732,12 +723,38 @@ struct PlocPassArgs {
     PlocClusters cl;
 };
 
+// Merges and stays of the list's positions [first, end), by one wave, from the
+// list itself: the counts that the tile which owns them publishes.
+__device__ uint2 ploc_tile_counts(const Box6* __restrict__ list, int first, int end, int r, int n) {
+    const auto nearest = [&](int i) {
+        const Box6 b = list[i];
+        float best = INFINITY;
+        uint32_t arg = kNone;
+        for (int j = max(i - r, 0); j < min(i + r + 1, n); ++j) {
+            const float d = merge_cost(b, list[j]);
+            const bool take = j != i && d < best;
+            best = take ? d : best;
+            arg = take ? (uint32_t)j : arg;
+        }
+        return arg;
+    };
+    uint2 counts = make_uint2(0u, 0u);
+    for (int i0 = first; i0 < end; i0 += 64) {
+        const int i = i0 + ((int)threadIdx.x & 63);
+        const uint32_t j = i < end ? nearest(i) : kNone;
+        const bool mutual = j != kNone && nearest((int)j) == (uint32_t)i;
+        counts.x += (uint32_t)__popcll(__ballot(mutual && (uint32_t)i < j));
+        counts.y += (uint32_t)__popcll(__ballot(i < end && !(mutual && j < (uint32_t)i)));
+    }
+    return counts;
+}
+
 __global__ __launch_bounds__(kPassThreads) void k_ploc_pass(PlocPassArgs a) {
     __shared__ Box6 s_box[kPassThreads + 64];
     __shared__ uint32_t s_nn[kPassThreads];
     __shared__ uint32_t s_w[kPassThreads / 64];
     __shared__ uint32_t s_hdr[5];  // tile, clusters, next merge id, list buffer, skip
-    __shared__ uint32_t s_excl[3]; // merges and stays before the tile, abort
+    __shared__ uint32_t s_excl[2]; // merges and stays before the tile
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = (int)a.radius;
     const uint32_t T = (uint32_t)(kPassThreads - 2 * r);
@@ -812,7 +829,6 @@ __global__ __launch_bounds__(kPassThreads) void k_ploc_pass(PlocPassArgs a) {
     if (wave == 0) {
         const uint32_t ax = total >> 16, ay = total & 0xFFFFu;
         uint32_t ex = 0, ey = 0;
-        bool failed = false;
         if (tile == 0) {
             if (lane == 0)
                 __hip_atomic_store(&a.tile_status[0], tile_word(kTilePre, ax, ay), __ATOMIC_RELAXED,
@@ -822,29 +838,27 @@ __global__ __launch_bounds__(kPassThreads) void k_ploc_pass(PlocPassArgs a) {
                 __hip_atomic_store(&a.tile_status[tile], tile_word(kTileAgg, ax, ay), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
             int64_t top = (int64_t)tile - 1;
-            uint32_t spins = 0;
+            uint32_t polls = 0;
             for (;;) {
                 const int64_t idx = top - lane;  // lane 0 = nearest tile
                 uint64_t w = kTilePre;           // before tile 0: an empty prefix
                 if (idx >= 0)
                     w = __hip_atomic_load(&a.tile_status[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                while (__ballot((w & kTileState) == 0) != 0) {
-                    if (++spins > kSpinLimit) {
-                        failed = true;
-                        break;
+                for (uint64_t missing; (missing = __ballot((w & kTileState) == 0)) != 0;) {
+                    if (++polls > kTilePatience) {
+                        const int m = __ffsll((long long)missing) - 1;
+                        const int first = (int)((top - m) * T);   // a whole tile: only the last may be short
+                        const uint2 c = ploc_tile_counts(b_in, first, first + (int)T, r, (int)iter);
+                        if (lane == m) w = publish_for(&a.tile_status[idx], tile_word(kTileAgg, c.x, c.y));
+                    } else {
+                        __builtin_amdgcn_s_sleep(1);
                     }
-                    __builtin_amdgcn_s_sleep(1);
                     if ((w & kTileState) == 0)
                         w = __hip_atomic_load(&a.tile_status[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
-                if (failed) break;
-                // nearest tile with counts through it (a prefix, or poison)
-                const unsigned long long pre = __ballot((w & kTileState) >= kTilePre);
+                // nearest tile with counts through it
+                const unsigned long long pre = __ballot((w & kTileState) == kTilePre);
                 const int stop = pre ? __ffsll((long long)pre) - 1 : 63;
-                if (pre && __shfl((uint32_t)(w >> 62), stop, 64) == 3u) {
-                    failed = true;
-                    break;
-                }
                 uint32_t cx = lane <= stop ? (uint32_t)(w >> 32) & 0x3FFFFFFFu : 0u;
                 uint32_t cy = lane <= stop ? (uint32_t)w : 0u;
 #pragma unroll
@@ -857,18 +871,14 @@ __global__ __launch_bounds__(kPassThreads) void k_ploc_pass(PlocPassArgs a) {
                 if (pre) break;
                 top -= 64;
             }
-            if (lane == 0) {
-                if (failed) atomicOr(a.err, kPlocErrSpin);
-                __hip_atomic_store(&a.tile_status[tile],
-                                   failed ? kTilePoison : tile_word(kTilePre, ex + ax, ey + ay), __ATOMIC_RELAXED,
+            if (lane == 0)
+                __hip_atomic_store(&a.tile_status[tile], tile_word(kTilePre, ex + ax, ey + ay), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
-            }
         }
         if (lane == 0) {
             s_excl[0] = ex;
             s_excl[1] = ey;
-            s_excl[2] = failed ? 1u : 0u;
-            if (!failed && tile == (iter - 1) / T) {  // the tile holding the last position ends the pass
+            if (tile == (iter - 1) / T) {  // the tile holding the last position ends the pass
                 a.st_out[0] = ey + ay;
                 a.st_out[1] = n_total + ex + ax;
                 a.st_out[2] = cur ^ 1u;
@@ -877,7 +887,7 @@ __global__ __launch_bounds__(kPassThreads) void k_ploc_pass(PlocPassArgs a) {
         }
     }
     __syncthreads();
-    if (s_excl[2] || !owned || !fy) return;
+    if (!owned || !fy) return;
 
     // merge and compaction (k_ploc_merge)
     const uint32_t ox = s_excl[0] + (local >> 16), oy = s_excl[1] + (local & 0xFFFFu);
@@ -1393,15 +1403,14 @@ __global__ __launch_bounds__(kThreads) void k_write_layout(
 inline uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + kThreads - 1) / kThreads); }
 
 // Shared front half of the build and of rtq_morton_codes: scene box + cube.
-// d_bounds holds 2 boxes, the words that a build reads back with them (8, the
-// first one zeroed here: the sort's errors), and 6 floats per
-// partial block (at most kBoundsPartials): kBoundsBoxes boxes of 32 B.
+// d_bounds holds 2 boxes followed by 6 floats per partial block (at most
+// kBoundsPartials): kBoundsBoxes boxes of 32 B.
 constexpr uint32_t kBoundsPartials = 1024;
-constexpr uint32_t kBoundsBoxes = 3 + (6 * kBoundsPartials + 7) / 8;
+constexpr uint32_t kBoundsBoxes = 2 + (6 * kBoundsPartials + 7) / 8;
 rtq_status compute_bounds(rtq_ctx* ctx, Scene* s, uint32_t pad_origin, rtq_aabb* d_bounds,
                           hipStream_t st) {
     const uint32_t nb = std::min<uint32_t>(blocks_for(s->n_tris), kBoundsPartials);
-    float* partial = reinterpret_cast<float*>(d_bounds + 3);
+    float* partial = reinterpret_cast<float*>(d_bounds + 2);
     hipLaunchKernelGGL(k_bounds_partial, dim3(nb), dim3(kThreads), 0, st, s->tris_ref, s->models,
                        s->n_tris, partial);
     RTQ_HIP(ctx, hipGetLastError());
@@ -1605,7 +1614,7 @@ private:
 
 // refit: the tree is the one the last build wrote the layouts for, with new
 // boxes: its placement is kept and the 8-wide nodes keep their children.
-// d_bounds: the scene's box, cube and words (compute_bounds), after a refit the
+// d_bounds: the scene's box and cube (compute_bounds), after a refit the
 // root cluster's box.
 rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipStream_t st, bool refit) {
     const uint32_t n = s->n_tris;
@@ -1684,7 +1693,6 @@ rtq_status write_layouts(rtq_ctx* ctx, Scene* s, const rtq_aabb* d_bounds, hipSt
     RTQ_HIP(ctx, hipStreamSynchronize(st));
     BuildReport h;
     std::memcpy(&h, report(ctx), sizeof h);
-    if (h.sort_err) return fail(ctx, RTQ_EINTERNAL, "build: a radix sort pass's look-back gave up");
     if (!refit) s->depth = h.depth;
     s->box_pad = box_pad_of(h.box);
     return RTQ_OK;
@@ -1769,8 +1777,7 @@ rtq_status build_scene(rtq_ctx* ctx, Scene* s, const rtq_build_params& prm) {
     hipLaunchKernelGGL(k_morton, dim3(blocks_for(n)), dim3(kThreads), 0, st, s->tris_ref, s->models, n,
                        d_bounds, s->sorted_codes, s->sorted_idx);
     RTQ_HIP(ctx, hipGetLastError());
-    rs = radix_sort_pairs(ctx, s->sorted_codes, s->sorted_idx, tk, tv, n, 30,
-                          reinterpret_cast<uint32_t*>(d_bounds + 2), st);
+    rs = radix_sort_pairs(ctx, s->sorted_codes, s->sorted_idx, tk, tv, n, 30, st);
     if (rs != RTQ_OK) return rs;
 
     // 2. PLOC

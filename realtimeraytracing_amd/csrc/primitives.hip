@@ -181,7 +181,6 @@ constexpr uint32_t kHistCopies = 8;
 constexpr uint32_t kDigitAgg = 1u << 30;
 constexpr uint32_t kDigitPre = 2u << 30;
 constexpr uint32_t kDigitFlags = 3u << 30;
-constexpr uint32_t kSortSpinLimit = 1u << 24;   // ~0.5 s of s_sleep(1) polls
 
 // Counts of every digit at every digit position in one read of the keys:
 // hist[p * 256 + d] = keys whose digit p (bits 8p .. 8p+7) is d, p < n_digits.
@@ -285,20 +284,21 @@ __device__ __forceinline__ uint32_t digit_totals(uint32_t (*counts)[256]) {
 
 // One digit pass in one launch (Adinets & Merrill, "Onesweep: A Faster Least
 // Significant Digit Radix Sort for GPUs", 2022): a workgroup takes the next
-// tile (take_tile, so every tile it waits on is already running), ranks its
+// tile (take_tile), ranks its
 // keys by digit, publishes its counts and sums those of the earlier tiles by
 // decoupled look-back per digit (Merrill & Garland 2016), 8 tiles at a time (a
 // tile waits for a chain of loads as long as the tiles that run beside it).  It
 // sorts its pairs in LDS, so that each digit's keys leave as one run: written
-// from where they were read they took a 64-B sector each.  A look-back that
-// waits longer than kSortSpinLimit polls sets *err and goes on.  5M pairs:
+// from where they were read they took a 64-B sector each.  A thread that has
+// waited for its digit's count of a tile for long (kTilePatience) counts that
+// tile's keys itself.  5M pairs:
 // 90.6 us a pass with 4,096-pair tiles written in place, 38.0 now (15 us of
 // memory traffic at the card's copy rate).
 template <int ITEMS>
 __global__ __launch_bounds__(kSortThreads) void k_onesweep(
     const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals, uint32_t n, uint32_t shift,
     const uint32_t* __restrict__ hist, uint32_t* __restrict__ tile_ctr, uint32_t* __restrict__ status,
-    uint32_t* __restrict__ err, uint32_t* __restrict__ out_k, uint32_t* __restrict__ out_v) {
+    uint32_t* __restrict__ out_k, uint32_t* __restrict__ out_v) {
     constexpr uint32_t kTile = kSortThreads * ITEMS;
     __shared__ uint2 s_kv[kTile];
     __shared__ uint32_t s_cnt[kSortWaves][256];
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(kSortThreads) void k_onesweep(
         uint32_t excl = 0;
         if (tile > 0) {
             constexpr uint32_t kAhead = 8;
-            uint32_t k = tile, spins = 0;   // tiles from k on are summed
+            uint32_t k = tile, polls = 0;   // tiles from k on are summed
             bool done = false;
             while (!done) {
                 uint32_t w[kAhead];
@@ -369,11 +369,15 @@ __global__ __launch_bounds__(kSortThreads) void k_onesweep(
                 }
                 k -= taken;
                 if (taken == 0) {
-                    if (++spins > kSortSpinLimit) {
-                        atomicOr(err, 1u);
-                        break;
+                    if (++polls > kTilePatience) {
+                        // tile k - 1, a whole one: only the last may be short
+                        const uint32_t* const missing = keys + (size_t)(k - 1) * kTile;
+                        uint32_t count = 0;
+                        for (uint32_t i = 0; i < kTile; ++i) count += ((missing[i] >> shift) & 0xFFu) == tid;
+                        publish_for(status + (size_t)(k - 1) * 256 + tid, kDigitAgg | count);
+                    } else {
+                        __builtin_amdgcn_s_sleep(1);
                     }
-                    __builtin_amdgcn_s_sleep(1);
                 }
             }
             __hip_atomic_store(mine, kDigitPre | (excl + c), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -468,7 +472,7 @@ rtq_status scan_u32x2_ws(rtq_ctx* ctx, const uint2* in, uint2* out, uint64_t n, 
 }
 
 rtq_status radix_sort_pairs(rtq_ctx* ctx, uint32_t* keys, uint32_t* vals, uint32_t* tmp_k,
-                            uint32_t* tmp_v, uint64_t n, uint32_t key_bits, uint32_t* err, hipStream_t st) {
+                            uint32_t* tmp_v, uint64_t n, uint32_t key_bits, hipStream_t st) {
     if (n == 0 || key_bits == 0) return RTQ_OK;
     if (n >= (1ull << 30)) return fail(ctx, RTQ_ECAPACITY, "sort: n must be < 2^30");
     const uint32_t nn = (uint32_t)n;
@@ -506,7 +510,7 @@ rtq_status radix_sort_pairs(rtq_ctx* ctx, uint32_t* keys, uint32_t* vals, uint32
         if (!one_clear) RTQ_HIP(ctx, hipMemsetAsync(status, 0, sizeof(uint32_t) * rows, st));
         const auto sweep = small_tiles ? &k_onesweep<4> : &k_onesweep<16>;
         hipLaunchKernelGGL(sweep, dim3(n_tiles), dim3(kSortThreads), 0, st, src_k, src_v, nn, 8 * p, hist + 256 * p,
-                           ctr + p * kTicketWords, status + (one_clear ? rows * p : 0), err, dst_k, dst_v);
+                           ctr + p * kTicketWords, status + (one_clear ? rows * p : 0), dst_k, dst_v);
         RTQ_HIP(ctx, hipGetLastError());
         std::swap(src_k, dst_k);
         std::swap(src_v, dst_v);

@@ -435,10 +435,9 @@ rtq_status write_top(rtq_ctx* ctx, Scene* s, const uint32_t* block_depth, uint32
 rtq_status ensure_ref_nodes(rtq_ctx* ctx, Scene* s, hipStream_t st);
 // Stable LSD radix sort of (key, value) pairs; `tmp_k`/`tmp_v` are n-entry buffers.
 // Queued on st and not waited for; digit counts and look-back words come from
-// the context's arena.  *err (device, zeroed by the caller) becomes non-zero
-// when a pass's look-back gave up: the order is then wrong and the caller fails.
+// the context's arena.
 rtq_status radix_sort_pairs(rtq_ctx* ctx, uint32_t* keys, uint32_t* vals, uint32_t* tmp_k,
-                            uint32_t* tmp_v, uint64_t n, uint32_t key_bits, uint32_t* err, hipStream_t st);
+                            uint32_t* tmp_v, uint64_t n, uint32_t key_bits, hipStream_t st);
 
 // ---- device helpers shared by the kernels
 
@@ -483,11 +482,32 @@ __device__ __forceinline__ void levels_up(const uint32_t* list, uint32_t count, 
 
 // Tile of this workgroup.  Workgroups are dispatched to the 8 XCDs in turn, and
 // the ones of each XCD number their tiles by a counter of their own: the k-th
-// one to start of those with blockIdx % 8 == x takes tile 8 k + x.  Every tile
-// before it is then taken by a workgroup that was dispatched before or with it
-// (or waits for a slot that only earlier tiles hold), so the look-back's waits
-// end; atomics on one word serialise (about 12 ns each, 50 us for the 4,361
-// tiles of a 2M-triangle terrain's first pass with one counter).
+// one to start of those with blockIdx % 8 == x takes tile 8 k + x.  Atomics on
+// one word serialise (about 12 ns each): with one counter a rebuild of 2,093,058
+// triangles takes 2,004 us instead of 1,917, a sort of 5M pairs 263 instead of
+// 234.
+// A tile may thus start before one that it takes counts from, which may even be
+// waiting for a slot that another program's waiting workgroups hold.  So no
+// look-back depends on another workgroup: once it has polled kTilePatience times
+// (about 1 ms) it counts a tile that has published nothing by itself, from the
+// pass's inputs, which no workgroup of the pass writes, and publishes the counts
+// in that tile's place.
+#ifndef RTQ_TILE_PATIENCE
+#define RTQ_TILE_PATIENCE 1024
+#endif
+constexpr uint32_t kTilePatience = RTQ_TILE_PATIENCE;
+
+// Publishes own counts w for a tile that may publish them itself at the same
+// time, or counts through it: whatever its word holds then.
+template <typename T>
+__device__ __forceinline__ T publish_for(T* word, T w) {
+    T seen = 0;
+    return __hip_atomic_compare_exchange_strong(word, &seen, w, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT)
+               ? w
+               : seen;
+}
+
 constexpr uint32_t kTicketStride = 32;             // words between the counters (128 B)
 constexpr uint32_t kTicketWords = 8 * kTicketStride;
 __device__ __forceinline__ uint32_t take_tile(uint32_t* ctr) {

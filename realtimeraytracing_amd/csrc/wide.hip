@@ -291,10 +291,7 @@ __device__ __forceinline__ float4 image_part(const uint32_t* img, uint32_t i) {
 // Tile status of the level scan: value in the low 32 bits, state on top.
 constexpr uint64_t kLvAgg = 1ull << 62;     // the tile's own count
 constexpr uint64_t kLvPre = 2ull << 62;     // the counts through the tile
-constexpr uint64_t kLvPoison = 3ull << 62;  // a wait at or before the tile gave up
 constexpr uint64_t kLvState = 3ull << 62;
-constexpr uint32_t kLvSpinLimit = 1u << 24;
-enum : uint32_t { kWideErrOverflow = 1, kWideErrScan = 2 };
 
 struct LevelArgs {
     uint32_t* lv;              // this level's words: count, first node, first status word, errors; then the next one's
@@ -319,11 +316,31 @@ struct LevelArgs {
     uint32_t* kids;            // 8 child clusters per node (kNone past the last)
 };
 
+// A child that becomes an 8-wide node of the next level: a merged cluster (ids
+// from nt on) of more than max_leaf triangles.
+__device__ __forceinline__ bool expandable(const LevelArgs& a, uint32_t c, uint32_t count) {
+    return c >= a.nt && count > a.max_leaf;
+}
+
+// Expandable children of a whole tile's nodes, by one wave: the count that the
+// tile publishes.
+__device__ uint32_t expandable_of_tile(const LevelArgs& a, uint32_t tile) {
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t total = 0;
+    for (uint32_t i = 0; i < kLevelNodes; i += 64 / kWidth) {
+        uint32_t c = 0;
+        const bool has = slot_child(a.items[tile * kLevelNodes + i + lane / kWidth], lane % kWidth, a.cleft, a.cright,
+                                    a.nt, a.choice, &c);
+        total += (uint32_t)__popcll(__ballot(has && expandable(a, c, a.ccount[c])));
+    }
+    return total;
+}
+
 // One level of the collapse in one launch, eight lanes per node of the level:
 // each lane finds its slot's child; the next level's nodes are numbered by an
 // exclusive scan of the nodes' expandable children in node order, across
-// workgroups by decoupled look-back (see take_tile; the wait is bounded and a
-// tile that gives up poisons its status and sets an error bit); then each lane
+// workgroups by decoupled look-back (a tile that has published nothing for long
+// is counted by the wave that waits for it, see take_tile); then each lane
 // quantises its child's box and the lanes of a node write its 128 B together.
 // The last tile writes the next level's words (lv[4..6]).  The grid covers an
 // upper bound of the level's count; workgroups past the count, and every
@@ -334,11 +351,15 @@ struct LevelArgs {
 // another), 171 us now; a level of a few nodes 20 us and 6 us.
 __global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
     constexpr uint32_t kWaves = kLevelThreads / 64;
-    __shared__ uint32_t s_tile, s_excl, s_bad, s_w[kWaves];
+    __shared__ uint32_t s_tile, s_excl, s_w[kWaves];
     __shared__ __align__(16) uint32_t s_img[kLevelNodes * kImageWords];
     const uint32_t count = a.lv[0];
     const uint32_t tiles = (count + kLevelNodes - 1) / kLevelNodes;
     if (blockIdx.x >= tiles) return;
+    if ((uint64_t)a.lv[2] + tiles > a.n_status) {   // more tiles than the levels can have: a broken invariant
+        if (threadIdx.x == 0) atomicOr(a.lv + 3, 1u);
+        return;
+    }
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     if (tid == 0) s_tile = take_tile(a.tickets);
     if (blockIdx.x == 0 && tid >= 64 && tid < 72) a.next_tickets[(tid - 64) * kTicketStride] = 0;
@@ -360,7 +381,7 @@ __global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
     const uint32_t cnt = has ? a.ccount[c] : 0u;
     const rtq_aabb box = a.cbox[c];
     const uint32_t first = has ? a.placed[c].y : 0u;
-    const bool expand = has && c >= a.nt && cnt > a.max_leaf;   // an 8-wide node of the next level
+    const bool expand = has && expandable(a, c, cnt);
     // exclusive sum of the expandable children over the workgroup
     const uint64_t em = __ballot(expand);
     const uint32_t in_wave = __builtin_amdgcn_mbcnt_hi((uint32_t)(em >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)em, 0u));
@@ -373,66 +394,58 @@ __global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
         total += s_w[w];
     }
 
+    uint64_t* const st = a.status + sbase;
+    if (tid == 0)
+        __hip_atomic_store(&st[tile], (tile == 0 ? kLvPre : kLvAgg) | total, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    // (before the look-back: a box in registers through it costs waves per SIMD)
+    uint32_t* const img = s_img + (tid / kWidth) * kImageWords;
+    wide_boxes(live, has, slot, n, box, box_pad_of(a.bounds[0]), img);
+
     // counts before this tile: decoupled look-back by wave 0
     if (wave == 0) {
-        bool failed = (uint64_t)sbase + tiles > a.n_status;
         uint32_t excl = 0;
-        if (!failed) {
-            uint64_t* const st = a.status + sbase;
-            if (tile == 0) {
-                if (lane == 0) __hip_atomic_store(&st[0], kLvPre | total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } else {
-                if (lane == 0)
-                    __hip_atomic_store(&st[tile], kLvAgg | total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                int64_t top = (int64_t)tile - 1;
-                uint32_t spins = 0;
-                for (;;) {
-                    const int64_t idx = top - (int64_t)lane;  // lane 0 = nearest tile
-                    uint64_t w = kLvPre;                       // before tile 0: an empty prefix
-                    if (idx >= 0) w = __hip_atomic_load(&st[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    while (__ballot((w & kLvState) == 0) != 0) {
-                        if (++spins > kLvSpinLimit) {
-                            failed = true;
-                            break;
-                        }
+        if (tile > 0) {
+            int64_t top = (int64_t)tile - 1;
+            uint32_t polls = 0;
+            for (;;) {
+                const int64_t idx = top - (int64_t)lane;  // lane 0 = nearest tile
+                uint64_t w = kLvPre;                       // before tile 0: an empty prefix
+                if (idx >= 0) w = __hip_atomic_load(&st[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (uint64_t missing; (missing = __ballot((w & kLvState) == 0)) != 0;) {
+                    if (++polls > kTilePatience) {
+                        const uint32_t m = (uint32_t)__builtin_ctzll(missing);
+                        const uint32_t c = expandable_of_tile(a, (uint32_t)top - m);
+                        if (lane == m) w = publish_for(&st[idx], kLvAgg | c);
+                    } else {
                         __builtin_amdgcn_s_sleep(1);
-                        if ((w & kLvState) == 0)
-                            w = __hip_atomic_load(&st[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     }
-                    if (failed) break;
-                    // nearest tile with counts through it (a prefix, or poison)
-                    const unsigned long long pre = __ballot((w & kLvState) >= kLvPre);
-                    const int stop = pre ? __ffsll((long long)pre) - 1 : 63;
-                    if (pre && __shfl((uint32_t)(w >> 62), stop, 64) == 3u) {
-                        failed = true;
-                        break;
-                    }
-                    uint32_t c = (int)lane <= stop ? (uint32_t)w : 0u;
-#pragma unroll
-                    for (int d = 32; d >= 1; d >>= 1) c += __shfl_xor(c, d, 64);
-                    excl += c;
-                    if (pre) break;
-                    top -= 64;
+                    if ((w & kLvState) == 0)
+                        w = __hip_atomic_load(&st[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
-                if (lane == 0)
-                    __hip_atomic_store(&st[tile], failed ? kLvPoison : (kLvPre | (uint64_t)(excl + total)),
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                // nearest tile with counts through it
+                const unsigned long long pre = __ballot((w & kLvState) == kLvPre);
+                const int stop = pre ? __ffsll((long long)pre) - 1 : 63;
+                uint32_t c = (int)lane <= stop ? (uint32_t)w : 0u;
+#pragma unroll
+                for (int d = 32; d >= 1; d >>= 1) c += __shfl_xor(c, d, 64);
+                excl += c;
+                if (pre) break;
+                top -= 64;
             }
+            if (lane == 0)
+                __hip_atomic_store(&st[tile], kLvPre | (uint64_t)(excl + total), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
         }
-        if (lane == 0) {
-            s_excl = excl;
-            s_bad = failed ? 1u : 0u;
-            if (failed) atomicOr(a.lv + 3, kWideErrScan);
-        }
+        if (lane == 0) s_excl = excl;
     }
     __syncthreads();
-    if (s_bad) return;
     const uint32_t excl = s_excl;
     const uint32_t next_base = level_base + count;
     if (tile == tiles - 1 && tid == 0) {
         uint32_t next_count = excl + total;
         if ((uint64_t)next_base + next_count > a.cap) {
-            atomicOr(a.lv + 3, kWideErrOverflow);   // more wide nodes than binary ones: a broken invariant
+            atomicOr(a.lv + 3, 1u);   // more wide nodes than binary ones: a broken invariant
             next_count = 0;
         }
         a.lv[4] = next_count;
@@ -440,8 +453,6 @@ __global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
         a.lv[6] = sbase + tiles;
     }
 
-    uint32_t* const img = s_img + (tid / kWidth) * kImageWords;
-    wide_boxes(live, has, slot, n, box, box_pad_of(a.bounds[0]), img);
     // an empty slot's box is inverted (wide_boxes); should a far ray still enter
     // it, its ref is the leaf of traversal triangle 0 alone: a real triangle, so
     // whatever that test reports is a genuine hit
@@ -452,7 +463,7 @@ __global__ __launch_bounds__(kLevelThreads) void k_wide_level(LevelArgs a) {
         if ((uint64_t)next_base + to < a.cap) {
             a.next_items[to] = c;
         } else {
-            atomicOr(a.lv + 3, kWideErrOverflow);
+            atomicOr(a.lv + 3, 1u);
         }
     } else if (has) {
         ref = leaf_ref(first, cnt);
@@ -618,7 +629,6 @@ rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const rtq_
             ++levels;
             n_wide = w[1] + w[0];
         }
-        if (err & kWideErrScan) return fail(ctx, RTQ_EINTERNAL, "wide collapse: a level scan gave up");
         if (err) return fail(ctx, RTQ_EINTERNAL, "wide collapse overflow");
         more = h_lv[kLvWords * (g1 - g0)] > 0;
         done = g1;
