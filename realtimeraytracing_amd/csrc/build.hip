@@ -454,7 +454,8 @@ __device__ __forceinline__ uint32_t nearest_in_window(const Box6* w, int i, int 
 // write everything of the others but the root's parent), the list they start as
 // and, unless null, the fused passes' state (kPlocHeadWords words).
 constexpr uint32_t kPlocBatch = 16;
-constexpr uint32_t kPlocHeadWords = 16 + 4 * kPlocBatch;   // state (8), errors and tail pass count (8), pass log
+constexpr uint32_t kPlocErrWord = 8, kTailCountWord = 9;   // errors and tail pass count, after the state
+constexpr uint32_t kPlocHeadWords = 16 + 4 * kPlocBatch;   // state (8), those two (8), pass log, then the tail's log
 constexpr uint32_t kTailPeek = 128;                        // tail log entries that reach the host with them
 constexpr uint32_t kPlocReportWords = kPlocHeadWords + 4 * kTailPeek;
 static_assert(kPlocReportWords <= kReportWords && kPlocReportWords <= 1024, "one word per thread of the tail");
@@ -1031,12 +1032,13 @@ __device__ __forceinline__ uint32_t tail_merge(TailLists& L, int tid, uint32_t m
 // and merges, so that a pass has two barriers.  960 clusters (19 passes): 112
 // us before these and the shorter search, 66 now; the last 33 passes of a
 // 2M-triangle terrain, whose first ones are long, 228 and 206.
-__global__ __launch_bounds__(kTailThreads) void k_ploc_tail(uint32_t* __restrict__ state, uint32_t radius,
-                                                            uint32_t* __restrict__ err, uint4* __restrict__ log,
-                                                            uint32_t* __restrict__ log_count, PlocLists lists,
-                                                            PlocClusters cl, uint32_t* __restrict__ host) {
+__global__ __launch_bounds__(kTailThreads) void k_ploc_tail(uint32_t* state, uint32_t radius, PlocLists lists,
+                                                            PlocClusters cl, uint32_t* host) {
     __shared__ TailLists L;
     __shared__ uint32_t s_hdr[4];
+    uint32_t* const err = state + kPlocErrWord;
+    uint32_t* const log_count = state + kTailCountWord;
+    uint4* const log = reinterpret_cast<uint4*>(state + kPlocHeadWords);
     Box6* const s_box = L.list + kRefRadius;
     const int tid = threadIdx.x;
     const int r = (int)radius;
@@ -1049,10 +1051,11 @@ __global__ __launch_bounds__(kTailThreads) void k_ploc_tail(uint32_t* __restrict
         if (s_hdr[3]) *log_count = 0;
     }
     __syncthreads();
-    // at the end, the head words and the log's first entries for the host: once
-    // every wave's own stores and atomics are done, read past the vector cache
+    // at the end, the head words and the log's first entries for the host: earlier
+    // launches and this workgroup wrote them, so the barrier orders the reads (a
+    // device-scope fence writes the L2 back: 4 us of a rebuild of 960 triangles);
+    // at device scope, where the error bits are set
     const auto tell = [&]() {
-        __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         if (tid < (int)kPlocReportWords)
             host[tid] = __hip_atomic_load(state + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1440,8 +1443,7 @@ rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
     const size_t ctl_words = kCtrWords + (size_t)kPlocBatch * max_tiles * 2;
     uint32_t* ctl = nullptr;
     if (n > kTailMax) RTQ_HIP(ctx, tmp.get(&ctl, ctl_words));
-    uint32_t* const err = state + 8;
-    uint32_t* const tail_count = err + 1;
+    uint32_t* const err = state + kPlocErrWord;
     uint4* const log = reinterpret_cast<uint4*>(state + 16);
     uint4* const tail_log = reinterpret_cast<uint4*>(state + kPlocHeadWords);
     PlocLists lists{{c0, c1}, {b0, b1}};
@@ -1463,8 +1465,7 @@ rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
             }
         }
         // the state of the batch's last pass is in slot 0 (kPlocBatch is even)
-        hipLaunchKernelGGL(k_ploc_tail, dim3(1), dim3(kTailThreads), 0, st, state, radius, err, tail_log, tail_count,
-                           lists, cl, report(ctx));
+        hipLaunchKernelGGL(k_ploc_tail, dim3(1), dim3(kTailThreads), 0, st, state, radius, lists, cl, report(ctx));
         RTQ_HIP(ctx, hipGetLastError());
         // the head block and the first tail log entries (those past the tail's
         // pass count are not used)
@@ -1472,7 +1473,7 @@ rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
         uint32_t h_head[kPlocReportWords];
         std::memcpy(h_head, report(ctx), sizeof h_head);
         const uint32_t* h_state = h_head;
-        const uint32_t* h_err = h_head + 8;
+        const uint32_t* h_err = h_head + kPlocErrWord;
         uint4 h_log[kPlocBatch];
         memcpy(h_log, h_head + 16, sizeof h_log);
         if (h_err[0] & kPlocErrNoMerge) return fail(ctx, RTQ_EINTERNAL, "PLOC pass made no merge");
@@ -1485,7 +1486,7 @@ rtq_status ploc_fused(rtq_ctx* ctx, Scene* s, uint32_t radius, Temps& tmp, uint3
                 if (e.y == 0) return fail(ctx, RTQ_EINTERNAL, "PLOC pass with %u clusters made no merge", e.z);
                 passes.emplace_back(e.x, e.y);
             }
-        const uint32_t nt = h_err[1];
+        const uint32_t nt = h_head[kTailCountWord];
         if (nt > kTailMax) return fail(ctx, RTQ_EINTERNAL, "PLOC tail ran %u passes", nt);
         if (nt) {
             h_tail.resize(nt);
