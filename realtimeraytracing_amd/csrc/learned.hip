@@ -124,6 +124,7 @@ __device__ __forceinline__ void child_hits(float4 n0, float4 n1, float4 n2, cons
 
 constexpr uint32_t kLogStack = 96;
 constexpr uint32_t kLogRecords = 32;       // samples of a ray kept until its wave ends
+constexpr uint64_t kLogLaunch = 1u << 24;  // logged rays per launch
 constexpr uint32_t kLogBudget = 1u << 14;  // node visits + triangle tests per sub-traversal
 // Lanes of a ray that prices 2 or 3 levels at a time: 2 + 4 or 2 + 4 + 8 of
 // them, rounded up to a power of two.
@@ -910,12 +911,16 @@ rtq_status rtq_order_log(rtq_ctx* ctx, uint32_t scene_id, const rtq_ray* rays_de
         const int ahead = threads <= 4 * 4 * 4 * (uint64_t)std::max(ctx->n_cu, 1) ? 3 : 2;
         const uint32_t per_wave = 64 / log_lanes(ahead);
         const uint32_t levels = std::min<uint32_t>(kLogStack, s->depth + 1);
-        hipLaunchKernelGGL(ahead == 3 ? &k_order_log<3> : &k_order_log<2>,
-                           dim3((uint32_t)((threads + per_wave - 1) / per_wave)), dim3(64),
-                           sizeof(uint32_t) * levels * 64, st, s->nodes, s->node_aux, s->tris, rays_dev,
-                           (uint32_t)n_rays, stride, (flags & RTQ_TRACE_ANY) ? 1u : 0u, samples_dev,
-                           (uint32_t)capacity, cnt);
-        e = hipGetLastError();
+        // (a launch has fewer than 2^32 threads, a ray 8 or 16 of them)
+        for (uint64_t first = 0; first < threads && e == hipSuccess; first += kLogLaunch) {
+            const uint64_t here = std::min<uint64_t>(threads - first, kLogLaunch), at = first * stride;
+            hipLaunchKernelGGL(ahead == 3 ? &k_order_log<3> : &k_order_log<2>,
+                               dim3((uint32_t)((here + per_wave - 1) / per_wave)), dim3(64),
+                               sizeof(uint32_t) * levels * 64, st, s->nodes, s->node_aux, s->tris, rays_dev + at,
+                               (uint32_t)std::min<uint64_t>(n_rays - at, here * stride), stride,
+                               (flags & RTQ_TRACE_ANY) ? 1u : 0u, samples_dev, (uint32_t)capacity, cnt);
+            e = hipGetLastError();
+        }
     }
     uint32_t h = 0;
     if (e == hipSuccess) e = hipMemcpyAsync(&h, cnt, sizeof h, hipMemcpyDeviceToHost, st);

@@ -70,3 +70,21 @@ def test_many_rays_give_the_samples_of_fewer(scene, torch_mod, any_hit):
     want = np.concatenate(parts)
     assert len(got) == len(want) < 24 * n
     assert np.array_equal(as_sorted(got).view(np.uint32), as_sorted(want).view(np.uint32))
+
+
+def test_more_rays_than_one_launch_has_lanes_for(scene, torch_mod):
+    """2^29 logged rays have 8 lanes each, more than a launch can start: the ones
+    that hit nothing (no direction) leave no samples, the others theirs."""
+    torch = torch_mod
+    n = 2 ** 29 + 5
+    if torch.cuda.mem_get_info()[0] < 2 * 32 * n:
+        pytest.skip("needs 34 GB of device memory")
+    rays = scenes.random_rays(3000, 15, (0, 0, 0), (1, 1, 1))
+    want = log(scene, torch, devmem.to_device(rays), len(rays), True, 1, 24 * len(rays))
+    words = torch.from_numpy(rays.view(np.float32).reshape(len(rays), 8))
+    every = torch.zeros((n, 8), dtype=torch.float32, device="cuda")
+    at = 2 ** 24 - 500          # across the first launch's end
+    every[:1000], every[at:at + 1000], every[n - 1000:] = (words[k:k + 1000].cuda() for k in (0, 1000, 2000))
+    got = log(scene, torch, every, n, True, 1, 24 * len(rays))
+    assert len(got) == len(want) > 100
+    assert np.array_equal(as_sorted(got).view(np.uint32), as_sorted(want).view(np.uint32))
