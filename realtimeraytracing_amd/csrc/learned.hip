@@ -374,6 +374,7 @@ __global__ __launch_bounds__(64) void k_order_log(const float4* __restrict__ nod
 
 constexpr int kTB = 64;  // samples per block
 constexpr int kGradThreads = 1024;
+constexpr uint32_t kGradLaunch = 1u << 16;   // blocks per launch
 // Row lengths of the LDS arrays: 20 or 44 mod 64 words, so that the matrix
 // operands read along a row (16 rows x 4 columns of a wave) lie in 64 distinct
 // banks and the ones read down a column (4 rows x 16 columns) in at most two
@@ -402,9 +403,10 @@ struct GradLds {
 };
 static_assert(sizeof(GradLds) <= 160 * 1024, "one workgroup per CU");
 
-// The order of an epoch: position i of a step holds sample (base + i * mul) % n,
-// base < n, mul < n < 2^31 and i < 2^16.  i * mul is exact in a double, its
-// quotient by n wrong by one at most (a 64-bit remainder is 1,000 cycles).
+// The order of an epoch: position i of a launch holds sample (base + i * mul) % n,
+// base < n, mul <= n, and i (under 64 kGradLaunch = 2^22) times mul under 2^53: it
+// is exact in a double, its quotient by n wrong by one at most (a 64-bit remainder
+// is 1,000 cycles).  Training has n < 2^31, a single gradient n < 2^32 and mul = 1.
 struct SampleOrder {
     uint32_t n, base, mul;
     double inv_n;
@@ -599,9 +601,17 @@ hipError_t queue_grad(const rtq_ctx* ctx, const float* params, const float* samp
                       uint32_t count, float* partial, float* loss_part, hipStream_t st) {
     const uint32_t blocks = (count + kTB - 1) / kTB;
     const int parts = grad_parts(ctx, blocks);
-    hipLaunchKernelGGL(parts == 4 ? &k_mlp_grad<4> : &k_mlp_grad<1>, dim3(blocks * parts), dim3(kGradThreads), 0, st,
-                       params, samples, order, count, partial, loss_part);
-    return hipGetLastError();
+    // (a launch has fewer than 2^32 threads, a sample 16 of them or more)
+    for (uint32_t b = 0; b < blocks; b += kGradLaunch) {
+        SampleOrder part = order;
+        part.base = (uint32_t)((order.base + (uint64_t)(kTB * b) * order.mul) % order.n);
+        hipLaunchKernelGGL(parts == 4 ? &k_mlp_grad<4> : &k_mlp_grad<1>, dim3(std::min(blocks - b, kGradLaunch) * parts),
+                           dim3(kGradThreads), 0, st, params, samples, part, count - kTB * b,
+                           partial + (size_t)b * kNP, loss_part + b);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 // The blocks' gradients of parameter j, summed in block order (deterministic)

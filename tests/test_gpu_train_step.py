@@ -66,3 +66,28 @@ def test_epoch_visits_every_sample_once(rtq_ctx, torch_mod, n, batch):
     rel = 2.0 ** -24 * (64 + n / 64) * 4
     assert losses[0] == pytest.approx(want, rel=rel)
     assert np.array_equal(dP.cpu().numpy(), P)
+
+
+def test_gradient_of_more_samples_than_one_launch_has_threads_for(rtq_ctx, torch_mod):
+    """2^28 samples have 16 threads each, more than a launch can start: the ones
+    without weight add nothing, the others what they give by themselves."""
+    torch = torch_mod
+    n, few = 2 ** 28 + 3, 900
+    if torch.cuda.mem_get_info()[0] < 180e9:   # the samples, and a row of sums per 64 of them
+        pytest.skip("needs 180 GB of device memory")
+    P, S = rand_params(4), rand_samples(few, 5)
+    every = torch.zeros((n, S.shape[1]), dtype=torch.float32, device="cuda")
+    rows = dev(S, torch)
+    at = 2 ** 22 - 150          # across the first launch's end
+    every[:300], every[at:at + 300], every[n - 300:] = rows[:300], rows[300:600], rows[600:]
+    g, dP = torch.zeros(ORDER_PARAMS, dtype=torch.float32, device="cuda"), dev(P, torch)
+    torch.cuda.synchronize()
+    loss = rtq_ctx.order_grad(dP.data_ptr(), every.data_ptr(), n, g.data_ptr())
+    want_loss, want = oracle.mlp_grad(P, S)
+    # the sums are those of the few samples (zeros add exactly), divided by n
+    want_loss, want = want_loss * few / n, want * few / n
+    rel = 2.0 ** -24 * (64 + few / 64) * 4
+    assert loss == pytest.approx(want_loss, rel=rel)
+    assert np.abs(g.cpu().numpy() - want).max() <= max(1e-5, rel) * np.abs(want).max()
+    del every
+    torch.cuda.empty_cache()
