@@ -223,13 +223,24 @@ rtq_status rtq_autotune(rtq_ctx* ctx, const rtq_batch_item* items, uint32_t n_it
         return RTQ_OK;
     };
     const uint32_t refills[] = {4, 8, 16, 32};
-    const uint32_t chunks[] = {128, 256, 512};
+    // chunk is the most rays that a wave takes at a time: settings that give
+    // these items the same chunks are one setting, timed as the one in force
+    // (launches of fewer than about 1,000 rays per wave take 64 under all of them)
+    const uint32_t chunks[] = {before.chunk, 128, 256, 512};
     for (uint32_t wide = 0; wide <= (any_wide ? 1u : 0u) && status == RTQ_OK; ++wide)
-        for (uint32_t rf : refills)
-            for (uint32_t ch : chunks)
-                if (status == RTQ_OK)
-                    status = consider(rtq_launch_params{rf, ch, wide, before.spec_slack, before.leaf_slack,
-                                                        before.stack_lds});
+        for (uint32_t rf : refills) {
+            std::vector<uint32_t> taken;
+            for (uint32_t ch : chunks) {
+                if (status != RTQ_OK) break;
+                const rtq_launch_params p{rf, ch, wide, before.spec_slack, before.leaf_slack, before.stack_lds};
+                apply(ctx, p);
+                status = trace_batch(ctx, items, n_items, nullptr, true, st);
+                const uint32_t rays = ctx->scratch.chunk;
+                if (status != RTQ_OK || std::find(taken.begin(), taken.end(), rays) != taken.end()) continue;
+                taken.push_back(rays);
+                status = consider(p);
+            }
+        }
     const rtq_launch_params stage1 = best;
     const uint32_t spec[] = {0, 4, 8, 16, 24, 32};
     const uint32_t leaf[] = {0, 8, 16, 24};

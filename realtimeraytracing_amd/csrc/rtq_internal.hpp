@@ -115,6 +115,7 @@ struct TraceScratch {
     // fixed: the spill buffer cannot grow (rtq_trace_noalloc); a launch takes
     // fewer workgroups instead, so every spill column fits in spill_words
     bool fixed = false;
+    uint32_t chunk = 0;   // rays of a chunk of the last launch queued or sized with it
 };
 }  // namespace rtq
 

@@ -920,6 +920,7 @@ rtq_status launch(rtq_ctx* ctx, TraceScratch& sc, uint64_t depth_entries, const 
     const uint64_t resident = (uint64_t)per_cu * (uint64_t)std::max(ctx->n_cu, 1);
     const WaveSplit split =
         split_rays(n, (uint64_t)kSimdsPerCu * std::max(ctx->n_cu, 1), resident * kWavesPerBlock, ctx->chunk);
+    sc.chunk = split.chunk;
     const uint32_t queue = queue_chunks(table, base.n_items, n, split.chunk);
     // whole rounds of the XCDs: every XCD's queue has the same chunks
     auto rounds = [](uint64_t waves) { return (waves + kXcds * kWavesPerBlock - 1) / (kXcds * kWavesPerBlock); };
