@@ -924,7 +924,8 @@ rtq_status launch(rtq_ctx* ctx, TraceScratch& sc, uint64_t depth_entries, const 
     const uint32_t queue = queue_chunks(table, base.n_items, n, split.chunk);
     // whole rounds of the XCDs: every XCD's queue has the same chunks
     auto rounds = [](uint64_t waves) { return (waves + kXcds * kWavesPerBlock - 1) / (kXcds * kWavesPerBlock); };
-    uint64_t blocks = std::min<uint64_t>(kXcds * std::min(rounds(split.waves), rounds((uint64_t)kXcds * queue)), resident);
+    const uint64_t most = std::min<uint64_t>(kXcds * rounds(split.waves), resident);
+    uint64_t blocks = std::min<uint64_t>(kXcds * rounds((uint64_t)kXcds * queue), most);   // few chunks: fewer
     if (blocks == 0) blocks = 1;
     constexpr uint32_t kStackLds = STACK;
     const uint64_t column = depth_entries > kStackLds ? depth_entries - kStackLds : 0;  // spill words per thread
@@ -939,10 +940,12 @@ rtq_status launch(rtq_ctx* ctx, TraceScratch& sc, uint64_t depth_entries, const 
         blocks = std::min(blocks, fit);
     }
     const uint64_t threads = blocks * kTraceThreads;
-    // sized for one wave per SIMD at least: a launch of fewer rays may take
-    // more workgroups than one of more rays does (split_rays), up to that many
+    // sized so that no launch of fewer rays needs more (it may be on a capturing
+    // stream): for every wave that the rays may have (a setting of long chunks
+    // takes fewer of them), and one per SIMD at least, since few rays may take
+    // more workgroups than some more rays do (split_rays), up to that many
     const uint64_t least = std::min<uint64_t>((uint64_t)std::max(ctx->n_cu, 1) * kSimdsPerCu / kWavesPerBlock, resident);
-    const uint64_t spill_words = column ? column * (sc.fixed ? threads : std::max(threads, least * kTraceThreads)) : 1;
+    const uint64_t spill_words = column ? column * (sc.fixed ? threads : std::max(most, least) * kTraceThreads) : 1;
     if (spill_words > sc.spill_words) {
         if (sc.fixed) return fail(ctx, RTQ_EINTERNAL, "trace: fixed scratch sizing");
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
