@@ -937,22 +937,27 @@ struct TailLists {
     uint32_t c[kTailMax];
     uint2 n[kTailMax];
     uint16_t nn[kTailMax];
-    uint32_t w[kTailThreads / 64];
+    uint32_t w[64];
 };
 
 // Flags, scan, merge and compaction of a list of m clusters whose neighbours
-// are found: thread t owns positions K t .. K t + K - 1.  Returns merges << 16 |
+// are found: thread t owns positions t, t + W, .., of W threads, so that
+// neighbouring lanes read and write neighbouring entries (four positions in a row
+// per thread lie 96 B apart: 4,095 passes of a list that loses one cluster each
+// 58.7 ms, 54.8 so).  Returns merges << 16 |
 // clusters left.  ONE_WAVE: the first wave alone (m <= 64 K), else every thread
-// (two barriers).  Both partners' state is read before anything depends on
-// it, so that a pass waits for LDS three times, not once per position and step.
+// (two barriers).  A position's own state is read before anything depends on
+// it, and by one wave its partner's too, so that a pass waits for LDS three
+// times, not once per position and step.
 template <int K, bool ONE_WAVE>
 __device__ __forceinline__ uint32_t tail_merge(TailLists& L, int tid, uint32_t m, uint32_t n_total,
                                                const PlocClusters& cl) {
+    constexpr int W = ONE_WAVE ? 64 : kTailThreads;
     Box6* const s_box = L.list + kRefRadius;
-    uint32_t j[K], back[K], f[K], sum = 0;
+    uint32_t j[K], back[K], f[K], run[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        const uint32_t i = (uint32_t)(K * tid + k);
+        const uint32_t i = (uint32_t)(tid + W * k);
         j[k] = L.nn[min(i, m - 1)];
     }
 #pragma unroll
@@ -965,46 +970,59 @@ __device__ __forceinline__ uint32_t tail_merge(TailLists& L, int tid, uint32_t m
     uint2 on[K], pn[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        const uint32_t i = min((uint32_t)(K * tid + k), m - 1);
+        const uint32_t i = min((uint32_t)(tid + W * k), m - 1);
         ob[k] = s_box[i];
         oc[k] = L.c[i];
         on[k] = L.n[i];
-        pb[k] = s_box[j[k]];
-        pc[k] = L.c[j[k]];
-        pn[k] = L.n[j[k]];
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        const uint32_t i = (uint32_t)(K * tid + k);
+        const uint32_t i = (uint32_t)(tid + W * k);
         const bool mutual = back[k] == i && j[k] != i;
         f[k] = i < m ? ((mutual && i < j[k]) ? 1u << 16 : 0u) | ((mutual && j[k] < i) ? 0u : 1u) : 0u;
-        sum += f[k];
     }
-    uint32_t run = wave_inclusive_sum(sum), total = 0;
-    if constexpr (ONE_WAVE) {
-        total = (uint32_t)__builtin_amdgcn_readlane((int)run, 63);
-        run -= sum;
-    } else {
-        if ((tid & 63) == 63) L.w[tid >> 6] = run;
-        __syncthreads();
-        run -= sum;
 #pragma unroll
-        for (int w = 0; w < kTailThreads / 64; ++w) {
-            const uint32_t x = L.w[w];
-            run += w < (tid >> 6) ? x : 0u;
-            total += x;
+    for (int k = 0; k < K; ++k)
+        if (ONE_WAVE || f[k] >> 16) {
+            pb[k] = s_box[j[k]];
+            pc[k] = L.c[j[k]];
+            pn[k] = L.n[j[k]];
         }
+    // flags before each position, and of all
+    uint32_t total = 0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) run[k] = wave_inclusive_sum(f[k]);
+    if constexpr (ONE_WAVE) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const uint32_t here = (uint32_t)__builtin_amdgcn_readlane((int)run[k], 63);
+            run[k] += total - f[k];
+            total += here;
+        }
+    } else {
+        // the sums of the waves, a lane for each wave's of each k
+        constexpr int kWaves = kTailThreads / 64;
+        static_assert(K * kWaves == 64, "one lane per sum");
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        if ((tid & 63) == 63)
+#pragma unroll
+            for (int k = 0; k < K; ++k) L.w[kWaves * k + wave] = run[k];
+        __syncthreads();
+        const uint32_t w = L.w[tid & 63], through = wave_inclusive_sum(w);
+        total = (uint32_t)__builtin_amdgcn_readlane((int)through, 63);
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            run[k] += (uint32_t)__builtin_amdgcn_readlane((int)(through - w), kWaves * k + wave) - f[k];
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        opos[k] = (f[k] & 0xFFFFu) ? run & 0xFFFFu : kNone;
+        opos[k] = (f[k] & 0xFFFFu) ? run[k] & 0xFFFFu : kNone;
         if (f[k] >> 16) {
-            const uint32_t id = n_total + (run >> 16);
+            const uint32_t id = n_total + (run[k] >> 16);
             on[k] = ploc_below_merged(cl, on[k], pn[k]);
             ploc_merge_store(cl, id, oc[k], pc[k], on[k], ob[k], pb[k]);
             oc[k] = id;
         }
-        run += f[k];
     }
     // every read of this pass's list is done: by the barrier above, or because
     // one wave's instructions keep their order
@@ -1022,16 +1040,15 @@ __device__ __forceinline__ uint32_t tail_merge(TailLists& L, int tid, uint32_t m
 }
 
 // All remaining passes once at most kTailMax clusters are left, in one
-// workgroup with the list in LDS (same arithmetic as k_ploc_pass).  Thread t
-// owns positions 4t .. 4t+3 for flags, scan and merge.  Does nothing unless
-// 1 < clusters <= kTailMax.
+// workgroup with the list in LDS (same arithmetic as k_ploc_pass).  Does nothing
+// unless 1 < clusters <= kTailMax.
 // One CU runs it, so its long passes are bound by the search's instructions
 // (merge_cost), its short ones (half of them have under 130 clusters) by a
 // pass's chain of dependent steps: up to 512 or 256 clusters a position's window
 // is shared by 2 or 4 lanes, and up to 256 the first wave alone flags, scans
 // and merges, so that a pass has two barriers.  960 clusters (19 passes): 112
-// us before these and the shorter search, 66 now; the last 33 passes of a
-// 2M-triangle terrain, whose first ones are long, 228 and 206.
+// us before these and the shorter search, 60 now; the last 33 passes of a
+// 2M-triangle terrain, whose first ones are long, 228 and 182.
 __global__ __launch_bounds__(kTailThreads) void k_ploc_tail(uint32_t* state, uint32_t radius, PlocLists lists,
                                                             PlocClusters cl, uint32_t* host) {
     __shared__ TailLists L;
