@@ -382,7 +382,7 @@ __host__ __device__ __forceinline__ float box_pad_of(const rtq_aabb& b) {
 // one-triangle scene.
 rtq_status build_wide(rtq_ctx* ctx, Scene* s, const uint32_t* choice, const rtq_aabb* bounds, hipStream_t st);
 // Clusters created by the passes from Scene::lds_from on: at most this many
-// (their placement state, 12 B each, and cost rows, 32 B each, in LDS).
+// (their places, 16 B each, and cost rows, 32 B each, in LDS).
 constexpr uint32_t kLdsClusters = 4096;
 constexpr int kLdsThreads = 1024;   // 4 clusters per thread
 // Those passes, (first cluster, merges) in build order, as a kernel argument:
@@ -394,7 +394,12 @@ struct TopPasses {
     uint2 inline_passes[kInlinePasses];
     const uint2* rest;
     __device__ __forceinline__ uint2 operator[](uint32_t k) const {
-        return k < kInlinePasses ? inline_passes[k] : rest[k - kInlinePasses];
+        if (k < kInlinePasses) return inline_passes[k];
+        // (constant memory: the kernels store to memory that it might be part of
+        // as far as the compiler knows, and each load would then be waited for)
+        using Words = const __attribute__((address_space(4))) uint32_t*;
+        const Words w = reinterpret_cast<Words>(reinterpret_cast<uintptr_t>(rest + (k - kInlinePasses)));
+        return make_uint2(w[0], w[1]);
     }
 };
 TopPasses top_passes(const Scene* s);
