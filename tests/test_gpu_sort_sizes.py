@@ -33,3 +33,10 @@ def test_sort_sizes(rtq_ctx, torch_mod, n, bits, kind):
     order = np.argsort(keys, kind="stable")
     assert np.array_equal(dk.cpu().numpy().view(np.uint32), keys[order])
     assert np.array_equal(dv.cpu().numpy().view(np.uint32), vals[order])
+
+
+@pytest.mark.parametrize("kind", ["random", "few"])
+def test_sort_with_one_set_of_status_words(rtq_ctx, torch_mod, kind):
+    """Past 2,048 tiles the passes share one set of look-back words, cleared before
+    each."""
+    test_sort_sizes(rtq_ctx, torch_mod, 2049 * 8192 - 5, 32, kind)
