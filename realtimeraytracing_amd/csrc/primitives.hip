@@ -485,8 +485,8 @@ rtq_status radix_sort_pairs(rtq_ctx* ctx, uint32_t* keys, uint32_t* vals, uint32
         RTQ_HIP(ctx, hipGetLastError());
         return RTQ_OK;
     }
-    // tiles of 8,192 pairs, or of 2,048 while those leave CUs idle
-    const bool small_tiles = nn <= 256u * 2048u;
+    // tiles of 8,192 pairs, or of 2,048 while one for each CU takes them all
+    const bool small_tiles = nn <= (uint32_t)std::max(ctx->n_cu, 1) * 2048u;
     const uint32_t tile = kSortThreads * (small_tiles ? 4 : 16);
     const uint32_t n_tiles = (nn + tile - 1) / tile;
     // digit counts and tile counters of every pass, then the passes' look-back
