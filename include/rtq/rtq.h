@@ -277,7 +277,8 @@ rtq_status rtq_trace_stats(rtq_ctx* ctx, uint32_t scene_id, const rtq_ray* rays_
  * persistent grid takes as many workgroups as that array holds stacks for, so
  * very deep trees trace with fewer workgroups; RTQ_ECAPACITY when not even one
  * workgroup's stacks fit.  A call that uses the counters clears them first
- * (one more small launch; a few hundred thousand rays need none).  All calls on
+ * (one more small launch): those with more 64-ray chunks than waves, from
+ * about 262,144 rays on (256 CUs), from fewer on very deep trees.  All calls on
  * one GPU share the array: calls that overlap on one GPU (any context, any
  * stream) race, and the caller must serialise them.  Asynchronous on `stream`;
  * device buffers. */

@@ -1116,7 +1116,7 @@ rtq_status trace_noalloc(rtq_ctx* ctx, const Scene* s, const rtq_ray* rays, uint
 rtq_status trace(rtq_ctx* ctx, const Scene* s, const rtq_ray* rays, uint64_t n, uint32_t flags, rtq_hit* hits,
                  uint32_t* stat_nodes, uint32_t* stat_tris, bool stats, hipStream_t st) {
     if (n == 0) return RTQ_OK;
-    // the counter runs past n by at most one chunk per wave: n <= 2^31 keeps it in range
+    // a lane holds its ray's number as an int, -1 for none: at most 2^31 of them
     if (n > 0x80000000ull) return fail(ctx, RTQ_ECAPACITY, "trace: n_rays must be <= 2^31");
     TraceArgs args{};
     args.tris = s->tris;
