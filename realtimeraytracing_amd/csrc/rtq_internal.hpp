@@ -495,7 +495,7 @@ __device__ __forceinline__ void levels_up(const uint32_t* list, uint32_t count, 
 // A tile may thus start before one that it takes counts from, which may even be
 // waiting for a slot that another program's waiting workgroups hold.  So no
 // look-back depends on another workgroup: once it has polled kTilePatience times
-// (about 1 ms) it counts a tile that has published nothing by itself, from the
+// (a load and a sleep each, 0.5 to 1 ms in all) it counts a tile that has published nothing by itself, from the
 // pass's inputs, which no workgroup of the pass writes, and publishes the counts
 // in that tile's place.
 #ifndef RTQ_TILE_PATIENCE
